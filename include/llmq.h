@@ -6,11 +6,7 @@
  *  - The caller owns every buffer (inputs, outputs, workspaces); the library allocates
  *    nothing, never synchronises with the host and launches on the stream it is given
  *    (0 = the null stream).  Calls are asynchronous.  State kept between calls: the
- *    *_force_plan tuning hooks, and a 1 MiB ring of arrival counters per GPU (a static device
- *    array) for the K split of the few-token AWQ kernel, which ends inside one launch.  The
- *    counters are zero between calls and every call takes fresh slots, so calls on different
- *    streams do not share any; a captured call replays on the slots it was captured with, so
- *    two replays of one graph must not run concurrently.
+ *    *_force_plan tuning hooks (per host thread) only.
  *  - Matrices are row-major; `ld*` is the row stride in ELEMENTS.
  *  - Return value: LLMQ_OK (0) or a negative llmq_status; llmq_status_string() names it.
  *  - Paths below are relative to the reference's runtime/ directory.
@@ -91,6 +87,17 @@ int llmq_quant_fp8_per_tensor(const void* x, int x_dtype, int64_t M, int64_t K, 
 int llmq_quant_fp8_static(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
                           uint8_t* q, const float* scale, int scale_is_f32_tensor,
                           llmq_stream_t stream);
+
+/* Per-tensor quantizers that also form the factor of the GEMM behind them, alpha = scale * w_scale (both fp32 device
+ * scalars), so that no elementwise launch sits between the two: fp8 == 0 is llmq_quant_i8_per_tensor with the product
+ * rounded to x_dtype (linear_sq.py:127), fp8 != 0 llmq_quant_fp8_per_tensor (linear_fp8.py:199-221), the static form
+ * llmq_quant_fp8_static (linear_fp8.py:296-308), both with the product in fp32.  scale: fp32, one element. */
+int llmq_quant_per_tensor_alpha(int fp8, const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
+                                void* q, float* scale, const float* w_scale, float* alpha,
+                                void* workspace, size_t workspace_bytes, llmq_stream_t stream);
+int llmq_quant_fp8_static_alpha(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
+                                uint8_t* q, const float* scale, int scale_is_f32_tensor,
+                                const float* w_scale, float* alpha, llmq_stream_t stream);
 
 /* Replaces quantize_weight_per_channel_absmax, utils/quantization_utils.py:27-38 (the offline weight
  * quantizer behind SqW8A8BBF16OBF16PerChannel.from_float).  w: [N, K] bf16 / f16 / f32, row stride ldw, any K;

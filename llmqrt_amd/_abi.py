@@ -32,6 +32,8 @@ SIGNATURES = {
     "llmq_quant_fp8_per_token": (_int, [_vp, _int, _i64, _i64, _i64, _vp, _vp, _vp]),
     "llmq_quant_fp8_per_tensor": (_int, [_vp, _int, _i64, _i64, _i64, _vp, _vp, _vp, _sz, _vp]),
     "llmq_quant_fp8_static": (_int, [_vp, _int, _i64, _i64, _i64, _vp, _vp, _int, _vp]),
+    "llmq_quant_per_tensor_alpha": (_int, [_int, _vp, _int, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "llmq_quant_fp8_static_alpha": (_int, [_vp, _int, _i64, _i64, _i64, _vp, _vp, _int, _vp, _vp, _vp]),
     "llmq_rmsnorm": (_int, [_vp, _int, _i64, _i64, _i64, _vp, _f32, _vp, _vp, _vp]),
     "llmq_rmsnorm_quant_i8_per_token": (_int, [_vp, _int, _i64, _i64, _i64, _vp, _f32, _vp, _vp, _vp, _int, _vp, _vp]),
     "llmq_rmsnorm_quant_fp8_per_token": (_int, [_vp, _int, _i64, _i64, _i64, _vp, _f32, _vp, _vp, _vp, _vp, _vp]),

@@ -7,6 +7,8 @@
 // The kernels reproduce exactly that sequence of roundings.  They are HBM-bound:
 // 2 bytes read + 1 byte written per element, one row per 256-thread block, the row held in
 // registers between the absmax pass and the quantize pass so x is read from HBM once.
+#include <type_traits>
+
 #include "llmq_common.h"
 #include "quant_math.h"
 
@@ -19,14 +21,30 @@ constexpr int kMaxPartials = 1024;  // per-tensor absmax partials (one per stage
 
 enum { SCALE_ROW = 0, SCALE_TENSOR = 1, SCALE_STATIC = 2 };
 
+// The factor the GEMM behind a per-tensor quantizer applies: activation scale x weight scale, formed by the quantizer
+// (one thread) instead of by separate elementwise launches.  round_dt: the product is rounded to the activation dtype
+// (SmoothQuant, linear_sq.py:127); otherwise it stays fp32 (linear_fp8.py:199-221, 296-308).  out may be null.
+struct TensorAlpha {
+    const float* w_scale;
+    float* out;
+    int round_dt;
+};
+template <int DT>
+__device__ __forceinline__ void store_alpha(const TensorAlpha& ta, float s) {
+    if (!ta.out) return;
+    const float a = s * ta.w_scale[0];
+    ta.out[0] = ta.round_dt ? Lo<DT>::round(a) : a;
+}
+
 // One block of NT threads per row.  NC > 0: the row's 16-byte chunks (8 elements) are kept in NC
 // registers per thread between the two passes; NC == 0: rows of any length, second pass
-// re-reads x (served by L2).
+// re-reads x (served by L2).  A tensor-wide or static scale needs no second look at the row and runs with NC == 0: fewer
+// registers and more rows in flight beat requesting the row ahead of the scale (static, 8192 x 3584: 18.0 against 21.9 us).
 template <int DT, int MODE, int SCALE, int NC, int NT = kThreads>
 __global__ __launch_bounds__(NT) void quant_rows_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, int64_t K, uint8_t* __restrict__ q,
     void* __restrict__ scale_out, int scale_dtype, const float* __restrict__ aux, int n_aux,
-    int static_f32, float floor) {
+    int static_f32, float floor, TensorAlpha ta) {
     __shared__ float smem[NT / kWave];
     const int64_t row = blockIdx.x;
     const int tid = threadIdx.x;
@@ -67,32 +85,28 @@ __global__ __launch_bounds__(NT) void quant_rows_kernel(
         if (scale_dtype == LLMQ_F32) ((float*)scale_out)[o] = s;
         else ((uint16_t*)scale_out)[o] = Lo<DT>::from_f32(s);
     }
+    if (SCALE != SCALE_ROW && row == 0 && tid == 0) store_alpha<DT>(ta, s);
     const float inv_s = 1.0f / s;
-    constexpr bool F32Q = (SCALE == SCALE_STATIC);
-    if (SCALE == SCALE_ROW && NC > 0) {
-        if (fin) {
+    auto store_row = [&](auto quot_c, auto fin_c) __attribute__((always_inline)) {
+        constexpr int QUOT = decltype(quot_c)::value;
+        constexpr bool FIN = decltype(fin_c)::value;
+        if (NC > 0) {
 #pragma unroll
             for (int c = 0; c < NC; c++) {
                 const int i = tid + c * NT;
-                if (i < nchunk) qr[i] = quant8<DT, MODE, Q_DT, true>(cache[c], s, inv_s);
+                if (i < nchunk) qr[i] = quant8<DT, MODE, QUOT, FIN>(cache[c], s, inv_s);
             }
         } else {
-#pragma unroll
-            for (int c = 0; c < NC; c++) {
-                const int i = tid + c * NT;
-                if (i < nchunk) qr[i] = quant8<DT, MODE, Q_DT>(cache[c], s, inv_s);
-            }
+            for (int i = tid; i < nchunk; i += NT) qr[i] = quant8<DT, MODE, QUOT, FIN>(xr[i], s, inv_s);
         }
-    } else if (F32Q) {
-        if (static_f32) {
-            for (int i = tid; i < nchunk; i += NT) qr[i] = quant8<DT, MODE, Q_DIV_F32>(xr[i], s, inv_s);
-        } else {
-            for (int i = tid; i < nchunk; i += NT) qr[i] = quant8<DT, MODE, Q_DIV_DT>(xr[i], s, inv_s);
-        }
+    };
+    if (SCALE == SCALE_STATIC) {
+        if (static_f32) store_row(std::integral_constant<int, Q_DIV_F32>{}, std::false_type{});
+        else store_row(std::integral_constant<int, Q_DIV_DT>{}, std::false_type{});
     } else if (fin) {
-        for (int i = tid; i < nchunk; i += NT) qr[i] = quant8<DT, MODE, Q_DT, true>(xr[i], s, inv_s);
+        store_row(std::integral_constant<int, Q_DT>{}, std::true_type{});
     } else {
-        for (int i = tid; i < nchunk; i += NT) qr[i] = quant8<DT, MODE, Q_DT>(xr[i], s, inv_s);
+        store_row(std::integral_constant<int, Q_DT>{}, std::false_type{});
     }
 }
 
@@ -139,19 +153,64 @@ __global__ __launch_bounds__(kThreads) void quant_rows_wave_kernel(
     }
 }
 
-// Stage 1 of the per-tensor quantizers: grid-stride absmax, one partial per block.
-template <int DT>
+// Stage 1 of the per-tensor quantizers: absmax partials, one per block.  A unit is kUnit consecutive chunks of a row
+// (a contiguous tensor is one long row), NL independent 16-byte loads per thread: 8, or 2 for strided rows shorter than
+// a unit of 8.  HBM-bound: 8192 x 3584 12.9 us (4.6 TB/s; one load at a time with a division per chunk 14.2), 4096 x 18944
+// 34.1 us (36.4).
+constexpr int kUnitLoads = 8;
+template <int DT, int NL>
 __global__ __launch_bounds__(kThreads) void absmax_partials_kernel(
-    const uint16_t* __restrict__ x, int64_t ldx, int64_t M, int64_t K, float* __restrict__ partials) {
+    const uint16_t* __restrict__ x, int64_t ldx, int64_t rows, int64_t cpr, float* __restrict__ partials) {
     __shared__ float smem[kNW];
-    const int64_t cpr = K >> 3, total = M * cpr;
+    constexpr int kUnit = NL * kThreads;
+    const int64_t upr = (cpr + kUnit - 1) / kUnit, units = rows * upr;
     float amax = 0.f;
-    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < total; i += (int64_t)gridDim.x * kThreads) {
-        const int64_t r = i / cpr, c = i - r * cpr;
-        amax = max_nonneg(amax, absmax8(reinterpret_cast<const uint4*>(x + r * ldx)[c], DT == LLMQ_BF16));
+    for (int64_t u = blockIdx.x; u < units; u += gridDim.x) {
+        const int64_t r = u / upr, c0 = (u - r * upr) * kUnit + threadIdx.x;
+        const uint4* xr = reinterpret_cast<const uint4*>(x + r * ldx);
+        uint4 v[NL];
+#pragma unroll
+        for (int i = 0; i < NL; i++) {
+            const int64_t c = c0 + i * kThreads;
+            v[i] = xr[c < cpr ? c : cpr - 1];  // past the end: the last chunk again, which changes no maximum
+        }
+#pragma unroll
+        for (int i = 0; i < NL; i++) amax = max_nonneg(amax, absmax8(v[i], DT == LLMQ_BF16));
     }
     amax = block_max<kNW>(amax, smem);
     if (threadIdx.x == 0) partials[blockIdx.x] = amax;
+}
+
+// Per-tensor quantizer of a small contiguous tensor in one launch: every block reduces the whole tensor by itself (it
+// sits in L2; what is saved is a launch and the gap in front of it), then quantizes its own 1024 chunks.  Bound by the
+// latency of launch, loads and reduction.
+constexpr int kSmallThreads = 1024;
+template <int DT, int MODE>
+__global__ __launch_bounds__(kSmallThreads) void quant_tensor_small_kernel(
+    const uint4* __restrict__ x, int total, uint2* __restrict__ q, void* __restrict__ scale_out, int scale_dtype,
+    float floor, TensorAlpha ta) {
+    __shared__ float smem[kSmallThreads / kWave];
+    const int tid = threadIdx.x, mine = blockIdx.x * kSmallThreads + tid;
+    const uint4 own = x[mine < total ? mine : total - 1];
+    float amax = 0.f;
+    for (int i0 = tid; i0 < total; i0 += kUnitLoads * kSmallThreads) {
+        uint4 v[kUnitLoads];
+#pragma unroll
+        for (int i = 0; i < kUnitLoads; i++) {
+            const int c = i0 + i * kSmallThreads;
+            v[i] = x[c < total ? c : total - 1];
+        }
+#pragma unroll
+        for (int i = 0; i < kUnitLoads; i++) amax = max_nonneg(amax, absmax8(v[i], DT == LLMQ_BF16));
+    }
+    amax = block_max<kSmallThreads / kWave>(amax, smem);
+    const float s = scale_from_amax<DT, MODE>(amax, floor);
+    if (mine == 0) {
+        if (scale_dtype == LLMQ_F32) ((float*)scale_out)[0] = s;
+        else ((uint16_t*)scale_out)[0] = Lo<DT>::from_f32(s);
+        store_alpha<DT>(ta, s);
+    }
+    if (mine < total) q[mine] = quant8<DT, MODE, Q_DT>(own, s, 1.0f / s);
 }
 
 // ---- RMSNorm fused with the per-token quantizer --------------------------------------------
@@ -399,7 +458,7 @@ int check_common(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, 
 
 template <int DT, int MODE, int SCALE>
 int launch_rows(const void* x, int64_t M, int64_t K, int64_t ldx, void* q, void* scale, int scale_dtype,
-                const float* aux, int n_aux, int static_f32, float floor, hipStream_t st) {
+                const float* aux, int n_aux, int static_f32, float floor, const TensorAlpha& ta, hipStream_t st) {
     const dim3 grid((unsigned)M), block(kThreads);
     const uint16_t* xp = (const uint16_t*)x;
     uint8_t* qp = (uint8_t*)q;
@@ -415,7 +474,7 @@ int launch_rows(const void* x, int64_t M, int64_t K, int64_t ldx, void* q, void*
         return launch_status();
     }
 #define LLMQ_LAUNCH_NCT(NC, NT) \
-    hipLaunchKernelGGL((quant_rows_kernel<DT, MODE, SCALE, NC, NT>), grid, dim3(NT), 0, st, xp, ldx, K, qp, scale, scale_dtype, aux, n_aux, static_f32, floor)
+    hipLaunchKernelGGL((quant_rows_kernel<DT, MODE, SCALE, NC, NT>), grid, dim3(NT), 0, st, xp, ldx, K, qp, scale, scale_dtype, aux, n_aux, static_f32, floor, ta)
 #define LLMQ_LAUNCH_NC(NC) LLMQ_LAUNCH_NCT(NC, kThreads)
     if (SCALE != SCALE_ROW) LLMQ_LAUNCH_NC(0);
     else if (half_blocks(M, K)) LLMQ_LAUNCH_NCT(4, kThreads / 2);
@@ -430,28 +489,50 @@ int launch_rows(const void* x, int64_t M, int64_t K, int64_t ldx, void* q, void*
 
 template <int MODE, int SCALE>
 int dispatch_rows(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, void* q, void* scale,
-                  int scale_dtype, const float* aux, int n_aux, int static_f32, float floor, hipStream_t st) {
+                  int scale_dtype, const float* aux, int n_aux, int static_f32, float floor, const TensorAlpha& ta,
+                  hipStream_t st) {
     if (x_dtype == LLMQ_BF16)
-        return launch_rows<LLMQ_BF16, MODE, SCALE>(x, M, K, ldx, q, scale, scale_dtype, aux, n_aux, static_f32, floor, st);
-    return launch_rows<LLMQ_F16, MODE, SCALE>(x, M, K, ldx, q, scale, scale_dtype, aux, n_aux, static_f32, floor, st);
+        return launch_rows<LLMQ_BF16, MODE, SCALE>(x, M, K, ldx, q, scale, scale_dtype, aux, n_aux, static_f32, floor, ta, st);
+    return launch_rows<LLMQ_F16, MODE, SCALE>(x, M, K, ldx, q, scale, scale_dtype, aux, n_aux, static_f32, floor, ta, st);
+}
+
+// Largest contiguous tensor (in chunks of 8 elements) that the one-launch per-tensor quantizer takes.  Measured (K = 3584,
+// back to back, one launch / two launches): 16 rows 3.7 / 6.2 us, 32 rows 4.6 / 6.8, 64 rows 6.4 / 6.8, 128 rows 10.5 / 6.9:
+// every block's pass over the whole tensor costs more than a launch from about 28000 chunks on.
+constexpr int64_t kSmallChunks = 16384;
+
+template <int DT, int MODE>
+int per_tensor_dt(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, void* q, void* scale, int scale_dtype,
+                  float* partials, float floor, const TensorAlpha& ta, hipStream_t st) {
+    const bool contiguous = ldx == K || M == 1;
+    const int64_t total = M * (K >> 3);
+    if (contiguous && total <= kSmallChunks) {
+        hipLaunchKernelGGL((quant_tensor_small_kernel<DT, MODE>), dim3((unsigned)((total + kSmallThreads - 1) / kSmallThreads)),
+                           dim3(kSmallThreads), 0, st, (const uint4*)x, (int)total, (uint2*)q, scale, scale_dtype, floor, ta);
+        return launch_status();
+    }
+    const int64_t rows = contiguous ? 1 : M, cpr = contiguous ? total : K >> 3;
+    const bool wide = cpr >= kUnitLoads * kThreads;
+    const int unit = (wide ? kUnitLoads : 2) * kThreads;
+    const int64_t units = rows * ((cpr + unit - 1) / unit);
+    const int nblk = (int)(units < kMaxPartials ? units : kMaxPartials);
+    if (wide)
+        hipLaunchKernelGGL((absmax_partials_kernel<DT, kUnitLoads>), dim3(nblk), dim3(kThreads), 0, st, (const uint16_t*)x,
+                           ldx, rows, cpr, partials);
+    else
+        hipLaunchKernelGGL((absmax_partials_kernel<DT, 2>), dim3(nblk), dim3(kThreads), 0, st, (const uint16_t*)x, ldx, rows,
+                           cpr, partials);
+    if (launch_status() != LLMQ_OK) return LLMQ_ERR_LAUNCH;
+    return dispatch_rows<MODE, SCALE_TENSOR>(x, x_dtype, M, K, ldx, q, scale, scale_dtype, partials, nblk, 0, floor, ta, st);
 }
 
 template <int MODE>
 int per_tensor(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, void* q, void* scale,
-               int scale_dtype, void* ws, size_t ws_bytes, float floor, hipStream_t st) {
+               int scale_dtype, void* ws, size_t ws_bytes, float floor, const TensorAlpha& ta, hipStream_t st) {
     if (!ws || ws_bytes < kMaxPartials * sizeof(float)) return LLMQ_ERR_WORKSPACE;
-    const int64_t total = M * (K >> 3);
-    int nblk = (int)((total + kThreads * 4 - 1) / (kThreads * 4));
-    nblk = nblk < 1 ? 1 : (nblk > kMaxPartials ? kMaxPartials : nblk);
-    float* partials = (float*)ws;
     if (x_dtype == LLMQ_BF16)
-        hipLaunchKernelGGL((absmax_partials_kernel<LLMQ_BF16>), dim3(nblk), dim3(kThreads), 0, st,
-                           (const uint16_t*)x, ldx, M, K, partials);
-    else
-        hipLaunchKernelGGL((absmax_partials_kernel<LLMQ_F16>), dim3(nblk), dim3(kThreads), 0, st,
-                           (const uint16_t*)x, ldx, M, K, partials);
-    if (launch_status() != LLMQ_OK) return LLMQ_ERR_LAUNCH;
-    return dispatch_rows<MODE, SCALE_TENSOR>(x, x_dtype, M, K, ldx, q, scale, scale_dtype, partials, nblk, 0, floor, st);
+        return per_tensor_dt<LLMQ_BF16, MODE>(x, x_dtype, M, K, ldx, q, scale, scale_dtype, (float*)ws, floor, ta, st);
+    return per_tensor_dt<LLMQ_F16, MODE>(x, x_dtype, M, K, ldx, q, scale, scale_dtype, (float*)ws, floor, ta, st);
 }
 
 // Per-output-channel int8 weight quantizer (an offline step: one pass when a module is built).  One block per
@@ -511,7 +592,7 @@ extern "C" int llmq_quant_i8_per_token_floor(const void* x, int x_dtype, int64_t
     if (scale_dtype != x_dtype && scale_dtype != LLMQ_F32) return LLMQ_ERR_DTYPE;
     if (K == 0) return LLMQ_ERR_SHAPE;
     return dispatch_rows<MODE_I8, SCALE_ROW>(x, x_dtype, M, K, ldx, q, scale, scale_dtype, nullptr, 0, 0, absmax_floor,
-                                             (hipStream_t)stream);
+                                             TensorAlpha{}, (hipStream_t)stream);
 }
 
 extern "C" int llmq_quant_i8_per_tensor(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
@@ -531,7 +612,7 @@ extern "C" int llmq_quant_i8_per_tensor_floor(const void* x, int x_dtype, int64_
     if (scale_dtype != x_dtype && scale_dtype != LLMQ_F32) return LLMQ_ERR_DTYPE;
     if (M == 0 || K == 0) return LLMQ_ERR_SHAPE;
     return per_tensor<MODE_I8>(x, x_dtype, M, K, ldx, q, scale, scale_dtype, workspace, workspace_bytes, absmax_floor,
-                               (hipStream_t)stream);
+                               TensorAlpha{}, (hipStream_t)stream);
 }
 
 extern "C" int llmq_quant_fp8_per_token(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
@@ -542,7 +623,7 @@ extern "C" int llmq_quant_fp8_per_token(const void* x, int x_dtype, int64_t M, i
     if (!scale) return LLMQ_ERR_NULL;
     if (K == 0) return LLMQ_ERR_SHAPE;
     return dispatch_rows<MODE_F8, SCALE_ROW>(x, x_dtype, M, K, ldx, q, scale, LLMQ_F32, nullptr, 0, 0,
-                                             QP<MODE_F8>::floor_, (hipStream_t)stream);
+                                             QP<MODE_F8>::floor_, TensorAlpha{}, (hipStream_t)stream);
 }
 
 extern "C" int llmq_quant_fp8_per_tensor(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
@@ -553,7 +634,34 @@ extern "C" int llmq_quant_fp8_per_tensor(const void* x, int x_dtype, int64_t M, 
     if (!scale) return LLMQ_ERR_NULL;
     if (M == 0 || K == 0) return LLMQ_ERR_SHAPE;
     return per_tensor<MODE_F8>(x, x_dtype, M, K, ldx, q, scale, LLMQ_F32, workspace, workspace_bytes,
-                               QP<MODE_F8>::floor_, (hipStream_t)stream);
+                               QP<MODE_F8>::floor_, TensorAlpha{}, (hipStream_t)stream);
+}
+
+extern "C" int llmq_quant_per_tensor_alpha(int fp8, const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, void* q,
+                                           float* scale, const float* w_scale, float* alpha, void* workspace,
+                                           size_t workspace_bytes, llmq_stream_t stream) {
+    int rc = check_common(x, x_dtype, M, K, ldx, q);
+    if (rc != LLMQ_OK) return rc;
+    if (!scale || !w_scale || !alpha) return LLMQ_ERR_NULL;
+    if (M == 0 || K == 0) return LLMQ_ERR_SHAPE;
+    const TensorAlpha ta{w_scale, alpha, fp8 ? 0 : 1};
+    if (fp8)
+        return per_tensor<MODE_F8>(x, x_dtype, M, K, ldx, q, scale, LLMQ_F32, workspace, workspace_bytes,
+                                   QP<MODE_F8>::floor_, ta, (hipStream_t)stream);
+    return per_tensor<MODE_I8>(x, x_dtype, M, K, ldx, q, scale, LLMQ_F32, workspace, workspace_bytes,
+                               QP<MODE_I8>::floor_, ta, (hipStream_t)stream);
+}
+
+extern "C" int llmq_quant_fp8_static_alpha(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, uint8_t* q,
+                                           const float* scale, int scale_is_f32_tensor, const float* w_scale, float* alpha,
+                                           llmq_stream_t stream) {
+    int rc = check_common(x, x_dtype, M, K, ldx, q);
+    if (rc != LLMQ_OK) return rc;
+    if (M == 0 || K == 0) return LLMQ_ERR_SHAPE;
+    if (!scale || !w_scale || !alpha) return LLMQ_ERR_NULL;
+    return dispatch_rows<MODE_F8, SCALE_STATIC>(x, x_dtype, M, K, ldx, q, nullptr, LLMQ_F32, scale, 1,
+                                                scale_is_f32_tensor ? 1 : 0, 0.f, TensorAlpha{w_scale, alpha, 0},
+                                                (hipStream_t)stream);
 }
 
 extern "C" int llmq_quant_fp8_static(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
@@ -564,7 +672,7 @@ extern "C" int llmq_quant_fp8_static(const void* x, int x_dtype, int64_t M, int6
     if (M == 0 || K == 0) return LLMQ_OK;
     if (!scale) return LLMQ_ERR_NULL;
     return dispatch_rows<MODE_F8, SCALE_STATIC>(x, x_dtype, M, K, ldx, q, nullptr, LLMQ_F32, scale, 1,
-                                                scale_is_f32_tensor ? 1 : 0, 0.f, (hipStream_t)stream);
+                                                scale_is_f32_tensor ? 1 : 0, 0.f, TensorAlpha{}, (hipStream_t)stream);
 }
 
 extern "C" int llmq_quant_i8_weight_per_channel(const void* w, int w_dtype, int64_t N, int64_t K, int64_t ldw,

@@ -9,7 +9,8 @@ from __future__ import annotations
 
 import torch
 
-from ..quantize import per_tensor_quantize, per_token_quantize, static_per_tensor_quantize
+from ..quantize import (per_tensor_quantize, per_tensor_quantize_with_alpha, per_token_quantize, static_per_tensor_quantize,
+                        static_per_tensor_quantize_with_alpha)
 from ..sq_fp8_kernels import (cutlass_f8f8bf16_rowwise_sm89, cutlass_f8f8bf16_tensorwise_sm89,
                               dynamic_linear_max_tokens, f8f8_tensorwise_quantized_output,
                               f8f8bf16_linear_dynamic_per_token)
@@ -106,8 +107,7 @@ class FP8DynamicLinear(_FP8LinearBase):
             return torch.zeros(out_shape, dtype=x.dtype, device=x.device)
         qweight = self._qweight_t()
         if self.per_tensor:
-            qinput, x_scale = per_tensor_quantize(x)
-            alpha = self.weight_scale * x_scale
+            qinput, alpha = per_tensor_quantize_with_alpha(x, self.weight_scale, fp8=True)
             output = cutlass_f8f8bf16_tensorwise_sm89(qinput.view(-1, x_shape[-1]), qweight, self.bias, alpha, 1.0,
                                                       dtype_to_str.get(self.dtype))
         else:
@@ -168,8 +168,7 @@ class FP8StaticLinear(_FP8LinearBase):
         if x.shape[0] == 0:
             return torch.zeros(out_shape, dtype=x.dtype, device=x.device)
         assert self.per_tensor, "[error!!] static activation quant only support per tensor!"
-        qinput = static_per_tensor_quantize(x, self.input_scale)
-        alpha = self.weight_scale * self.input_scale
+        qinput, alpha = static_per_tensor_quantize_with_alpha(x, self.input_scale, self.weight_scale)
         if self.quantize_output:
             # output / output_scale -> e4m3fn -> * output_scale (linear_fp8.py:309-311) inside the GEMM epilogue:
             # one launch, fp32 result as the reference's `qoutput.to(dtype) * output_scale`

@@ -9,7 +9,7 @@ from __future__ import annotations
 
 import torch
 
-from ..quantize import (quantize_activation_per_tensor_absmax, quantize_weight_per_channel_absmax,
+from ..quantize import (per_tensor_quantize_with_alpha, quantize_activation_per_tensor_absmax, quantize_weight_per_channel_absmax,
                         quantize_activation_per_token_absmax,
                         quantize_activation_per_token_absmax_f32)
 from ..sq_fp8_kernels import (dynamic_linear_max_tokens, w8a8_int8_linear_bbf16_obf16_per_channel,
@@ -68,10 +68,9 @@ class SqW8A8BBF16OBF16PerTensor(LinearBase):
         assert self.input_scale.device == self.qweight.device, "when sq linear fwd, scale and qweight must be same device!"
         x_shape = x.shape
         x2 = x.reshape(-1, x_shape[-1])
-        qx, input_scale = quantize_activation_per_tensor_absmax(x2)
-        # alpha stays on the device: the product is rounded to the activation dtype as the
-        # reference's `input_scale * weight_scale.item()` is, then read by the kernel
-        alpha = (input_scale.float() * self.weight_scale.float()).to(input_scale.dtype)
+        # alpha stays on the device: the quantizer forms the product, rounded to the activation dtype as the
+        # reference's `input_scale * weight_scale.item()` is, and the GEMM reads it
+        qx, alpha = per_tensor_quantize_with_alpha(x2, self.weight_scale, fp8=False)
         y = w8a8_int8_linear_bbf16_obf16_per_tensor(qx, self.qweight.t(), self._bias_or_zeros(x.dtype, x.device),
                                                     alpha, 1.0)
         return y.view(*x_shape[:-1], -1)

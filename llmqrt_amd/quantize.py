@@ -143,6 +143,41 @@ def static_per_tensor_quantize(tensor: torch.Tensor, scale) -> torch.Tensor:
     return q.view(*tensor.shape)
 
 
+def _alpha_operands(t: torch.Tensor, w_scale: torch.Tensor):
+    x = _as_rows(t)
+    M, K = x.shape
+    ws = w_scale.detach()
+    return (x, M, K, x.stride(0) if M > 1 else K, ws if ws.dtype == torch.float32 else ws.float(),
+            torch.empty(2, dtype=torch.float32, device=x.device))
+
+
+@torch.no_grad()
+def per_tensor_quantize_with_alpha(t: torch.Tensor, w_scale: torch.Tensor, fp8: bool):
+    """quantize_activation_per_tensor_absmax (int8) or per_tensor_quantize (fp8), and the factor scale * w_scale of the
+    GEMM that follows, formed by the quantizer's own kernel: -> (codes like t, alpha as a 0-dim fp32 tensor).  For int8
+    the product is rounded to t's dtype (linear_sq.py:127)."""
+    x, M, K, ldx, ws, s = _alpha_operands(t, w_scale)
+    q = torch.empty((M, K), dtype=torch.float8_e4m3fn if fp8 else torch.int8, device=x.device)
+    scratch = _abi.workspaces.get(x.device, _abi.lib().llmq_quant_workspace_bytes())
+    _abi.check(_abi.lib().llmq_quant_per_tensor_alpha(
+        int(fp8), x.data_ptr(), _abi.dtype_code(x.dtype), M, K, ldx, q.data_ptr(), s.data_ptr(), ws.data_ptr(),
+        s.data_ptr() + 4, scratch.data_ptr(), scratch.numel(), _abi.stream_of(x)), "llmq_quant_per_tensor_alpha")
+    return q.view(t.shape), s[1]
+
+
+@torch.no_grad()
+def static_per_tensor_quantize_with_alpha(t: torch.Tensor, scale: torch.Tensor, w_scale: torch.Tensor):
+    """static_per_tensor_quantize on a one-element fp32 GPU tensor, and scale * w_scale: -> (codes like t, alpha)."""
+    x, M, K, ldx, ws, s = _alpha_operands(t, w_scale)
+    sdev = scale.detach().reshape(-1)[:1].to(device=x.device, dtype=torch.float32)
+    q = torch.empty((M, K), dtype=torch.float8_e4m3fn, device=x.device)
+    _abi.check(_abi.lib().llmq_quant_fp8_static_alpha(
+        x.data_ptr(), _abi.dtype_code(x.dtype), M, K, ldx, q.data_ptr(), sdev.data_ptr(),
+        int(scale.dim() > 0 and scale.dtype == torch.float32), ws.data_ptr(), s.data_ptr(), _abi.stream_of(x)),
+        "llmq_quant_fp8_static_alpha")
+    return q.view(t.shape), s[0]
+
+
 @torch.no_grad()
 def quantize_weight_per_channel_absmax(w: torch.Tensor):
     """Replaces quantize_weight_per_channel_absmax (utils/quantization_utils.py:27-38): w [N, K] bf16 / fp16 / fp32 on

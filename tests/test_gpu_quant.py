@@ -277,3 +277,34 @@ def test_dynamic_quantizers_with_the_1e8_floor(cuda, M, K, dtype):
     qt_ref, st_ref = R.dynamic_quantize_activation_per_tensor_absmax(tiny)
     qt, st = dynamic_quantize_activation_per_tensor_absmax(tiny.to(cuda))
     assert _same_with_nans(st.cpu(), st_ref) and torch.equal(qt.cpu(), qt_ref)
+
+
+# one-launch kernel (contiguous, up to 16384 chunks of 8 elements): one chunk, a block's 1024 chunks and its neighbours, the
+# largest; two-launch kernels: the smallest contiguous, strided rows with short (2 loads a thread) and long (8) units
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("M,K,pad", [(1, 8, 0), (1, 8192, 0), (9, 1032, 0), (32, 4096, 0), (32, 4104, 0), (3, 2056, 8),
+                                     (70, 16392, 8), (1030, 2048, 0)])
+def test_per_tensor_with_alpha(cuda, M, K, pad, fp8, dtype):
+    """Codes as the plain per-tensor quantizer's oracle, alpha = scale x weight scale (int8: rounded to the dtype), exact."""
+    from llmqrt_amd.quantize import per_tensor_quantize_with_alpha, static_per_tensor_quantize_with_alpha
+    x = _acts(M, K, 17 * M + K, dtype)
+    x[M - 1, K - 1] = 300.0 if M > 1 else 50.0  # the maximum sits in the last chunk
+    buf = torch.zeros(M, K + pad, dtype=dtype, device=cuda)
+    buf[:, :K] = x.to(cuda)
+    xd = buf[:, :K]
+    ws = torch.tensor(0.0137, dtype=torch.float32)
+    q, a = per_tensor_quantize_with_alpha(xd, ws.to(cuda), fp8)
+    if fp8:
+        q_ref, s_ref = R.fp8_per_tensor_quantize(x)
+        a_ref = s_ref.float() * ws
+        assert torch.equal(q.cpu().view(torch.uint8), q_ref.view(torch.uint8))
+        sx = torch.tensor([0.21], dtype=torch.float32)
+        qs, sa = static_per_tensor_quantize_with_alpha(xd, sx.to(cuda), ws.to(cuda))
+        qs_ref = R.fp8_static_per_tensor_quantize(x, sx)
+        assert torch.equal(qs.cpu().view(torch.uint8), qs_ref.view(torch.uint8)) and torch.equal(sa.cpu().reshape(()), (sx * ws).reshape(()))
+    else:
+        q_ref, s_ref = R.quantize_activation_per_tensor_absmax(x)
+        a_ref = (s_ref.float() * ws).to(dtype).float()
+        assert torch.equal(q.cpu(), q_ref)
+    assert a.dtype == torch.float32 and torch.equal(a.cpu().reshape(()), a_ref.reshape(()))
