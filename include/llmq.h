@@ -281,6 +281,15 @@ int llmq_awq_gemm(const void* x, int64_t ldx, const int32_t* qweight, const void
 
 size_t llmq_awq_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
+/* llmq_awq_gemm for a bf16 model: x and out are bf16.  The activations are rounded to fp16 inside the kernel and the fp16
+ * result is widened to bf16, the values of the reference's conversions around the op (linear_awq.py:245-262).  Only where
+ * llmq_awq_gemm_bf16_supported says 1 (the few-token kernel); otherwise LLMQ_ERR_DTYPE, before any launch. */
+int llmq_awq_gemm_bf16(const void* x, int64_t ldx, const int32_t* qweight, const void* scales,
+                       const int32_t* qzeros, const void* bias, void* out,
+                       int64_t M, int64_t N, int64_t K, int64_t group,
+                       void* workspace, size_t workspace_bytes, llmq_stream_t stream);
+int llmq_awq_gemm_bf16_supported(int64_t M, int64_t N, int64_t K, int64_t group);
+
 /* No counterpart in the reference (its split-K ends in fp16 atomics on the output, awq_kernels.py:253-267):
  * size of the counter area at the start of an AWQ workspace, and a launch on `stream` that zeroes it. */
 size_t llmq_awq_workspace_ticket_bytes(void);

@@ -84,6 +84,24 @@ def awq_gemm_triton(input: torch.Tensor, qweight: torch.Tensor, scales: torch.Te
                     split_k_iters: int, block_size_m: int = 32, block_size_n: int = 32,
                     block_size_k: int = 32, *, bias: torch.Tensor | None = None) -> torch.Tensor:
     """input fp16 [M, K] x dequant(qweight) -> fp16 [M, N] (fp32 accumulation, deterministic)."""
+    assert input.dtype == torch.float16
+    return _awq_gemm(input, qweight, scales, qzeros, split_k_iters, bias)
+
+
+def awq_gemm_bf16_supported(M: int, N: int, K: int, group_size: int) -> bool:
+    """Whether ``awq_gemm_bf16`` takes this shape: the few-token kernel, which converts on the way in and out."""
+    return bool(_abi.lib().llmq_awq_gemm_bf16_supported(M, N, K, group_size))
+
+
+@torch.no_grad()
+def awq_gemm_bf16(input: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor, qzeros: torch.Tensor,
+                  bias: torch.Tensor | None = None) -> torch.Tensor:
+    """``awq_gemm_triton(input.half(), ...).bfloat16()`` in one launch, for shapes that awq_gemm_bf16_supported takes."""
+    assert input.dtype == torch.bfloat16
+    return _awq_gemm(input, qweight, scales, qzeros, 1, bias)
+
+
+def _awq_gemm(input, qweight, scales, qzeros, split_k_iters, bias):
     M, K = input.shape
     N = qweight.shape[1] * 8
     group_size = qweight.shape[0] // qzeros.shape[0]
@@ -91,14 +109,15 @@ def awq_gemm_triton(input: torch.Tensor, qweight: torch.Tensor, scales: torch.Te
     assert split_k_iters & (split_k_iters - 1) == 0 and split_k_iters != 0
     assert split_k_iters <= 32
     _check_layout(qweight, scales, qzeros, K, N, group_size)
-    assert input.dtype == torch.float16 and input.device == qweight.device
+    assert input.device == qweight.device
     x = input
     if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:
         x = x.contiguous()
-    result = torch.empty((M, N), dtype=scales.dtype, device=input.device)
+    result = torch.empty((M, N), dtype=input.dtype, device=input.device)
     L = _abi.lib()
     ws = _abi.awq_workspaces.get(x.device, L.llmq_awq_gemm_workspace_bytes(M, N, K))
-    _abi.check(L.llmq_awq_gemm(x.data_ptr(), x.stride(0), qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(),
-                               _abi.ptr(bias), result.data_ptr(), M, N, K, group_size, _abi.ptr(ws),
-                               ws.numel() if ws is not None else 0, _abi.stream_of(x)), "llmq_awq_gemm")
+    fn = L.llmq_awq_gemm if input.dtype == torch.float16 else L.llmq_awq_gemm_bf16
+    _abi.check(fn(x.data_ptr(), x.stride(0), qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(),
+                  _abi.ptr(bias), result.data_ptr(), M, N, K, group_size, _abi.ptr(ws),
+                  ws.numel() if ws is not None else 0, _abi.stream_of(x)), "llmq_awq_gemm")
     return result

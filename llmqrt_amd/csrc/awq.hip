@@ -812,9 +812,11 @@ extern "C" int llmq_awq_workspace_init(void* workspace, size_t workspace_bytes, 
     return awq_clear_tickets(workspace, workspace_bytes, (hipStream_t)stream);
 }
 
-extern "C" int llmq_awq_gemm(const void* x, int64_t ldx, const int32_t* qweight, const void* scales,
-                             const int32_t* qzeros, const void* bias, void* out, int64_t M, int64_t N, int64_t K,
-                             int64_t group, void* workspace, size_t workspace_bytes, llmq_stream_t stream) {
+namespace {
+
+int awq_gemm_entry(const void* x, int64_t ldx, const int32_t* qweight, const void* scales, const int32_t* qzeros,
+                   const void* bias, void* out, int64_t M, int64_t N, int64_t K, int64_t group, bool bf16_io,
+                   void* workspace, size_t workspace_bytes, llmq_stream_t stream) {
     if (M < 0 || N < 0 || K < 0) return LLMQ_ERR_SHAPE;
     if (M == 0 || N == 0) return LLMQ_OK;
     if (!x || !qweight || !scales || !qzeros || !out) return LLMQ_ERR_NULL;
@@ -834,6 +836,7 @@ extern "C" int llmq_awq_gemm(const void* x, int64_t ldx, const int32_t* qweight,
     const uint16_t* sc = (const uint16_t*)scales;
     const uint16_t* bs = (const uint16_t*)bias;
     const int Ni = (int)N, Ki = (int)K, Gi = (int)group;
+    if (bf16_io && (tile_path(M) || !decode16_path(M, N, K, group))) return LLMQ_ERR_DTYPE;
     if (tile_path(M)) {
         const AwqTilePlan t = tile_plan(M, N, K);
         if (t.splits > 1 && (!ws || workspace_bytes < (size_t)t.splits * M * N * sizeof(float))) return LLMQ_ERR_WORKSPACE;
@@ -851,7 +854,7 @@ extern "C" int llmq_awq_gemm(const void* x, int64_t ldx, const int32_t* qweight,
     if (decode16_path(M, N, K, group)) {
         const AwqDecodePlan d = decode16_plan(M, N, K);
         if (d.splits > 1 && (!ws || workspace_bytes < awq_decode_workspace_bytes(d, M, N))) return LLMQ_ERR_WORKSPACE;
-        return launch_awq_decode(d, (const uint16_t*)x, ldx, qw, sc, qz, bs, (uint16_t*)out, tickets, ws, (int)M, Ni, Ki, st);
+        return launch_awq_decode(d, (const uint16_t*)x, ldx, qw, sc, qz, bs, (uint16_t*)out, tickets, ws, (int)M, Ni, Ki, bf16_io, st);
     }
     // tokens are processed in slabs of at most 64 rows (4 MFMA token tiles per weight pass)
     for (int64_t m0 = 0; m0 < M; m0 += 64) {
@@ -893,6 +896,24 @@ extern "C" int llmq_awq_gemm(const void* x, int64_t ldx, const int32_t* qweight,
         }
     }
     return LLMQ_OK;
+}
+
+}  // namespace
+
+extern "C" int llmq_awq_gemm(const void* x, int64_t ldx, const int32_t* qweight, const void* scales,
+                             const int32_t* qzeros, const void* bias, void* out, int64_t M, int64_t N, int64_t K,
+                             int64_t group, void* workspace, size_t workspace_bytes, llmq_stream_t stream) {
+    return awq_gemm_entry(x, ldx, qweight, scales, qzeros, bias, out, M, N, K, group, false, workspace, workspace_bytes, stream);
+}
+
+extern "C" int llmq_awq_gemm_bf16_supported(int64_t M, int64_t N, int64_t K, int64_t group) {
+    return !tile_path(M) && g_force_v == 0 && decode16_path(M, N, K, group);
+}
+
+extern "C" int llmq_awq_gemm_bf16(const void* x, int64_t ldx, const int32_t* qweight, const void* scales,
+                                  const int32_t* qzeros, const void* bias, void* out, int64_t M, int64_t N, int64_t K,
+                                  int64_t group, void* workspace, size_t workspace_bytes, llmq_stream_t stream) {
+    return awq_gemm_entry(x, ldx, qweight, scales, qzeros, bias, out, M, N, K, group, true, workspace, workspace_bytes, stream);
 }
 
 extern "C" int llmq_awq_dequant(const int32_t* qweight, const void* scales, const int32_t* qzeros, void* out,

@@ -36,6 +36,24 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));  // a first-class 16-byte value (HIP's uint4 is a struct: copies of it become memcpy)
 
+// Activations and outputs of a bf16 model (BF): the 4-bit weights are fp16 by definition, so the activations are rounded to
+// fp16 on their way into LDS and the fp16 result is widened back, the same values as separate conversions around the
+// op (linear_awq.py:245-262) without their two launches and two passes over the output.
+__device__ __forceinline__ u4 bf16x8_to_f16(u4 v) {
+    u4 r;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t w = v[i];
+        r[i] = Lo<LLMQ_F16>::pack2(Lo<LLMQ_BF16>::lo_f32(w), Lo<LLMQ_BF16>::hi_f32(w));
+    }
+    return r;
+}
+template <bool BF>
+__device__ __forceinline__ uint32_t pack_out(float a, float b) {
+    const uint32_t h = (uint32_t)Lo<LLMQ_F16>::from_f32(a) | ((uint32_t)Lo<LLMQ_F16>::from_f32(b) << 16);
+    return BF ? Lo<LLMQ_BF16>::pack2(Lo<LLMQ_F16>::lo_f32(h), Lo<LLMQ_F16>::hi_f32(h)) : h;
+}
+
 constexpr int kGroup = 128;      // quantization group = 2 stages of 64 rows = 4 MFMA chunks of 32 rows
 constexpr int kStageRows = 64;
 
@@ -53,7 +71,7 @@ __host__ __device__ constexpr int rev_nibble_d(int j) { return ((j & 1) << 2) | 
 // Tickets of neighbouring tiles are 256 bytes apart so that their atomics land in different memory channels
 // (adjacent words were measured 1-3 us slower per launch).
 constexpr int kTicketStride = 64;  // in 4-byte words
-template <int TILE_CH, int NT>
+template <int TILE_CH, int NT, bool BF>
 __device__ __forceinline__ void finish_split_tile(const float* ptile, int M, int N, int tile, int ks, int splits,
                                                   float* partials, int64_t plane, unsigned int* tickets,
                                                   const uint16_t* bias, uint16_t* out) {
@@ -68,9 +86,7 @@ __device__ __forceinline__ void finish_split_tile(const float* ptile, int M, int
             lo1 = Lo<LLMQ_F16>::to_f32(Lo<LLMQ_F16>::from_f32(lo1)) + Lo<LLMQ_F16>::to_f32(bias[nn + 2]);
             hi1 = Lo<LLMQ_F16>::to_f32(Lo<LLMQ_F16>::from_f32(hi1)) + Lo<LLMQ_F16>::to_f32(bias[nn + 3]);
         }
-        *reinterpret_cast<uint2*>(out + (int64_t)m * N + nn) =
-            make_uint2((uint32_t)Lo<LLMQ_F16>::from_f32(lo0) | ((uint32_t)Lo<LLMQ_F16>::from_f32(hi0) << 16),
-                       (uint32_t)Lo<LLMQ_F16>::from_f32(lo1) | ((uint32_t)Lo<LLMQ_F16>::from_f32(hi1) << 16));
+        *reinterpret_cast<uint2*>(out + (int64_t)m * N + nn) = make_uint2(pack_out<BF>(lo0, hi0), pack_out<BF>(lo1, hi1));
     };
     if (splits == 1) {
         for (int idx = tid; idx < M * tile_q; idx += NT) {
@@ -160,7 +176,8 @@ __device__ __forceinline__ void finish_split_tile(const float* ptile, int M, int
 // RM: token rows per lane that can be live (min(M, 4)).  KS: K slices inside the block - KS sets of CS wavefronts, each
 // with its own LDS stages, take consecutive shares of the block's groups (KS x the bytes in flight per block at the
 // same number of cross-block arrivals) and add their sums through LDS in slice order before the block publishes.
-template <int CS, int PD, int RM, int KS>
+// BF: x and out are bf16.
+template <int CS, int PD, int RM, int KS, bool BF>
 __global__ __launch_bounds__(CS * KS * kWave, KS == 4 ? 2 : 3) void awq_decode_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, const uint32_t* __restrict__ qw,
     const uint16_t* __restrict__ scales, const uint32_t* __restrict__ qz, const uint16_t* __restrict__ bias,
@@ -272,7 +289,7 @@ __global__ __launch_bounds__(CS * KS * kWave, KS == 4 ? 2 : 3) void awq_decode_k
         *reinterpret_cast<u4*>(tile_lds + st_slot + RPL * STRIDE) = cur.w1;
         *reinterpret_cast<u4*>(tile_lds + st_slot + 2 * RPL * STRIDE) = cur.w2;
         *reinterpret_cast<u4*>(tile_lds + st_slot + 3 * RPL * STRIDE) = cur.w3;
-        if (x_loader) *reinterpret_cast<u4*>(ldx_s[buf] + x_slot) = x_ok ? cur.x0 : u4{0u, 0u, 0u, 0u};  // rows past M read as 0
+        if (x_loader) *reinterpret_cast<u4*>(ldx_s[buf] + x_slot) = x_ok ? (BF ? bf16x8_to_f16(cur.x0) : cur.x0) : u4{0u, 0u, 0u, 0u};  // rows past M read as 0
         if ((st & 1) == 0) {
             z_cur = z_next;
             s_cur = s_next;
@@ -362,7 +379,7 @@ __global__ __launch_bounds__(CS * KS * kWave, KS == 4 ? 2 : 3) void awq_decode_k
                 lo = Lo<LLMQ_F16>::to_f32(Lo<LLMQ_F16>::from_f32(lo)) + Lo<LLMQ_F16>::to_f32(bias[nn + 2 * j]);
                 hi = Lo<LLMQ_F16>::to_f32(Lo<LLMQ_F16>::from_f32(hi)) + Lo<LLMQ_F16>::to_f32(bias[nn + 2 * j + 1]);
             }
-            o[j] = (uint32_t)Lo<LLMQ_F16>::from_f32(lo) | ((uint32_t)Lo<LLMQ_F16>::from_f32(hi) << 16);
+            o[j] = pack_out<BF>(lo, hi);
         }
         *reinterpret_cast<uint4*>(out + (int64_t)m * N + nn) = make_uint4(o[0], o[1], o[2], o[3]);
     };
@@ -401,7 +418,7 @@ __global__ __launch_bounds__(CS * KS * kWave, KS == 4 ? 2 : 3) void awq_decode_k
         }
         __syncthreads();
     }
-    finish_split_tile<TILE_CH, NT>(ptile, M, N, tile, ks, splits, partials, (int64_t)Mtot * N, tickets, bias, out);
+    finish_split_tile<TILE_CH, NT, BF>(ptile, M, N, tile, ks, splits, partials, (int64_t)Mtot * N, tickets, bias, out);
 }
 
 inline int cdiv_d(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
@@ -492,21 +509,29 @@ int awq_clear_tickets(void* workspace, size_t bytes, hipStream_t st) {
 
 int launch_awq_decode(const AwqDecodePlan& p, const uint16_t* x, int64_t ldx, const uint32_t* qw, const uint16_t* scales,
                       const uint32_t* qz, const uint16_t* bias, uint16_t* out, unsigned int* tickets, float* ws, int M,
-                      int N, int K, hipStream_t st) {
+                      int N, int K, bool bf16_io, hipStream_t st) {
     const int tiles_n = cdiv_d(N / 8, 16 * p.cs);
     const int slabs = cdiv_d(M, 16), work = tiles_n * p.splits;
     const dim3 grid((unsigned)(slabs == 1 ? work : cdiv_d(work, 8) * 8 * slabs));
     if (p.splits > 1 && (!tickets || (size_t)tiles_n * slabs * kTicketStride * sizeof(unsigned int) > kAwqTicketBytes))
         return LLMQ_ERR_WORKSPACE;
-#define LLMQ_DECODE_RM(CS_, PD_, RM_, KS_)                                                                            \
-    hipLaunchKernelGGL((awq_decode_kernel<CS_, PD_, RM_, KS_>), grid, dim3(CS_ * KS_ * kWave), 0, st, x, ldx, qw, scales, \
-                       qz, bias, out, ws, tickets, M, N, K, p.groups_per_block, tiles_n, p.splits, slabs)
-#define LLMQ_DECODE(CS_, PD_, KS_)                         \
-    do {                                                   \
-        if (M == 1) LLMQ_DECODE_RM(CS_, PD_, 1, KS_);      \
-        else if (M == 2) LLMQ_DECODE_RM(CS_, PD_, 2, KS_); \
-        else LLMQ_DECODE_RM(CS_, PD_, 4, KS_);             \
+#define LLMQ_DECODE_RM(CS_, PD_, RM_, KS_, BF_)                                                                       \
+    hipLaunchKernelGGL((awq_decode_kernel<CS_, PD_, RM_, KS_, BF_>), grid, dim3(CS_ * KS_ * kWave), 0, st, x, ldx, qw,  \
+                       scales, qz, bias, out, ws, tickets, M, N, K, p.groups_per_block, tiles_n, p.splits, slabs)
+#define LLMQ_DECODE_BF(CS_, PD_, KS_, BF_)                      \
+    do {                                                        \
+        if (M == 1) LLMQ_DECODE_RM(CS_, PD_, 1, KS_, BF_);      \
+        else if (M == 2) LLMQ_DECODE_RM(CS_, PD_, 2, KS_, BF_); \
+        else LLMQ_DECODE_RM(CS_, PD_, 4, KS_, BF_);             \
     } while (0)
+#define LLMQ_DECODE(CS_, PD_, KS_) LLMQ_DECODE_BF(CS_, PD_, KS_, false)
+    if (bf16_io) {
+        if (p.cs != 2 || p.pd != 1) return LLMQ_ERR_DTYPE;  // built for the tile that the plan picks
+        if (p.ks == 4) LLMQ_DECODE_BF(2, 1, 4, true);
+        else if (p.ks == 2) LLMQ_DECODE_BF(2, 1, 2, true);
+        else LLMQ_DECODE_BF(2, 1, 1, true);
+        return launch_status();
+    }
     if (p.cs == 4 && p.pd == 2) LLMQ_DECODE(4, 2, 1);
     else if (p.cs == 4) LLMQ_DECODE(4, 1, 1);
     else if (p.pd == 2) LLMQ_DECODE(2, 2, 1);
@@ -514,6 +539,7 @@ int launch_awq_decode(const AwqDecodePlan& p, const uint16_t* x, int64_t ldx, co
     else if (p.ks == 2) LLMQ_DECODE(2, 1, 2);
     else LLMQ_DECODE(2, 1, 1);
 #undef LLMQ_DECODE
+#undef LLMQ_DECODE_BF
 #undef LLMQ_DECODE_RM
     return launch_status();
 }

@@ -29,6 +29,6 @@ AwqDecodePlan make_awq_decode_plan(int64_t M, int64_t N, int64_t K, int force_cs
 size_t awq_decode_workspace_bytes(const AwqDecodePlan& p, int64_t M, int64_t N);
 int launch_awq_decode(const AwqDecodePlan& p, const uint16_t* x, int64_t ldx, const uint32_t* qw, const uint16_t* scales,
                       const uint32_t* qz, const uint16_t* bias, uint16_t* out, unsigned int* tickets, float* ws, int M,
-                      int N, int K, hipStream_t st);
+                      int N, int K, bool bf16_io, hipStream_t st);
 
 }  // namespace llmq

@@ -5,7 +5,8 @@ from __future__ import annotations
 
 import torch
 
-from ..awq_kernels import awq_dequantize_transposed, awq_dequantize_triton, awq_gemm_triton, gemm_f16
+from ..awq_kernels import (awq_dequantize_transposed, awq_dequantize_triton, awq_gemm_bf16, awq_gemm_bf16_supported,
+                           awq_gemm_triton, gemm_f16)
 from .linear_base import LinearBase
 
 AWQ_ORDER = (0, 2, 4, 6, 1, 3, 5, 7)
@@ -122,6 +123,12 @@ class WQLinear_GEMM(LinearBase):
         if x.shape[0] == 0:
             return torch.zeros(out_shape, dtype=x.dtype, device=x.device)
         input_dtype = x.dtype
+        tokens = x.numel() // x.shape[-1]
+        if input_dtype == torch.bfloat16 and awq_gemm_bf16_supported(tokens, self.out_features, self.in_features,
+                                                                    self.group_size):
+            # a few tokens of a bf16 model: the kernel converts in and out itself
+            return awq_gemm_bf16(x.reshape(-1, x.shape[-1]), self.qweight, self.scales, self.qzeros,
+                                 self.bias).view(out_shape)
         if input_dtype != torch.float16:
             x = x.to(torch.float16)
         with torch.no_grad():

@@ -517,3 +517,26 @@ def test_module_many_token_path_is_own_kernels(cuda):
         torch.matmul = real_matmul
     assert y.shape == (2, T // 2, N)
     assert rel_err(y.reshape(T, N), ref) <= REL_TOL
+
+
+# the plans behind the bf16 form: no split with one slice per block cannot occur; K splits with 1 (wide N), 2 and 4 slices,
+# 4 slices without a split (wide N, 9-16 tokens), slabs of 16 with a ragged last one, a ragged last column tile
+@pytest.mark.parametrize("M,K,N,with_bias", [(1, 512, 32, True), (2, 3584, 1152, False), (5, 1024, 288, True), (16, 2304, 544, True),
+                                             (3, 1536, 16640, True), (12, 768, 16640, False), (17, 1024, 1056, True), (64, 4864, 896, False)])
+def test_bf16_activations_equal_separate_conversions(cuda, M, K, N, with_bias):
+    """awq_gemm_bf16 and the module on bf16 activations: bit for bit the fp16 op between x.half() and .bfloat16()."""
+    from llmqrt_amd import workloads as W
+    from llmqrt_amd.awq_kernels import awq_gemm_bf16, awq_gemm_bf16_supported, awq_gemm_triton
+    from llmqrt_amd.linear import WQLinear_GEMM
+    qw, qz, s = (t.to(cuda) for t in W.awq_weights(N, K, K + N))
+    bias = (0.3 * torch.randn(N, generator=torch.Generator().manual_seed(N))).half().to(cuda) if with_bias else None
+    x = W.activations(M, K, M + 3, dtype=torch.bfloat16).to(cuda)
+    assert awq_gemm_bf16_supported(M, N, K, 128) and not awq_gemm_bf16_supported(65, N, K, 128)
+    ref = awq_gemm_triton(x.half(), qw, s, qz, 8, bias=bias).bfloat16()
+    assert torch.equal(awq_gemm_bf16(x, qw, s, qz, bias), ref)
+    mod = WQLinear_GEMM(4, 128, K, N, with_bias, cuda)
+    mod.qweight.copy_(qw); mod.qzeros.copy_(qz); mod.scales.copy_(s)
+    if with_bias:
+        mod.bias.copy_(bias)
+    y = mod(x.view(M, 1, K))
+    assert y.dtype == torch.bfloat16 and torch.equal(y.view(M, N), ref)
