@@ -290,6 +290,15 @@ int llmq_awq_gemm_bf16(const void* x, int64_t ldx, const int32_t* qweight, const
                        void* workspace, size_t workspace_bytes, llmq_stream_t stream);
 int llmq_awq_gemm_bf16_supported(int64_t M, int64_t N, int64_t K, int64_t group);
 
+/* The same (x_dtype LLMQ_F16 or LLMQ_BF16) with the two halves of the workspace given apart: the counter area
+ * (llmq_awq_workspace_ticket_bytes() bytes, zero before and after a call) and the partial sums of this one call
+ * (llmq_awq_gemm_partials_bytes, contents irrelevant; both may be NULL when that is 0). */
+int llmq_awq_gemm_tickets(const void* x, int x_dtype, int64_t ldx, const int32_t* qweight, const void* scales,
+                          const int32_t* qzeros, const void* bias, void* out,
+                          int64_t M, int64_t N, int64_t K, int64_t group,
+                          void* tickets, void* partials, size_t partials_bytes, llmq_stream_t stream);
+size_t llmq_awq_gemm_partials_bytes(int64_t M, int64_t N, int64_t K, int64_t group);
+
 /* No counterpart in the reference (its split-K ends in fp16 atomics on the output, awq_kernels.py:253-267):
  * size of the counter area at the start of an AWQ workspace, and a launch on `stream` that zeroes it. */
 size_t llmq_awq_workspace_ticket_bytes(void);

@@ -816,7 +816,7 @@ namespace {
 
 int awq_gemm_entry(const void* x, int64_t ldx, const int32_t* qweight, const void* scales, const int32_t* qzeros,
                    const void* bias, void* out, int64_t M, int64_t N, int64_t K, int64_t group, bool bf16_io,
-                   void* workspace, size_t workspace_bytes, llmq_stream_t stream) {
+                   void* ticket_area, void* partials, size_t workspace_bytes, llmq_stream_t stream) {
     if (M < 0 || N < 0 || K < 0) return LLMQ_ERR_SHAPE;
     if (M == 0 || N == 0) return LLMQ_OK;
     if (!x || !qweight || !scales || !qzeros || !out) return LLMQ_ERR_NULL;
@@ -824,13 +824,12 @@ int awq_gemm_entry(const void* x, int64_t ldx, const int32_t* qweight, const voi
         return LLMQ_ERR_SHAPE;
     if (N > 0x7fffffffLL || K > 0x7fffffffLL || M > 0x7fffffffLL || ldx * 16 > 0x7fffffffLL) return LLMQ_ERR_SHAPE;
     if (!aligned16(x) || !aligned16(scales) || !aligned16(out) || (reinterpret_cast<uintptr_t>(qweight) & 15u) ||
-        (reinterpret_cast<uintptr_t>(qzeros) & 15u) || (reinterpret_cast<uintptr_t>(workspace) & 15u))
+        (reinterpret_cast<uintptr_t>(qzeros) & 15u) || (reinterpret_cast<uintptr_t>(ticket_area) & 15u) ||
+        (reinterpret_cast<uintptr_t>(partials) & 15u))
         return LLMQ_ERR_ALIGN;
     hipStream_t st = (hipStream_t)stream;
-    // workspace = arrival counters (kAwqTicketBytes, zero between calls), then partial sums (contents irrelevant)
-    unsigned int* tickets = workspace_bytes > kAwqTicketBytes ? (unsigned int*)workspace : nullptr;
-    float* ws = tickets ? (float*)((unsigned char*)workspace + kAwqTicketBytes) : nullptr;
-    workspace_bytes = tickets ? workspace_bytes - kAwqTicketBytes : 0;
+    unsigned int* tickets = (unsigned int*)ticket_area;
+    float* ws = tickets ? (float*)partials : nullptr;
     const uint32_t* qw = (const uint32_t*)qweight;
     const uint32_t* qz = (const uint32_t*)qzeros;
     const uint16_t* sc = (const uint16_t*)scales;
@@ -898,12 +897,23 @@ int awq_gemm_entry(const void* x, int64_t ldx, const int32_t* qweight, const voi
     return LLMQ_OK;
 }
 
+// workspace = arrival counters (kAwqTicketBytes, zero between calls), then partial sums (contents irrelevant)
+int awq_gemm_workspace(const void* x, int64_t ldx, const int32_t* qweight, const void* scales, const int32_t* qzeros,
+                       const void* bias, void* out, int64_t M, int64_t N, int64_t K, int64_t group, bool bf16_io,
+                       void* workspace, size_t workspace_bytes, llmq_stream_t stream) {
+    const bool usable = workspace && workspace_bytes > kAwqTicketBytes;
+    if (!usable && (reinterpret_cast<uintptr_t>(workspace) & 15u) && M > 0 && N > 0) return LLMQ_ERR_ALIGN;
+    return awq_gemm_entry(x, ldx, qweight, scales, qzeros, bias, out, M, N, K, group, bf16_io, usable ? workspace : nullptr,
+                          usable ? (unsigned char*)workspace + kAwqTicketBytes : nullptr,
+                          usable ? workspace_bytes - kAwqTicketBytes : 0, stream);
+}
+
 }  // namespace
 
 extern "C" int llmq_awq_gemm(const void* x, int64_t ldx, const int32_t* qweight, const void* scales,
                              const int32_t* qzeros, const void* bias, void* out, int64_t M, int64_t N, int64_t K,
                              int64_t group, void* workspace, size_t workspace_bytes, llmq_stream_t stream) {
-    return awq_gemm_entry(x, ldx, qweight, scales, qzeros, bias, out, M, N, K, group, false, workspace, workspace_bytes, stream);
+    return awq_gemm_workspace(x, ldx, qweight, scales, qzeros, bias, out, M, N, K, group, false, workspace, workspace_bytes, stream);
 }
 
 extern "C" int llmq_awq_gemm_bf16_supported(int64_t M, int64_t N, int64_t K, int64_t group) {
@@ -913,7 +923,33 @@ extern "C" int llmq_awq_gemm_bf16_supported(int64_t M, int64_t N, int64_t K, int
 extern "C" int llmq_awq_gemm_bf16(const void* x, int64_t ldx, const int32_t* qweight, const void* scales,
                                   const int32_t* qzeros, const void* bias, void* out, int64_t M, int64_t N, int64_t K,
                                   int64_t group, void* workspace, size_t workspace_bytes, llmq_stream_t stream) {
-    return awq_gemm_entry(x, ldx, qweight, scales, qzeros, bias, out, M, N, K, group, true, workspace, workspace_bytes, stream);
+    return awq_gemm_workspace(x, ldx, qweight, scales, qzeros, bias, out, M, N, K, group, true, workspace, workspace_bytes, stream);
+}
+
+extern "C" size_t llmq_awq_gemm_partials_bytes(int64_t M, int64_t N, int64_t K, int64_t group) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    if (tile_path(M)) {
+        const AwqTilePlan t = tile_plan(M, N, K);
+        return t.splits > 1 ? (size_t)t.splits * M * N * sizeof(float) : 0;
+    }
+    if (decode16_path(M, N, K, group)) return awq_decode_workspace_bytes(decode16_plan(M, N, K), M, N);
+    size_t total = 0;
+    for (int64_t m0 = 0; m0 < M; m0 += 64) {
+        const int64_t mm = M - m0 < 64 ? M - m0 : 64;
+        const int splits = decode_path(mm, group) ? make_decode_plan(mm, N, K).splits : make_awq_plan(mm, N, K).splits;
+        const size_t need = splits > 1 ? (size_t)splits * mm * N * sizeof(float) : 0;
+        if (need > total) total = need;
+    }
+    return total;
+}
+
+extern "C" int llmq_awq_gemm_tickets(const void* x, int x_dtype, int64_t ldx, const int32_t* qweight, const void* scales,
+                                     const int32_t* qzeros, const void* bias, void* out, int64_t M, int64_t N, int64_t K,
+                                     int64_t group, void* tickets, void* partials, size_t partials_bytes,
+                                     llmq_stream_t stream) {
+    if (x_dtype != LLMQ_BF16 && x_dtype != LLMQ_F16) return LLMQ_ERR_DTYPE;
+    return awq_gemm_entry(x, ldx, qweight, scales, qzeros, bias, out, M, N, K, group, x_dtype == LLMQ_BF16, tickets, partials,
+                          tickets ? partials_bytes : 0, stream);
 }
 
 extern "C" int llmq_awq_dequant(const int32_t* qweight, const void* scales, const int32_t* qzeros, void* out,

@@ -136,6 +136,19 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, double mfma_scale = 1.0, bool fp
     return best;
 }
 
+// The plan of a problem by operand format (0 int8, 1 fp8, 2 fp16; K in bytes).  Searching it takes microseconds of host
+// time and a call needs it for its workspace and for its launch, so each host thread remembers the last plans it made
+// (a pure function of sizes and format; a forced plan is not remembered).
+Plan plan_for(int op, int64_t M, int64_t N, int64_t K) {
+    const double scale = op == 2 ? 2.0 : 1.0;
+    if (g_force_cfg >= 0) return make_plan(M, N, K, scale, op == 1);
+    struct Entry { int64_t M, N, K; int op; Plan plan; };
+    static thread_local Entry cache[64] = {};
+    Entry& e = cache[((uint64_t)(M * 31 + N * 17 + K * 7 + op) * 0x9E3779B97F4A7C15ull) >> 58];
+    if (e.M != M || e.N != N || e.K != K || e.op != op) e = Entry{M, N, K, op, make_plan(M, N, K, scale, op == 1)};
+    return e.plan;
+}
+
 // op: 0 int8, 1 fp8 (a_format picks the A format), 2 fp16 (K, lda, ldb in bytes, i.e. twice the element counts)
 // out_scale (device scalar, may be null): out is fp32 [M, N] holding the out_dtype result after a round trip through
 // e4m3fn on that scale (tile kernel's general epilogue; no few-token kernel, no tail split)
@@ -159,7 +172,7 @@ int gemm_entry(int op, int a_format, const uint8_t* A, int64_t lda, const uint8_
         return launch_gemm_skinny(fp8, a_format == LLMQ_E5M2 ? 1 : 0, sk_t, sk_nw, A, lda, B, ldb, (int)M, (int)N, (int)K, sep,
                                   out, ldo, acc_dump, st);
     }
-    Plan p = make_plan(M, N, K, op == 2 ? 2.0 : 1.0, fp8);
+    Plan p = plan_for(op, M, N, K);
     // fp8 fragments are twice as wide: the 8-wave prefill tile runs ~5 % faster with 128-byte K tiles
     if (fp8 && g_force_cfg < 0 && p.cfg == 1 && p.splits == 1) p.cfg = 6;
     // int8 with direct loads: no staging registers, so the 128-byte K tile fits (half the barriers, whole lines per row)
@@ -255,7 +268,7 @@ extern "C" size_t llmq_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     int sk_t, sk_nw;
     if (skinny_plan(M, N, K, sk_t, sk_nw)) return 0;
-    const Plan p = make_plan(M, N, K), p8 = make_plan(M, N, K, 1.0, true);  // the int8 and the fp8 plan may differ
+    const Plan p = plan_for(0, M, N, K), p8 = plan_for(1, M, N, K);  // the int8 and the fp8 plan may differ
     const int splits = p.splits > p8.splits ? p.splits : p8.splits;
     return splits > 1 ? (size_t)splits * M * N * 4 : 0;
 }
@@ -293,13 +306,13 @@ extern "C" int llmq_gemm_fp8_quantized_output(const uint8_t* A, int a_format, in
 
 extern "C" size_t llmq_gemm_fp8_quantized_output_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
-    const Plan p = make_plan(M, N, K, 1.0, true);
+    const Plan p = plan_for(1, M, N, K);
     return p.splits > 1 ? (size_t)p.splits * M * N * 4 : 0;
 }
 
 extern "C" size_t llmq_gemm_f16_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
-    const Plan p = make_plan(M, N, 2 * K, 2.0);
+    const Plan p = plan_for(2, M, N, 2 * K);
     return p.splits > 1 ? (size_t)p.splits * M * N * 4 : 0;
 }
 

@@ -5,6 +5,7 @@ from __future__ import annotations
 
 import torch
 
+from .._native import host
 from ..awq_kernels import (awq_dequantize_transposed, awq_dequantize_triton, awq_gemm_bf16, awq_gemm_bf16_supported,
                            awq_gemm_triton, gemm_f16)
 from .linear_base import LinearBase
@@ -116,6 +117,13 @@ class WQLinear_GEMM(LinearBase):
         return awq_linear
 
     def forward(self, x):
+        b = self._buffers
+        many = dequant_matmul_token_threshold(self.in_features, self.out_features) if USE_DEQUANT_MATMUL else 1 << 62
+        y = host().awq(x, b["qweight"], b["qzeros"], b["scales"], b["bias"] if "bias" in b else self.bias, self.group_size, many)
+        return self._forward_general(x) if y is None else y
+
+    def _forward_general(self, x):
+        """Inputs outside the native call's layout (strided rows, other dtypes), and its error messages."""
         assert x.device == self.qweight.device, "when awq linear fwd, input and qweight must be same device!"
         assert self.qzeros.device == self.qweight.device, "when awq linear fwd, qzeros and qweight must be same device!"
         assert self.scales.device == self.qweight.device, "when awq linear fwd, scales and qweight must be same device!"
@@ -123,7 +131,7 @@ class WQLinear_GEMM(LinearBase):
         if x.shape[0] == 0:
             return torch.zeros(out_shape, dtype=x.dtype, device=x.device)
         input_dtype = x.dtype
-        tokens = x.numel() // x.shape[-1]
+        tokens = x.numel() // max(x.shape[-1], 1)
         if input_dtype == torch.bfloat16 and awq_gemm_bf16_supported(tokens, self.out_features, self.in_features,
                                                                     self.group_size):
             # a few tokens of a bf16 model: the kernel converts in and out itself

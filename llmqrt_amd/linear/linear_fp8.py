@@ -3,12 +3,14 @@
 Parameter names/shapes/dtypes follow the reference (``weight`` is kept in the model dtype holding
 fp8-representable values, ``weight_scale`` fp32 [1] or [N, 1], ``bias``, static: ``input_scale``,
 ``output_scale``).  Unlike the reference, the fp8 copy of the weight is made once and reused
-until the parameter changes, instead of being re-cast on every forward.
+until the parameter changes, instead of being re-cast on every forward.  ``forward`` hands the tensors to
+one native call; what that call does not take runs through ``_forward_general``, which converts or raises.
 """
 from __future__ import annotations
 
 import torch
 
+from .._native import host
 from ..quantize import (per_tensor_quantize, per_tensor_quantize_with_alpha, per_token_quantize, static_per_tensor_quantize,
                         static_per_tensor_quantize_with_alpha)
 from ..sq_fp8_kernels import (cutlass_f8f8bf16_rowwise_sm89, cutlass_f8f8bf16_tensorwise_sm89,
@@ -43,7 +45,7 @@ class _FP8LinearBase(LinearBase):
 
     def _wscale_flat(self):
         """The per-channel weight scales as a contiguous fp32 [N] vector, made once and kept like the fp8 weight."""
-        s = self.weight_scale
+        s = self._parameters["weight_scale"]
         key = (id(s), s.data_ptr(), s._version, s.device)
         if self._s_cache is None or self._s_cache[0] != key:
             self._s_cache = (key, s.detach().to(torch.float32).reshape(-1).contiguous())
@@ -53,11 +55,19 @@ class _FP8LinearBase(LinearBase):
         """[K, N] column-major fp8 view of the weight.  The cast is made once and kept until the parameter is
         replaced, moved, re-versioned (an in-place op on the Parameter) or a state dict is loaded; a write
         through ``weight.data`` changes none of these and needs an explicit ``invalidate_cache()``."""
-        w = self.weight
+        return self._qweight().t()
+
+    def _qweight(self):
+        """The same as [N, K] rows."""
+        w = self._parameters["weight"]
         key = (id(w), w.data_ptr(), w._version, w.device)
         if self._q_cache is None or self._q_cache[0] != key:
             self._q_cache = (key, w.detach().to(self.qdtype).contiguous())
-        return self._q_cache[1].t()
+        return self._q_cache[1]
+
+    def _bias_param(self):
+        p = self._parameters
+        return p["bias"] if "bias" in p else self.bias
 
     def invalidate_cache(self):
         """Drop the cached fp8 copy of the weight and the flat copy of its scales; the next forward makes them again."""
@@ -97,8 +107,15 @@ class FP8DynamicLinear(_FP8LinearBase):
             lin.bias.data = module.bias.data.to(dtype)
         return lin
 
-    @torch.no_grad()
     def forward(self, x):
+        if self.per_tensor:
+            y = host().fp8_tensor(x, self._qweight(), self._parameters["weight_scale"], self._bias_param(), self.dtype, None, None)
+        else:
+            y = host().fp8_token(x, self._qweight(), self._wscale_flat(), self._bias_param())
+        return self._forward_general(x) if y is None else y
+
+    @torch.no_grad()
+    def _forward_general(self, x):
         assert x.device == self.weight.device, "when fp8 linear fwd, input and qweight must be same device!"
         assert self.weight_scale.device == self.weight.device, "when fp8 linear fwd, scale and qweight must be same device!"
         x_shape = x.shape
@@ -122,11 +139,15 @@ class FP8DynamicLinear(_FP8LinearBase):
                                                    x_scale.view(-1, 1), self.weight_scale.to(torch.float32).t(), True)
         return output.view(*x_shape[:-1], -1)
 
-    @torch.no_grad()
     def forward_quantized(self, qinput, x_scale):
         """Per-channel forward for activations already quantized per token (e4m3fn qinput, fp32 scales
         [.., 1]), e.g. by the fused RMSNorm + quantizer kernel; no counterpart in the reference."""
         assert not self.per_tensor, "pre-quantized activations carry per-token scales"
+        y = host().fp8_prequantized(qinput, x_scale, self._qweight(), self._wscale_flat(), self._bias_param())
+        return self._forward_quantized_general(qinput, x_scale) if y is None else y
+
+    @torch.no_grad()
+    def _forward_quantized_general(self, qinput, x_scale):
         output = cutlass_f8f8bf16_rowwise_sm89(qinput.reshape(-1, qinput.shape[-1]), self._qweight_t(), self.bias,
                                                x_scale.reshape(-1, 1), self.weight_scale.to(torch.float32).t(), True)
         return output.view(*qinput.shape[:-1], -1)
@@ -159,8 +180,17 @@ class FP8StaticLinear(_FP8LinearBase):
             lin.bias.data = module.bias.data.to(dtype)
         return lin
 
-    @torch.no_grad()
     def forward(self, x):
+        if self.per_tensor:
+            p = self._parameters
+            y = host().fp8_tensor(x, self._qweight(), p["weight_scale"], self._bias_param(), self.dtype, p["input_scale"],
+                                  p["output_scale"] if self.quantize_output else None)
+            if y is not None:
+                return y
+        return self._forward_general(x)
+
+    @torch.no_grad()
+    def _forward_general(self, x):
         assert x.device == self.weight.device, "when fp8 linear fwd, input and qweight must be same device!"
         assert self.weight_scale.device == self.weight.device, "when fp8 linear fwd, scale and qweight must be same device!"
         x_shape = x.shape

@@ -3,15 +3,18 @@
 Buffer names, shapes and dtypes match the reference so its checkpoints load unchanged:
 ``qweight`` int8 [N, K], ``bias`` [N] (model dtype), ``weight_scale`` / ``input_scale``.
 The forward pass is two HIP kernels (activation quantizer, int8 MFMA GEMM with fused
-dequant epilogue) and no host synchronisation.
+dequant epilogue) and no host synchronisation.  ``forward`` hands the tensors to one native
+call; what that call does not take (strided rows, mixed devices, other dtypes) runs through
+``_forward_general``, which converts or raises.
 """
 from __future__ import annotations
 
 import torch
 
-from ..quantize import (per_tensor_quantize_with_alpha, quantize_activation_per_tensor_absmax, quantize_weight_per_channel_absmax,
-                        quantize_activation_per_token_absmax,
-                        quantize_activation_per_token_absmax_f32)
+from .._native import host
+from ..quantize import (per_tensor_quantize_with_alpha, quantize_activation_per_tensor_absmax,
+                        quantize_activation_per_token_absmax, quantize_activation_per_token_absmax_f32,
+                        quantize_weight_per_channel_absmax)
 from ..sq_fp8_kernels import (dynamic_linear_max_tokens, w8a8_int8_linear_bbf16_obf16_per_channel,
                               w8a8_int8_linear_bbf16_obf16_per_tensor, w8a8_int8_linear_dynamic_per_token)
 from .linear_base import LinearBase
@@ -61,8 +64,13 @@ class SqW8A8BBF16OBF16PerTensor(LinearBase):
             z = self._zero_bias = torch.zeros(self.out_features, dtype=dtype, device=device)
         return z
 
-    @torch.no_grad()
     def forward(self, x):
+        b = self._buffers
+        y = host().sq_tensor(x, b["qweight"], b["weight_scale"], b["bias"] if "bias" in b else self.bias, b["input_scale"])
+        return self._forward_general(x) if y is None else y
+
+    @torch.no_grad()
+    def _forward_general(self, x):
         assert x.device == self.qweight.device, "when sq linear fwd, input and qweight must be same device!"
         assert self.weight_scale.device == self.qweight.device, "when sq linear fwd, scale and qweight must be same device!"
         assert self.input_scale.device == self.qweight.device, "when sq linear fwd, scale and qweight must be same device!"
@@ -114,8 +122,13 @@ class SqW8A8BBF16OBF16PerChannel(LinearBase):
 
     _bias_or_zeros = SqW8A8BBF16OBF16PerTensor._bias_or_zeros
 
-    @torch.no_grad()
     def forward(self, x):
+        b = self._buffers
+        y = host().sq_token(x, b["qweight"], b["weight_scale"], b["bias"] if "bias" in b else self.bias)
+        return self._forward_general(x) if y is None else y
+
+    @torch.no_grad()
+    def _forward_general(self, x):
         assert x.device == self.qweight.device, "when sq linear fwd, input and qweight must be same device!"
         assert self.weight_scale.device == self.qweight.device, "when sq linear fwd, scale and qweight must be same device!"
         x_shape = x.shape
@@ -130,10 +143,16 @@ class SqW8A8BBF16OBF16PerChannel(LinearBase):
                                                      input_scale, self.weight_scale)
         return y.view(*x_shape[:-1], -1)
 
-    @torch.no_grad()
     def forward_quantized(self, qx, input_scale, out_dtype):
         """Same as forward for activations that are already quantized per token (int8 qx, fp32 scales
         [.., 1]), e.g. by the fused RMSNorm + quantizer kernel; no counterpart in the reference."""
+        b = self._buffers
+        y = host().sq_prequantized(qx, input_scale, b["qweight"], b["weight_scale"], b["bias"] if "bias" in b else self.bias,
+                                   out_dtype)
+        return self._forward_quantized_general(qx, input_scale, out_dtype) if y is None else y
+
+    @torch.no_grad()
+    def _forward_quantized_general(self, qx, input_scale, out_dtype):
         q2 = qx.reshape(-1, qx.shape[-1])
         y = w8a8_int8_linear_bbf16_obf16_per_channel(q2, self.qweight.t(), self._bias_or_zeros(out_dtype, qx.device),
                                                      input_scale.reshape(-1, 1), self.weight_scale)

@@ -11,6 +11,7 @@ import torch
 from torch import nn
 
 from . import _abi
+from ._native import host
 from .quantize import _as_rows
 
 
@@ -83,10 +84,15 @@ class RMSNorm(nn.Module):
         self.variance_epsilon = eps
 
     def forward(self, hidden_states):
-        return rmsnorm(hidden_states, self.weight, self.variance_epsilon)
+        y = host().rmsnorm(hidden_states, self.weight, self.variance_epsilon)
+        return rmsnorm(hidden_states, self.weight, self.variance_epsilon) if y is None else y
 
     def forward_quantized(self, hidden_states, fp8: bool = False, return_normed: bool = False):
         """Normalise and quantize per token in one pass, for a W8A8 / FP8 Linear that accepts (q, scale)."""
+        if not return_normed:
+            out = host().rmsnorm_quant(hidden_states, self.weight, self.variance_epsilon, fp8)
+            if out is not None:
+                return out
         if fp8:
             return rmsnorm_per_token_quantize(hidden_states, self.weight, self.variance_epsilon, return_normed)
         return rmsnorm_quantize_activation_per_token_absmax(hidden_states, self.weight, self.variance_epsilon,

@@ -1,0 +1,89 @@
+"""The native forward passes of the modules (csrc/host_ops.cpp) against the general Python path of the same module."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+K, N = 1024, 544
+
+
+def _modules(dtype, bias):
+    from llmqrt_amd.linear import (FP8DynamicLinear, FP8StaticLinear, SqW8A8BBF16OBF16PerChannel,
+                                   SqW8A8BBF16OBF16PerTensor, WQLinear_GEMM)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    lin = torch.nn.Linear(K, N, bias=bias, device="cuda")
+    lin.weight.data = 0.02 * torch.randn(N, K, device="cuda", generator=g)
+    if bias:
+        lin.bias.data = torch.randn(N, device="cuda", generator=g)
+    mods = {"sq": SqW8A8BBF16OBF16PerTensor.from_linear(lin, 8, 0, False, dtype=dtype),
+            "sq_channel": SqW8A8BBF16OBF16PerChannel.from_linear(lin, 8, 0, False, dtype=dtype),
+            "fp8": FP8DynamicLinear.from_linear(lin, init_only=False, dtype=dtype, per_tensor=True)}
+    for name, quantized in (("static", False), ("static_out", True)):
+        m = FP8StaticLinear.from_linear(lin, init_only=False, dtype=dtype, quantize_output=quantized)
+        m.input_scale.data.fill_(0.15)
+        m.output_scale.data.fill_(0.05)
+        mods[name] = m
+    if dtype == torch.bfloat16:
+        mods["fp8_token"] = FP8DynamicLinear.from_linear(lin, init_only=False, dtype=dtype, per_tensor=False)
+    w = lin.weight.t().reshape(K // 128, 128, N)
+    s = ((w.amax(1) - w.amin(1)) / 15).clamp(min=1e-5).half()
+    z = (-w.amin(1) / s.float()).round().clamp(0, 15)
+    mods["awq"] = WQLinear_GEMM.from_linear(lin, 4, 128, scales=s, zeros=z)
+    return mods
+
+
+# 1 / 4 tokens: one-launch linears; 5: quantizer + few-token kernel; 70: tile kernels; 300: AWQ dequantize + GEMM
+@pytest.mark.parametrize("M", [1, 4, 5, 70, 300])
+@pytest.mark.parametrize("dtype,bias", [(torch.bfloat16, True), (torch.float16, False)])
+def test_native_forward_equals_general_path(cuda, M, dtype, bias):
+    x = torch.randn(M, 1, K, device=cuda, generator=torch.Generator(device="cuda").manual_seed(M)).to(dtype)
+    strided = torch.zeros(M, 1, K + 8, dtype=dtype, device=cuda)
+    strided[..., :K] = x
+    for name, mod in _modules(dtype, bias).items():
+        y, ref = mod(x), mod._forward_general(x)
+        assert y.shape == (M, 1, N) and y.dtype == ref.dtype, name
+        assert torch.equal(y, ref), name
+        assert torch.equal(mod(strided[..., :K]), ref), name  # not contiguous: the general path from forward()
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_native_norm_and_prequantized(cuda, fp8):
+    from llmqrt_amd.norm import RMSNorm, rmsnorm, rmsnorm_per_token_quantize, rmsnorm_quantize_activation_per_token_absmax
+    mods = _modules(torch.bfloat16, True)
+    mod = mods["fp8_token" if fp8 else "sq_channel"]
+    g = torch.Generator(device="cuda").manual_seed(9)
+    x = torch.randn(2, 37, K, device=cuda, generator=g).bfloat16()
+    norm = RMSNorm((1 + 0.1 * torch.randn(K, device=cuda, generator=g)).bfloat16(), 1e-6)
+    assert torch.equal(norm(x), rmsnorm(x, norm.weight, 1e-6))
+    q, s = norm.forward_quantized(x, fp8=fp8)
+    if fp8:
+        q2, s2 = rmsnorm_per_token_quantize(x, norm.weight, 1e-6)
+        y, ref = mod.forward_quantized(q, s), mod._forward_quantized_general(q, s)
+    else:
+        q2, s2 = rmsnorm_quantize_activation_per_token_absmax(x, norm.weight, 1e-6, torch.float32)
+        y, ref = mod.forward_quantized(q, s, x.dtype), mod._forward_quantized_general(q, s, x.dtype)
+    assert torch.equal(q.view(torch.uint8), q2.view(torch.uint8)) and torch.equal(s, s2)
+    assert q.shape == x.shape and s.shape == (2, 37, 1) and y.shape == (2, 37, N) and torch.equal(y, ref)
+
+
+def test_native_awq_counters_by_stream(cuda):
+    """K splits that end in arrival counters: calls overlapping on two streams, and a captured call replayed beside them."""
+    mod = _modules(torch.bfloat16, False)["awq"]
+    g = torch.Generator(device="cuda").manual_seed(3)
+    xs = [torch.randn(4, K, device=cuda, generator=g).bfloat16() for _ in range(2)]
+    refs = [mod._forward_general(x) for x in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = mod(xs[0])
+    outs = [[], []]
+    for _ in range(20):
+        for i, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                outs[i].append(mod(xs[i]))
+        graph.replay()
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(torch.equal(y, refs[i]) for y in outs[i])
+    assert torch.equal(captured, refs[0])
