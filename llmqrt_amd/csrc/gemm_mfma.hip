@@ -53,6 +53,13 @@ bool skinny_plan(int64_t M, int64_t N, int64_t K, int& t, int& nw) {
     // 10.9 against 15.7 / 15.5); a narrow N keeps the lead to 64 tokens with 16 wavefronts along K (o: 11.3 against
     // 13.5 us).  For gate_up (N = 37888) the tile kernel already streams at 5.5 TB/s.
     if (N > 8192) return false;
+    // Short K: more wavefronts along K would own a step or two each and wait for the block's reduction, so four and one
+    // channel tile (4 / 8 / 16 wavefronts, us: 16 x 896 x 896 fp8 4.2 / 5.5 / 5.5, 40 x 896 x 1792 5.7 / 5.6 / 8.7,
+    // 64 x 2048 x 896 4.9 / 6.5 / 6.7, int8 48 x 1152 x 896 4.6 / 5.9 / 9.2; at K = 3584 eight win, 5.3 against 5.8).
+    if (K <= 2048 && N < 4096) {
+        t = 1, nw = 4;
+        return true;
+    }
     if (K >= 8192) {
         if (M > 8) return false;
         t = 1, nw = 8;
@@ -76,9 +83,11 @@ bool skinny_plan(int64_t M, int64_t N, int64_t K, int& t, int& nw) {
 
 // Pick the tile shape and K split with the smallest modelled time:
 // waves of blocks over the CUs x per-block MFMA time, with a floor from the bytes each block streams.
-// mfma_scale: matrix-core time per K byte relative to int8 / fp8 (fp16: 2)
+// The matrix cores take the same time per byte of K for int8, fp8 and fp16 (half the K elements at half the rate), so one
+// table serves all three.  (Priced at twice the time per byte, fp16 was split five ways along K at 777 x 3584 x 18944: 138-140
+// us with 55 MB of partial sums, against 132-136 us for the two-way split picked here.)
 // fp8: the 64-byte K tiles have one MFMA sub-step there and keep the register-staged loop (measured ~20 % slower)
-Plan make_plan(int64_t M, int64_t N, int64_t K, double mfma_scale = 1.0, bool fp8 = false) {
+Plan make_plan(int64_t M, int64_t N, int64_t K, bool fp8 = false) {
     int ocfg, osp;
     if (plan_override(ocfg, osp) && ocfg < 100) {
         const TileShape s = kShapes[ocfg < kNumShapes ? ocfg : kNumShapes - 1];
@@ -98,17 +107,18 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, double mfma_scale = 1.0, bool fp
         {2, 1, 0.60, 12.0},  // 256x128
         {3, 1, 0.27, 8.0},   // 128x128
         {4, 1, 0.17, 7.0},   // 64x128 (0.15 with its operands in the Infinity Cache; 0.17 is what it takes with weights out of HBM)
-        {5, 1, 0.10, 6.0},   // 32x128
+        {5, 1, 0.115, 4.1},  // 32x128: a chain of load latencies, the same however many CUs are busy
         {7, 1, 0.45, 8.0},   // 128x256, 8 waves
     };
     Plan best{1, 1, (int)K};
     double best_t = 1e300;
     for (const Model& md : kModels) {
         const TileShape s = kShapes[md.cfg];
-        // skinny tiles are for small M; the 64-row tile also serves up to 1024 rows when 128x128 tiles
-        // could not even fill the CUs once and K is short (measured: o and qkv at M = 512)
-        if (M > 128 && md.cfg == 5) continue;
-        if (M > 128 && md.cfg == 4 && (M > 1024 || (int64_t)cdiv(M, 128) * cdiv(N, 128) >= 2 * kNumCu)) continue;
+        // small tiles are for small M; the 64-row tile also serves up to 1024 rows when 128x128 tiles
+        // could not even fill the CUs once and K is short (measured: o and qkv at M = 512), and any M whose 64-row
+        // grid fits the chip at once (fp8 2048 x 896 x 4864: 16.7 us against 28.5 with 128x256 tiles)
+        if (M > 128 && md.cfg == 4 && (M > 1024 ? (int64_t)cdiv(M, 64) * cdiv(N, 128) > kNumCu
+                                              : (int64_t)cdiv(M, 128) * cdiv(N, 128) >= 2 * kNumCu)) continue;
         if (md.cfg < 5 && M <= s.bm / 2) continue;            // mostly padding
         // 128x256 tiles are for grids that 256x256 tiles cannot fill twice over (measured: o / down at M = 2048,
         // gate_up at M = 512, qkv at M = 4096: 8-17 % ahead; with more tiles the big tile's lower operand traffic wins)
@@ -120,16 +130,20 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, double mfma_scale = 1.0, bool fp
             const int eff_sp = cdiv(K, kps);
             if (eff_sp != sp) continue;
             const int64_t slots = (int64_t)kNumCu * md.per_cu, blocks = tiles * sp;
+            // past 128 rows the 32-row tile is for grids that fit the chip at once (fp8, us, 64-row tile / 32-row tile:
+            // 200 x 512 x 3584 12.7 / 9.0 with its K split, 256 x 896 x 4864 15.0 / 11.3, 1000 x 896 x 896 7.6 / 5.7);
+            // beyond one round its operand traffic loses (1000 x 896 x 4864 as two splits 19.0 against 14.3 unsplit)
+            if (md.cfg == 5 && M > 128 && blocks > slots) break;
             const int64_t full_rounds = blocks / slots, rest = blocks % slots;
             // fp8: the 64-byte K tiles run the slower register-staged loop; unsplit, config 1 is launched as the
             // 128-byte-tile config 6 (gemm_entry), which does not
-            const double tt = md.t_tile * mfma_scale * (fp8 && s.bk == 64 && !(md.cfg == 1 && sp == 1) ? 1.2 : 1.0);
+            const double tt = md.t_tile * (fp8 && s.bk == 64 && !(md.cfg == 1 && sp == 1) ? 1.2 : 1.0);
             double t = full_rounds * (kps / 64.0 * tt + md.fixed);
-            if (rest) t += kps / 64.0 * tt * (0.52 + 0.48 * (double)rest / slots) + md.fixed;
+            if (rest) t += kps / 64.0 * tt * (md.cfg == 5 ? 1.0 : 0.52 + 0.48 * (double)rest / slots) + md.fixed;
             // two 64-row blocks fit a CU side by side and share its load path: between one and two blocks per CU the
             // launch is one stretched round, not two (measured: 288 blocks of K = 3584 take 20 us, 224 take 14)
             if (md.cfg == 4 && blocks > slots && blocks <= 2 * slots) t = kps / 64.0 * tt * blocks / slots + md.fixed + 3.0;
-            if (sp > 1) t += 5.0 + (double)M * N * sp * 8.0 / 8.0e6;
+            if (sp > 1) t += 3.5 + (double)M * N * sp * 8.0 / 8.0e6;
             if (t < best_t) { best_t = t; best = Plan{md.cfg, sp, kps}; }
         }
     }
@@ -140,12 +154,11 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, double mfma_scale = 1.0, bool fp
 // time and a call needs it for its workspace and for its launch, so each host thread remembers the last plans it made
 // (a pure function of sizes and format; a forced plan is not remembered).
 Plan plan_for(int op, int64_t M, int64_t N, int64_t K) {
-    const double scale = op == 2 ? 2.0 : 1.0;
-    if (g_force_cfg >= 0) return make_plan(M, N, K, scale, op == 1);
+    if (g_force_cfg >= 0) return make_plan(M, N, K, op == 1);
     struct Entry { int64_t M, N, K; int op; Plan plan; };
     static thread_local Entry cache[64] = {};
     Entry& e = cache[((uint64_t)(M * 31 + N * 17 + K * 7 + op) * 0x9E3779B97F4A7C15ull) >> 58];
-    if (e.M != M || e.N != N || e.K != K || e.op != op) e = Entry{M, N, K, op, make_plan(M, N, K, scale, op == 1)};
+    if (e.M != M || e.N != N || e.K != K || e.op != op) e = Entry{M, N, K, op, make_plan(M, N, K, op == 1)};
     return e.plan;
 }
 

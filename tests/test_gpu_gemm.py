@@ -611,3 +611,32 @@ def test_skinny_kernel_is_deterministic_and_ignores_rows_past_m(cuda):
     y2 = w8a8_int8_linear_bbf16_obf16_per_channel(a, qw.to(cuda).t(), bias.to(cuda), sx.to(cuda), sw.to(cuda))
     assert torch.equal(y, y2)
     assert rel_err(y, R.w8a8_epilogue_per_token_per_channel(R.int8_gemm_exact(qx, qw), sx, sw, bias, torch.bfloat16)) <= REL_TOL
+
+
+# Both sides of the planner's lines for small grids: 32-row tiles past 128 rows (one round of blocks, with and without a K
+# split), 64-row tiles past 1024 rows, four wavefronts along a short K up to 64 tokens
+@pytest.mark.parametrize("M,N,K", [(129, 512, 3584), (200, 516, 3584), (256, 896, 4864), (1024, 1024, 896), (1025, 1024, 896),
+                                   (2049, 896, 1152), (1, 896, 2048), (33, 1000, 896), (64, 4088, 2064), (64, 4096, 2048)])
+def test_small_grid_plans(cuda, M, N, K):
+    from llmqrt_amd.sq_fp8_kernels import w8a8_int8_linear_bbf16_obf16_per_channel
+    qx, sx, qw, sw, bias = _int8_problem(M, N, K, 40 + M)
+    acc_ref = R.int8_gemm_exact(qx, qw)
+    dump = torch.empty((M, N), dtype=torch.int32, device=cuda)
+    y = w8a8_int8_linear_bbf16_obf16_per_channel(qx.to(cuda), qw.to(cuda).t(), bias.to(cuda), sx.to(cuda).view(-1, 1),
+                                                 sw.to(cuda).view(1, -1), _acc_dump=dump)
+    assert torch.equal(dump.cpu(), acc_ref)
+    assert rel_err(y, R.w8a8_epilogue_per_token_per_channel(acc_ref, sx, sw, bias, torch.bfloat16)) <= REL_TOL
+
+
+@pytest.mark.parametrize("N", [512, 520, 514])
+def test_split_finish_forms_agree(cuda, force_plan, N):
+    """int8 sums do not depend on the split: the four-channel finish (N % 4 == 0), the element-wise one and the unsplit
+    epilogue give the same bits."""
+    from llmqrt_amd.sq_fp8_kernels import w8a8_int8_linear_bbf16_obf16_per_channel
+    qx, sx, qw, sw, bias = _int8_problem(70, N, 3072, 11)
+    args = (qx.to(cuda), qw.to(cuda).t(), bias.to(cuda), sx.to(cuda).view(-1, 1), sw.to(cuda).view(1, -1))
+    force_plan(5, 1)
+    ref = w8a8_int8_linear_bbf16_obf16_per_channel(*args)
+    for splits in (2, 4, 5, 6):
+        force_plan(5, splits)
+        assert torch.equal(w8a8_int8_linear_bbf16_obf16_per_channel(*args), ref), splits
