@@ -9,7 +9,8 @@
 //
 // Scratch comes from the caching allocator per call (stream-ordered, so safe with any number of threads and streams).
 // The one thing kept between calls is the arrival counters of the few-token AWQ kernel: 512 KiB per device and stream,
-// zeroed once and left zero by every call; calls on one stream run in order, calls on two streams use two sets.
+// zeroed once and left zero by every call; calls on one stream run in order, calls on two streams use two sets, a captured
+// call has a set of its own.
 #include <Python.h>
 
 #include <ATen/core/Tensor.h>
@@ -266,15 +267,19 @@ std::optional<Tensor> fp8_tensor(const Tensor& x, const Tensor& w, const Tensor&
 // ---- AWQ -------------------------------------------------------------------------------------------------------
 class TicketPool {
   public:
-    // The counters of the current stream.  During a capture nothing new is kept: the zero fill would be recorded instead of
-    // executed, so a stream without counters gets a set of the capture's own, zeroed by a node of the graph.
+    static constexpr size_t kMaxSets = 256;  // 128 MiB over all devices; torch's own pool has 32 streams per device
+    // The counters of the current stream.  A capture always gets a set of its own, zeroed by a node of the graph: the graph
+    // may be replayed on any stream, beside eager calls on the stream it was captured on, and after release().  The pool is
+    // bounded; streams past the bound pay for a zero fill per call.
     Tensor get(const at::Device& dev, llmq_stream_t stream) {
+        auto fresh = [&] { return at::zeros({(int64_t)llmq_awq_workspace_ticket_bytes()}, at::TensorOptions().dtype(at::kByte).device(dev)); };
+        if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return fresh();
         const Key key{dev.index(), stream};
         std::lock_guard<std::mutex> lock(mutex_);
         const auto it = pool_.find(key);
         if (it != pool_.end()) return it->second;
-        Tensor t = at::zeros({(int64_t)llmq_awq_workspace_ticket_bytes()}, at::TensorOptions().dtype(at::kByte).device(dev));
-        if (c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None) pool_.emplace(key, t);
+        Tensor t = fresh();
+        if (pool_.size() < kMaxSets) pool_.emplace(key, t);
         return t;
     }
     void release() {

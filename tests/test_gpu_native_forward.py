@@ -87,3 +87,30 @@ def test_native_awq_counters_by_stream(cuda):
     for i in range(2):
         assert all(torch.equal(y, refs[i]) for y in outs[i])
     assert torch.equal(captured, refs[0])
+
+
+def test_captured_awq_call_owns_its_counters(cuda):
+    """A graph captured on a stream that already has counters keeps none of them: they may go, or count for eager calls."""
+    from llmqrt_amd._native import host
+    mod = _modules(torch.bfloat16, False)["awq"]
+    x = torch.randn(4, K, device=cuda, generator=torch.Generator(device="cuda").manual_seed(3)).bfloat16()
+    st, other = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(st):
+        ref = mod(x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        captured = mod(x)
+    outs = []
+    for _ in range(10):
+        with torch.cuda.stream(st):
+            outs.append(mod(x))
+        with torch.cuda.stream(other):
+            graph.replay()
+    torch.cuda.synchronize()
+    host().release_tickets()
+    outs.append(mod(x))
+    with torch.cuda.stream(other):
+        graph.replay()
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, ref) for y in outs) and torch.equal(captured, ref)
