@@ -242,6 +242,13 @@ int llmq_linear_fp8_dynamic(const void* x, int x_dtype, int64_t ldx, const uint8
                             const void* bias, int bias_dtype, void* out, int out_dtype, int64_t ldo, int64_t M, int64_t N,
                             int64_t K, uint8_t* q_dump, float* scale_dump, float* acc_dump, llmq_stream_t stream);
 int llmq_linear_dynamic_max_tokens(int64_t K);
+/* The same with one dynamic scale for the whole tensor: what llmq_quant_per_tensor_alpha followed by llmq_gemm_w8a8
+ * (llmq_gemm_fp8) with that alpha gives.  w_scale: one device scalar.  Up to llmq_linear_per_tensor_max_tokens(K) tokens
+ * (M * K <= 16384); more return LLMQ_ERR_SHAPE. */
+int llmq_linear_per_tensor_dynamic(int fp8, const void* x, int x_dtype, int64_t ldx, const void* B, int64_t ldb,
+                                   const float* w_scale, const void* bias, int bias_dtype, void* out, int out_dtype,
+                                   int64_t ldo, int64_t M, int64_t N, int64_t K, llmq_stream_t stream);
+int llmq_linear_per_tensor_max_tokens(int64_t K);
 /* Tuning / test hook: 0 = two 16-channel tiles per wavefront x 4 wavefronts per block, 1 = one tile x 8 wavefronts,
  * -1 = built-in choice.  Per host thread (thread-local state): it affects only calls made later by the thread that set it. */
 int llmq_linear_dynamic_force_variant(int v);

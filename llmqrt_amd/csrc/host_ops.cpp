@@ -84,6 +84,8 @@ struct Launch {
     explicit Launch(const at::Device& dev) : guard(dev), stream(c10::hip::getCurrentHIPStream(dev.index()).stream()) {}
 };
 
+bool one_launch_tensor(const Rows& r) { return r.M <= llmq_linear_per_tensor_max_tokens(r.K); }
+
 // The weight side of an 8-bit Linear: [N, K] bytes, K % 16 == 0.
 bool weight_ok(const Tensor& w, at::ScalarType dtype, const at::Device& dev, int64_t K) {
     return w.defined() && w.scalar_type() == dtype && w.dim() == 2 && w.size(1) == K && w.size(0) > 0 && K % 16 == 0 &&
@@ -135,6 +137,14 @@ std::optional<Tensor> sq_tensor(const Tensor& x, const Tensor& w, const Tensor& 
         return std::nullopt;
     const at::ScalarType odt = bias ? bias->scalar_type() : x.scalar_type();
     const Launch l(x.device());
+    if (one_launch_tensor(r)) {
+        Tensor out = make(out_size(x, w.size(0)), odt, x.device());
+        check(llmq_linear_per_tensor_dynamic(0, x.data_ptr(), code(x.scalar_type()), r.K, w.data_ptr(), r.K,
+                                             (const float*)w_scale.data_ptr(), ptr(bias), code(odt), out.data_ptr(), code(odt),
+                                             w.size(0), r.M, w.size(0), r.K, l.stream),
+              "llmq_linear_per_tensor_dynamic");
+        return out;
+    }
     // codes, then {scale, alpha}, then the quantizer's partial maxima
     const int64_t codes = round16(r.M * r.K), part = (int64_t)llmq_quant_workspace_bytes();
     Tensor tmp = make({codes + 16 + part}, at::kByte, x.device());
@@ -235,6 +245,14 @@ std::optional<Tensor> fp8_tensor(const Tensor& x, const Tensor& w, const Tensor&
         (output_scale && !scale_ok(*output_scale, x.device(), 1)))
         return std::nullopt;
     const Launch l(x.device());
+    if (!input_scale && !output_scale && one_launch_tensor(r)) {
+        Tensor out = make(out_size(x, N), odt, x.device());
+        check(llmq_linear_per_tensor_dynamic(1, x.data_ptr(), code(x.scalar_type()), r.K, w.data_ptr(), r.K,
+                                             (const float*)w_scale.data_ptr(), ptr(bias), code(odt), out.data_ptr(), code(odt), N,
+                                             r.M, N, r.K, l.stream),
+              "llmq_linear_per_tensor_dynamic");
+        return out;
+    }
     const int64_t codes = round16(r.M * r.K), part = input_scale ? 0 : (int64_t)llmq_quant_workspace_bytes();
     Tensor tmp = make({codes + 16 + part}, at::kByte, x.device());
     uint8_t* p = (uint8_t*)tmp.data_ptr();

@@ -24,6 +24,14 @@
 // the quantizer's load -> reduce -> quantize chain now precedes every block's first MFMA.  What it saves is a launch on
 // the host side.  (Quantizing in the operand registers of every wavefront instead of once per block was measured
 // 40-100 % slower: 15 of 16 MFMA rows repeat the same token's work at one token.)
+//
+// TENSOR: the same with one scale for the whole activation tensor (SqW8A8BBF16OBF16PerTensor, per-tensor
+// FP8DynamicLinear; linear_sq.py:44-54, linear_fp8.py:11-27), for M * K <= 16384.  A block spreads the tensor's 16-byte pieces
+// over all its threads and keeps them in registers from the maximum to the codes: two loads' latency and one block
+// reduction instead of a launch that every GEMM block would wait for.
+// Ahead of the pair at every size tried (us, one launch / two, int8, weights out of HBM): 1 x 3584 x 3584 7.0 / 8.0, 4 x 3584 x
+// 3584 7.7 / 9.0, 16 x 896 x 896 5.4 / 7.6, 1 x 896 x 4864 7.7 / 9.5, 16 x 9728 x 896 9.4 / 9.7, 4 x 37888 x 3584 29.9 / 31.0,
+// 1 x 4096 x 16384 14.7 / 16.3.  The line at 16384 elements is what the block holds in 32 registers a thread.
 #include <algorithm>
 #include <type_traits>
 
@@ -52,17 +60,19 @@ struct FusedArgs {
     int bias_dtype, out_dtype;
 };
 
+constexpr int kTensorChunks = 2048;  // TENSOR: 16-byte pieces of the activation tensor a block holds in registers
 constexpr int kRowPad = 16;        // bytes between LDS rows beyond K: consecutive tokens start 4 banks apart
 constexpr int kMaxLdsBytes = 65536 - 256;
 constexpr int kRowChunks = 10;     // 16-byte pieces of a row a lane keeps in registers (K <= 10 * 64 * 8 = 5120); longer rows are re-read
 
-template <bool FP8, int DT, int T, int NW, int D>
+template <bool FP8, int DT, int T, int NW, int D, bool TENSOR>
 __global__ __launch_bounds__(NW * kWave) void linear_fused_kernel(FusedArgs a) {
     constexpr int MODE = FP8 ? MODE_F8 : MODE_I8;
     constexpr int NT = NW * kWave, KSTEP = FP8 ? 128 : 64, P = FP8 ? 2 : 1, LB = 16 * P;  // LB codes per lane and step
     using acc_t = typename std::conditional<FP8, v4f, v4i>::type;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];  // [M][K + kRowPad] codes; after the main loop: red[NW][T][64]
-    __shared__ float s_scale[16];
+    __shared__ float s_scale[16];  // TENSOR: [0] = activation scale x weight scale
+    __shared__ float s_red[TENSOR ? NW : 1];
 
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -95,11 +105,39 @@ __global__ __launch_bounds__(NW * kWave) void linear_fused_kernel(FusedArgs a) {
     };
 
     Batch ba, bb;
+    // TENSOR: the activations are requested first (loads complete in order: behind the weights they would wait for HBM)
+    constexpr int CH = TENSOR ? kTensorChunks / NT : 1;
+    uint4 act[CH];
+    if constexpr (TENSOR) {
+        const int cpr = K >> 3, total = M * cpr;
+#pragma unroll
+        for (int c = 0; c < CH; c++) {
+            const int i = min(tid + c * NT, total - 1), m = i / cpr;  // past the end: the last piece, which changes no maximum
+            act[c] = reinterpret_cast<const uint4*>(a.x + (int64_t)m * a.ldx)[i - m * cpr];
+        }
+    }
     if (s_begin < s_end) load_batch(s_begin, ba);  // weights start streaming before the activations are quantized
+    if constexpr (TENSOR) {
+        const int cpr = K >> 3, total = M * cpr;
+        float amax = 0.f;
+#pragma unroll
+        for (int c = 0; c < CH; c++) amax = max_nonneg(amax, absmax8(act[c], DT == LLMQ_BF16));
+        amax = block_max<NW>(amax, s_red);
+        const float s = scale_from_amax<DT, MODE>(amax), inv_s = 1.0f / s;
+        if (tid == 0) {
+            const float alpha = s * a.w_scale[0];
+            s_scale[0] = FP8 ? alpha : Lo<DT>::round(alpha);  // int8: rounded to the activation dtype, as store_alpha does
+        }
+#pragma unroll
+        for (int c = 0; c < CH; c++) {
+            const int i = tid + c * NT, m = i / cpr;
+            if (i < total) *reinterpret_cast<uint2*>(smem + m * row_bytes + 8 * (i - m * cpr)) = quant8<DT, MODE, Q_DT>(act[c], s, inv_s);
+        }
+    }
 
     // ---- quantize: wavefront w takes tokens w, w + NW, ...; a lane owns the 16-byte pieces lane, lane + 64, ...
     const int nchunk = K >> 3;
-    for (int m = wave; m < M; m += NW) {
+    for (int m = TENSOR ? M : wave; m < M; m += NW) {
         const uint4* row = reinterpret_cast<const uint4*>(a.x + (int64_t)m * a.ldx);
         uint4 cache[kRowChunks];
         float amax = 0.f;
@@ -196,14 +234,14 @@ __global__ __launch_bounds__(NW * kWave) void linear_fused_kernel(FusedArgs a) {
         // lane l of that accumulator: token l % 16, channels n0 + 16 t + 4 (l / 16) .. + 3
         const int m = l & 15, n = n0 + 16 * t + 4 * (l >> 4);
         if (m >= M || n >= N) continue;
-        const float sa = s_scale[m];
+        const float sa = TENSOR ? 1.f : s_scale[m], alpha = TENSOR ? s_scale[0] : 1.f;
         uint16_t h[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int ne = min(n + e, N - 1);
-            const float sw = a.w_scale ? a.w_scale[ne] : 1.f;
+            const float sw = !TENSOR && a.w_scale ? a.w_scale[ne] : 1.f;
             const float bb2 = a.bias ? load_as_f32(a.bias, a.bias_dtype, ne) : 0.f;
-            const float v = epi_value((float)sum[e], sa, sw, 1.0f, bb2);
+            const float v = epi_value((float)sum[e], sa, sw, alpha, bb2);
             h[e] = a.out_dtype == LLMQ_BF16 ? Lo<LLMQ_BF16>::from_f32(v) : Lo<LLMQ_F16>::from_f32(v);
         }
         uint16_t* orow = reinterpret_cast<uint16_t*>(a.out) + (int64_t)m * a.ldo + n;
@@ -227,28 +265,34 @@ __global__ __launch_bounds__(NW * kWave) void linear_fused_kernel(FusedArgs a) {
 
 thread_local int g_force_fused_variant = -1;  // tuning hook (per host thread): 0 = 2 channel tiles x 4 wavefronts, 1 = 1 x 8
 
-template <bool FP8, int DT>
+template <bool FP8, int DT, bool TENSOR>
 int launch_fused(const FusedArgs& a, hipStream_t st) {
     constexpr int D = FP8 ? 2 : 4;  // steps per batch: ~64 registers per batch
-    // same split as the few-token GEMM: short K and many channels -> wider channel tiles, otherwise more wavefronts along K
-    bool wide = a.K < 8192 && a.N >= 4096;
-    if (g_force_fused_variant >= 0) wide = g_force_fused_variant == 0;
+    // same split as the few-token GEMM (fp32 sums in the same order): short K and many channels -> wider channel tiles,
+    // very short K -> four wavefronts, otherwise more wavefronts along K
+    const bool wide = g_force_fused_variant >= 0 ? g_force_fused_variant == 0 : a.K < 8192 && a.N >= 4096;
+    const bool four = g_force_fused_variant < 0 && a.K <= 2048 && a.N < 4096;
     const size_t lds = std::max<size_t>((size_t)a.M * (a.K + kRowPad), (size_t)8 * 1 * kWave * 16);  // codes, then the reduction
     if (wide) {
-        hipLaunchKernelGGL((linear_fused_kernel<FP8, DT, 2, 4, D>), dim3((a.N + 31) / 32), dim3(4 * kWave), lds, st, a);
+        hipLaunchKernelGGL((linear_fused_kernel<FP8, DT, 2, 4, D, TENSOR>), dim3((a.N + 31) / 32), dim3(4 * kWave), lds, st, a);
+    } else if (four) {
+        hipLaunchKernelGGL((linear_fused_kernel<FP8, DT, 1, 4, D, TENSOR>), dim3((a.N + 15) / 16), dim3(4 * kWave), lds, st, a);
     } else {
-        hipLaunchKernelGGL((linear_fused_kernel<FP8, DT, 1, 8, D>), dim3((a.N + 15) / 16), dim3(8 * kWave), lds, st, a);
+        hipLaunchKernelGGL((linear_fused_kernel<FP8, DT, 1, 8, D, TENSOR>), dim3((a.N + 15) / 16), dim3(8 * kWave), lds, st, a);
     }
     return launch_status();
 }
 
+int64_t tensor_max_tokens(int64_t K) { return K <= 0 ? 0 : std::min<int64_t>(16, kTensorChunks * 8 / K); }
+
 int fused_entry(bool fp8, const void* x, int x_dtype, int64_t ldx, const uint8_t* B, int64_t ldb, const float* w_scale,
                 const void* bias, int bias_dtype, void* out, int out_dtype, int64_t ldo, int64_t M, int64_t N, int64_t K,
-                uint8_t* q_dump, float* scale_dump, void* acc_dump, hipStream_t st) {
+                uint8_t* q_dump, float* scale_dump, void* acc_dump, hipStream_t st, bool tensor = false) {
     if (M < 0 || N < 0 || K < 0) return LLMQ_ERR_SHAPE;
     if (M > 16 || M * (K + kRowPad) > kMaxLdsBytes) return LLMQ_ERR_SHAPE;  // llmq_linear_dynamic_max_tokens(K)
+    if (tensor && M > tensor_max_tokens(K)) return LLMQ_ERR_SHAPE;
     if (M == 0 || N == 0) return LLMQ_OK;
-    if (!x || !B || !out) return LLMQ_ERR_NULL;
+    if (!x || !B || !out || (tensor && !w_scale)) return LLMQ_ERR_NULL;
     if (x_dtype != LLMQ_BF16 && x_dtype != LLMQ_F16) return LLMQ_ERR_DTYPE;
     if (out_dtype != LLMQ_BF16 && out_dtype != LLMQ_F16) return LLMQ_ERR_DTYPE;
     if (bias && bias_dtype != LLMQ_BF16 && bias_dtype != LLMQ_F16 && bias_dtype != LLMQ_F32) return LLMQ_ERR_DTYPE;
@@ -257,8 +301,15 @@ int fused_entry(bool fp8, const void* x, int x_dtype, int64_t ldx, const uint8_t
     if (!aligned16(x) || !aligned16(B) || (q_dump && !aligned16(q_dump))) return LLMQ_ERR_ALIGN;
     const FusedArgs a{(const uint16_t*)x, B, w_scale, bias, out, q_dump, scale_dump, acc_dump, ldx, ldb, ldo,
                       (int)M, (int)N, (int)K, bias_dtype, out_dtype};
-    if (fp8) return x_dtype == LLMQ_BF16 ? launch_fused<true, LLMQ_BF16>(a, st) : launch_fused<true, LLMQ_F16>(a, st);
-    return x_dtype == LLMQ_BF16 ? launch_fused<false, LLMQ_BF16>(a, st) : launch_fused<false, LLMQ_F16>(a, st);
+    auto launch = [&](auto fp8_c, auto dt_c) {
+        constexpr bool F = decltype(fp8_c)::value;
+        constexpr int DT = decltype(dt_c)::value;
+        return tensor ? launch_fused<F, DT, true>(a, st) : launch_fused<F, DT, false>(a, st);
+    };
+    using BF = std::integral_constant<int, LLMQ_BF16>;
+    using HF = std::integral_constant<int, LLMQ_F16>;
+    if (fp8) return x_dtype == LLMQ_BF16 ? launch(std::true_type{}, BF{}) : launch(std::true_type{}, HF{});
+    return x_dtype == LLMQ_BF16 ? launch(std::false_type{}, BF{}) : launch(std::false_type{}, HF{});
 }
 
 }  // namespace
@@ -292,4 +343,13 @@ extern "C" int llmq_linear_fp8_dynamic(const void* x, int x_dtype, int64_t ldx, 
                                        float* acc_dump, llmq_stream_t stream) {
     return fused_entry(true, x, x_dtype, ldx, B, ldb, w_scale, bias, bias_dtype, out, out_dtype, ldo, M, N, K, q_dump,
                        scale_dump, acc_dump, (hipStream_t)stream);
+}
+
+extern "C" int llmq_linear_per_tensor_max_tokens(int64_t K) { return (int)tensor_max_tokens(K); }
+
+extern "C" int llmq_linear_per_tensor_dynamic(int fp8, const void* x, int x_dtype, int64_t ldx, const void* B, int64_t ldb,
+                                              const float* w_scale, const void* bias, int bias_dtype, void* out, int out_dtype,
+                                              int64_t ldo, int64_t M, int64_t N, int64_t K, llmq_stream_t stream) {
+    return fused_entry(fp8 != 0, x, x_dtype, ldx, (const uint8_t*)B, ldb, w_scale, bias, bias_dtype, out, out_dtype, ldo, M, N, K,
+                       nullptr, nullptr, nullptr, (hipStream_t)stream, true);
 }

@@ -122,3 +122,28 @@ def test_modules_take_the_one_launch_path_with_identical_results(cuda, tokens):
     assert torch.equal(part, full[:tokens])   # int32 accumulation is exact, the epilogue arithmetic is shared
     full, part = f8(x), f8(x[:tokens])    # fp32 accumulation: the two kernels add in different orders
     assert ((part.float() - full[:tokens].float()).abs().max() / full.float().abs().max()).item() <= 1e-2
+
+
+# One launch with a tensor-wide scale (M * K <= 16384): one token, the most tokens of a K, rows past the MFMA's 16-byte steps,
+# one channel tile / two / ragged N; one token more runs as quantizer + GEMM.  int8: the same bits as quantizer + GEMM; fp8: fp32
+# sums of the same products, in another order where the GEMM is the tile kernel, then one rounding: a bf16 step is 2^-8.
+@pytest.mark.parametrize("M,N,K", [(1, 3584, 3584), (4, 3584, 3584), (5, 3584, 3584), (16, 896, 896), (16, 1000, 1024), (2, 4104, 8192),
+                                   (1, 520, 16384), (3, 9728, 912), (1, 5000, 2064), (16, 24, 16)])
+@pytest.mark.parametrize("dtype,bias", [(torch.bfloat16, True), (torch.float16, False)])
+def test_per_tensor_one_launch(cuda, M, N, K, dtype, bias):
+    from llmqrt_amd.linear import FP8DynamicLinear, SqW8A8BBF16OBF16PerTensor
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    lin = torch.nn.Linear(K, N, bias=bias, device="cuda")
+    lin.weight.data = 0.02 * torch.randn(N, K, device="cuda", generator=g)
+    x = torch.randn(M, K, device="cuda", generator=g).to(dtype)
+    x[-1, -1] = 50.0  # the largest value in the last piece of the last row
+    sq = SqW8A8BBF16OBF16PerTensor.from_linear(lin, 8, 0, False, dtype=dtype)
+    f8 = FP8DynamicLinear.from_linear(lin, init_only=False, dtype=dtype, per_tensor=True)
+    for v in (x, torch.zeros_like(x)):
+        assert torch.equal(sq(v), sq._forward_general(v))
+        y, ref = f8(v).double(), f8._forward_general(v).double()
+        assert torch.equal(y.isnan(), ref.isnan())  # fp16 zeros: the quantizer's floor is 0 in fp16, and 0 / 0 is NaN either way
+        y, ref = y.nan_to_num(), ref.nan_to_num()
+        assert (y - ref).abs().max() <= 2.0 ** -8 * ref.abs().max()
+    x[0, 3] = float("nan")
+    assert torch.equal(f8(x).isnan(), f8._forward_general(x).isnan())
