@@ -81,6 +81,8 @@ bool skinny_plan(int64_t M, int64_t N, int64_t K, int& t, int& nw) {
     return false;
 }
 
+constexpr size_t kStaticScratchBytes = (size_t)32 << 20;  // the library's own scratch (llmq_gemm_w8a8_static)
+
 // Pick the tile shape and K split with the smallest modelled time:
 // waves of blocks over the CUs x per-block MFMA time, with a floor from the bytes each block streams.
 // The matrix cores take the same time per byte of K for int8, fp8 and fp16 (half the K elements at half the rate), so one
@@ -143,7 +145,9 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, bool fp8 = false) {
             // two 64-row blocks fit a CU side by side and share its load path: between one and two blocks per CU the
             // launch is one stretched round, not two (measured: 288 blocks of K = 3584 take 20 us, 224 take 14)
             if (md.cfg == 4 && blocks > slots && blocks <= 2 * slots) t = kps / 64.0 * tt * blocks / slots + md.fixed + 3.0;
-            if (sp > 1) t += 3.5 + (double)M * N * sp * 8.0 / 8.0e6;
+            // the finishing launch, then the round trip of the partial sums.  Past the library's own scratch a split keeps the
+            // dearer price it was calibrated with, so that llmq_gemm_w8a8_static goes on taking what it took
+            if (sp > 1) t += ((size_t)M * N * sp * 4 > kStaticScratchBytes ? 5.0 : 3.5) + (double)M * N * sp * 8.0 / 8.0e6;
             if (t < best_t) { best_t = t; best = Plan{md.cfg, sp, kps}; }
         }
     }
@@ -224,7 +228,6 @@ int gemm_entry(int op, int a_format, const uint8_t* A, int64_t lda, const uint8_
 
 // ---- scratch owned by the library, for the entry point that takes no workspace ---------------------
 // One copy of this array exists on every GPU the library is loaded on, for the life of the process.
-constexpr size_t kStaticScratchBytes = (size_t)32 << 20;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 // `scratch` is a host-side stand-in for the symbol, not a device address: the address of each GPU's copy
 // is looked up once per device and only that pointer is ever handed to a kernel.

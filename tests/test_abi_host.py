@@ -175,3 +175,11 @@ def test_bench_refuses_more_than_one_gpu():
     r = subprocess.run([sys.executable, str(root / "bench.py"), "--gpus", "2"], capture_output=True, text=True, timeout=300)
     assert r.returncode != 0
     assert "one GPU" in r.stderr and r.stdout.strip() == ""
+
+
+@pytest.mark.parametrize("M,N,K", [(2313, 1824, 18288), (410, 21624, 18512), (509, 8528, 16832), (6162, 1440, 18320), (1230, 8088, 19872)])
+def test_plans_fit_the_static_scratch(M, N, K):
+    """Problems near the line between one pass and a K split, which llmq_gemm_w8a8_static takes in one pass."""
+    from llmqrt_amd import _abi
+    L = _abi.lib()
+    assert L.llmq_gemm_workspace_bytes(M, N, K) <= L.llmq_gemm_static_scratch_bytes()
