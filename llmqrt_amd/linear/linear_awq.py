@@ -119,11 +119,13 @@ class WQLinear_GEMM(LinearBase):
     def forward(self, x):
         b = self._buffers
         many = dequant_matmul_token_threshold(self.in_features, self.out_features) if USE_DEQUANT_MATMUL else 1 << 62
-        y = host().awq(x, b["qweight"], b["qzeros"], b["scales"], b["bias"] if "bias" in b else self.bias, self.group_size, many)
+        y = host().awq(x, b.get("qweight"), b.get("qzeros"), b.get("scales"), b["bias"] if "bias" in b else self.bias,
+                       self.group_size, many)
         return self._forward_general(x) if y is None else y
 
     def _forward_general(self, x):
-        """Inputs outside the native call's layout (strided rows, other dtypes), and its error messages."""
+        """Inputs outside the native call's layout (strided rows, other dtypes), tensors that are not registered buffers
+        (a DataParallel replica's, a parametrization's), and the error messages."""
         assert x.device == self.qweight.device, "when awq linear fwd, input and qweight must be same device!"
         assert self.qzeros.device == self.qweight.device, "when awq linear fwd, qzeros and qweight must be same device!"
         assert self.scales.device == self.qweight.device, "when awq linear fwd, scales and qweight must be same device!"

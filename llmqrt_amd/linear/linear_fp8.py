@@ -4,7 +4,8 @@ Parameter names/shapes/dtypes follow the reference (``weight`` is kept in the mo
 fp8-representable values, ``weight_scale`` fp32 [1] or [N, 1], ``bias``, static: ``input_scale``,
 ``output_scale``).  Unlike the reference, the fp8 copy of the weight is made once and reused
 until the parameter changes, instead of being re-cast on every forward.  ``forward`` hands the tensors to
-one native call; what that call does not take runs through ``_forward_general``, which converts or raises.
+one native call; what that call does not take, or tensors that are not registered parameters (a DataParallel
+replica's, a parametrization's), run through ``_forward_general``, which reads the attributes and converts or raises.
 """
 from __future__ import annotations
 
@@ -45,7 +46,9 @@ class _FP8LinearBase(LinearBase):
 
     def _wscale_flat(self):
         """The per-channel weight scales as a contiguous fp32 [N] vector, made once and kept like the fp8 weight."""
-        s = self._parameters["weight_scale"]
+        s = self._parameters.get("weight_scale")
+        if s is None:  # not a registered parameter: a DataParallel replica's attribute, a parametrization's property
+            s = self.weight_scale
         key = (id(s), s.data_ptr(), s._version, s.device)
         if self._s_cache is None or self._s_cache[0] != key:
             self._s_cache = (key, s.detach().to(torch.float32).reshape(-1).contiguous())
@@ -59,7 +62,9 @@ class _FP8LinearBase(LinearBase):
 
     def _qweight(self):
         """The same as [N, K] rows."""
-        w = self._parameters["weight"]
+        w = self._parameters.get("weight")
+        if w is None:
+            w = self.weight
         key = (id(w), w.data_ptr(), w._version, w.device)
         if self._q_cache is None or self._q_cache[0] != key:
             self._q_cache = (key, w.detach().to(self.qdtype).contiguous())
@@ -109,7 +114,8 @@ class FP8DynamicLinear(_FP8LinearBase):
 
     def forward(self, x):
         if self.per_tensor:
-            y = host().fp8_tensor(x, self._qweight(), self._parameters["weight_scale"], self._bias_param(), self.dtype, None, None)
+            y = host().fp8_tensor(x, self._qweight(), self._parameters.get("weight_scale"), self._bias_param(), self.dtype,
+                                  None, None)
         else:
             y = host().fp8_token(x, self._qweight(), self._wscale_flat(), self._bias_param())
         return self._forward_general(x) if y is None else y
@@ -181,9 +187,9 @@ class FP8StaticLinear(_FP8LinearBase):
         return lin
 
     def forward(self, x):
-        if self.per_tensor:
-            p = self._parameters
-            y = host().fp8_tensor(x, self._qweight(), p["weight_scale"], self._bias_param(), self.dtype, p["input_scale"],
+        p = self._parameters
+        if self.per_tensor and "input_scale" in p and "output_scale" in p:
+            y = host().fp8_tensor(x, self._qweight(), p.get("weight_scale"), self._bias_param(), self.dtype, p["input_scale"],
                                   p["output_scale"] if self.quantize_output else None)
             if y is not None:
                 return y

@@ -4,8 +4,9 @@ Buffer names, shapes and dtypes match the reference so its checkpoints load unch
 ``qweight`` int8 [N, K], ``bias`` [N] (model dtype), ``weight_scale`` / ``input_scale``.
 The forward pass is two HIP kernels (activation quantizer, int8 MFMA GEMM with fused
 dequant epilogue) and no host synchronisation.  ``forward`` hands the tensors to one native
-call; what that call does not take (strided rows, mixed devices, other dtypes) runs through
-``_forward_general``, which converts or raises.
+call; what that call does not take (strided rows, mixed devices, other dtypes, tensors that are not
+registered buffers, as in a DataParallel replica or under a parametrization) runs through
+``_forward_general``, which reads the attributes and converts or raises.
 """
 from __future__ import annotations
 
@@ -65,8 +66,9 @@ class SqW8A8BBF16OBF16PerTensor(LinearBase):
         return z
 
     def forward(self, x):
-        b = self._buffers
-        y = host().sq_tensor(x, b["qweight"], b["weight_scale"], b["bias"] if "bias" in b else self.bias, b["input_scale"])
+        b = self._buffers  # a tensor that is not a registered buffer gives None, which the native call refuses
+        y = host().sq_tensor(x, b.get("qweight"), b.get("weight_scale"), b["bias"] if "bias" in b else self.bias,
+                             b.get("input_scale"))
         return self._forward_general(x) if y is None else y
 
     @torch.no_grad()
@@ -124,7 +126,7 @@ class SqW8A8BBF16OBF16PerChannel(LinearBase):
 
     def forward(self, x):
         b = self._buffers
-        y = host().sq_token(x, b["qweight"], b["weight_scale"], b["bias"] if "bias" in b else self.bias)
+        y = host().sq_token(x, b.get("qweight"), b.get("weight_scale"), b["bias"] if "bias" in b else self.bias)
         return self._forward_general(x) if y is None else y
 
     @torch.no_grad()
@@ -147,8 +149,8 @@ class SqW8A8BBF16OBF16PerChannel(LinearBase):
         """Same as forward for activations that are already quantized per token (int8 qx, fp32 scales
         [.., 1]), e.g. by the fused RMSNorm + quantizer kernel; no counterpart in the reference."""
         b = self._buffers
-        y = host().sq_prequantized(qx, input_scale, b["qweight"], b["weight_scale"], b["bias"] if "bias" in b else self.bias,
-                                   out_dtype)
+        y = host().sq_prequantized(qx, input_scale, b.get("qweight"), b.get("weight_scale"),
+                                   b["bias"] if "bias" in b else self.bias, out_dtype)
         return self._forward_quantized_general(qx, input_scale, out_dtype) if y is None else y
 
     @torch.no_grad()

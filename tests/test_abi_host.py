@@ -183,3 +183,51 @@ def test_plans_fit_the_static_scratch(M, N, K):
     from llmqrt_amd import _abi
     L = _abi.lib()
     assert L.llmq_gemm_workspace_bytes(M, N, K) <= L.llmq_gemm_static_scratch_bytes()
+
+
+def _moved_tensors(mod, how):
+    """The module's tensors where nn.Module's dictionaries do not hold them under their names."""
+    if how == "replica":  # as torch.nn.parallel.replicate leaves a module: parameters are plain attributes
+        rep = mod._replicate_for_data_parallel()
+        for name, p in mod._parameters.items():
+            if p is not None:
+                setattr(rep, name, p.detach())
+        return rep
+    if how == "attributes":
+        for store in (mod._parameters, mod._buffers):
+            for name in [n for n, t in store.items() if t is not None]:
+                t = store.pop(name)
+                object.__setattr__(mod, name, t.detach())
+        return mod
+    for store in (mod._parameters, mod._buffers):
+        for name in [n for n, t in store.items() if t is not None and t.is_floating_point()]:
+            if store is mod._buffers:
+                mod.register_parameter(name, torch.nn.Parameter(store.pop(name), requires_grad=False))
+            torch.nn.utils.parametrize.register_parametrization(mod, name, torch.nn.Identity())
+    return mod
+
+
+def _all_modules():
+    from llmqrt_amd.linear import (FP8DynamicLinear, FP8StaticLinear, SqW8A8BBF16OBF16PerChannel,
+                                   SqW8A8BBF16OBF16PerTensor, WQLinear_GEMM)
+    lin = torch.nn.Linear(128, 64, bias=True)
+    return {"sq": SqW8A8BBF16OBF16PerTensor.from_linear(lin, 8, 0, True), "sq_channel": SqW8A8BBF16OBF16PerChannel.from_linear(lin, 8, 0, True),
+            "fp8": FP8DynamicLinear.from_linear(lin), "fp8_token": FP8DynamicLinear.from_linear(lin, per_tensor=False),
+            "static": FP8StaticLinear.from_linear(lin), "static_out": FP8StaticLinear.from_linear(lin, quantize_output=True),
+            "awq": WQLinear_GEMM.from_linear(lin, 4, 64, True)}
+
+
+@pytest.mark.parametrize("how", ["replica", "attributes", "parametrized"])
+def test_forward_takes_tensors_that_are_not_registered(how):
+    """The general path, which reads the attributes, takes such a module; off the GPU it says so instead of a KeyError."""
+    x = torch.zeros(2, 128, dtype=torch.bfloat16)
+    for name, mod in _all_modules().items():
+        mod = _moved_tensors(mod, how)
+        with pytest.raises((RuntimeError, AssertionError)):
+            mod(x)
+        if name == "sq_channel":
+            with pytest.raises(RuntimeError, match="GPU"):
+                mod.forward_quantized(x.to(torch.int8), torch.ones(2, 1), torch.bfloat16)
+        if name == "fp8_token":
+            with pytest.raises(RuntimeError, match="GPU"):
+                mod.forward_quantized(x.to(torch.float8_e4m3fn), torch.ones(2, 1))

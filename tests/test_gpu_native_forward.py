@@ -114,3 +114,13 @@ def test_captured_awq_call_owns_its_counters(cuda):
         graph.replay()
     torch.cuda.synchronize()
     assert all(torch.equal(y, ref) for y in outs) and torch.equal(captured, ref)
+
+
+def test_replica_forward_equals_module(cuda):
+    """A DataParallel replica: its parameters are plain attributes, so the general path serves the fp8 modules."""
+    x = torch.randn(5, K, device=cuda, generator=torch.Generator(device="cuda").manual_seed(1)).bfloat16()
+    for name, mod in _modules(torch.bfloat16, True).items():
+        rep = mod._replicate_for_data_parallel()
+        for key, p in mod._parameters.items():
+            setattr(rep, key, p.detach())
+        assert torch.equal(rep(x), mod._forward_general(x)), name
