@@ -26,6 +26,12 @@ __all__ = ["FP8DynamicLinear", "FP8StaticLinear", "per_tensor_quantize", "per_to
 dtype_to_str = {torch.bfloat16: "bfloat16", torch.float16: "float16"}
 
 
+def _made_from(cache, t):
+    """Whether ``cache`` = (source, copy, address, version) was made from ``t`` as it is.  The source itself is kept, so that
+    no later tensor can take its place in memory and pass for it."""
+    return cache is not None and cache[0] is t and cache[2] == t.data_ptr() and cache[3] == t._version
+
+
 class _FP8LinearBase(LinearBase):
     def _init_common(self, in_features, out_features, bias, dev, dtype, qdtype, per_channel_scale):
         self.dtype = dtype
@@ -49,9 +55,8 @@ class _FP8LinearBase(LinearBase):
         s = self._parameters.get("weight_scale")
         if s is None:  # not a registered parameter: a DataParallel replica's attribute, a parametrization's property
             s = self.weight_scale
-        key = (id(s), s.data_ptr(), s._version, s.device)
-        if self._s_cache is None or self._s_cache[0] != key:
-            self._s_cache = (key, s.detach().to(torch.float32).reshape(-1).contiguous())
+        if not _made_from(self._s_cache, s):
+            self._s_cache = (s, s.detach().to(torch.float32).reshape(-1).contiguous(), s.data_ptr(), s._version)
         return self._s_cache[1]
 
     def _qweight_t(self):
@@ -65,9 +70,8 @@ class _FP8LinearBase(LinearBase):
         w = self._parameters.get("weight")
         if w is None:
             w = self.weight
-        key = (id(w), w.data_ptr(), w._version, w.device)
-        if self._q_cache is None or self._q_cache[0] != key:
-            self._q_cache = (key, w.detach().to(self.qdtype).contiguous())
+        if not _made_from(self._q_cache, w):
+            self._q_cache = (w, w.detach().to(self.qdtype).contiguous(), w.data_ptr(), w._version)
         return self._q_cache[1]
 
     def _bias_param(self):

@@ -231,3 +231,22 @@ def test_forward_takes_tensors_that_are_not_registered(how):
         if name == "fp8_token":
             with pytest.raises(RuntimeError, match="GPU"):
                 mod.forward_quantized(x.to(torch.float8_e4m3fn), torch.ones(2, 1))
+
+
+def test_fp8_copies_follow_a_parametrized_tensor():
+    """A parametrization makes a new tensor on each access, often at the address of the one before: the fp8 copy of the
+    weight and the flat scales must come from the tensor of this access."""
+    class Double(torch.nn.Module):
+        def forward(self, t):
+            return t * 2
+
+    mod = _all_modules()["fp8_token"]
+    for name in ("weight", "weight_scale"):
+        torch.nn.utils.parametrize.register_parametrization(mod, name, Double())
+    values = [(torch.full((64, 128), float(i)), torch.full((64, 1), 0.5 * i)) for i in range(1, 5)]
+    with torch.no_grad():
+        for w, s in values:
+            mod.parametrizations.weight.original.copy_(w)
+            mod.parametrizations.weight_scale.original.copy_(s)
+            q, flat = mod._qweight(), mod._wscale_flat()
+            assert torch.equal(q.float(), 2 * w) and torch.equal(flat, 2 * s.reshape(-1))
