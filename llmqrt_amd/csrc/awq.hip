@@ -779,8 +779,13 @@ extern "C" int llmq_awq_force_plan(int v, int splits, int k_waves) {
     return LLMQ_OK;
 }
 
+// No problem that llmq_awq_gemm takes has fewer than 8 channels or 32 rows of weights; the plans divide by counts of both.
+static bool awq_sizes_ok(int64_t M, int64_t N, int64_t K) {
+    return M > 0 && N >= 8 && K >= 32 && M <= 0x7fffffffLL && N <= 0x7fffffffLL && K <= 0x7fffffffLL;
+}
+
 extern "C" size_t llmq_awq_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    if (!awq_sizes_ok(M, N, K)) return 0;
     size_t total = 0;
     if (tile_path(M)) {
         const AwqTilePlan t = tile_plan(M, N, K);
@@ -927,7 +932,7 @@ extern "C" int llmq_awq_gemm_bf16(const void* x, int64_t ldx, const int32_t* qwe
 }
 
 extern "C" size_t llmq_awq_gemm_partials_bytes(int64_t M, int64_t N, int64_t K, int64_t group) {
-    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    if (!awq_sizes_ok(M, N, K)) return 0;
     if (tile_path(M)) {
         const AwqTilePlan t = tile_plan(M, N, K);
         return t.splits > 1 ? (size_t)t.splits * M * N * sizeof(float) : 0;

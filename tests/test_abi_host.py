@@ -250,3 +250,16 @@ def test_fp8_copies_follow_a_parametrized_tensor():
             mod.parametrizations.weight_scale.original.copy_(s)
             q, flat = mod._qweight(), mod._wscale_flat()
             assert torch.equal(q.float(), 2 * w) and torch.equal(flat, 2 * s.reshape(-1))
+
+
+def test_awq_size_queries_answer_for_any_sizes():
+    """In a child process: a division by a plan's zero tile count would end the whole process, not raise."""
+    import subprocess
+    import sys
+    code = ("import itertools; from llmqrt_amd import _abi; L = _abi.lib(); v = (-1, 0, 1, 7, 8, 16, 31, 32, 33, 64, 65, 128, 300)\n"
+            "for m, n, k in itertools.product(v, v, v):\n"
+            "    L.llmq_awq_gemm_workspace_bytes(m, n, k)\n"
+            "    for g in (-1, 0, 8, 32, 128): L.llmq_awq_gemm_partials_bytes(m, n, k, g)\n"
+            "assert L.llmq_awq_gemm_workspace_bytes(1, 4608, 3584) > L.llmq_awq_gemm_partials_bytes(1, 4608, 3584, 128) > 0")
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
