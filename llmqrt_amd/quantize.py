@@ -147,6 +147,8 @@ def _alpha_operands(t: torch.Tensor, w_scale: torch.Tensor):
     x = _as_rows(t)
     M, K = x.shape
     ws = w_scale.detach()
+    if ws.device != x.device or ws.numel() == 0:
+        raise RuntimeError("the weight scale must be a one-element tensor on the device of the activations")
     return (x, M, K, x.stride(0) if M > 1 else K, ws if ws.dtype == torch.float32 else ws.float(),
             torch.empty(2, dtype=torch.float32, device=x.device))
 
@@ -155,7 +157,11 @@ def _alpha_operands(t: torch.Tensor, w_scale: torch.Tensor):
 def per_tensor_quantize_with_alpha(t: torch.Tensor, w_scale: torch.Tensor, fp8: bool):
     """quantize_activation_per_tensor_absmax (int8) or per_tensor_quantize (fp8), and the factor scale * w_scale of the
     GEMM that follows, formed by the quantizer's own kernel: -> (codes like t, alpha as a 0-dim fp32 tensor).  For int8
-    the product is rounded to t's dtype (linear_sq.py:127)."""
+    the product is rounded to t's dtype (linear_sq.py:127).  A w_scale in another dtype than fp32 (a module cast to 16 bits)
+    makes fp8's product one of that dtype, as torch's promotion does (linear_fp8.py:199-221)."""
+    if fp8 and w_scale.dtype != torch.float32:
+        q, s = per_tensor_quantize(t)
+        return q, (w_scale * s).reshape(-1)[0].float()
     x, M, K, ldx, ws, s = _alpha_operands(t, w_scale)
     q = torch.empty((M, K), dtype=torch.float8_e4m3fn if fp8 else torch.int8, device=x.device)
     scratch = _abi.workspaces.get(x.device, _abi.lib().llmq_quant_workspace_bytes())
@@ -167,14 +173,16 @@ def per_tensor_quantize_with_alpha(t: torch.Tensor, w_scale: torch.Tensor, fp8: 
 
 @torch.no_grad()
 def static_per_tensor_quantize_with_alpha(t: torch.Tensor, scale: torch.Tensor, w_scale: torch.Tensor):
-    """static_per_tensor_quantize on a one-element fp32 GPU tensor, and scale * w_scale: -> (codes like t, alpha)."""
+    """static_per_tensor_quantize, and scale * w_scale in torch's promoted dtype: -> (codes like t, alpha as a 0-dim fp32
+    tensor).  One kernel for fp32 scales on t's device."""
+    if scale.dtype != torch.float32 or w_scale.dtype != torch.float32 or scale.device != t.device:
+        return static_per_tensor_quantize(t, scale), (w_scale * scale).reshape(-1)[0].float()
     x, M, K, ldx, ws, s = _alpha_operands(t, w_scale)
-    sdev = scale.detach().reshape(-1)[:1].to(device=x.device, dtype=torch.float32)
+    sdev = scale.detach().reshape(-1)[:1]
     q = torch.empty((M, K), dtype=torch.float8_e4m3fn, device=x.device)
     _abi.check(_abi.lib().llmq_quant_fp8_static_alpha(
         x.data_ptr(), _abi.dtype_code(x.dtype), M, K, ldx, q.data_ptr(), sdev.data_ptr(),
-        int(scale.dim() > 0 and scale.dtype == torch.float32), ws.data_ptr(), s.data_ptr(), _abi.stream_of(x)),
-        "llmq_quant_fp8_static_alpha")
+        int(scale.dim() > 0), ws.data_ptr(), s.data_ptr(), _abi.stream_of(x)), "llmq_quant_fp8_static_alpha")
     return q.view(t.shape), s[0]
 
 

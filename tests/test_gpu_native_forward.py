@@ -124,3 +124,35 @@ def test_replica_forward_equals_module(cuda):
         for key, p in mod._parameters.items():
             setattr(rep, key, p.detach())
         assert torch.equal(rep(x), mod._forward_general(x)), name
+
+
+@pytest.mark.parametrize("M", [3, 70])
+@pytest.mark.parametrize("cast", [torch.bfloat16, torch.float16])
+def test_fp8_modules_cast_to_16_bits(cuda, M, cast):
+    """module.to(16-bit dtype) casts the scales too: activation scale x weight scale is then torch's product of the two."""
+    from llmqrt_amd.quantize import per_tensor_quantize, static_per_tensor_quantize
+    from llmqrt_amd.sq_fp8_kernels import cutlass_f8f8bf16_tensorwise_sm89
+    x = torch.randn(M, K, device=cuda, generator=torch.Generator(device="cuda").manual_seed(M)).to(cast)
+    mods = _modules(cast, True)
+    for name in ("fp8", "static"):
+        mod = mods[name].to(cast)
+        assert mod.weight_scale.dtype == cast
+        if name == "fp8":
+            q, s = per_tensor_quantize(x)
+        else:
+            q, s = static_per_tensor_quantize(x, mod.input_scale), mod.input_scale
+        ref = cutlass_f8f8bf16_tensorwise_sm89(q, mod._qweight_t(), mod.bias, mod.weight_scale * s, 1.0,
+                                               "bfloat16" if cast == torch.bfloat16 else "float16")
+        assert torch.equal(mod(x), ref), name
+
+
+def test_static_input_scale_off_the_gpu_is_refused(cuda):
+    """A one-dimensional host scale: torch refuses the product with the weight's scale, and so does the module."""
+    mod = _modules(torch.bfloat16, True)["static"]
+    mod.input_scale.data = mod.input_scale.data.cpu()
+    x = torch.randn(3, K, device=cuda).bfloat16()
+    with pytest.raises(RuntimeError):
+        mod(x)
+    from llmqrt_amd.quantize import per_tensor_quantize_with_alpha
+    with pytest.raises(RuntimeError, match="weight scale"):
+        per_tensor_quantize_with_alpha(x, torch.ones(1), True)
