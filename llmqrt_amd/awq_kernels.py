@@ -22,6 +22,15 @@ def _check_layout(qweight, scales, zeros, K, N, group_size):
     assert group_size in AWQ_TRITON_SUPPORTED_GROUP_SIZES or group_size == K
 
 
+def _bias_vector(bias, N, device):
+    """The bias as the kernels read it: N values in a row on the operands' device."""
+    if bias is None:
+        return None
+    if bias.device != device or bias.numel() != N:
+        raise RuntimeError(f"bias must hold {N} values on {device}, got {list(bias.shape)} on {bias.device}")
+    return bias.reshape(-1).contiguous()
+
+
 @torch.no_grad()
 def awq_dequantize_triton(qweight: torch.Tensor, scales: torch.Tensor, zeros: torch.Tensor,
                           block_size_x: int = 32, block_size_y: int = 32) -> torch.Tensor:
@@ -67,6 +76,7 @@ def gemm_f16(x: torch.Tensor, w_nk: torch.Tensor, bias: torch.Tensor | None = No
         x = x.contiguous()
     if w_nk.stride(1) != 1 or w_nk.stride(0) % 8 or w_nk.data_ptr() % 16:
         w_nk = w_nk.contiguous()
+    bias = _bias_vector(bias, N, x.device)
     out = torch.empty((M, N), dtype=torch.float16, device=x.device)
     if M == 0 or N == 0:
         return out
@@ -113,6 +123,9 @@ def _awq_gemm(input, qweight, scales, qzeros, split_k_iters, bias):
     x = input
     if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:
         x = x.contiguous()
+    bias = _bias_vector(bias, N, x.device)
+    if bias is not None:
+        bias = bias.to(torch.float16)  # what the kernels read
     result = torch.empty((M, N), dtype=input.dtype, device=input.device)
     L = _abi.lib()
     ws = _abi.awq_workspaces.get(x.device, L.llmq_awq_gemm_workspace_bytes(M, N, K))

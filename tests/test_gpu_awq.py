@@ -540,3 +540,22 @@ def test_bf16_activations_equal_separate_conversions(cuda, M, K, N, with_bias):
         mod.bias.copy_(bias)
     y = mod(x.view(M, 1, K))
     assert y.dtype == torch.bfloat16 and torch.equal(y.view(M, N), ref)
+
+
+def test_bias_is_checked_and_converted(cuda):
+    """The kernels read N fp16 values on the GPU: another dtype is converted, a host or short bias is refused."""
+    from llmqrt_amd import workloads as W
+    from llmqrt_amd.awq_kernels import awq_dequantize_transposed, awq_gemm_bf16, awq_gemm_triton, gemm_f16
+    N, K = 64, 256
+    qw, qz, s = (t.to(cuda) for t in W.awq_weights(N, K, 3))
+    x = W.activations(4, K, 5, dtype=torch.float16).to(cuda)
+    bias = torch.arange(N, device=cuda, dtype=torch.float16) / 8
+    ref = awq_gemm_triton(x, qw, s, qz, 8, bias=bias)
+    for b in (bias.float(), bias.bfloat16(), bias.view(1, N), bias.repeat_interleave(2)[::2]):
+        assert torch.equal(awq_gemm_triton(x, qw, s, qz, 8, bias=b), ref)
+    w = awq_dequantize_transposed(qw, s, qz)
+    for b in (bias.cpu(), bias[:-1]):
+        for call in (lambda: awq_gemm_triton(x, qw, s, qz, 8, bias=b), lambda: gemm_f16(x, w, b),
+                     lambda: awq_gemm_bf16(x.bfloat16(), qw, s, qz, b)):
+            with pytest.raises(RuntimeError, match="bias"):
+                call()
