@@ -36,9 +36,6 @@ namespace {
 
 using at::Tensor;
 
-// As many tokens as the one-launch linear serves no slower than quantizer + GEMM (measured on the 7B projections).
-constexpr int64_t kOneLaunchTokens = 4, kOneLaunchMaxK = 8192;
-
 void check(int status, const char* what) {
     if (status != LLMQ_OK)
         throw std::runtime_error(std::string(what) + ": " + llmq_status_string(status) + " (llmq status " +
@@ -158,7 +155,15 @@ std::optional<Tensor> sq_tensor(const Tensor& x, const Tensor& w, const Tensor& 
     return out;
 }
 
-std::optional<Tensor> sq_token(const Tensor& x, const Tensor& w, const Tensor& w_scale, const std::optional<Tensor>& bias) {
+// The line between the one-launch linear and quantizer + GEMM for per-token scales comes from the module: up to `tokens` rows
+// of fewer than `k` elements.
+struct OneLaunch {
+    int64_t tokens, k;
+    bool takes(const Rows& r) const { return r.M <= tokens && r.K < k && r.M <= llmq_linear_dynamic_max_tokens(r.K); }
+};
+
+std::optional<Tensor> sq_token(const Tensor& x, const Tensor& w, const Tensor& w_scale, const std::optional<Tensor>& bias,
+                               const OneLaunch& line) {
     const Rows r = rows_of(x);
     if (!r.ok || !is16(x.scalar_type()) || !weight_ok(w, at::kChar, x.device(), r.K)) return std::nullopt;
     const int64_t N = w.size(0);
@@ -168,7 +173,7 @@ std::optional<Tensor> sq_token(const Tensor& x, const Tensor& w, const Tensor& w
     const Launch l(x.device());
     const float* ws = (const float*)w_scale.data_ptr();
     Tensor out = make(out_size(x, N), odt, x.device());
-    if (r.M <= kOneLaunchTokens && r.K < kOneLaunchMaxK && r.M <= llmq_linear_dynamic_max_tokens(r.K)) {
+    if (line.takes(r)) {
         check(llmq_linear_i8_dynamic(x.data_ptr(), code(x.scalar_type()), r.K, (const int8_t*)w.data_ptr(), r.K, ws, ptr(bias),
                                      code(odt), out.data_ptr(), code(odt), N, r.M, N, r.K, nullptr, nullptr, nullptr, l.stream),
               "llmq_linear_i8_dynamic");
@@ -206,7 +211,8 @@ std::optional<Tensor> prequantized(bool fp8, const Tensor& q, const Tensor& a_sc
 }
 
 // ---- FP8 (e4m3fn) ----------------------------------------------------------------------------------------------
-std::optional<Tensor> fp8_token(const Tensor& x, const Tensor& w, const Tensor& w_scale, const std::optional<Tensor>& bias) {
+std::optional<Tensor> fp8_token(const Tensor& x, const Tensor& w, const Tensor& w_scale, const std::optional<Tensor>& bias,
+                                const OneLaunch& line) {
     const Rows r = rows_of(x);
     if (!r.ok || !is16(x.scalar_type()) || !weight_ok(w, at::kFloat8_e4m3fn, x.device(), r.K)) return std::nullopt;
     const int64_t N = w.size(0);
@@ -216,7 +222,7 @@ std::optional<Tensor> fp8_token(const Tensor& x, const Tensor& w, const Tensor& 
     const Launch l(x.device());
     const float* ws = (const float*)w_scale.data_ptr();
     Tensor out = make(out_size(x, N), at::kBFloat16, x.device());
-    if (r.M <= kOneLaunchTokens && r.K < kOneLaunchMaxK && r.M <= llmq_linear_dynamic_max_tokens(r.K)) {
+    if (line.takes(r)) {
         check(llmq_linear_fp8_dynamic(x.data_ptr(), code(x.scalar_type()), r.K, (const uint8_t*)w.data_ptr(), r.K, ws, ptr(bias),
                                       bias ? code(bias->scalar_type()) : LLMQ_BF16, out.data_ptr(), LLMQ_BF16, N, r.M, N, r.K,
                                       nullptr, nullptr, nullptr, l.stream),
@@ -460,12 +466,14 @@ LLMQ_PY(py_sq_tensor, 5)
     return wrap(std::move(y));
 LLMQ_PY_END
 
-LLMQ_PY(py_sq_token, 4)
+LLMQ_PY(py_sq_token, 6)
     const Tensor &x = in.tensor(0), &w = in.tensor(1), &s = in.tensor(2);
     const auto bias = in.optional(3);
     LLMQ_PY_TENSORS;
+    const OneLaunch line{PyLong_AsLongLong(argv[4]), PyLong_AsLongLong(argv[5])};
+    if (PyErr_Occurred()) return nullptr;
     std::optional<Tensor> y;
-    { NoGil g; y = sq_token(x, w, s, bias); }
+    { NoGil g; y = sq_token(x, w, s, bias, line); }
     return wrap(std::move(y));
 LLMQ_PY_END
 
@@ -488,12 +496,14 @@ LLMQ_PY(py_fp8_prequantized, 5)
     return wrap(std::move(y));
 LLMQ_PY_END
 
-LLMQ_PY(py_fp8_token, 4)
+LLMQ_PY(py_fp8_token, 6)
     const Tensor &x = in.tensor(0), &w = in.tensor(1), &s = in.tensor(2);
     const auto bias = in.optional(3);
     LLMQ_PY_TENSORS;
+    const OneLaunch line{PyLong_AsLongLong(argv[4]), PyLong_AsLongLong(argv[5])};
+    if (PyErr_Occurred()) return nullptr;
     std::optional<Tensor> y;
-    { NoGil g; y = fp8_token(x, w, s, bias); }
+    { NoGil g; y = fp8_token(x, w, s, bias, line); }
     return wrap(std::move(y));
 LLMQ_PY_END
 

@@ -24,15 +24,17 @@ __all__ = ["SqW8A8BBF16OBF16PerTensor", "SqW8A8BBF16OBF16PerChannel",
            "quantize_activation_per_tensor_absmax", "quantize_activation_per_token_absmax"]
 
 
-# Up to this many tokens (and K < 8192) the one-launch linear is as fast on the GPU as quantizer + GEMM and saves a
-# launch on the host; beyond, the two launches are faster (measured on MI355X at the Qwen2-7B shapes).
+# Up to this many tokens, and for shorter rows than ONE_LAUNCH_K, the one-launch linear is as fast on the GPU as quantizer +
+# GEMM and saves a launch on the host; beyond, the two launches are faster (measured on MI355X at the Qwen2-7B shapes).
+# The native forwards take both numbers from here.
 ONE_LAUNCH_MAX_TOKENS = 4
+ONE_LAUNCH_K = 8192
 
 
 def _fusable(x2: torch.Tensor) -> bool:
     """Layout the one-launch linear takes: 16-bit activations, contiguous rows, K % 16 == 0, 16-byte aligned."""
     return (x2.is_cuda and x2.dtype in (torch.bfloat16, torch.float16) and x2.stride(-1) == 1 and x2.shape[-1] % 16 == 0
-            and x2.shape[-1] < 8192
+            and x2.shape[-1] < ONE_LAUNCH_K
             and x2.stride(0) % 8 == 0 and x2.data_ptr() % 16 == 0)
 
 
@@ -126,7 +128,8 @@ class SqW8A8BBF16OBF16PerChannel(LinearBase):
 
     def forward(self, x):
         b = self._buffers
-        y = host().sq_token(x, b.get("qweight"), b.get("weight_scale"), b["bias"] if "bias" in b else self.bias)
+        y = host().sq_token(x, b.get("qweight"), b.get("weight_scale"), b["bias"] if "bias" in b else self.bias,
+                            ONE_LAUNCH_MAX_TOKENS, ONE_LAUNCH_K)
         return self._forward_general(x) if y is None else y
 
     @torch.no_grad()
