@@ -156,3 +156,50 @@ def test_static_input_scale_off_the_gpu_is_refused(cuda):
     from llmqrt_amd.quantize import per_tensor_quantize_with_alpha
     with pytest.raises(RuntimeError, match="weight scale"):
         per_tensor_quantize_with_alpha(x, torch.ones(1), True)
+
+
+def _allocations():
+    return torch.cuda.memory_stats()["allocation.all.allocated"]
+
+
+@pytest.mark.parametrize("form", ["module"])
+def test_capture_zeroes_counters_once(cuda, form):
+    """A captured AWQ call with a K split allocates its output and partial sums; the counters are one set per capture and
+    stream.  Replays beside eager work, with a second stream inside the graph and the pool released in between, stay right."""
+    from llmqrt_amd._native import host
+    from llmqrt_amd.awq_kernels import awq_gemm_triton
+    mod = _modules(torch.bfloat16, False)["awq"]
+    g = torch.Generator(device="cuda").manual_seed(8)
+    xs = [torch.randn(4, K, device=cuda, generator=g).half() for _ in range(4)]
+    call = mod if form == "module" else lambda x: awq_gemm_triton(x, mod.qweight, mod.scales, mod.qzeros, 8)
+    refs = [call(x) for x in xs]
+    torch.cuda.synchronize()
+    st, side = torch.cuda.Stream(), torch.cuda.Stream()
+    graphs, counts = [], []
+    for calls in (1, 3):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=st):
+            before = _allocations()
+            ys = [call(xs[i]) for i in range(calls)]
+            counts.append(_allocations() - before)
+            ptr = host().awq_counters(xs[0]).data_ptr()
+            assert host().awq_counters(xs[0]).data_ptr() == ptr
+            side.wait_stream(st)
+            with torch.cuda.stream(side):
+                ys.append(call(xs[3]))
+                assert host().awq_counters(xs[0]).data_ptr() != ptr
+            st.wait_stream(side)
+        graphs.append((graph, ys, refs[:calls] + refs[3:]))
+    assert counts[1] - counts[0] == 2 * 2  # output and partial sums of two more calls
+    for turn in range(5):
+        for graph, ys, want in graphs:
+            for y in ys:
+                y.zero_()
+            graph.replay()
+            with torch.cuda.stream(st):
+                eager = call(xs[turn % 4])
+            torch.cuda.synchronize()
+            assert torch.equal(eager, refs[turn % 4])
+            assert all(torch.equal(y, r) for y, r in zip(ys, want))
+        if turn == 2:
+            host().release_tickets()
