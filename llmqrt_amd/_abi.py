@@ -117,25 +117,31 @@ def stream_of(t: torch.Tensor) -> int:
 
 
 class _Workspaces:
-    """One grow-only scratch tensor per (device, stream): the C library never allocates.
-    zeroed: every new buffer starts as zeros (the AWQ workspace begins with arrival counters that must be zero before
-    the first call and that every call leaves zero)."""
+    """One grow-only scratch tensor per (device, stream): the C library never allocates.  Under capture every call gets
+    memory of the graph instead: an eager call's buffer may be replaced by a larger one while the graph still replays on
+    it, and a graph's buffer must not serve eager calls."""
 
-    def __init__(self, zeroed: bool = False):
+    def __init__(self):
         self._buf = {}
-        self._zeroed = zeroed
+
+    @staticmethod
+    def _capturing(device: torch.device) -> bool:
+        if device.index == torch.cuda.current_device():
+            return torch.cuda.is_current_stream_capturing()
+        with torch.cuda.device(device):
+            return torch.cuda.is_current_stream_capturing()
 
     def get(self, device: torch.device, nbytes: int) -> torch.Tensor | None:
         if nbytes == 0:
             return None
+        if self._capturing(device):
+            return torch.empty(nbytes, dtype=torch.uint8, device=device)
         key = (device.index, torch.cuda.current_stream(device).cuda_stream)
         buf = self._buf.get(key)
         if buf is None or buf.numel() < nbytes:
-            alloc = torch.zeros if self._zeroed else torch.empty
-            buf = alloc(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+            buf = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
             self._buf[key] = buf
         return buf
 
 
 workspaces = _Workspaces()
-awq_workspaces = _Workspaces(zeroed=True)  # never shared with another op: their partial sums would overwrite the counters

@@ -7,6 +7,7 @@ from __future__ import annotations
 import torch
 
 from . import _abi
+from ._native import host
 
 AWQ_TRITON_SUPPORTED_GROUP_SIZES = [-1, 32, 64, 128]
 
@@ -128,9 +129,12 @@ def _awq_gemm(input, qweight, scales, qzeros, split_k_iters, bias):
         bias = bias.to(torch.float16)  # what the kernels read
     result = torch.empty((M, N), dtype=input.dtype, device=input.device)
     L = _abi.lib()
-    ws = _abi.awq_workspaces.get(x.device, L.llmq_awq_gemm_workspace_bytes(M, N, K))
-    fn = L.llmq_awq_gemm if input.dtype == torch.float16 else L.llmq_awq_gemm_bf16
-    _abi.check(fn(x.data_ptr(), x.stride(0), qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(),
-                  _abi.ptr(bias), result.data_ptr(), M, N, K, group_size, _abi.ptr(ws),
-                  ws.numel() if ws is not None else 0, _abi.stream_of(x)), "llmq_awq_gemm")
+    # the arrival counters are the native forwards' own, one set per stream and one per capture; the partial sums are this call's
+    partials = L.llmq_awq_gemm_partials_bytes(M, N, K, group_size)
+    ws = _abi.workspaces.get(x.device, partials)
+    counters = host().awq_counters(x) if partials else None
+    _abi.check(L.llmq_awq_gemm_tickets(x.data_ptr(), _abi.dtype_code(input.dtype), x.stride(0), qweight.data_ptr(),
+                                       scales.data_ptr(), qzeros.data_ptr(), _abi.ptr(bias), result.data_ptr(), M, N, K,
+                                       group_size, _abi.ptr(counters), _abi.ptr(ws), ws.numel() if ws is not None else 0,
+                                       _abi.stream_of(x)), "llmq_awq_gemm")
     return result

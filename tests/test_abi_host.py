@@ -263,3 +263,22 @@ def test_awq_size_queries_answer_for_any_sizes():
             "assert L.llmq_awq_gemm_workspace_bytes(1, 4608, 3584) > L.llmq_awq_gemm_partials_bytes(1, 4608, 3584, 128) > 0")
     r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stderr[-2000:]
+
+
+def test_captured_calls_keep_no_shared_workspace(monkeypatch):
+    """A capture neither uses a cached buffer, which a larger eager call would replace under the graph, nor leaves one."""
+    from llmqrt_amd import _abi
+    state = {"capturing": False}
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: None)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state["capturing"])
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: type("S", (), {"cuda_stream": 7})())
+    cache, cpu = _abi._Workspaces(), torch.device("cpu")
+    assert cache.get(cpu, 0) is None
+    eager = cache.get(cpu, 100)
+    assert cache.get(cpu, 1 << 20) is eager and cache.get(cpu, (1 << 20) + 1) is not eager
+    eager = cache.get(cpu, 1)
+    state["capturing"] = True
+    first, second = cache.get(cpu, 100), cache.get(cpu, 4 << 20)
+    assert first is not eager and second is not eager and second is not first and second.numel() >= 4 << 20
+    state["capturing"] = False
+    assert cache.get(cpu, 100) is eager

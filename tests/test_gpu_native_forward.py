@@ -162,7 +162,7 @@ def _allocations():
     return torch.cuda.memory_stats()["allocation.all.allocated"]
 
 
-@pytest.mark.parametrize("form", ["module"])
+@pytest.mark.parametrize("form", ["module", "op"])
 def test_capture_zeroes_counters_once(cuda, form):
     """A captured AWQ call with a K split allocates its output and partial sums; the counters are one set per capture and
     stream.  Replays beside eager work, with a second stream inside the graph and the pool released in between, stay right."""
