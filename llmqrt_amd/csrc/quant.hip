@@ -153,29 +153,41 @@ __global__ __launch_bounds__(kThreads) void quant_rows_wave_kernel(
     }
 }
 
-// Stage 1 of the per-tensor quantizers: absmax partials, one per block.  A unit is kUnit consecutive chunks of a row
-// (a contiguous tensor is one long row), NL independent 16-byte loads per thread: 8, or 2 for strided rows shorter than
-// a unit of 8.  HBM-bound: 8192 x 3584 12.9 us (4.6 TB/s; one load at a time with a division per chunk 14.2), 4096 x 18944
-// 34.1 us (36.4).
-constexpr int kUnitLoads = 8;
-template <int DT, int NL>
+// Stage 1 of the per-tensor quantizers: absmax partials, one per block.  The tensor's chunks, row after row, are cut into
+// units of kUnit; a thread takes kUnitLoads independent 16-byte loads of a unit.  HBM-bound: 8192 x 3584 12.9 us (4.6 TB/s;
+// one load at a time with a division per chunk 14.2), 4096 x 18944 34.1 us (36.4).
+// STRIDED: rows of cpr chunks lie ldx apart.  A thread divides once per unit to find its first chunk and steps from there:
+// step_rows, step_chunks = kThreads / cpr, kThreads % cpr.  Units follow the chunks and not the rows, so that short rows fill
+// them too.
+constexpr int kUnitLoads = 8, kUnit = kUnitLoads * kThreads;
+template <int DT, bool STRIDED>
 __global__ __launch_bounds__(kThreads) void absmax_partials_kernel(
-    const uint16_t* __restrict__ x, int64_t ldx, int64_t rows, int64_t cpr, float* __restrict__ partials) {
+    const uint16_t* __restrict__ x, int64_t ldx, int64_t cpr, int64_t total, int64_t step_rows, int64_t step_chunks,
+    float* __restrict__ partials) {
     __shared__ float smem[kNW];
-    constexpr int kUnit = NL * kThreads;
-    const int64_t upr = (cpr + kUnit - 1) / kUnit, units = rows * upr;
+    const uint4* first = reinterpret_cast<const uint4*>(x);
+    const uint4* last = STRIDED ? reinterpret_cast<const uint4*>(x + (total / cpr - 1) * ldx) + (cpr - 1) : first + (total - 1);
     float amax = 0.f;
-    for (int64_t u = blockIdx.x; u < units; u += gridDim.x) {
-        const int64_t r = u / upr, c0 = (u - r * upr) * kUnit + threadIdx.x;
-        const uint4* xr = reinterpret_cast<const uint4*>(x + r * ldx);
-        uint4 v[NL];
+    for (int64_t base = (int64_t)blockIdx.x * kUnit; base < total; base += (int64_t)gridDim.x * kUnit) {
+        const int64_t at = base + threadIdx.x;
+        int64_t r = 0, c = at;
+        if (STRIDED) {
+            r = total <= 0xffffffffLL ? (int64_t)((uint32_t)at / (uint32_t)cpr) : at / cpr;
+            c = at - r * cpr;
+        }
+        uint4 v[kUnitLoads];
 #pragma unroll
-        for (int i = 0; i < NL; i++) {
-            const int64_t c = c0 + i * kThreads;
-            v[i] = xr[c < cpr ? c : cpr - 1];  // past the end: the last chunk again, which changes no maximum
+        for (int i = 0; i < kUnitLoads; i++) {
+            const uint4* src = STRIDED ? reinterpret_cast<const uint4*>(x + r * ldx) + c : first + (at + i * kThreads);
+            v[i] = *(at + i * kThreads < total ? src : last);  // past the end: the last chunk again, which changes no maximum
+            if (STRIDED) {
+                r += step_rows;
+                c += step_chunks;
+                if (c >= cpr) c -= cpr, r++;
+            }
         }
 #pragma unroll
-        for (int i = 0; i < NL; i++) amax = max_nonneg(amax, absmax8(v[i], DT == LLMQ_BF16));
+        for (int i = 0; i < kUnitLoads; i++) amax = max_nonneg(amax, absmax8(v[i], DT == LLMQ_BF16));
     }
     amax = block_max<kNW>(amax, smem);
     if (threadIdx.x == 0) partials[blockIdx.x] = amax;
@@ -511,17 +523,14 @@ int per_tensor_dt(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
                            dim3(kSmallThreads), 0, st, (const uint4*)x, (int)total, (uint2*)q, scale, scale_dtype, floor, ta);
         return launch_status();
     }
-    const int64_t rows = contiguous ? 1 : M, cpr = contiguous ? total : K >> 3;
-    const bool wide = cpr >= kUnitLoads * kThreads;
-    const int unit = (wide ? kUnitLoads : 2) * kThreads;
-    const int64_t units = rows * ((cpr + unit - 1) / unit);
+    const int64_t cpr = K >> 3, units = (total + kUnit - 1) / kUnit;
     const int nblk = (int)(units < kMaxPartials ? units : kMaxPartials);
-    if (wide)
-        hipLaunchKernelGGL((absmax_partials_kernel<DT, kUnitLoads>), dim3(nblk), dim3(kThreads), 0, st, (const uint16_t*)x,
-                           ldx, rows, cpr, partials);
+    if (contiguous)
+        hipLaunchKernelGGL((absmax_partials_kernel<DT, false>), dim3(nblk), dim3(kThreads), 0, st, (const uint16_t*)x, ldx, cpr,
+                           total, 0, 0, partials);
     else
-        hipLaunchKernelGGL((absmax_partials_kernel<DT, 2>), dim3(nblk), dim3(kThreads), 0, st, (const uint16_t*)x, ldx, rows,
-                           cpr, partials);
+        hipLaunchKernelGGL((absmax_partials_kernel<DT, true>), dim3(nblk), dim3(kThreads), 0, st, (const uint16_t*)x, ldx, cpr,
+                           total, kThreads / cpr, kThreads % cpr, partials);
     if (launch_status() != LLMQ_OK) return LLMQ_ERR_LAUNCH;
     return dispatch_rows<MODE, SCALE_TENSOR>(x, x_dtype, M, K, ldx, q, scale, scale_dtype, partials, nblk, 0, floor, ta, st);
 }
