@@ -9,7 +9,7 @@ import importlib.machinery
 import importlib.util
 import pathlib
 
-import torch  # noqa: F401  (the extension's torch and HIP libraries must be in the process first)
+import torch  # the extension's torch and HIP libraries must be in the process first
 
 from . import _abi
 
@@ -24,6 +24,9 @@ def _load():
     loader = importlib.machinery.ExtensionFileLoader("_llmq_host", str(_PATH))
     module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_llmq_host", loader))
     loader.exec_module(module)
+    if module.torch_version != torch.__version__:
+        raise RuntimeError(f"{_PATH} was built against torch {module.torch_version} and this is torch {torch.__version__}: "
+                           "build it again with `python -m llmqrt_amd.csrc.build`")
     return module
 
 

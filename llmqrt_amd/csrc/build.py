@@ -50,7 +50,8 @@ def _build_host() -> None:
     import torch
     torch_dir = pathlib.Path(torch.__file__).resolve().parent
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-Wno-deprecated-declarations",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DLLMQ_TORCH_VERSION="{torch.__version__}"',
+           "-Wno-deprecated-declarations",
            "-isystem", str(torch_dir / "include"), "-isystem", str(torch_dir / "include/torch/csrc/api/include"),
            "-isystem", sysconfig.get_paths()["include"], "-isystem", "/opt/rocm/include", f"-I{ROOT / 'include'}",
            str(HERE / "host_ops.cpp"), "-o", str(HOST_LIB), f"-L{OUT_DIR}", "-l:libllmq_gfx950.so", f"-L{torch_dir / 'lib'}",

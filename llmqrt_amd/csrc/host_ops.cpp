@@ -622,4 +622,9 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_llmq_host", "native forward p
 
 }  // namespace
 
-extern "C" PyObject* PyInit__llmq_host(void) { return PyModule_Create(&module_def); }
+extern "C" PyObject* PyInit__llmq_host(void) {
+    PyObject* m = PyModule_Create(&module_def);
+    // the tensors that cross this boundary have the layout of the torch it was compiled against
+    if (m && PyModule_AddStringConstant(m, "torch_version", LLMQ_TORCH_VERSION) != 0) Py_CLEAR(m);
+    return m;
+}

@@ -282,3 +282,11 @@ def test_captured_calls_keep_no_shared_workspace(monkeypatch):
     assert first is not eager and second is not eager and second is not first and second.numel() >= 4 << 20
     state["capturing"] = False
     assert cache.get(cpu, 100) is eager
+
+
+def test_native_library_of_another_torch_is_refused(monkeypatch):
+    from llmqrt_amd import _native
+    assert _native.host().torch_version == torch.__version__
+    monkeypatch.setattr(torch, "__version__", "0.0.0")
+    with pytest.raises(RuntimeError, match="built against torch"):
+        _native._load()
