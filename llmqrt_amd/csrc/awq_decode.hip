@@ -116,11 +116,17 @@ __device__ __forceinline__ void finish_split_tile(const float* ptile, int M, int
     if (!s_last) return;
     // Eight splits at a time, added in split order.  Every coherent load goes to memory, so the read-back costs one round
     // trip per pass: where a pass has more pieces than threads (16 tokens on 512 threads), a thread takes two pieces,
-    // sixteen 16-byte loads in flight.
+    // sixteen 16-byte loads in flight.  The loads and the wait for them are one statement: the compiler takes the outputs of a
+    // statement as written at its end.  (s_nop: the wait states between a vector instruction that writes a scalar register and a
+    // load that reads it, which the compiler does not place in front of a statement.)  A split's plane is a scalar base, a piece's place in it a 32-bit offset (at most 16 rows of
+    // the 130816 channels that the tickets allow).
     const int items = M * tile_q;
-    auto ld = [&](const float* src, int sp, v4f& t) __attribute__((always_inline)) {
-        const float* q = src + (int64_t)min(sp, splits - 1) * plane;
-        asm volatile("global_load_dwordx4 %0, %1, off sc1" : "=v"(t) : "v"(q) : "memory");
+    auto offset_of = [&](int idx) __attribute__((always_inline)) {
+        const int m = idx / tile_q;
+        return 4u * (uint32_t)(m * N + tile_n0 + 4 * (idx - m * tile_q));
+    };
+    auto plane_of = [&](int sp) __attribute__((always_inline)) {
+        return partials + (uint32_t)min(sp, splits - 1) * (uint32_t)plane;  // at most 64 splits of 64 rows: below 2^32 elements
     };
     auto add8 = [&](v4f& acc, int left, v4f t0, v4f t1, v4f t2, v4f t3, v4f t4, v4f t5, v4f t6, v4f t7) __attribute__((always_inline)) {
         acc += t0;
@@ -132,45 +138,49 @@ __device__ __forceinline__ void finish_split_tile(const float* ptile, int M, int
         if (left > 6) acc += t6;
         if (left > 7) acc += t7;
     };
+#define LLMQ_LD(OUT, OFF, BASE) "global_load_dwordx4 %" #OUT ", %" #OFF ", %" #BASE " sc1\n\t"
     for (int base = 0; base < items; base += 2 * NT) {
         const int idx = base + tid, idx1 = idx + NT;
         if (base + NT < items) {  // block-uniform: the second half of the pass is not empty
             const bool two = idx1 < items;  // a lane without a second piece loads its first one twice
             const int ia = idx, ib = two ? idx1 : idx;
-            const int ma = ia / tile_q, na = tile_n0 + 4 * (ia - ma * tile_q);
-            const int mb = ib / tile_q, nb = tile_n0 + 4 * (ib - mb * tile_q);
-            const float* srca = partials + (int64_t)ma * N + na;
-            const float* srcb = partials + (int64_t)mb * N + nb;
+            const uint32_t oa = offset_of(ia), ob = offset_of(ib);
             v4f acca = {0.f, 0.f, 0.f, 0.f}, accb = {0.f, 0.f, 0.f, 0.f};
             for (int sp = 0; sp < splits; sp += 8) {
                 v4f a0, a1, a2, a3, a4, a5, a6, a7, b0, b1, b2, b3, b4, b5, b6, b7;
-                ld(srca, sp, a0), ld(srca, sp + 1, a1), ld(srca, sp + 2, a2), ld(srca, sp + 3, a3);
-                ld(srca, sp + 4, a4), ld(srca, sp + 5, a5), ld(srca, sp + 6, a6), ld(srca, sp + 7, a7);
-                ld(srcb, sp, b0), ld(srcb, sp + 1, b1), ld(srcb, sp + 2, b2), ld(srcb, sp + 3, b3);
-                ld(srcb, sp + 4, b4), ld(srcb, sp + 5, b5), ld(srcb, sp + 6, b6), ld(srcb, sp + 7, b7);
-                asm volatile("s_waitcnt vmcnt(0)"
-                             : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(a4), "+v"(a5), "+v"(a6), "+v"(a7), "+v"(b0),
-                               "+v"(b1), "+v"(b2), "+v"(b3), "+v"(b4), "+v"(b5), "+v"(b6), "+v"(b7)::"memory");
+                asm volatile("s_nop 4\n\t" LLMQ_LD(0, 16, 18) LLMQ_LD(1, 16, 19) LLMQ_LD(2, 16, 20) LLMQ_LD(3, 16, 21)
+                             LLMQ_LD(4, 16, 22) LLMQ_LD(5, 16, 23) LLMQ_LD(6, 16, 24) LLMQ_LD(7, 16, 25)
+                             LLMQ_LD(8, 17, 18) LLMQ_LD(9, 17, 19) LLMQ_LD(10, 17, 20) LLMQ_LD(11, 17, 21)
+                             LLMQ_LD(12, 17, 22) LLMQ_LD(13, 17, 23) LLMQ_LD(14, 17, 24) LLMQ_LD(15, 17, 25)
+                             "s_waitcnt vmcnt(0)"
+                             : "=&v"(a0), "=&v"(a1), "=&v"(a2), "=&v"(a3), "=&v"(a4), "=&v"(a5), "=&v"(a6), "=&v"(a7), "=&v"(b0),
+                               "=&v"(b1), "=&v"(b2), "=&v"(b3), "=&v"(b4), "=&v"(b5), "=&v"(b6), "=&v"(b7)
+                             : "v"(oa), "v"(ob), "s"(plane_of(sp)), "s"(plane_of(sp + 1)), "s"(plane_of(sp + 2)), "s"(plane_of(sp + 3)),
+                               "s"(plane_of(sp + 4)), "s"(plane_of(sp + 5)), "s"(plane_of(sp + 6)), "s"(plane_of(sp + 7))
+                             : "memory");
                 add8(acca, splits - sp, a0, a1, a2, a3, a4, a5, a6, a7);
                 add8(accb, splits - sp, b0, b1, b2, b3, b4, b5, b6, b7);
             }
-            store4(acca, ma, na);
-            if (two) store4(accb, mb, nb);
+            store4(acca, ia / tile_q, tile_n0 + 4 * (ia % tile_q));
+            if (two) store4(accb, ib / tile_q, tile_n0 + 4 * (ib % tile_q));
         } else if (idx < items) {
-            const int ia = idx;
-            const int ma = ia / tile_q, na = tile_n0 + 4 * (ia - ma * tile_q);
-            const float* srca = partials + (int64_t)ma * N + na;
+            const uint32_t oa = offset_of(idx);
             v4f acca = {0.f, 0.f, 0.f, 0.f};
             for (int sp = 0; sp < splits; sp += 8) {
                 v4f a0, a1, a2, a3, a4, a5, a6, a7;
-                ld(srca, sp, a0), ld(srca, sp + 1, a1), ld(srca, sp + 2, a2), ld(srca, sp + 3, a3);
-                ld(srca, sp + 4, a4), ld(srca, sp + 5, a5), ld(srca, sp + 6, a6), ld(srca, sp + 7, a7);
-                asm volatile("s_waitcnt vmcnt(0)" : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(a4), "+v"(a5), "+v"(a6), "+v"(a7)::"memory");
+                asm volatile("s_nop 4\n\t" LLMQ_LD(0, 8, 9) LLMQ_LD(1, 8, 10) LLMQ_LD(2, 8, 11) LLMQ_LD(3, 8, 12)
+                             LLMQ_LD(4, 8, 13) LLMQ_LD(5, 8, 14) LLMQ_LD(6, 8, 15) LLMQ_LD(7, 8, 16)
+                             "s_waitcnt vmcnt(0)"
+                             : "=&v"(a0), "=&v"(a1), "=&v"(a2), "=&v"(a3), "=&v"(a4), "=&v"(a5), "=&v"(a6), "=&v"(a7)
+                             : "v"(oa), "s"(plane_of(sp)), "s"(plane_of(sp + 1)), "s"(plane_of(sp + 2)), "s"(plane_of(sp + 3)),
+                               "s"(plane_of(sp + 4)), "s"(plane_of(sp + 5)), "s"(plane_of(sp + 6)), "s"(plane_of(sp + 7))
+                             : "memory");
                 add8(acca, splits - sp, a0, a1, a2, a3, a4, a5, a6, a7);
             }
-            store4(acca, ma, na);
+            store4(acca, idx / tile_q, tile_n0 + 4 * (idx % tile_q));
         }
     }
+#undef LLMQ_LD
 }
 
 // RM: token rows per lane that can be live (min(M, 4)).  KS: K slices inside the block - KS sets of CS wavefronts, each

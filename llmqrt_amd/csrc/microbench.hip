@@ -81,9 +81,11 @@ __global__ __launch_bounds__(512) void lds_kernel(const uint4* __restrict__ src,
     if (MODE == 0) {
         for (int i = 0; i < iters; i++) {
             u4 r[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r[j]) : "v"(la), "n"(j * 1024) : "memory");
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            asm volatile("ds_read_b128 %0, %8\n\tds_read_b128 %1, %8 offset:1024\n\tds_read_b128 %2, %8 offset:2048\n\t"
+                         "ds_read_b128 %3, %8 offset:3072\n\tds_read_b128 %4, %8 offset:4096\n\tds_read_b128 %5, %8 offset:5120\n\t"
+                         "ds_read_b128 %6, %8 offset:6144\n\tds_read_b128 %7, %8 offset:7168\n\ts_waitcnt lgkmcnt(0)"
+                         : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7])
+                         : "v"(la) : "memory");
 #pragma unroll
             for (int j = 0; j < 8; j++) acc += r[j].x;
         }
