@@ -5,8 +5,9 @@
  *  - Every pointer is a DEVICE pointer unless its comment says "host".
  *  - The caller owns every buffer (inputs, outputs, workspaces); the library allocates
  *    nothing, never synchronises with the host and launches on the stream it is given
- *    (0 = the null stream).  Calls are asynchronous.  State kept between calls: the
- *    *_force_plan tuning hooks (per host thread) only.
+ *    (0 = the null stream).  Calls are asynchronous.  State kept between calls, all of
+ *    it per host thread: the *_force_plan tuning hooks, and the last GEMM plans (a function of sizes
+ *    and format alone).  llmq_gemm_w8a8_static has a scratch array per GPU.
  *  - Matrices are row-major; `ld*` is the row stride in ELEMENTS.
  *  - Return value: LLMQ_OK (0) or a negative llmq_status; llmq_status_string() names it.
  *  - Paths below are relative to the reference's runtime/ directory.

@@ -13,3 +13,11 @@ Layout:
   workloads.py     seeded synthetic inputs of the benchmark configurations
 """
 __version__ = "0.1.0"
+
+
+def release_workspaces() -> None:
+    """Give back the scratch that is kept per device and stream between calls: the Python ops' workspaces and the arrival
+    counters of the few-token AWQ kernel.  Calls that are running keep theirs; later calls allocate again."""
+    from . import _abi, _native
+    _abi.workspaces.release()
+    _native.host().release_tickets()

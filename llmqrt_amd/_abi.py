@@ -121,8 +121,13 @@ class _Workspaces:
     memory of the graph instead: an eager call's buffer may be replaced by a larger one while the graph still replays on
     it, and a graph's buffer must not serve eager calls."""
 
+    _MAX_STREAMS = 256
+
     def __init__(self):
         self._buf = {}
+
+    def release(self):
+        self._buf.clear()
 
     @staticmethod
     def _capturing(device: torch.device) -> bool:
@@ -140,6 +145,8 @@ class _Workspaces:
         buf = self._buf.get(key)
         if buf is None or buf.numel() < nbytes:
             buf = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+            if len(self._buf) >= self._MAX_STREAMS:
+                self._buf.clear()
             self._buf[key] = buf
         return buf
 

@@ -284,6 +284,22 @@ def test_captured_calls_keep_no_shared_workspace(monkeypatch):
     assert cache.get(cpu, 100) is eager
 
 
+def test_workspaces_are_bounded_and_given_back(monkeypatch):
+    import llmqrt_amd
+    from llmqrt_amd import _abi
+    stream = {"id": 0}
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: None)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: type("S", (), {"cuda_stream": stream["id"]})())
+    cache, cpu = _abi._Workspaces(), torch.device("cpu")
+    monkeypatch.setattr(_abi, "workspaces", cache)
+    monkeypatch.setattr(_abi._Workspaces, "_MAX_STREAMS", 4)
+    for stream["id"] in range(9):
+        assert cache.get(cpu, 8) is cache.get(cpu, 8) and len(cache._buf) <= 4
+    llmqrt_amd.release_workspaces()
+    assert not cache._buf
+
+
 def test_native_library_of_another_torch_is_refused(monkeypatch):
     from llmqrt_amd import _native
     assert _native.host().torch_version == torch.__version__

@@ -203,3 +203,30 @@ def test_capture_zeroes_counters_once(cuda, form):
             assert all(torch.equal(y, r) for y, r in zip(ys, want))
         if turn == 2:
             host().release_tickets()
+
+
+def test_more_streams_than_counter_sets(cuda):
+    """256 streams keep a counter set; a call on one more zeroes a set of its own, and gives the same result."""
+    import ctypes
+    import llmqrt_amd
+    from llmqrt_amd._native import host
+    hip = ctypes.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+    mod = _modules(torch.bfloat16, False)["awq"]
+    x = torch.randn(4, K, device=cuda, generator=torch.Generator(device="cuda").manual_seed(2)).bfloat16()
+    ref = mod(x)
+    torch.cuda.synchronize()
+    llmqrt_amd.release_workspaces()
+    kept = []
+    for i in range(258):
+        ptr = ctypes.c_void_p()
+        assert hip.hipStreamCreate(ctypes.byref(ptr)) == 0
+        with torch.cuda.stream(torch.cuda.ExternalStream(ptr.value)):
+            host().awq_counters(x)
+            before = _allocations()
+            host().awq_counters(x)
+            kept.append(_allocations() == before)
+            y = mod(x) if i in (0, 255, 256, 257) else None
+        torch.cuda.synchronize()
+        assert y is None or torch.equal(y, ref), i
+    assert kept == [True] * 256 + [False] * 2
+    llmqrt_amd.release_workspaces()
