@@ -82,14 +82,66 @@ bool skinny_plan(int64_t M, int64_t N, int64_t K, int& t, int& nw) {
 }
 
 constexpr size_t kStaticScratchBytes = (size_t)32 << 20;  // the library's own scratch (llmq_gemm_w8a8_static)
+inline size_t partials_bytes(const Plan& p, int64_t M, int64_t N) { return p.splits > 1 ? (size_t)p.splits * M * N * 4 : 0; }
 
-// Pick the tile shape and K split with the smallest modelled time:
+// More than 128 rows, fewer than two rounds of 256x256 tiles, up to 20480 elements of K: the plan with the smallest modelled time.
+// The table is fitted to the times (us) of 311 000 plans, every configuration and K split of 12 600 random problems of the three
+// formats, each with weights out of HBM and with weights in the Infinity Cache.
+//   step      time per 64 bytes of K of a round of up to 256 blocks (a partly filled round takes as long as a full one)
+//   fixed     prologue and epilogue of a round
+//   ragged    factor on step where rows are no whole number of 128-byte lines (K % 128 != 0)
+//   shared    64- and 32-row tiles, which share a CU: past 256 blocks, time per 64 bytes of K and 256 blocks
+//   finish, partial   finishing launch of a K split, and us per 8 MB of partial sums written and read
+// The rounds model below had these sizes as well, tuned on the 7B projections.  It priced one pass of small tiles too low (fp16
+// 435 x 5504 x 7936 at 109 us, measured 182 where 108 were to be had; fp8 130 x 3584 x 7936 18.4 / 29.4 / 19.1), which left 4-8 % of the
+// problems of 129-1024 rows more than 5 % slower than the planner before it.  18 700 other random problems with this table: 1.9 %
+// faster than the rounds model in the mean, 9 % faster than that planner, 1.1 % of them more than 5 % behind it (two runs of one plan
+// differ by as much on 1 %), 0.2 % more than 10 %.
+// A split whose partial sums exceed the 32 MB of the L2s must win by a tenth (without that margin 1.3 % of the problems end
+// more than 5 % behind the rounds model, with it 0.6 %).
+constexpr int64_t kTableMaxK = 20480;  // elements
+struct TileCost { int cfg; double step, fixed, ragged, shared, finish, partial; };
+Plan table_plan(int op, int64_t M, int64_t N, int64_t K, size_t max_partials) {
+    static const TileCost kInt8F16[] = {{1, 0.707, 8.52, 1.248, 0, 3.91, 1.425},  // 256x256
+                                        {2, 0.484, 8.53, 1.236, 0, 1.92, 1.319},  // 256x128
+                                        {3, 0.275, 5.99, 1.298, 0, 3.77, 0.999}}; // 128x128
+    static const TileCost kFp8[] = {{1, 0.659, 10.33, 1.455, 0, 3.67, 1.630},
+                                    {2, 0.629, 9.83, 1.113, 0, 1.94, 1.251},
+                                    {3, 0.399, 6.36, 1.250, 0, 4.51, 0.446}};
+    static const TileCost kAll[] = {{4, 0.173, 3.60, 1.585, 0.225, 3.47, 1.522},  // 64x128
+                                    {5, 0.167, 0.87, 1.400, 0.254, 3.77, 1.623},  // 32x128
+                                    {7, 0.359, 6.97, 1.454, 0, 2.42, 1.867}};     // 128x256
+    const bool ragged = K % 128 != 0;
+    Plan best{1, 1, (int)K};
+    double best_t = 1e300;
+    for (int row = 0; row < 6; row++) {
+        const TileCost& c = row >= 3 ? kAll[row - 3] : (op == 1 ? kFp8 : kInt8F16)[row];
+        const TileShape s = kShapes[c.cfg];
+        const int64_t tiles = (int64_t)cdiv(M, s.bm) * cdiv(N, s.bn);
+        const double step = c.step * (ragged ? c.ragged : 1.0), shared = c.shared * (ragged ? c.ragged : 1.0);
+        for (int sp = 1; sp <= 16; sp += sp < 8 ? 1 : 2) {
+            const size_t partials = sp > 1 ? (size_t)M * N * sp * 4 : 0;
+            if (sp > 1 && (K / sp < 512 || partials > (size_t)256 << 20 || partials > max_partials)) break;
+            const int kps = cdiv(cdiv(K, sp), s.bk) * s.bk;
+            if (cdiv(K, kps) != sp) continue;
+            const double steps = kps / 64.0, x = (double)tiles * sp / kNumCu, rounds = (double)cdiv(tiles * sp, kNumCu);
+            double t = rounds * (steps * step + c.fixed);
+            if (c.shared > 0 && x > 1) t = steps * std::max(shared * x, step) + c.fixed * 0.5 * (1 + rounds);
+            if (sp > 1) t += c.finish + c.partial * partials * 2 / 8.0e6;
+            if (partials > kStaticScratchBytes) t *= 1.1;
+            if (t < best_t) best_t = t, best = Plan{c.cfg, sp, kps};
+        }
+    }
+    return best;
+}
+
+// The rounds model, for up to 128 rows, for grids of two rounds and more, and for a longer K:
 // waves of blocks over the CUs x per-block MFMA time, with a floor from the bytes each block streams.
 // The matrix cores take the same time per byte of K for int8, fp8 and fp16 (half the K elements at half the rate), so one
 // table serves all three.  (Priced at twice the time per byte, fp16 was split five ways along K at 777 x 3584 x 18944: 138-140
 // us with 55 MB of partial sums, against 132-136 us for the two-way split picked here.)
 // fp8: the 64-byte K tiles have one MFMA sub-step there and keep the register-staged loop (measured ~20 % slower)
-Plan make_plan(int64_t M, int64_t N, int64_t K, bool fp8 = false) {
+Plan rounds_plan(int64_t M, int64_t N, int64_t K, bool fp8) {
     int ocfg, osp;
     if (plan_override(ocfg, osp) && ocfg < 100) {
         const TileShape s = kShapes[ocfg < kNumShapes ? ocfg : kNumShapes - 1];
@@ -154,15 +206,28 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, bool fp8 = false) {
     return best;
 }
 
-// The plan of a problem by operand format (0 int8, 1 fp8, 2 fp16; K in bytes).  Searching it takes microseconds of host
-// time and a call needs it for its workspace and for its launch, so each host thread remembers the last plans it made
-// (a pure function of sizes and format; a forced plan is not remembered).
+// The plan of a problem by operand format (0 int8, 1 fp8, 2 fp16; K in bytes).  kStaticInt8: int8 on the library's own scratch,
+// which refuses what the rounds model splits past its size and runs the rest with a plan that fits.  With a ragged 8-bit K, whose
+// price is the least certain, the other entry points stay within that size too where the rounds model does.
+constexpr int kStaticInt8 = 3;
+Plan make_plan(int op, int64_t M, int64_t N, int64_t K) {
+    const Plan rounds = rounds_plan(M, N, K, op == 1);
+    const bool forced = g_force_cfg >= 0 && g_force_cfg < 100;
+    if (forced || M <= 128 || (int64_t)cdiv(M, 256) * cdiv(N, 256) >= 2 * kNumCu || K > kTableMaxK * (op == 2 ? 2 : 1)) return rounds;
+    const bool fits = partials_bytes(rounds, M, N) <= kStaticScratchBytes;
+    if (op == kStaticInt8 && !fits) return rounds;
+    const bool keep = op == kStaticInt8 || (op != 2 && K % 128 != 0 && fits);
+    return table_plan(op, M, N, K, keep ? kStaticScratchBytes : SIZE_MAX);
+}
+
+// Searching a plan takes microseconds of host time and a call needs it for its workspace and for its launch, so each host
+// thread remembers the last plans it made (a pure function of sizes and format; a forced plan is not remembered).
 Plan plan_for(int op, int64_t M, int64_t N, int64_t K) {
-    if (g_force_cfg >= 0) return make_plan(M, N, K, op == 1);
+    if (g_force_cfg >= 0) return make_plan(op, M, N, K);
     struct Entry { int64_t M, N, K; int op; Plan plan; };
     static thread_local Entry cache[64] = {};
     Entry& e = cache[((uint64_t)(M * 31 + N * 17 + K * 7 + op) * 0x9E3779B97F4A7C15ull) >> 58];
-    if (e.M != M || e.N != N || e.K != K || e.op != op) e = Entry{M, N, K, op, make_plan(M, N, K, op == 1)};
+    if (e.M != M || e.N != N || e.K != K || e.op != op) e = Entry{M, N, K, op, make_plan(op, M, N, K)};
     return e.plan;
 }
 
@@ -172,7 +237,8 @@ Plan plan_for(int op, int64_t M, int64_t N, int64_t K) {
 int gemm_entry(int op, int a_format, const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ldb,
                const float* a_scale, const float* w_scale, float alpha, const float* alpha_dev, const void* bias,
                int bias_dtype, float beta, void* out, int out_dtype, int64_t ldo, int64_t M, int64_t N, int64_t K,
-               void* acc_dump, void* ws, size_t ws_bytes, hipStream_t st, const float* out_scale = nullptr) {
+               void* acc_dump, void* ws, size_t ws_bytes, hipStream_t st, const float* out_scale = nullptr,
+               bool static_scratch = false) {
     const bool fp8 = op == 1;
     if (M < 0 || N < 0 || K < 0) return LLMQ_ERR_SHAPE;
     if (M == 0 || N == 0) return LLMQ_OK;
@@ -189,14 +255,12 @@ int gemm_entry(int op, int a_format, const uint8_t* A, int64_t lda, const uint8_
         return launch_gemm_skinny(fp8, a_format == LLMQ_E5M2 ? 1 : 0, sk_t, sk_nw, A, lda, B, ldb, (int)M, (int)N, (int)K, sep,
                                   out, ldo, acc_dump, st);
     }
-    Plan p = plan_for(op, M, N, K);
+    Plan p = plan_for(static_scratch ? kStaticInt8 : op, M, N, K);
     // fp8 fragments are twice as wide: the 8-wave prefill tile runs ~5 % faster with 128-byte K tiles
     if (fp8 && g_force_cfg < 0 && p.cfg == 1 && p.splits == 1) p.cfg = 6;
     // int8 with direct loads: no staging registers, so the 128-byte K tile fits (half the barriers, whole lines per row)
     if (!fp8 && g_force_cfg < 0 && p.cfg == 1 && K % 128 == 0 && p.k_per_split % 128 == 0) p.cfg = 6;
-    if (p.splits > 1) {
-        if (!ws || ws_bytes < (size_t)p.splits * M * N * 4) return LLMQ_ERR_WORKSPACE;
-    }
+    if (p.splits > 1 && (!ws || ws_bytes < partials_bytes(p, M, N))) return LLMQ_ERR_WORKSPACE;
     auto run = [&](const Plan& pl, const uint8_t* Bp, const float* wsc, const void* bs, void* o, int64_t n) {
         Epilogue ep{a_scale, wsc, alpha_dev, bs, alpha, beta, bias_dtype, out_dtype, out_scale};
         const bool dma = g_force_dma != 0;
@@ -260,11 +324,10 @@ extern "C" int llmq_gemm_w8a8_static(const int8_t* A, int64_t lda, const int8_t*
     int rc = static_scratch(&ws);
     if (rc != LLMQ_OK) return rc;
     // The common entry validates the arguments first and then checks the partial sums of the plan it is about to
-    // launch (the int8 plan of this problem) against the size it is given: a plan that does not fit the array is
-    // refused there, before any launch.
+    // launch against the size it is given: a plan that does not fit the array is refused there, before any launch.
     rc = gemm_entry(0, 0, (const uint8_t*)A, lda, (const uint8_t*)B, ldb, a_scale, w_scale, alpha, alpha_dev, bias,
                     bias_dtype, beta, out, out_dtype, ldo, M, N, K, nullptr, ws, kStaticScratchBytes,
-                    (hipStream_t)stream);
+                    (hipStream_t)stream, nullptr, true);
     return rc == LLMQ_ERR_WORKSPACE ? LLMQ_ERR_SCRATCH : rc;
 }
 
@@ -285,8 +348,7 @@ extern "C" size_t llmq_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     int sk_t, sk_nw;
     if (skinny_plan(M, N, K, sk_t, sk_nw)) return 0;
     const Plan p = plan_for(0, M, N, K), p8 = plan_for(1, M, N, K);  // the int8 and the fp8 plan may differ
-    const int splits = p.splits > p8.splits ? p.splits : p8.splits;
-    return splits > 1 ? (size_t)splits * M * N * 4 : 0;
+    return std::max(partials_bytes(p, M, N), partials_bytes(p8, M, N));
 }
 
 extern "C" int llmq_gemm_w8a8(const int8_t* A, int64_t lda, const int8_t* B, int64_t ldb, const float* a_scale,
@@ -323,13 +385,13 @@ extern "C" int llmq_gemm_fp8_quantized_output(const uint8_t* A, int a_format, in
 extern "C" size_t llmq_gemm_fp8_quantized_output_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     const Plan p = plan_for(1, M, N, K);
-    return p.splits > 1 ? (size_t)p.splits * M * N * 4 : 0;
+    return partials_bytes(p, M, N);
 }
 
 extern "C" size_t llmq_gemm_f16_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     const Plan p = plan_for(2, M, N, 2 * K);
-    return p.splits > 1 ? (size_t)p.splits * M * N * 4 : 0;
+    return partials_bytes(p, M, N);
 }
 
 extern "C" int llmq_gemm_f16(const void* A, int64_t lda, const void* B, int64_t ldb, float alpha, const void* bias,

@@ -640,3 +640,39 @@ def test_split_finish_forms_agree(cuda, force_plan, N):
     for splits in (2, 4, 5, 6):
         force_plan(5, splits)
         assert torch.equal(w8a8_int8_linear_bbf16_obf16_per_channel(*args), ref), splits
+
+
+# Plans past 128 rows: 12 and 16 splits of 32-row tiles, the longest K of the planner's table and one beyond, ragged K with 8 and with
+# 16 splits, one pass of every tile shape, a K split of 128x128 tiles; the first grid of two rounds of 256x256 tiles and the last below
+@pytest.mark.parametrize("M,N,K", [(129, 512, 40960), (129, 512, 41088), (300, 128, 24576), (129, 520, 5072), (257, 264, 30000),
+                                   (500, 4104, 512), (1000, 2056, 1024), (2000, 2056, 1152), (3000, 3000, 640), (1025, 1025, 8192),
+                                   (1792, 18688, 128), (2048, 16384, 128)])
+@pytest.mark.parametrize("fmt", ["int8", "fp8", "fp16"])
+def test_plans_past_128_rows(cuda, fmt, M, N, K):
+    """int8 sums exact; fp8 and fp16 sums against fp64 within the accumulation tolerances used above."""
+    from llmqrt_amd.awq_kernels import gemm_f16
+    from llmqrt_amd.sq_fp8_kernels import cutlass_f8f8bf16_rowwise_sm89, w8a8_int8_linear_bbf16_obf16_per_channel
+    g = torch.Generator(device=cuda).manual_seed(M + N + K)
+    one_m, one_n = torch.ones(M, 1, device=cuda), torch.ones(1, N, device=cuda)
+    if fmt == "int8":
+        a = torch.randint(-128, 128, (M, K), dtype=torch.int8, device=cuda, generator=g)
+        b = torch.randint(-128, 128, (N, K), dtype=torch.int8, device=cuda, generator=g)
+        dump = torch.empty(M, N, dtype=torch.int32, device=cuda)
+        bias = torch.zeros(N, device=cuda, dtype=torch.bfloat16)
+        y = w8a8_int8_linear_bbf16_obf16_per_channel(a, b.t(), bias, one_m, one_n, _acc_dump=dump)
+    elif fmt == "fp8":
+        a = torch.randn(M, K, device=cuda, generator=g).to(torch.float8_e4m3fn)
+        b = torch.randn(N, K, device=cuda, generator=g).to(torch.float8_e4m3fn)
+        dump = torch.empty(M, N, dtype=torch.float32, device=cuda)
+        y = cutlass_f8f8bf16_rowwise_sm89(a, b.t(), None, one_m, one_n, True, _acc_dump=dump)
+    else:
+        a = torch.randn(M, K, device=cuda, generator=g).half()
+        b = torch.randn(N, K, device=cuda, generator=g).half()
+        dump = torch.empty(M, N, dtype=torch.float32, device=cuda)
+        y = gemm_f16(a, b, _acc_dump=dump)
+    acc = a.double() @ b.double().t()
+    if fmt == "int8":
+        assert torch.equal(dump.double(), acc)
+    else:
+        assert ((dump.double() - acc).abs().max() / acc.abs().max()).item() <= FP8_ACC_TOL
+    assert ((y.double() - acc).abs().max() / acc.abs().max()).item() <= REL_TOL

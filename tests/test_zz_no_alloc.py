@@ -63,3 +63,15 @@ def test_static_scratch_gemm_rejects_oversized_problems(cuda):
     assert L.llmq_gemm_workspace_bytes(M, N, K) > L.llmq_gemm_static_scratch_bytes()
     rc = L.llmq_gemm_w8a8_static(0x1000, K, 0x1000, K, None, None, 1.0, None, None, 0, 0.0, 0x1000, 0, N, M, N, K, None)
     assert rc == -7 and b"scratch" in L.llmq_status_string(rc)
+
+
+def test_static_scratch_takes_a_plan_that_fits(cuda):
+    """A problem whose fastest plan splits K past the array: the static entry point runs one that fits, with the same bits."""
+    from llmqrt_amd import _abi
+    L = _abi.lib()
+    M, N, K = 5603, 520, 14336
+    assert L.llmq_gemm_workspace_bytes(M, N, K) > L.llmq_gemm_static_scratch_bytes()
+    p = _problem(M, N, K, 3, cuda)
+    want = _run(L, _abi, False, p, M, N, K, cuda)
+    got = _run(L, _abi, True, p, M, N, K, cuda)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
