@@ -519,7 +519,7 @@ def test_module_many_token_path_is_own_kernels(cuda):
     assert rel_err(y.reshape(T, N), ref) <= REL_TOL
 
 
-# the plans behind the bf16 form: no split with one slice per block cannot occur; K splits with 1 (wide N), 2 and 4 slices,
+# the plans behind the bf16 form: K splits with 1 (wide N), 2 and 4 slices per block,
 # 4 slices without a split (wide N, 9-16 tokens), slabs of 16 with a ragged last one, a ragged last column tile
 @pytest.mark.parametrize("M,K,N,with_bias", [(1, 512, 32, True), (2, 3584, 1152, False), (5, 1024, 288, True), (16, 2304, 544, True),
                                              (3, 1536, 16640, True), (12, 768, 16640, False), (17, 1024, 1056, True), (64, 4864, 896, False)])

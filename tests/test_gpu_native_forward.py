@@ -230,3 +230,37 @@ def test_more_streams_than_counter_sets(cuda):
         assert y is None or torch.equal(y, ref), i
     assert kept == [True] * 256 + [False] * 2
     llmqrt_amd.release_workspaces()
+
+
+@pytest.mark.parametrize("M", [1, 5, 70, 300])
+@pytest.mark.parametrize("dtype,bias", [(torch.bfloat16, True), (torch.float16, False)])
+def test_contiguous_rows_take_the_native_call(cuda, M, dtype, bias, monkeypatch):
+    """What the comparisons of this file rest on: contiguous activations never reach the general path, strided ones do."""
+    from llmqrt_amd import norm as norm_module
+
+    class General(Exception):
+        pass
+
+    def general(*args, **kwargs):
+        raise General
+
+    wide = torch.randn(M, 1, K + 8, device=cuda, generator=torch.Generator(device="cuda").manual_seed(M)).to(dtype)
+    x, strided = wide[..., :K].contiguous(), wide[..., :K]
+    norm = norm_module.RMSNorm(torch.ones(K, device=cuda, dtype=dtype))
+    mods = _modules(dtype, bias)
+    for name in ("rmsnorm", "rmsnorm_per_token_quantize", "rmsnorm_quantize_activation_per_token_absmax"):
+        monkeypatch.setattr(norm_module, name, general)
+    calls = [norm, norm.forward_quantized, lambda t: norm.forward_quantized(t, fp8=True)]
+    for mod in mods.values():
+        monkeypatch.setattr(mod, "_forward_general", general)
+        calls.append(mod)
+    for call in calls:
+        call(x)
+        if M > 1:
+            with pytest.raises(General):
+                call(strided)
+    quantized = {"sq_channel": (torch.int8, (dtype,)), "fp8_token": (torch.float8_e4m3fn, ())}
+    for name, (qdtype, more) in quantized.items():
+        if name in mods:
+            monkeypatch.setattr(mods[name], "_forward_quantized_general", general)
+            mods[name].forward_quantized(x.to(qdtype), torch.ones(M, 1, 1, device=cuda), *more)
