@@ -264,3 +264,37 @@ def test_contiguous_rows_take_the_native_call(cuda, M, dtype, bias, monkeypatch)
         if name in mods:
             monkeypatch.setattr(mods[name], "_forward_quantized_general", general)
             mods[name].forward_quantized(x.to(qdtype), torch.ones(M, 1, 1, device=cuda), *more)
+
+
+def test_native_forward_from_threads(cuda):
+    """Four threads on a stream each share the modules and the counter pool while a fifth gives the pool back."""
+    import threading
+    from llmqrt_amd._native import host
+    mods = list(_modules(torch.bfloat16, True).items())
+    g = torch.Generator(device="cuda").manual_seed(6)
+    xs = [torch.randn(m, 1, K, device=cuda, generator=g).bfloat16() for m in (1, 4, 5, 70)]
+    refs = [[mod._forward_general(x) for _, mod in mods] for x in xs]
+    torch.cuda.synchronize()
+    wrong, done = [], threading.Event()
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(20):
+                ys = [mod(xs[i]) for _, mod in mods]
+                torch.cuda.current_stream().synchronize()
+                wrong.extend((i, name) for (name, _), y, ref in zip(mods, ys, refs[i]) if not torch.equal(y, ref))
+
+    def release():
+        while not done.wait(0.002):
+            host().release_tickets()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    releaser = threading.Thread(target=release)
+    releaser.start()
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    done.set()
+    releaser.join(10)
+    assert not wrong and not any(t.is_alive() for t in threads + [releaser])
