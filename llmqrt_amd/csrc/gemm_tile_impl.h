@@ -93,6 +93,15 @@ __device__ __forceinline__ void tile_coords(int bid, int nblk, int tiles_m, int 
     tn = (pid % width) / gsize;
 }
 
+// f(integral_constant<B>) .. f(integral_constant<E - 1>)
+template <int B, int E, class F>
+__device__ __forceinline__ void unrolled(F&& f) {
+    if constexpr (B < E) {
+        f(std::integral_constant<int, B>{});
+        unrolled<B + 1, E>(f);
+    }
+}
+
 template <class C, bool KFULL>
 __global__ __launch_bounds__(C::NT) void gemm_tile_kernel(
     const uint8_t* __restrict__ A, int64_t lda, const uint8_t* __restrict__ B, int64_t ldb,
@@ -179,51 +188,42 @@ __global__ __launch_bounds__(C::NT) void gemm_tile_kernel(
     // freshly published stage overlap the last MFMAs of the previous tile).
     using frag_t = typename std::conditional<C::FP8, v8i, v4i>::type;
     frag_t fa[C::PIPE ? 2 : 1][C::TM], fb[C::PIPE ? 2 : 1][C::TN];
-    auto read_frags = [&](int stage, int ks, frag_t* af, frag_t* bf) {
-        const uint4* sA = lds + stage * C::STAGE_CHUNKS;
-        const uint4* sB = sA + C::BM * C::CPR;
+    auto read_frag = [&](const uint4* src, int row, int ks, frag_t& f) __attribute__((always_inline)) {
         if constexpr (C::FP8) {
             const int c0 = ks * 4 + khalf * 2;
-#pragma unroll
-            for (int i = 0; i < C::TM; i++) {
-                const int row = a_row0 + i * 32;
-                const uint4 lo = sA[lds_chunk<C::CPR>(row, c0)], hi = sA[lds_chunk<C::CPR>(row, c0 + 1)];
-                af[i] = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-            }
-#pragma unroll
-            for (int j = 0; j < C::TN; j++) {
-                const int row = b_row0 + j * 32;
-                const uint4 lo = sB[lds_chunk<C::CPR>(row, c0)], hi = sB[lds_chunk<C::CPR>(row, c0 + 1)];
-                bf[j] = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-            }
+            const uint4 lo = src[lds_chunk<C::CPR>(row, c0)], hi = src[lds_chunk<C::CPR>(row, c0 + 1)];
+            f = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
         } else {
-            const int c0 = ks * 2 + khalf;
-#pragma unroll
-            for (int i = 0; i < C::TM; i++) {
-                const uint4 v = sA[lds_chunk<C::CPR>(a_row0 + i * 32, c0)];
-                af[i] = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
-            }
-#pragma unroll
-            for (int j = 0; j < C::TN; j++) {
-                const uint4 v = sB[lds_chunk<C::CPR>(b_row0 + j * 32, c0)];
-                bf[j] = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
-            }
+            const uint4 v = src[lds_chunk<C::CPR>(row, ks * 2 + khalf)];
+            f = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
         }
+    };
+    auto read_frag_a = [&](int stage, int ks, int i, frag_t& f) __attribute__((always_inline)) {
+        read_frag(lds + stage * C::STAGE_CHUNKS, a_row0 + i * 32, ks, f);
+    };
+    auto read_frag_b = [&](int stage, int ks, int j, frag_t& f) __attribute__((always_inline)) {
+        read_frag(lds + stage * C::STAGE_CHUNKS + C::BM * C::CPR, b_row0 + j * 32, ks, f);
+    };
+    auto read_frags = [&](int stage, int ks, frag_t* af, frag_t* bf) {
+#pragma unroll
+        for (int i = 0; i < C::TM; i++) read_frag_a(stage, ks, i, af[i]);
+#pragma unroll
+        for (int j = 0; j < C::TN; j++) read_frag_b(stage, ks, j, bf[j]);
+    };
+    auto mfma_one = [&](int i, int j, const frag_t* af, const frag_t* bf) __attribute__((always_inline)) {
+        if constexpr (C::FP8)
+            acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bf[j], af[i], acc[i][j], 0, C::AFMT, 0, 0, 0, 0);
+        else if constexpr (C::F16)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, bf[j]), __builtin_bit_cast(v8h, af[i]),
+                                                               acc[i][j], 0, 0, 0);
+        else
+            acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[j], af[i], acc[i][j], 0, 0, 0);
     };
     auto mfma_step = [&](const frag_t* af, const frag_t* bf) {
 #pragma unroll
         for (int i = 0; i < C::TM; i++)
 #pragma unroll
-            for (int j = 0; j < C::TN; j++) {
-                if constexpr (C::FP8)
-                    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bf[j], af[i], acc[i][j], 0, C::AFMT,
-                                                                                0, 0, 0, 0);
-                else if constexpr (C::F16)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, bf[j]), __builtin_bit_cast(v8h, af[i]),
-                                                                       acc[i][j], 0, 0, 0);
-                else
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[j], af[i], acc[i][j], 0, 0, 0);
-            }
+            for (int j = 0; j < C::TN; j++) mfma_one(i, j, af, bf);
     };
     // Scheduling directive for one sub-step: issue the LDS reads of the next fragments one by one
     // between the MFMAs of the current fragments (reads first), instead of after them.
@@ -313,69 +313,106 @@ __global__ __launch_bounds__(C::NT) void gemm_tile_kernel(
         // which would wait for every outstanding load before any later LDS read, does not see them.
         static_assert(C::KSUB % 2 == 0 && C::KSUB >= 2, "fragment parity must return to 0 at every tile");
         static_assert(KFULL, "the direct loads cannot zero a ragged K tail");
-        constexpr int LPT = C::A_LOADS + C::B_LOADS;  // loads per thread and tile
+        constexpr int NS = C::STAGES, LPT = C::A_LOADS + C::B_LOADS;  // loads per thread and tile
+        constexpr int SLOTS = C::TM * C::TN;                          // MFMAs per sub-step
+        constexpr int PER = (LPT + C::KSUB * SLOTS - 1) / (C::KSUB * SLOTS);  // loads requested behind one MFMA
+        constexpr int STEP = SLOTS * PER;                                     // ... and in one sub-step
+        // Global addresses: one scalar base per operand that moves along K, one 32-bit offset per piece that does not.
         const int swz = (ld_row / (16 / C::CPR)) & (C::CPR - 1);
-        const uint8_t* pa[C::A_LOADS];
-        const uint8_t* pb[C::B_LOADS];
+        uint32_t off[LPT];
 #pragma unroll
-        for (int i = 0; i < C::A_LOADS; i++) pa[i] = A + (int64_t)m0 * lda + k_begin + a_off[i] + (ld_c ^ swz) * 16;
+        for (int i = 0; i < C::A_LOADS; i++) off[i] = (uint32_t)a_off[i] + (uint32_t)((ld_c ^ swz) * 16);
 #pragma unroll
-        for (int i = 0; i < C::B_LOADS; i++) pb[i] = B + (int64_t)n0 * ldb + k_begin + b_off[i] + (ld_c ^ swz) * 16;
-        const uint32_t lds_base = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)smem_raw);
-        const uint32_t wave_off = (uint32_t)__builtin_amdgcn_readfirstlane(wave) * 1024u;
+        for (int i = 0; i < C::B_LOADS; i++) off[C::A_LOADS + i] = (uint32_t)b_off[i] + (uint32_t)((ld_c ^ swz) * 16);
+        const uint8_t* sA = A + (int64_t)m0 * lda + k_begin;
+        const uint8_t* sB = B + (int64_t)n0 * ldb + k_begin;
+        const uint32_t lds_base = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)smem_raw) +
+                                  (uint32_t)__builtin_amdgcn_readfirstlane(wave) * 1024u;
         // int32 accumulators (any summation order gives the same bits): every XCD starts its walk over K at another
         // eighth and wraps around (blockIdx.x % 8 is the XCD), so the eight L2s ask the fabric for different lines of the
         // shared panels at any moment instead of all for the same ones.  The blocks of one XCD stay in step, which is what
         // lets them share a panel through their L2.  fp32 accumulators keep the natural order: their bits would
         // otherwise depend on where in the grid a tile sits.
         const int krot = C::FACC ? 0 : (int)((blockIdx.x % kNumXcd) * (unsigned)ktiles / kNumXcd);
-        auto issue_tile = [&](int kt, int stage) {
-            int kr = min(kt, ktiles - 1) + krot;  // past the end: the last tile again, into a stage nobody reads
-            kr -= kr >= ktiles ? ktiles : 0;
-            const int koff = kr * C::BK;
-            const uint32_t sbase = lds_base + (uint32_t)stage * (C::STAGE_CHUNKS * 16u) + wave_off;
-#pragma unroll
-            for (int i = 0; i < C::A_LOADS; i++) {
-                const uint32_t m0v = sbase + (uint32_t)i * (C::NT * 16u);
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m0v), "v"(pa[i] + koff) : "memory", "m0");
-            }
-#pragma unroll
-            for (int i = 0; i < C::B_LOADS; i++) {
-                const uint32_t m0v = sbase + (uint32_t)(C::BM * C::CPR * 16) + (uint32_t)i * (C::NT * 16u);
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m0v), "v"(pb[i] + koff) : "memory", "m0");
-            }
+        int ld_kt = krot;  // K tile that the next loads fetch
+        auto issue = [&](int stage, auto d_c) __attribute__((always_inline)) {  // piece d of tile ld_kt into an LDS stage
+            constexpr int d = decltype(d_c)::value;
+            const uint8_t* base = (d < C::A_LOADS ? sA : sB) + (int64_t)ld_kt * C::BK;
+            const uint32_t voff = off[d], m0v = lds_base + (uint32_t)stage * (C::STAGE_CHUNKS * 16u) + (uint32_t)d * (C::NT * 16u);
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0v), "v"(voff), "s"(base) : "memory", "m0");
         };
-        constexpr int NS = C::STAGES;
-        auto wait_next_tile = [] {  // at most the NS - 2 youngest tiles may still be in flight
-            constexpr int N = (NS - 2) * LPT;
-            static_assert(N < 64, "vmcnt is a 6-bit counter");
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+        static_assert(C::A_LOADS * C::NT * 16 == C::BM * C::CPR * 16, "the B pieces follow the A pieces in a stage");
+        auto next_kt = [&]() __attribute__((always_inline)) { ld_kt = ld_kt + 1 == ktiles ? 0 : ld_kt + 1; };
+        // the tile behind the one being computed has landed when at most `younger` later tiles are still in flight
+        auto wait_next_tile = [](int younger) __attribute__((always_inline)) {
+            static_assert((NS - 2) * LPT < 64, "vmcnt is a 6-bit counter");
+            if (younger >= NS - 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * LPT) : "memory");
+            else if (NS > 3 && younger == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NS > 3 ? LPT : 0) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         };
-#pragma unroll
-        for (int t = 0; t < NS - 1; t++) issue_tile(t, t);
-        wait_next_tile();
+        // One sub-step: the fragments of the next one (sub-step ks_rd of stage rd) are read between the MFMAs of this one,
+        // and with LOAD the pieces D0 .. D0 + STEP - 1 of a later tile are requested, PER behind each.
+        // Requested all at once at the top of a tile they hold every wavefront until the CU's address path (16 clocks each) has
+        // taken them, with nothing queued for the matrix cores: us before / with the requests spread and the last, unread
+        // tiles not requested, weights out of HBM, int8 1000 x 4608 x 3584 32.1 / 30.0, 2048 x 4608 x 3584 50.8 / 44.1, 8192 x
+        // 37888 x 3584 996 / 975, fp8 512 x 37888 x 3584 93.0 / 88.7, 4096 x 3584 x 18944 249 / 226, fp16 777 x 3584 x 18944 140 / 132.
+        // (Level or slower: two requests behind an MFMA, s_setprio around the MFMAs, all fragment reads first.)
+        auto sub_step = [&](int rd, int ks_rd, auto par_c, auto d0_c, auto load_c, int ld_stage) __attribute__((always_inline)) {
+            constexpr int par = decltype(par_c)::value, D0 = decltype(d0_c)::value;
+            constexpr bool LOAD = decltype(load_c)::value && D0 < LPT;
+            unrolled<0, SLOTS>([&](auto m_c) __attribute__((always_inline)) {
+                constexpr int m = decltype(m_c)::value, FR = C::TM + C::TN, RPS = (FR + SLOTS - 1) / SLOTS;
+                unrolled<(m * RPS < FR ? m * RPS : FR), ((m + 1) * RPS < FR ? (m + 1) * RPS : FR)>([&](auto r_c) __attribute__((always_inline)) {
+                    constexpr int r = decltype(r_c)::value;  // the order of first use: A 0, B 0 .. TN - 1, A 1 ..
+                    if constexpr (r >= 1 && r <= C::TN) read_frag_b(rd, ks_rd, r - 1, fb[par ^ 1][r - 1]);
+                    else read_frag_a(rd, ks_rd, r ? r - C::TN : 0, fa[par ^ 1][r ? r - C::TN : 0]);
+                });
+                mfma_one(m / C::TN, m % C::TN, fa[par], fb[par]);
+                if constexpr (LOAD)
+                    unrolled<(D0 + m * PER < LPT ? D0 + m * PER : LPT), (D0 + (m + 1) * PER < LPT ? D0 + (m + 1) * PER : LPT)>(
+                        [&](auto d) __attribute__((always_inline)) { issue(ld_stage, d); });
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        };
+        unrolled<0, NS - 1>([&](auto t_c) __attribute__((always_inline)) {
+            constexpr int t = decltype(t_c)::value;
+            if (t < ktiles) {
+                unrolled<0, LPT>([&](auto d) __attribute__((always_inline)) { issue(t, d); });
+                next_kt();
+            }
+        });
+        wait_next_tile(min(ktiles, NS - 1) - 1);
         lds_barrier();
         read_frags(0, 0, fa[0], fb[0]);
-        int stage = 0;
-#pragma unroll 1
-        for (int kt = 0; kt < ktiles; kt++) {
+        // the stage NS - 1 is free from the start: the part of its tile that the loop requests behind a barrier comes first
+        if (NS - 1 < ktiles)
+            unrolled<0, (STEP < LPT ? STEP : LPT)>([&](auto d) __attribute__((always_inline)) { issue(NS - 1, d); });
+        int stage = 0, kt = 0;
+        // rest: the part of tile kt + NS - 1 that the last iteration did not request; first: tile kt + NS exists
+        auto k_tile = [&](auto rest_c, auto first_c) __attribute__((always_inline)) {
             const int prev = stage == 0 ? NS - 1 : stage - 1, next = stage == NS - 1 ? 0 : stage + 1;
-            issue_tile(kt + NS - 1, prev);  // the stage of tile kt-1: every wavefront passed the last barrier after reading it
-#pragma unroll
-            for (int ks = 0; ks < C::KSUB - 1; ks++) {
-                read_frags(stage, ks + 1, fa[(ks + 1) & 1], fb[(ks + 1) & 1]);
-                mfma_step(fa[ks & 1], fb[ks & 1]);
-                interleave_reads_with_mfma();
-                __builtin_amdgcn_sched_barrier(0);
+            unrolled<0, C::KSUB - 1>([&](auto ks_c) __attribute__((always_inline)) {
+                constexpr int ks = decltype(ks_c)::value;
+                sub_step(stage, ks + 1, std::integral_constant<int, ks & 1>{}, std::integral_constant<int, (ks + 1) * STEP>{}, rest_c, prev);
+            });
+            if constexpr (decltype(rest_c)::value) {
+                next_kt();
+                wait_next_tile(NS - 2);
+            } else {
+                wait_next_tile(ktiles - 2 - kt);  // tile kt+1 has landed
             }
-            wait_next_tile();  // tile kt+1 has landed
             lds_barrier();
-            read_frags(next, 0, fa[0], fb[0]);
-            mfma_step(fa[(C::KSUB - 1) & 1], fb[(C::KSUB - 1) & 1]);
-            interleave_reads_with_mfma();
-            __builtin_amdgcn_sched_barrier(0);
+            // every wavefront has read the whole of stage kt: it takes tile kt + NS
+            sub_step(next, 0, std::integral_constant<int, (C::KSUB - 1) & 1>{}, std::integral_constant<int, 0>{}, first_c, stage);
             stage = next;
-        }
+            kt++;
+        };
+#pragma unroll 1
+        while (kt < ktiles - NS) k_tile(std::true_type{}, std::true_type{});
+        if (kt == ktiles - NS) k_tile(std::true_type{}, std::false_type{});
+        // Past the last request nothing is fetched: a block that ends waits for no load that nobody reads.
+#pragma unroll 1
+        while (kt < ktiles) k_tile(std::false_type{}, std::false_type{});
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be landing in LDS when it is reused or released
         lds_barrier();
     } else if constexpr (C::RS == 2) {
