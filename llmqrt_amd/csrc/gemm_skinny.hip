@@ -29,6 +29,7 @@ struct SkinnyEpilogue {
     const void* bias;        // [N] or null
     float alpha, beta;
     int bias_dtype, out_dtype;
+    const float* out_scale;  // device scalar or null: out is fp32 and holds the value after a round trip through e4m3fn on it
 };
 
 namespace {
@@ -50,6 +51,10 @@ __global__ __launch_bounds__(NW * kWave) void gemm_skinny_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int r16 = lane & 15, kq = lane >> 4;
     const int n0 = blockIdx.x * (16 * T);
+    // token slab of 16 * MT rows
+    const int row0 = blockIdx.y * (16 * MT);
+    A += (int64_t)row0 * lda;
+    M -= row0;
     const int steps = (K + KSTEP - 1) / KSTEP, spw = (steps + NW - 1) / NW;
     const int s_begin = min(steps, wave * spw), s_end = min(steps, s_begin + spw);
 
@@ -142,8 +147,8 @@ __global__ __launch_bounds__(NW * kWave) void gemm_skinny_kernel(
 #pragma unroll
         for (int w = 1; w < NW; w++) sum += red[w][q][l];
         // lane l of that accumulator: token 16 mt + l % 16, channels n0 + 16 t + 4 (l / 16) .. + 3
-        const int m = 16 * mt + (l & 15), n = n0 + 16 * t + 4 * (l >> 4);
-        if (m >= M || n >= N) continue;
+        const int ml = 16 * mt + (l & 15), m = row0 + ml, n = n0 + 16 * t + 4 * (l >> 4);
+        if (ml >= M || n >= N) continue;
         const float sa = ep.a_scale ? ep.a_scale[m] : 1.f;
         uint16_t h[4];
 #pragma unroll
@@ -155,7 +160,15 @@ __global__ __launch_bounds__(NW * kWave) void gemm_skinny_kernel(
             h[e] = ep.out_dtype == LLMQ_BF16 ? Lo<LLMQ_BF16>::from_f32(v) : Lo<LLMQ_F16>::from_f32(v);
         }
         uint16_t* orow = reinterpret_cast<uint16_t*>(out) + (int64_t)m * ldo + n;
-        if (n + 3 < N && ((reinterpret_cast<uintptr_t>(orow) & 7u) == 0)) {
+        if (ep.out_scale) {
+            float* frow = reinterpret_cast<float*>(out) + (int64_t)m * ldo + n;
+            const float os = *ep.out_scale;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float f = ep.out_dtype == LLMQ_BF16 ? Lo<LLMQ_BF16>::to_f32(h[e]) : Lo<LLMQ_F16>::to_f32(h[e]);
+                if (n + e < N) frow[e] = fp8_round_trip(f, os);
+            }
+        } else if (n + 3 < N && ((reinterpret_cast<uintptr_t>(orow) & 7u) == 0)) {
             *reinterpret_cast<uint2*>(orow) = make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
         } else {
 #pragma unroll
@@ -179,7 +192,7 @@ void launch_skinny_d(const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ld
     // steps per batch: about 96 to 128 registers for the two batches in flight
     constexpr int D = FP8 ? (MT == 4 ? 1 : 2) : (MT == 4 ? 2 : 4);
     const int blocks = (N + 16 * T - 1) / (16 * T);
-    hipLaunchKernelGGL((gemm_skinny_kernel<FP8, AFMT, MT, T, NW, D>), dim3(blocks), dim3(NW * kWave), 0, st, A, lda, B, ldb, M,
+    hipLaunchKernelGGL((gemm_skinny_kernel<FP8, AFMT, MT, T, NW, D>), dim3(blocks, (M + 16 * MT - 1) / (16 * MT)), dim3(NW * kWave), 0, st, A, lda, B, ldb, M,
                        N, K, ep, out, ldo, acc_dump);
 }
 
@@ -201,13 +214,11 @@ void launch_skinny_mt(int t, int nw, const uint8_t* A, int64_t lda, const uint8_
 
 }  // namespace
 
-bool gemm_skinny_supported(int64_t M) { return M >= 1 && M <= 64; }
-
-// t: 16-channel tiles per wavefront (1 | 2), nw: wavefronts per block (4 | 8 | 16); a_format: 0 e4m3, 1 e5m2 (fp8 only)
-int launch_gemm_skinny(bool fp8, int a_format, int t, int nw, const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ldb,
+// mt: 16-token tiles per block (1 | 2 | 4), t: 16-channel tiles per wavefront (1 | 2), nw: wavefronts per block (4 | 8 | 16; 4 | 8 for
+// mt = 4 and t = 2); a_format: 0 e4m3, 1 e5m2 (fp8 only)
+int launch_gemm_skinny(bool fp8, int a_format, int mt, int t, int nw, const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ldb,
                        int M, int N, int K, const SkinnyEpilogue& ep, void* out, int64_t ldo, void* acc_dump,
                        hipStream_t st) {
-    const int mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
 #define LLMQ_SK_MT(FP8_, AF_)                                                                                       \
     do {                                                                                                            \
         if (mt == 1) launch_skinny_mt<FP8_, AF_, 1>(t, nw, A, lda, B, ldb, M, N, K, ep, out, ldo, acc_dump, st);      \

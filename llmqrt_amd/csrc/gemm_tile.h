@@ -21,10 +21,12 @@ struct Epilogue {
 };
 
 struct Plan {
-    int cfg;     // index into the config table
+    int cfg;     // index into the config table; kSkinnyCfg + v: the few-token kernel
     int splits;  // K splits (1 = fused epilogue)
     int k_per_split;
+    int mt = 0;  // few-token kernel: 16-token tiles per block
 };
+constexpr int kSkinnyCfg = 100;  // + v: 1 + (v & 1) channel tiles per wavefront, 4 << (v >> 1) wavefronts per block
 
 constexpr int kNumCu = 256;
 inline int cdiv(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
@@ -38,6 +40,9 @@ constexpr TileShape kShapes[] = {
     {32, 128, 128},   // 5: 4 waves x (32x32), decode
     {256, 256, 128},  // 6: 8 waves x (128x64), whole 128-byte lines per row (fp8 prefill)
     {128, 256, 128},  // 7: 8 waves x (64x64): twice the tiles of config 6 for grids that would leave CUs idle
+    {128, 128, 128},  // 8: 8 waves x (64x32)  } direct loads only: K in whole 128-byte tiles
+    {192, 128, 128},  // 9: 8 waves x (96x32)  }
+    {256, 128, 128},  // 10: 8 waves x (64x64) }
 };
 constexpr int kNumShapes = sizeof(kShapes) / sizeof(kShapes[0]);
 

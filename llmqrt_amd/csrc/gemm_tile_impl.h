@@ -537,6 +537,64 @@ __global__ __launch_bounds__(C::NT) void gemm_tile_kernel(
                 }
                 return;
             }
+            // 128-channel tiles whose wavefronts own less than 64 x 64: the finished tile is put together in LDS and the block stores whole
+            // 256-byte rows.  Stored from the registers, a row of such a wavefront is two pieces of 32 bytes of a line (us, from registers /
+            // through LDS: int8 6831 x 2432 x 896 34.8 / 31.6 with 192x128, 36.5 / 31.5 with 128x128, 34.1 / 30.3 with 64x128 tiles, fp8 512 x
+            // 3584 x 3584 16.8 / 16.1, 512 x 4608 x 3584 20.2 / 19.5).
+            constexpr bool BLOCK_EPI = C::DMA && C::BN == 128 && C::LDS_BYTES >= (size_t)C::BM * C::BN * 2u;
+            if constexpr (BLOCK_EPI) {
+                float sa_r[C::TM], sw_r[C::TN][16], bb_r[C::TN][16];  // fetched before any store is issued (see above)
+#pragma unroll
+                for (int i = 0; i < C::TM; i++) sa_r[i] = ep.a_scale ? ep.a_scale[m0 + wm * C::WTM + i * 32 + l32] : 1.f;
+#pragma unroll
+                for (int j = 0; j < C::TN; j++)
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        const int n = n0 + wn * C::WTN + j * 32 + 8 * g + 4 * khalf;
+                        const float4 v = ep.w_scale ? *reinterpret_cast<const float4*>(ep.w_scale + n) : make_float4(1.f, 1.f, 1.f, 1.f);
+                        sw_r[j][4 * g] = v.x, sw_r[j][4 * g + 1] = v.y, sw_r[j][4 * g + 2] = v.z, sw_r[j][4 * g + 3] = v.w;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) bb_r[j][4 * g + e] = ep.bias ? ep.beta * load_as_f32(ep.bias, ep.bias_dtype, n + e) : 0.f;
+                    }
+                // (the barrier behind the main loop: every wavefront is done reading the operand stages)
+#pragma unroll
+                for (int i = 0; i < C::TM; i++)
+#pragma unroll
+                    for (int j = 0; j < C::TN; j++) {
+                        const int row = wm * C::WTM + i * 32 + l32;
+                        uint32_t pk[4][2];
+#pragma unroll
+                        for (int g = 0; g < 4; g++) {
+                            uint16_t h[4];
+#pragma unroll
+                            for (int e = 0; e < 4; e++) {
+                                const auto av = acc[i][j][4 * g + e];
+                                h[e] = Lo<ODT>::from_f32(epi_value<PLAIN>((float)av, sa_r[i], sw_r[j][4 * g + e], alpha, bb_r[j][4 * g + e]));
+                            }
+                            pk[g][0] = (uint32_t)h[0] | ((uint32_t)h[1] << 16);
+                            pk[g][1] = (uint32_t)h[2] | ((uint32_t)h[3] << 16);
+                        }
+#pragma unroll
+                        for (int g = 0; g < 2; g++) {
+#pragma unroll
+                            for (int x = 0; x < 2; x++) {
+                                const auto sw2 = __builtin_amdgcn_permlane32_swap(pk[2 * g][x], pk[2 * g + 1][x], false, false);
+                                pk[2 * g][x] = sw2[0];
+                                pk[2 * g + 1][x] = sw2[1];
+                            }
+                            const int chunk = (wn * C::WTN + j * 32) / 8 + 2 * g + khalf;  // 8 channels = 16 bytes; 16 rows of a column hit 16 places
+                            lds[row * 16 + (chunk ^ (row & 15))] = make_uint4(pk[2 * g][0], pk[2 * g][1], pk[2 * g + 1][0], pk[2 * g + 1][1]);
+                        }
+                    }
+                __syncthreads();
+                uint16_t* obase = reinterpret_cast<uint16_t*>(out) + (int64_t)m0 * ldo + n0;
+#pragma unroll
+                for (int it = 0; it < C::BM * 16 / C::NT; it++) {
+                    const int q = it * C::NT + tid, row = q >> 4, c = q & 15;
+                    store_streaming(obase + (int64_t)row * ldo + 8 * c, lds[row * 16 + (c ^ (row & 15))]);
+                }
+                return;
+            }
             float sa_r[C::TM];  // fetched before any store is issued (see above)
 #pragma unroll
             for (int i = 0; i < C::TM; i++) sa_r[i] = ep.a_scale ? ep.a_scale[m0 + wm * C::WTM + i * 32 + l32] : 1.f;
@@ -819,6 +877,9 @@ int launch_shape(const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ldb, i
         case 4: return launch_cfg<GemmCfg<64, 128, 128, 2, 2, FP8, AFMT, 2, DMA>>(A, lda, B, ldb, M, N, K, p, ep, out, ldo, acc_dump, ws, st);
         case 6: return launch_cfg<GemmCfg<256, 256, 128, 2, 4, FP8, AFMT, 1, DMA>>(A, lda, B, ldb, M, N, K, p, ep, out, ldo, acc_dump, ws, st);
         case 7: return launch_cfg<GemmCfg<128, 256, 128, 2, 4, FP8, AFMT, 1, DMA>>(A, lda, B, ldb, M, N, K, p, ep, out, ldo, acc_dump, ws, st);
+        case 8: if constexpr (DMA) return launch_cfg<GemmCfg<128, 128, 128, 2, 4, FP8, AFMT, 1, true>>(A, lda, B, ldb, M, N, K, p, ep, out, ldo, acc_dump, ws, st);
+        case 9: if constexpr (DMA) return launch_cfg<GemmCfg<192, 128, 128, 2, 4, FP8, AFMT, 1, true>>(A, lda, B, ldb, M, N, K, p, ep, out, ldo, acc_dump, ws, st);
+        case 10: if constexpr (DMA) return launch_cfg<GemmCfg<256, 128, 128, 4, 2, FP8, AFMT, 1, true>>(A, lda, B, ldb, M, N, K, p, ep, out, ldo, acc_dump, ws, st);
         default: return launch_cfg<GemmCfg<32, 128, 128, 1, 4, FP8, AFMT, 2, DMA>>(A, lda, B, ldb, M, N, K, p, ep, out, ldo, acc_dump, ws, st);
     }
 }
@@ -831,8 +892,10 @@ int launch_gemm(const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ldb, in
     // the 64-byte K tiles have a single sub-step there and stay register-staged.
     const int bk = kShapes[p.cfg].bk;
     const bool dma = allow_dma && K % bk == 0 && p.k_per_split % bk == 0;
+    Plan staged = p;  // tiles that exist with direct loads only: a forced plan on a ragged K takes the staged tile next in size
+    if (p.cfg >= 8) staged.cfg = p.cfg == 8 ? 3 : 2;
     int rc = dma ? launch_shape<FP8, AFMT, true>(A, lda, B, ldb, M, N, K, p, ep, out, ldo, acc_dump, ws, st)
-                 : launch_shape<FP8, AFMT, false>(A, lda, B, ldb, M, N, K, p, ep, out, ldo, acc_dump, ws, st);
+                 : launch_shape<FP8, AFMT, false>(A, lda, B, ldb, M, N, K, staged, ep, out, ldo, acc_dump, ws, st);
     if (rc != LLMQ_OK || p.splits == 1) return rc;
     constexpr bool kF32 = FP8 || AFMT == 2;
     const int64_t total = (int64_t)M * N;

@@ -1,0 +1,79 @@
+"""Few-token GEMM in slabs of tokens (17 and more tokens, few channels) and the tiles of whole 128-byte lines, at the edges of slabs, tiles and
+of the sizes where the planner lets them compete."""
+import pytest
+import torch
+
+from oracle import ref_math as R
+
+pytestmark = pytest.mark.gpu
+
+# 16-, 32- and 64-token slabs with a full, a one-row and a ragged last slab; ragged channels; short and long K; both sides of
+# the token and channel limits
+SHAPES = [(60, 640, 1664), (40, 1152, 6528), (45, 1160, 1280), (17, 520, 2048), (33, 1000, 1536), (65, 768, 1664), (82, 776, 1664),
+          (128, 2048, 896), (129, 1024, 896), (200, 512, 3584), (256, 1024, 1024), (257, 1024, 1024), (5, 1024, 18944), (64, 8192, 896)]
+
+
+def _ints(shape, seed, dtype=torch.int8):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randint(-127, 128, shape, generator=g, dtype=torch.int32).to(dtype)
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_int8_accumulators_exact(cuda, M, N, K):
+    from llmqrt_amd.sq_fp8_kernels import w8a8_int8_linear_bbf16_obf16_per_channel
+    g = torch.Generator().manual_seed(M + N)
+    qx, qw = _ints((M, K), M), _ints((N, K), N)
+    sx, sw = torch.rand(M, generator=g) * 0.01 + 1e-3, torch.rand(N, generator=g) * 0.01 + 1e-3
+    bias = torch.randn(N, generator=g).bfloat16()
+    acc = R.int8_gemm_exact(qx, qw)
+    dump = torch.full((M, N), -1, dtype=torch.int32, device=cuda)
+    args = (qx.to(cuda), qw.to(cuda).t(), bias.to(cuda), sx.to(cuda).view(-1, 1), sw.to(cuda).view(1, -1))
+    y = w8a8_int8_linear_bbf16_obf16_per_channel(*args, _acc_dump=dump)
+    assert torch.equal(dump.cpu(), acc)
+    ref = R.w8a8_epilogue_per_token_per_channel(acc, sx, sw, bias, torch.bfloat16)
+    assert torch.equal(y.cpu().view(torch.int16), ref.view(torch.int16))
+    assert torch.equal(w8a8_int8_linear_bbf16_obf16_per_channel(*args).view(torch.int16), y.view(torch.int16))
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_fp8_with_and_without_output_quantization(cuda, M, N, K):
+    """The GEMM against float64 (fp8 products are exact; 2e-4 of the largest is what the matrix cores' accumulation window loses, half a
+    bf16 step the output), then its quantized output against the three steps on that GEMM result, bit for bit."""
+    from llmqrt_amd.quantize import static_per_tensor_quantize
+    from llmqrt_amd.sq_fp8_kernels import cutlass_f8f8bf16_tensorwise_sm89, f8f8_tensorwise_quantized_output
+    g = torch.Generator().manual_seed(M * N)
+    a = (torch.randn(M, K, generator=g) * 30).clamp(-448, 448).to(torch.float8_e4m3fn)
+    b = (torch.randn(N, K, generator=g) * 30).clamp(-448, 448).to(torch.float8_e4m3fn)
+    bias = (50 * torch.randn(N, generator=g)).bfloat16()
+    alpha = torch.tensor(0.01)
+    ref = a.double() @ b.double().t() * 0.01 + bias.double()
+    y = cutlass_f8f8bf16_tensorwise_sm89(a.to(cuda), b.to(cuda).t(), bias.to(cuda), alpha.to(cuda), 1.0, "bfloat16")
+    assert ((y.cpu().double() - ref).abs() <= 2e-4 * ref.abs().max() + ref.abs() / 256).all()
+    scale = torch.tensor([float(ref.abs().max()) / 300], device=cuda)
+    q = static_per_tensor_quantize(y, scale)
+    want = q.to(torch.bfloat16).float() * scale
+    got = f8f8_tensorwise_quantized_output(a.to(cuda), b.to(cuda).t(), bias.to(cuda), alpha.to(cuda), 1.0, "bfloat16", scale)
+    assert got.dtype == torch.float32 and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("cfg", [4, 5, 8, 9, 10])
+@pytest.mark.parametrize("M,N,K", [(192, 128, 128), (193, 256, 256), (384, 384, 384), (127, 136, 512), (576, 120, 1152)])
+@pytest.mark.parametrize("splits", [1, 2])
+def test_tiles_of_whole_lines(cuda, cfg, M, N, K, splits):
+    """One to nine K tiles (fewer and more than LDS stages), interior and edge tiles of the block-wide epilogue, fp16 output with bias."""
+    from llmqrt_amd import _abi
+    from llmqrt_amd.sq_fp8_kernels import w8a8_int8_linear_bbf16_obf16_per_channel
+    if K // splits < 128:
+        pytest.skip("a split holds at least one K tile")
+    qx, qw = _ints((M, K), 1), _ints((N, K), 2)
+    g = torch.Generator().manual_seed(3)
+    sx, sw, bias = torch.rand(M, generator=g) * 1e-3, torch.rand(N, generator=g) * 1e-2, torch.randn(N, generator=g).half()
+    ref = R.w8a8_epilogue_per_token_per_channel(R.int8_gemm_exact(qx, qw), sx, sw, bias, torch.float16)
+    L = _abi.lib()
+    _abi.check(L.llmq_gemm_force_plan(cfg, splits), "force_plan")
+    try:
+        y = w8a8_int8_linear_bbf16_obf16_per_channel(qx.to(cuda), qw.to(cuda).t(), bias.to(cuda), sx.to(cuda).view(-1, 1),
+                                                     sw.to(cuda).view(1, -1))
+    finally:
+        L.llmq_gemm_force_plan(-1, 1)
+    assert torch.equal(y.cpu().view(torch.int16), ref.view(torch.int16))
