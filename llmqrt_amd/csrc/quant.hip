@@ -408,16 +408,29 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_quant_rows_wave_kernel(
 // (quantizer) / 9.7 us (RMSNorm + quantizer) against 9.3 / 13.7 us for a block per row; at K = 3584 a block per row is
 // ahead by 5 % (17.2 against 18.0 us) and by 1.3 us at a few rows, so longer rows keep it.
 inline bool wave_rows(int64_t M, int64_t K) { return (K >> 3) <= 2 * kWave && M >= 256; }
-// Rows of 257-512 chunks (K = 3584: 448) with enough rows to fill the chip run on half-size blocks with four chunks
-// per thread: the per-row arithmetic that every wavefront repeats (two reductions, the scale, its reciprocal) is spread
-// over twice the elements.  Fused RMSNorm + int8 quantizer at 8192 x 3584 from HBM: 21.6 us against 23.6.
-inline bool half_blocks(int64_t M, int64_t K) { return (K >> 3) > kThreads && (K >> 3) <= 2 * kThreads && M >= 256; }
+// A block per row: threads and chunks per thread, by how many rows have to fill the chip.  A few rows are a chain of latencies (load, two
+// reductions, codes), which more threads with less each shorten; many rows are arithmetic that every wavefront repeats per row (reductions,
+// scale, reciprocal), which fewer threads with more each spread over more elements.  Fused RMSNorm + int8 quantizer / quantizer alone, us:
+//   257-512 chunks (K = 3584)    512 x 1      256 x 2      128 x 4          1025-2560 chunks (K = 18944)   1024 x 3      512 x 5     256 x 10
+//   32 rows                      3.19 / 2.68  3.41 / 2.74  3.42 / 2.72      32 rows                        5.14 / 3.75   5.19 / 3.79  6.41 / 3.99
+//   256                          3.57 / 3.03  3.79 / 3.09  4.30 / 3.31      128                            5.90 / 4.47   5.96 / 4.49  7.20 / 4.74
+//   512                          4.43 / 3.61  4.36 / 3.60  5.01 / 3.94      512                           10.65 / 8.14  10.34 / 8.22  11.2 / 8.51
+//   2048                         9.20 / 7.06  8.13 / 6.35  8.47 / 6.68      2048                           32.0 / 21.2   31.3 / 20.6  31.0 / 20.4
+//   8192                         --           23.6 / --    21.6 / --
+enum RowShape { R512x1, R256x1, R256x2, R128x4, R256x4, R1024x3, R512x5, R256x10, RLong };
+inline RowShape row_shape(int64_t M, int64_t K) {
+    const int64_t chunks = K >> 3;
+    if (chunks <= 256) return R256x1;
+    if (chunks <= 512) return M < 400 ? R512x1 : M < 6144 ? R256x2 : R128x4;
+    if (chunks <= 1024) return R256x4;
+    if (chunks <= 2560) return M <= 256 ? R1024x3 : M <= 1024 ? R512x5 : R256x10;
+    return RLong;
+}
 
 template <int DT, int QMODE>
 int launch_norm(const void* x, int64_t M, int64_t K, int64_t ldx, const void* weight, float eps, void* y, void* q,
                 void* scale, int scale_dtype, float* inv_out, hipStream_t st) {
     const dim3 grid((unsigned)M), block(kThreads);
-    const int64_t per_thread = ((K >> 3) + kThreads - 1) / kThreads;
     if (wave_rows(M, K)) {
         const dim3 wgrid((unsigned)((M + kNW - 1) / kNW));
         const int64_t per_lane = ((K >> 3) + kWave - 1) / kWave;
@@ -432,14 +445,17 @@ int launch_norm(const void* x, int64_t M, int64_t K, int64_t ldx, const void* we
 #define LLMQ_LAUNCH_NCT(NC, NT)                                                                                          \
     hipLaunchKernelGGL((rmsnorm_quant_rows_kernel<DT, QMODE, NC, NT>), grid, dim3(NT), 0, st, (const uint16_t*)x, ldx, K, \
                        (const uint16_t*)weight, eps, (uint16_t*)y, (uint8_t*)q, scale, scale_dtype, inv_out)
-#define LLMQ_LAUNCH_NC(NC) LLMQ_LAUNCH_NCT(NC, kThreads)
-    if (half_blocks(M, K)) LLMQ_LAUNCH_NCT(4, kThreads / 2);
-    else if (per_thread <= 1) LLMQ_LAUNCH_NC(1);
-    else if (per_thread <= 2) LLMQ_LAUNCH_NC(2);
-    else if (per_thread <= 4) LLMQ_LAUNCH_NC(4);
-    else if (per_thread <= 10) LLMQ_LAUNCH_NC(10);
-    else LLMQ_LAUNCH_NC(0);
-#undef LLMQ_LAUNCH_NC
+    switch (row_shape(M, K)) {
+        case R512x1: LLMQ_LAUNCH_NCT(1, 512); break;
+        case R256x1: LLMQ_LAUNCH_NCT(1, 256); break;
+        case R256x2: LLMQ_LAUNCH_NCT(2, 256); break;
+        case R128x4: LLMQ_LAUNCH_NCT(4, 128); break;
+        case R256x4: LLMQ_LAUNCH_NCT(4, 256); break;
+        case R1024x3: LLMQ_LAUNCH_NCT(3, 1024); break;
+        case R512x5: LLMQ_LAUNCH_NCT(5, 512); break;
+        case R256x10: LLMQ_LAUNCH_NCT(10, 256); break;
+        default: LLMQ_LAUNCH_NCT(0, 256);
+    }
 #undef LLMQ_LAUNCH_NCT
     return launch_status();
 }
@@ -474,7 +490,6 @@ int launch_rows(const void* x, int64_t M, int64_t K, int64_t ldx, void* q, void*
     const dim3 grid((unsigned)M), block(kThreads);
     const uint16_t* xp = (const uint16_t*)x;
     uint8_t* qp = (uint8_t*)q;
-    const int64_t per_thread = ((K >> 3) + kThreads - 1) / kThreads;
     if (SCALE == SCALE_ROW && wave_rows(M, K)) {
         const dim3 wgrid((unsigned)((M + kNW - 1) / kNW));
         const int64_t per_lane = ((K >> 3) + kWave - 1) / kWave;
@@ -487,15 +502,18 @@ int launch_rows(const void* x, int64_t M, int64_t K, int64_t ldx, void* q, void*
     }
 #define LLMQ_LAUNCH_NCT(NC, NT) \
     hipLaunchKernelGGL((quant_rows_kernel<DT, MODE, SCALE, NC, NT>), grid, dim3(NT), 0, st, xp, ldx, K, qp, scale, scale_dtype, aux, n_aux, static_f32, floor, ta)
-#define LLMQ_LAUNCH_NC(NC) LLMQ_LAUNCH_NCT(NC, kThreads)
-    if (SCALE != SCALE_ROW) LLMQ_LAUNCH_NC(0);
-    else if (half_blocks(M, K)) LLMQ_LAUNCH_NCT(4, kThreads / 2);
-    else if (per_thread <= 1) LLMQ_LAUNCH_NC(1);
-    else if (per_thread <= 2) LLMQ_LAUNCH_NC(2);
-    else if (per_thread <= 4) LLMQ_LAUNCH_NC(4);
-    else if (per_thread <= 10) LLMQ_LAUNCH_NC(10);
-    else LLMQ_LAUNCH_NC(0);
-#undef LLMQ_LAUNCH_NC
+    if constexpr (SCALE != SCALE_ROW) LLMQ_LAUNCH_NCT(0, kThreads);
+    else switch (row_shape(M, K)) {
+        case R512x1: LLMQ_LAUNCH_NCT(1, 512); break;
+        case R256x1: LLMQ_LAUNCH_NCT(1, 256); break;
+        case R256x2: LLMQ_LAUNCH_NCT(2, 256); break;
+        case R128x4: LLMQ_LAUNCH_NCT(4, 128); break;
+        case R256x4: LLMQ_LAUNCH_NCT(4, 256); break;
+        case R1024x3: LLMQ_LAUNCH_NCT(3, 1024); break;
+        case R512x5: LLMQ_LAUNCH_NCT(5, 512); break;
+        case R256x10: LLMQ_LAUNCH_NCT(10, 256); break;
+        default: LLMQ_LAUNCH_NCT(0, 256);
+    }
     return launch_status();
 }
 
