@@ -314,6 +314,9 @@ Plan make_plan(int op, int64_t M, int64_t N, int64_t K) {
     const Plan plan = few ? skinny(skinny_mt(M), t, nw, K) : tile_plan(op, M, N, K);
     if (g_force_cfg >= 0 || !slab_problem(op, M, N, K)) return plan;
     if (op == kStaticInt8 && partials_bytes(plan, M, N) > kStaticScratchBytes) return plan;  // refused, as before
+    // Sixteen wavefronts along a K of a few thousand in one block row: measured best there (slabs 8 % slower in the mean at 33-64 tokens of
+    // more than 3000 channels, level at 2049-3000; 18-43 % faster with fewer channels, 40 % with a longer K).
+    if (few && M > 32 && N > 2048 && K > 2048 && K <= 4096) return plan;
     // The plan of the rules stays unless another is modelled as clearly faster.
     double now = 1e300, best_t;
     if (few) now = skinny_time(op, M, N, K, skinny_mt(M), t, nw);
@@ -331,7 +334,9 @@ Plan make_plan(int op, int64_t M, int64_t N, int64_t K) {
     }
     // By a tenth (2.1 % of 8600 random problems here end more than 5 % behind the rules, against 4.0 % without a margin, for 1.113 of the
     // 1.118 in the mean), by more where the rules pick the few-token kernel themselves: most of those were such problems with a short K.
-    return best_t < (few ? (K <= 1024 ? 0.75 : 0.85) : 0.9) * now ? best : plan;
+    // A K split gives way to one launch of slabs at the same modelled time: the gap before its finishing launch is not in the model.
+    const bool one_launch = best.cfg >= kSkinnyCfg && plan.splits > 1;
+    return best_t < (few ? (K <= 1024 ? 0.75 : 0.85) : one_launch ? 1.0 : 0.9) * now ? best : plan;
 }
 
 // Searching a plan takes microseconds of host time and a call needs it for its workspace and for its launch, so each host
