@@ -85,7 +85,7 @@ inline bool table_problem(int op, int64_t M, int64_t N, int64_t K) {  // K in by
     return M > (K % 128 ? 128 : 64) && (int64_t)cdiv(M, 256) * cdiv(N, 256) < 2 * kNumCu && K <= kTableMaxK * (op == 2 ? 2 : 1);
 }
 
-// K in whole 128-byte tiles, more than 64 rows: every operand goes global -> LDS directly.  Time (us) of a launch of x * 256
+// More than 64 rows of whole 128-byte lines, more than 128 of others (whose K tail goes through registers).  Time (us) of a launch of x * 256
 // blocks over `steps` times 64 bytes of K: each round of 256 blocks takes steps * step + fixed, a partly filled one with a share f
 // of the CUs steps * step * (lo + (1 - lo) f) + fixed (fewer blocks share the supply and the clock is higher); the 64- and 32-row tiles
 // share a CU: a block beside another takes `first` of its time.  Otherwise `first` is paid once.  The weights bound a launch from below (weights us per MB + base),
@@ -168,8 +168,8 @@ bool slab_problem(int op, int64_t M, int64_t N, int64_t K) {
     return op != 2 && (M > 16 || M * (K + 16) > 65280) && M <= 256 && K % 128 == 0 && K <= kTableMaxK && N <= (M <= 64 ? 8192 : M <= 128 ? 2048 : 1024);
 }
 
-// The configurations that have a register-staged loop, for rows that are no whole number of 128-byte lines (more than 128 rows): the
-// ragged tail of K goes through registers.  Fitted the same way to 311 000 plans of 12 600 random problems.
+// The plan among the configurations without the tiles of whole lines 8-10: what the table has to beat, and the bound of the workspace
+// query.  Fitted the same way to 311 000 plans of 12 600 random problems.
 //   step      time per 64 bytes of K of a round of up to 256 blocks (a partly filled round takes as long as a full one)
 //   fixed     prologue and epilogue of a round
 //   ragged    factor on step where K % 128 != 0
@@ -294,9 +294,8 @@ Plan tile_plan(int op, int64_t M, int64_t N, int64_t K) {
     if (forced || !table_problem(op, M, N, K)) return rounds;
     const bool fits = partials_bytes(rounds, M, N) <= kStaticScratchBytes;
     if (op == kStaticInt8 && !fits) return rounds;
-    if (K % 128 != 0) return staged_plan(op, M, N, K, op == kStaticInt8 || (op != 2 && fits) ? kStaticScratchBytes : SIZE_MAX);
     double best_t;
-    const size_t most = op == kStaticInt8 ? kStaticScratchBytes : SIZE_MAX;
+    const size_t most = op == kStaticInt8 || (K % 128 != 0 && op != 2 && fits) ? kStaticScratchBytes : SIZE_MAX;
     const Plan best = table_plan(op, M, N, K, most, best_t);
     // The plan without the tiles of whole lines stays unless the table's is modelled as 6 % faster: of 2100 random problems of 300-8192
     // rows 4.4 % end more than 5 % behind it, without the margin 7.1 %, at the same mean.
@@ -375,10 +374,11 @@ int gemm_entry(int op, int a_format, const uint8_t* A, int64_t lda, const uint8_
         return launch_gemm_skinny(fp8, a_format == LLMQ_E5M2 ? 1 : 0, p.mt, 1 + (v & 1), 4 << (v >> 1), A, lda, B, ldb, (int)M, (int)N,
                                   (int)K, sep, out, ldo, acc_dump, st);
     }
-    // fp8 fragments are twice as wide: the 8-wave prefill tile runs ~5 % faster with 128-byte K tiles
-    if (fp8 && g_force_cfg < 0 && p.cfg == 1 && p.splits == 1) p.cfg = 6;
-    // int8 with direct loads: no staging registers, so the 128-byte K tile fits (half the barriers, whole lines per row)
-    if (!fp8 && g_force_cfg < 0 && p.cfg == 1 && K % 128 == 0 && p.k_per_split % 128 == 0) p.cfg = 6;
+    // The 256x256 tile runs with 128-byte K tiles (half the barriers, whole lines per row) where the split allows it.
+    if (g_force_cfg < 0 && p.cfg == 1 && (p.splits == 1 || p.k_per_split % 128 == 0)) {
+        p.cfg = 6;
+        if (p.splits == 1) p.k_per_split = cdiv(K, 128) * 128;
+    }
     if (p.splits > 1 && (!ws || ws_bytes < partials_bytes(p, M, N))) return LLMQ_ERR_WORKSPACE;
     auto run = [&](const Plan& pl, const uint8_t* Bp, const float* wsc, const void* bs, void* o, int64_t n) {
         Epilogue ep{a_scale, wsc, alpha_dev, bs, alpha, beta, bias_dtype, out_dtype, out_scale};
@@ -393,7 +393,7 @@ int gemm_entry(int op, int a_format, const uint8_t* A, int64_t lda, const uint8_
     // whole number of rounds: the first part keeps the big tiles and ends with every CU busy, the rest runs as one
     // round of 128x256 tiles (twice the blocks, half the time each).  Measured: 8192 x 4608 x 3584 (2.25 rounds)
     // and 8192 x 37888 x 3584 (18.5 rounds).
-    if (g_force_cfg < 0 && p.cfg == 6 && p.splits == 1 && !acc_dump && !out_scale && K % 128 == 0) {
+    if (g_force_cfg < 0 && p.cfg == 6 && p.splits == 1 && !acc_dump && !out_scale) {
         const int64_t tm = cdiv(M, 256), tn = cdiv(N, 256), tiles = tm * tn, tail = tiles % kNumCu, full = tiles - tail;
         if (full >= kNumCu && tail > 0 && tail <= 160 && full % tm == 0) {
             const int64_t n1 = full / tm * 256, n2 = N - n1;
@@ -401,7 +401,7 @@ int gemm_entry(int op, int a_format, const uint8_t* A, int64_t lda, const uint8_
                 const int rc = run(p, B, w_scale, bias, out, n1);
                 if (rc != LLMQ_OK) return rc;
                 const int64_t be = bias_dtype == LLMQ_F32 ? 4 : 2;
-                return run(Plan{7, 1, (int)K}, B + n1 * ldb, w_scale ? w_scale + n1 : nullptr,
+                return run(Plan{7, 1, cdiv(K, 128) * 128}, B + n1 * ldb, w_scale ? w_scale + n1 : nullptr,
                            bias ? static_cast<const uint8_t*>(bias) + n1 * be : nullptr, static_cast<uint8_t*>(out) + n1 * 2, n2);
             }
         }

@@ -312,7 +312,10 @@ __global__ __launch_bounds__(C::NT) void gemm_tile_kernel(
         // the block barrier that publishes the stage.  The loads are issued from assembly so that the compiler,
         // which would wait for every outstanding load before any later LDS read, does not see them.
         static_assert(C::KSUB % 2 == 0 && C::KSUB >= 2, "fragment parity must return to 0 at every tile");
-        static_assert(KFULL, "the direct loads cannot zero a ragged K tail");
+        // whole K tiles of this split; the direct loads cannot zero a ragged tail, which goes through registers behind them (us, all of K
+        // through registers / only its tail, weights out of HBM: int8 1000 x 4608 x 3600 45.0 / 29.3, 4096 x 18944 x 3600 354 / 295, fp8
+        // 4096 x 3584 x 3600 72.0 / 63.1, fp16 1000 x 4608 x 3592 77.4 / 59.8; the tiles differ too)
+        const int kfull = KFULL ? ktiles : (k_end - k_begin) / C::BK;
         constexpr int NS = C::STAGES, LPT = C::A_LOADS + C::B_LOADS;  // loads per thread and tile
         constexpr int SLOTS = C::TM * C::TN;                          // MFMAs per sub-step
         constexpr int PER = (LPT + C::KSUB * SLOTS - 1) / (C::KSUB * SLOTS);  // loads requested behind one MFMA
@@ -333,7 +336,7 @@ __global__ __launch_bounds__(C::NT) void gemm_tile_kernel(
         // shared panels at any moment instead of all for the same ones.  The blocks of one XCD stay in step, which is what
         // lets them share a panel through their L2.  fp32 accumulators keep the natural order: their bits would
         // otherwise depend on where in the grid a tile sits.
-        const int krot = C::FACC ? 0 : (int)((blockIdx.x % kNumXcd) * (unsigned)ktiles / kNumXcd);
+        const int krot = C::FACC ? 0 : (int)((blockIdx.x % kNumXcd) * (unsigned)kfull / kNumXcd);
         int ld_kt = krot;  // K tile that the next loads fetch
         auto issue = [&](int stage, auto d_c) __attribute__((always_inline)) {  // piece d of tile ld_kt into an LDS stage
             constexpr int d = decltype(d_c)::value;
@@ -342,7 +345,7 @@ __global__ __launch_bounds__(C::NT) void gemm_tile_kernel(
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0v), "v"(voff), "s"(base) : "memory", "m0");
         };
         static_assert(C::A_LOADS * C::NT * 16 == C::BM * C::CPR * 16, "the B pieces follow the A pieces in a stage");
-        auto next_kt = [&]() __attribute__((always_inline)) { ld_kt = ld_kt + 1 == ktiles ? 0 : ld_kt + 1; };
+        auto next_kt = [&]() __attribute__((always_inline)) { ld_kt = ld_kt + 1 == kfull ? 0 : ld_kt + 1; };
         // the tile behind the one being computed has landed when at most `younger` later tiles are still in flight
         auto wait_next_tile = [](int younger) __attribute__((always_inline)) {
             static_assert((NS - 2) * LPT < 64, "vmcnt is a 6-bit counter");
@@ -376,16 +379,16 @@ __global__ __launch_bounds__(C::NT) void gemm_tile_kernel(
         };
         unrolled<0, NS - 1>([&](auto t_c) __attribute__((always_inline)) {
             constexpr int t = decltype(t_c)::value;
-            if (t < ktiles) {
+            if (t < kfull) {
                 unrolled<0, LPT>([&](auto d) __attribute__((always_inline)) { issue(t, d); });
                 next_kt();
             }
         });
-        wait_next_tile(min(ktiles, NS - 1) - 1);
+        wait_next_tile(min(kfull, NS - 1) - 1);
         lds_barrier();
         read_frags(0, 0, fa[0], fb[0]);
         // the stage NS - 1 is free from the start: the part of its tile that the loop requests behind a barrier comes first
-        if (NS - 1 < ktiles)
+        if (NS - 1 < kfull)
             unrolled<0, (STEP < LPT ? STEP : LPT)>([&](auto d) __attribute__((always_inline)) { issue(NS - 1, d); });
         int stage = 0, kt = 0;
         // rest: the part of tile kt + NS - 1 that the last iteration did not request; first: tile kt + NS exists
@@ -399,7 +402,7 @@ __global__ __launch_bounds__(C::NT) void gemm_tile_kernel(
                 next_kt();
                 wait_next_tile(NS - 2);
             } else {
-                wait_next_tile(ktiles - 2 - kt);  // tile kt+1 has landed
+                wait_next_tile(kfull - 2 - kt);  // tile kt+1 has landed
             }
             lds_barrier();
             // every wavefront has read the whole of stage kt: it takes tile kt + NS
@@ -408,13 +411,26 @@ __global__ __launch_bounds__(C::NT) void gemm_tile_kernel(
             kt++;
         };
 #pragma unroll 1
-        while (kt < ktiles - NS) k_tile(std::true_type{}, std::true_type{});
-        if (kt == ktiles - NS) k_tile(std::true_type{}, std::false_type{});
+        while (kt < kfull - NS) k_tile(std::true_type{}, std::true_type{});
+        if (kt == kfull - NS) k_tile(std::true_type{}, std::false_type{});
         // Past the last request nothing is fetched: a block that ends waits for no load that nobody reads.
 #pragma unroll 1
-        while (kt < ktiles) k_tile(std::false_type{}, std::false_type{});
+        while (kt < kfull) k_tile(std::false_type{}, std::false_type{});
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be landing in LDS when it is reused or released
         lds_barrier();
+        if constexpr (!KFULL) {
+            if (kfull < ktiles) {  // block-uniform
+                load_tile(kfull, ra[0], rb[0]);
+                store_tile(0, kfull, ra[0], rb[0]);
+                lds_barrier();
+#pragma unroll
+                for (int ks = 0; ks < C::KSUB; ks++) {
+                    read_frags(0, ks, fa[0], fb[0]);
+                    mfma_step(fa[0], fb[0]);
+                }
+                lds_barrier();
+            }
+        }
     } else if constexpr (C::RS == 2) {
         load_tile(0, ra[0], rb[0]);
         load_tile(1, ra[1], rb[1]);
@@ -843,7 +859,7 @@ int launch_cfg(const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ldb, int
             if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tile_kernel<C, true>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::LDS_BYTES) != hipSuccess)
                 return LLMQ_ERR_LAUNCH;
-            if constexpr (!C::DMA)
+            if constexpr (!C::DMA || C::BK == 128)
                 if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_tile_kernel<C, false>),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::LDS_BYTES) != hipSuccess)
                     return LLMQ_ERR_LAUNCH;
@@ -853,7 +869,7 @@ int launch_cfg(const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ldb, int
     const int tiles = cdiv(M, C::BM) * cdiv(N, C::BN);
     // every split covers whole K tiles -> the loads need no K predicate
     const bool kfull = (K % C::BK == 0) && (p.k_per_split % C::BK == 0);
-    if constexpr (C::DMA) {
+    if constexpr (C::DMA && C::BK != 128) {
         if (!kfull) return LLMQ_ERR_SHAPE;  // callers route ragged K to the register-staged kernel
         hipLaunchKernelGGL((gemm_tile_kernel<C, true>), dim3(tiles, p.splits), dim3(C::NT), C::LDS_BYTES, st, A, lda, B,
                            ldb, M, N, K, p.k_per_split, ep, out, ldo, acc_dump, ws);
@@ -887,11 +903,11 @@ int launch_shape(const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ldb, i
 template <bool FP8, int AFMT>
 int launch_gemm(const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ldb, int M, int N, int K, const Plan& p,
                 const Epilogue& ep, void* out, int64_t ldo, void* acc_dump, void* ws, bool allow_dma, hipStream_t st) {
-    // Operand tiles go straight into LDS whenever every split covers whole K tiles (the direct loads cannot zero a
-    // ragged tail); llmq_gemm_force_plan(cfg | 64, .) keeps the register-staged loop.  The fp8 K step is 64 bytes, so
-    // the 64-byte K tiles have a single sub-step there and stay register-staged.
+    // Operand tiles go straight into LDS; llmq_gemm_force_plan(cfg | 64, .) keeps the register-staged loop.  The 128-byte K
+    // tiles add a ragged tail of the last split through registers; the 64-byte ones need whole tiles (the fp8 K step is 64
+    // bytes, so they have a single sub-step there and stay register-staged).
     const int bk = kShapes[p.cfg].bk;
-    const bool dma = allow_dma && K % bk == 0 && p.k_per_split % bk == 0;
+    const bool dma = allow_dma && p.k_per_split % bk == 0 && (K % bk == 0 || bk == 128);
     Plan staged = p;  // tiles that exist with direct loads only: a forced plan on a ragged K takes the staged tile next in size
     if (p.cfg >= 8) staged.cfg = p.cfg == 8 ? 3 : 2;
     int rc = dma ? launch_shape<FP8, AFMT, true>(A, lda, B, ldb, M, N, K, p, ep, out, ldo, acc_dump, ws, st)

@@ -77,3 +77,33 @@ def test_tiles_of_whole_lines(cuda, cfg, M, N, K, splits):
     finally:
         L.llmq_gemm_force_plan(-1, 1)
     assert torch.equal(y.cpu().view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("cfg", [4, 5, 6, 7, 8, 9, 10])
+@pytest.mark.parametrize("M,N,K", [(65, 136, 16), (192, 128, 112), (300, 264, 144), (256, 256, 272), (130, 512, 1264), (257, 384, 2032)])
+def test_ragged_tail_behind_direct_loads(cuda, cfg, M, N, K):
+    """K that ends inside a 128-byte tile: no whole tile, one, a few and more than LDS stages in front of tails of 16 to 112 bytes, without
+    a split and with the tail in the last of two, against the register-staged loop bit for bit and the exact accumulators."""
+    from llmqrt_amd import _abi
+    from llmqrt_amd.sq_fp8_kernels import cutlass_f8f8bf16_rowwise_sm89, w8a8_int8_linear_bbf16_obf16_per_channel
+    qx, qw = _ints((M, K), 1), _ints((N, K), 2)
+    g = torch.Generator().manual_seed(3)
+    sx, sw = torch.rand(M, generator=g) * 1e-3, torch.rand(N, generator=g) * 1e-2
+    ref = R.w8a8_epilogue_per_token_per_channel(R.int8_gemm_exact(qx, qw), sx, sw, None, torch.bfloat16)
+    a8 = (torch.randn(M, K, generator=g) * 20).to(torch.float8_e4m3fn).to(cuda)
+    b8 = (torch.randn(N, K, generator=g) * 20).to(torch.float8_e4m3fn).to(cuda)
+    zero = torch.zeros(N, dtype=torch.bfloat16, device=cuda)
+    L = _abi.lib()
+    try:
+        for splits in (1, 2):
+            if K // splits < 128 and splits > 1:
+                continue
+            f8 = []
+            for force in (cfg, cfg | 64):
+                _abi.check(L.llmq_gemm_force_plan(force, splits), "force_plan")
+                y = w8a8_int8_linear_bbf16_obf16_per_channel(qx.to(cuda), qw.to(cuda).t(), zero, sx.to(cuda).view(-1, 1), sw.to(cuda).view(1, -1))
+                assert torch.equal(y.cpu().view(torch.int16), ref.view(torch.int16))
+                f8.append(cutlass_f8f8bf16_rowwise_sm89(a8, b8.t(), None, sx.to(cuda).view(-1, 1), sw.to(cuda).view(1, -1), True))
+            assert torch.equal(f8[0].view(torch.int16), f8[1].view(torch.int16))
+    finally:
+        L.llmq_gemm_force_plan(-1, 1)
