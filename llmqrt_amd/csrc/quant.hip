@@ -55,14 +55,18 @@ __global__ __launch_bounds__(NT) void quant_rows_kernel(
     uint4 cache[NC > 0 ? NC : 1];
     float s;
     bool fin = false;  // block-uniform: the absmax behind the scale is finite, so no quotient can be NaN
+    // The row is requested before the scale is known, also where it comes from elsewhere: its latency runs beside that of the partials
+    // or of the scale.
+    if (NC > 0) {
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            const int i = tid + c * NT;
+            cache[c] = (i < nchunk) ? xr[i] : make_uint4(0, 0, 0, 0);
+        }
+    }
     if (SCALE == SCALE_ROW) {
         float amax = 0.f;
         if (NC > 0) {
-#pragma unroll
-            for (int c = 0; c < NC; c++) {
-                const int i = tid + c * NT;
-                cache[c] = (i < nchunk) ? xr[i] : make_uint4(0, 0, 0, 0);
-            }
 #pragma unroll
             for (int c = 0; c < NC; c++) amax = max_nonneg(amax, absmax8(cache[c], DT == LLMQ_BF16));
         } else {
@@ -502,16 +506,23 @@ int launch_rows(const void* x, int64_t M, int64_t K, int64_t ldx, void* q, void*
     }
 #define LLMQ_LAUNCH_NCT(NC, NT) \
     hipLaunchKernelGGL((quant_rows_kernel<DT, MODE, SCALE, NC, NT>), grid, dim3(NT), 0, st, xp, ldx, K, qp, scale, scale_dtype, aux, n_aux, static_f32, floor, ta)
-    if constexpr (SCALE != SCALE_ROW) LLMQ_LAUNCH_NCT(0, kThreads);
-    else switch (row_shape(M, K)) {
+    // A scale that comes from elsewhere: rows in registers hide their latency behind the partials' or the scale's while a block or two per CU
+    // cover the rows; with more, blocks that loop and need fewer registers are ahead.  Loop of 256 threads / rows in registers, us,
+    // absmax + quantizer (static scale):
+    //            K = 3584                    9728                        18944
+    //   64 rows  4.82 / 4.77 (2.58 / 2.29)   6.86 / 5.49 (4.03 / 2.96)   8.74 / 6.37 (7.56 / 4.60)
+    //   200      5.73 / 5.45 (2.82 / 2.53)   7.23 / 6.13 (5.02 / 3.64)   10.0 / 7.84 (8.12 / 5.61)
+    //   512      6.27 / 6.06 (3.66 / 3.71)   9.15 / 8.67 (6.25 / 6.00)   13.8 / 13.4 (12.2 / 10.4)
+    //   1000     7.40 / 7.59 (4.65 / 4.80)   12.7 / 13.4 (9.72 / 9.29)   19.7 / 20.3 (16.0 / 16.3)
+    switch (SCALE != SCALE_ROW && M > 512 ? RLong : row_shape(M, K)) {
         case R512x1: LLMQ_LAUNCH_NCT(1, 512); break;
         case R256x1: LLMQ_LAUNCH_NCT(1, 256); break;
         case R256x2: LLMQ_LAUNCH_NCT(2, 256); break;
-        case R128x4: LLMQ_LAUNCH_NCT(4, 128); break;
+        case R128x4: if constexpr (SCALE == SCALE_ROW) LLMQ_LAUNCH_NCT(4, 128); break;  // (M >= 6144)
         case R256x4: LLMQ_LAUNCH_NCT(4, 256); break;
         case R1024x3: LLMQ_LAUNCH_NCT(3, 1024); break;
         case R512x5: LLMQ_LAUNCH_NCT(5, 512); break;
-        case R256x10: LLMQ_LAUNCH_NCT(10, 256); break;
+        case R256x10: if constexpr (SCALE == SCALE_ROW) LLMQ_LAUNCH_NCT(10, 256); break;  // (M > 1024)
         default: LLMQ_LAUNCH_NCT(0, 256);
     }
     return launch_status();

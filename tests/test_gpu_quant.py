@@ -114,6 +114,33 @@ def test_static_fp8(cuda, dtype):
         assert torch.equal(got_f.cpu().view(torch.uint8), ref_f.view(torch.uint8))
 
 
+# both sides of the row counts and row lengths at which a per-tensor or static row changes its block, up to the longest in registers
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K", [(9, 2048), (9, 2056), (399, 4096), (400, 4096), (512, 3592), (513, 3592), (70, 4104), (70, 8192), (256, 8200),
+                                 (257, 8200), (3, 20480), (3, 20488), (512, 1024), (513, 1024)])
+def test_per_tensor_and_static_row_blocks(cuda, M, K, dtype):
+    """Codes and scales of strided rows with the largest value in the last chunk, finite and with an infinity, bit for bit."""
+    from llmqrt_amd.quantize import per_tensor_quantize, quantize_activation_per_tensor_absmax, static_per_tensor_quantize
+    x = _acts(M, K, 31 * M + K, dtype)
+    x[M - 1, K - 1] = 300.0
+    buf = torch.full((M, K + 8), 1000.0, dtype=dtype, device=cuda)
+    buf[:, :K] = x.to(cuda)
+    q, s = quantize_activation_per_tensor_absmax(buf[:, :K])
+    q_ref, s_ref = R.quantize_activation_per_tensor_absmax(x)
+    assert torch.equal(s.cpu(), s_ref) and torch.equal(q.cpu(), q_ref)
+    f, fs = per_tensor_quantize(buf[:, :K])
+    f_ref, fs_ref = R.fp8_per_tensor_quantize(x)
+    assert torch.equal(fs.cpu(), fs_ref) and torch.equal(f.cpu().view(torch.uint8), f_ref.view(torch.uint8))
+    for scale in (torch.tensor([0.21], dtype=torch.float32), 0.21):
+        st = scale.to(cuda) if torch.is_tensor(scale) else scale
+        ref = R.fp8_static_per_tensor_quantize(x, scale)
+        assert torch.equal(static_per_tensor_quantize(buf[:, :K], st).cpu().view(torch.uint8), ref.view(torch.uint8))
+    x[M // 2, 8] = float("inf")
+    f, fs = per_tensor_quantize(x.to(cuda))
+    f_ref, fs_ref = R.fp8_per_tensor_quantize(x)
+    assert torch.equal(fs.cpu(), fs_ref) and _same_with_nans(f.cpu(), f_ref)
+
+
 def test_strided_input_and_3d(cuda):
     from llmqrt_amd.quantize import quantize_activation_per_token_absmax
     x = _acts(8, 1024, 3, torch.bfloat16)
