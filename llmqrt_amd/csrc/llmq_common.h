@@ -150,17 +150,17 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-// sum over a block of NW wavefronts in a fixed order; every thread gets the same result.
+// sum over the NW wavefronts of a block from wavefront w0 on, in a fixed order; every thread of the block gets the same result.
 template <int NW>
-__device__ __forceinline__ float block_sum(float v, float* smem) {
+__device__ __forceinline__ float block_sum(float v, float* smem, int w0 = 0) {
     v = wave_sum(v);
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     __syncthreads();
     if (lane == 0) smem[w] = v;
     __syncthreads();
-    float r = smem[0];
+    float r = smem[w0];
 #pragma unroll
-    for (int i = 1; i < NW; i++) r += smem[i];
+    for (int i = 1; i < NW; i++) r += smem[w0 + i];
     return r;
 }
 

@@ -237,8 +237,9 @@ __global__ __launch_bounds__(kSmallThreads) void quant_tensor_small_kernel(
 //   h = fp32(x);  inv = 1 / sqrt(mean(h^2) + eps);  n = round_dt(h * inv);  y = round_dt(w * n)
 //   then exactly the per-token quantizer above on y.
 // Everything after `inv` is bit-identical to the reference evaluated with the same inv; inv itself
-// depends on the summation order of mean() (here: per-thread FMA chain, wavefront butterfly, then the
-// wavefronts in order) and can differ from another order in the last bits.
+// depends on the summation order of mean() and can differ from another order in the last bits.  The order here: LANES running sums, sum t
+// an FMA chain over the row's 16-byte chunks t, t + LANES, ..; a butterfly over each 64 of them; the results of the 64s in order.  LANES
+// follows from the size alone and not from the block that does the work (norm_shape below).
 template <int DT>
 __device__ __forceinline__ float sumsq8(uint4 r, float acc) {
     const uint32_t w[4] = {r.x, r.y, r.z, r.w};
@@ -271,16 +272,20 @@ __device__ __forceinline__ uint4 norm8(uint4 r, uint4 wv, float inv) {
     return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// QMODE: -1 = no quantizer (plain RMSNorm), MODE_I8, MODE_F8.
-template <int DT, int QMODE, int NC, int NT = kThreads>
+// QMODE: -1 = no quantizer (plain RMSNorm), MODE_I8, MODE_F8.  G = 2: two halves of LANES threads; thread t of the lower one owns the chunks
+// t + c LANES, of the upper one t + (NC + c) LANES.  The upper half reads the lower one's chunks as well and forms the running sums alone: a
+// wait for the lower half's through LDS takes longer (one-token layer 50.4 / 49.6 us).
+template <int DT, int QMODE, int NC, int NT = kThreads, int G = 1>
 __global__ __launch_bounds__(NT) void rmsnorm_quant_rows_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, int64_t K, const uint16_t* __restrict__ weight, float eps,
     uint16_t* __restrict__ y, uint8_t* __restrict__ q, void* __restrict__ scale_out, int scale_dtype,
     float* __restrict__ inv_out) {
+    constexpr int QM = QMODE < 0 ? MODE_I8 : QMODE, LANES = NT / G;
+    static_assert(LANES % kWave == 0 && (G == 1 || (G == 2 && NC > 0)), "halves of whole wavefronts, rows in registers");
     __shared__ float smem[NT / kWave];
-    constexpr int QM = QMODE < 0 ? MODE_I8 : QMODE;
     const int64_t row = blockIdx.x;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, upper = G > 1 ? __builtin_amdgcn_readfirstlane(tid / LANES) : 0;
+    const int first = tid + upper * (NC - 1) * LANES;  // the thread's first chunk; the others follow LANES apart
     const int nchunk = (int)(K >> 3);
     const uint4* xr = reinterpret_cast<const uint4*>(x + row * ldx);
     const uint4* wr = reinterpret_cast<const uint4*>(weight);
@@ -292,15 +297,26 @@ __global__ __launch_bounds__(NT) void rmsnorm_quant_rows_kernel(
     if (NC > 0) {
 #pragma unroll
         for (int c = 0; c < NC; c++) {
-            const int i = tid + c * NT;
+            const int i = first + c * LANES;
             cache[c] = (i < nchunk) ? xr[i] : make_uint4(0, 0, 0, 0);
+        }
+        if (upper) {
+            uint4 low[NC > 0 ? NC : 1];  // (a lower chunk past the row has no upper one behind it)
+#pragma unroll
+            for (int c = 0; c < NC; c++) {
+                const int i = tid + (c - 1) * LANES;
+                low[c] = (i < nchunk) ? xr[i] : make_uint4(0, 0, 0, 0);
+            }
+#pragma unroll
+            for (int c = 0; c < NC; c++) ss = sumsq8<DT>(low[c], ss);
         }
 #pragma unroll
         for (int c = 0; c < NC; c++) ss = sumsq8<DT>(cache[c], ss);
     } else {
         for (int i = tid; i < nchunk; i += NT) ss = sumsq8<DT>(xr[i], ss);
     }
-    ss = block_sum<NT / kWave>(ss, smem);
+    // the last LANES threads hold the sums
+    ss = block_sum<LANES / kWave>(ss, smem, (G - 1) * (LANES / kWave));
     const float inv = 1.0f / sqrtf(ss / (float)K + eps);
     if (inv_out && tid == 0) inv_out[row] = inv;
 
@@ -308,7 +324,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_quant_rows_kernel(
     if (NC > 0) {
 #pragma unroll
         for (int c = 0; c < NC; c++) {
-            const int i = tid + c * NT;
+            const int i = first + c * LANES;
             if (i < nchunk) {
                 cache[c] = norm8<DT>(cache[c], wr[i], inv);
                 if (yr) yr[i] = cache[c];
@@ -333,13 +349,13 @@ __global__ __launch_bounds__(NT) void rmsnorm_quant_rows_kernel(
     if (NC > 0 && amax < __builtin_inff() && s > 0.f) {  // block-uniform: no quotient can be NaN
 #pragma unroll
         for (int c = 0; c < NC; c++) {
-            const int i = tid + c * NT;
+            const int i = first + c * LANES;
             if (i < nchunk) qr[i] = quant8<DT, QM, Q_DT, true>(cache[c], s, inv_s);
         }
     } else if (NC > 0) {
 #pragma unroll
         for (int c = 0; c < NC; c++) {
-            const int i = tid + c * NT;
+            const int i = first + c * LANES;
             if (i < nchunk) qr[i] = quant8<DT, QM, Q_DT>(cache[c], s, inv_s);
         }
     } else {
@@ -414,13 +430,12 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_quant_rows_wave_kernel(
 inline bool wave_rows(int64_t M, int64_t K) { return (K >> 3) <= 2 * kWave && M >= 256; }
 // A block per row: threads and chunks per thread, by how many rows have to fill the chip.  A few rows are a chain of latencies (load, two
 // reductions, codes), which more threads with less each shorten; many rows are arithmetic that every wavefront repeats per row (reductions,
-// scale, reciprocal), which fewer threads with more each spread over more elements.  Fused RMSNorm + int8 quantizer / quantizer alone, us:
-//   257-512 chunks (K = 3584)    512 x 1      256 x 2      128 x 4          1025-2560 chunks (K = 18944)   1024 x 3      512 x 5     256 x 10
-//   32 rows                      3.19 / 2.68  3.41 / 2.74  3.42 / 2.72      32 rows                        5.14 / 3.75   5.19 / 3.79  6.41 / 3.99
-//   256                          3.57 / 3.03  3.79 / 3.09  4.30 / 3.31      128                            5.90 / 4.47   5.96 / 4.49  7.20 / 4.74
-//   512                          4.43 / 3.61  4.36 / 3.60  5.01 / 3.94      512                           10.65 / 8.14  10.34 / 8.22  11.2 / 8.51
-//   2048                         9.20 / 7.06  8.13 / 6.35  8.47 / 6.68      2048                           32.0 / 21.2   31.3 / 20.6  31.0 / 20.4
-//   8192                         --           23.6 / --    21.6 / --
+// scale, reciprocal), which fewer threads with more each spread over more elements.  int8 per-token quantizer, us:
+//   257-512 chunks (K = 3584)    512 x 1   256 x 2   128 x 4       1025-2560 chunks (K = 18944)   1024 x 3   512 x 5   256 x 10
+//   32 rows                      2.68      2.74      2.72          32 rows                        3.75       3.79      3.99
+//   256                          3.03      3.09      3.31          128                            4.47       4.49      4.74
+//   512                          3.61      3.60      3.94          512                            8.14       8.22      8.51
+//   2048                         7.06      6.35      6.68          2048                           21.2       20.6      20.4
 enum RowShape { R512x1, R256x1, R256x2, R128x4, R256x4, R1024x3, R512x5, R256x10, RLong };
 inline RowShape row_shape(int64_t M, int64_t K) {
     const int64_t chunks = K >> 3;
@@ -428,6 +443,24 @@ inline RowShape row_shape(int64_t M, int64_t K) {
     if (chunks <= 512) return M < 400 ? R512x1 : M < 6144 ? R256x2 : R128x4;
     if (chunks <= 1024) return R256x4;
     if (chunks <= 2560) return M <= 256 ? R1024x3 : M <= 1024 ? R512x5 : R256x10;
+    return RLong;
+}
+
+// RMSNorm: LANES, the order of the sum of squares, is fixed by the size (128 for 257-512 chunks and 256 rows or more, else 256), so wider
+// blocks read half of their row twice, and the lines lie elsewhere.  RMSNorm + int8 quantizer, rows in cache, us:
+//   K = 3584     512 x 1   256 x 2   128 x 4      K = 18944    512 x 5   256 x 10
+//   1 row        2.40      2.80                   32 rows      5.32      6.40
+//   128          3.40      3.76                   128          5.76      6.80
+//   256                    3.84      4.44         256          6.92      7.32
+//   512                    4.24      4.84         512          10.5      8.92
+//   768                    4.88      4.96         1024         16.3      17.0
+//   1024                   5.56      5.16         2048         28.5      28.4
+inline RowShape norm_shape(int64_t M, int64_t K) {
+    const int64_t chunks = K >> 3;
+    if (chunks <= 256) return R256x1;
+    if (chunks <= 512) return M < 256 ? R512x1 : M < 768 ? R256x2 : R128x4;
+    if (chunks <= 1024) return R256x4;
+    if (chunks <= 2560) return M <= 256 ? R512x5 : R256x10;
     return RLong;
 }
 
@@ -446,19 +479,18 @@ int launch_norm(const void* x, int64_t M, int64_t K, int64_t ldx, const void* we
 #undef LLMQ_LAUNCH_NCW
         return launch_status();
     }
-#define LLMQ_LAUNCH_NCT(NC, NT)                                                                                          \
-    hipLaunchKernelGGL((rmsnorm_quant_rows_kernel<DT, QMODE, NC, NT>), grid, dim3(NT), 0, st, (const uint16_t*)x, ldx, K, \
+#define LLMQ_LAUNCH_NCT(NC, NT, G)                                                                                          \
+    hipLaunchKernelGGL((rmsnorm_quant_rows_kernel<DT, QMODE, NC, NT, G>), grid, dim3(NT), 0, st, (const uint16_t*)x, ldx, K, \
                        (const uint16_t*)weight, eps, (uint16_t*)y, (uint8_t*)q, scale, scale_dtype, inv_out)
-    switch (row_shape(M, K)) {
-        case R512x1: LLMQ_LAUNCH_NCT(1, 512); break;
-        case R256x1: LLMQ_LAUNCH_NCT(1, 256); break;
-        case R256x2: LLMQ_LAUNCH_NCT(2, 256); break;
-        case R128x4: LLMQ_LAUNCH_NCT(4, 128); break;
-        case R256x4: LLMQ_LAUNCH_NCT(4, 256); break;
-        case R1024x3: LLMQ_LAUNCH_NCT(3, 1024); break;
-        case R512x5: LLMQ_LAUNCH_NCT(5, 512); break;
-        case R256x10: LLMQ_LAUNCH_NCT(10, 256); break;
-        default: LLMQ_LAUNCH_NCT(0, 256);
+    switch (norm_shape(M, K)) {
+        case R512x1: LLMQ_LAUNCH_NCT(1, 512, 2); break;
+        case R256x1: LLMQ_LAUNCH_NCT(1, 256, 1); break;
+        case R256x2: LLMQ_LAUNCH_NCT(2, 256, 2); break;
+        case R128x4: LLMQ_LAUNCH_NCT(4, 128, 1); break;
+        case R256x4: LLMQ_LAUNCH_NCT(4, 256, 1); break;
+        case R512x5: LLMQ_LAUNCH_NCT(5, 512, 2); break;
+        case R256x10: LLMQ_LAUNCH_NCT(10, 256, 1); break;
+        default: LLMQ_LAUNCH_NCT(0, 256, 1);
     }
 #undef LLMQ_LAUNCH_NCT
     return launch_status();

@@ -81,6 +81,51 @@ def test_rmsnorm_fp8_fused(cuda, M, K, dtype):
     assert torch.equal(q.cpu().view(torch.uint8), q_ref.view(torch.uint8))
 
 
+def _mean_square_in_order(x, M):
+    """mean(x^2) in the kernels' order of fp32 additions for a problem of M rows (the square of a 16-bit float is exact in fp32, so an FMA
+    adds like a plain addition): LANES running sums over the 16-byte chunks t, t + LANES, .., a butterfly over each 64 of them, the 64s in
+    order."""
+    rows, K = x.shape
+    chunks = K // 8
+    lanes = 64 if chunks <= 128 and M >= 256 else 128 if 256 < chunks <= 512 and M >= 256 else 256
+    per_lane = -(-chunks // lanes)
+    sq = torch.zeros(rows, per_lane * lanes, 8)
+    sq[:, :chunks] = x.float().square().view(rows, chunks, 8)
+    sq = sq.view(rows, per_lane, lanes, 8)
+    acc = torch.zeros(rows, lanes)
+    for c in range(per_lane):
+        for e in range(8):
+            acc = acc + sq[:, c, :, e]
+    acc = acc.view(rows, lanes // 64, 64)
+    for o in (32, 16, 8, 4, 2, 1):
+        acc = acc + acc[..., torch.arange(64) ^ o]
+    total = acc[:, 0, 0]
+    for w in range(1, lanes // 64):
+        total = total + acc[:, w, 0]
+    return total / float(K)
+
+
+# both sides of every row count at which the block of a row changes, every row length class; K is a power of two, so the mean is exact
+@pytest.mark.parametrize("M,K", [(8, 1024), (300, 1024), (8, 2048), (300, 2048), (1, 4096), (255, 4096), (256, 4096), (399, 4096), (400, 4096),
+                                 (767, 4096), (768, 4096), (6143, 4096), (6144, 4096), (9, 8192), (300, 8192), (3, 16384), (256, 16384),
+                                 (257, 16384), (1024, 16384), (1025, 16384), (3, 32768)])
+def test_order_of_the_sum_of_squares(cuda, M, K):
+    """The bits of the sum follow from the size of the problem, whatever block adds it up.  The rows are permutations of one row, and eps takes
+    all but a thousandth of its mean square away: one last bit of the sum (6e-8 of it) moves the result by 3e-5, a few last bits of the root
+    and the reciprocal by 5e-7."""
+    from llmqrt_amd.norm import rmsnorm
+    g = torch.Generator().manual_seed(M + K)
+    base = torch.randn(K, generator=g).bfloat16()
+    rows = min(M, 64)
+    x = torch.stack([base[torch.randperm(K, generator=g)] for _ in range(rows)]).repeat(-(-M // rows), 1)[:M].contiguous()
+    mean = _mean_square_in_order(x[:rows], M)
+    eps = torch.tensor(-0.999 * float(base.double().square().mean()), dtype=torch.float32)
+    inv = torch.empty(M, dtype=torch.float32, device=cuda)
+    rmsnorm(x.to(cuda), torch.ones(K, dtype=torch.bfloat16, device=cuda), float(eps), _inv_dump=inv)
+    want = (1.0 / torch.sqrt((mean + eps).double())).repeat(-(-M // rows))[:M]
+    assert ((inv.cpu().double() - want).abs() <= 1e-6 * want).all()
+
+
 def test_strided_rows_and_3d(cuda):
     from llmqrt_amd.norm import RMSNorm
     x = torch.randn(2, 5, 1024, generator=torch.Generator().manual_seed(3)).bfloat16()
