@@ -288,6 +288,18 @@ Plan rounds_plan(int64_t M, int64_t N, int64_t K, bool fp8) {
 // price is the least certain, the other entry points stay within that size too where the rounds model does.
 constexpr int kStaticInt8 = 3;
 
+// The plan without slabs and without the table of the tiles of whole lines.  Its partial sums are what a size was first served with: a
+// workspace of that size is still taken (gemm_entry) where the faster plan asks for more.
+Plan rules_plan(int op, int64_t M, int64_t N, int64_t K) {
+    int t, nw;
+    if (op != 2 && skinny_plan(M, N, K, t, nw)) return skinny(skinny_mt(M), t, nw, K);
+    const Plan rounds = rounds_plan(M, N, K, op == 1);
+    if (M <= 128 || (int64_t)cdiv(M, 256) * cdiv(N, 256) >= 2 * kNumCu || K > kTableMaxK * (op == 2 ? 2 : 1)) return rounds;
+    const bool fits = partials_bytes(rounds, M, N) <= kStaticScratchBytes;
+    if (op == kStaticInt8 && !fits) return rounds;
+    return staged_plan(op, M, N, K, op == kStaticInt8 || (op != 2 && K % 128 != 0 && fits) ? kStaticScratchBytes : SIZE_MAX);
+}
+
 Plan tile_plan(int op, int64_t M, int64_t N, int64_t K) {
     const Plan rounds = rounds_plan(M, N, K, op == 1);
     const bool forced = g_force_cfg >= 0 && g_force_cfg < 100;
@@ -367,7 +379,11 @@ int gemm_entry(int op, int a_format, const uint8_t* A, int64_t lda, const uint8_
     if (bias && bias_dtype != LLMQ_BF16 && bias_dtype != LLMQ_F16 && bias_dtype != LLMQ_F32) return LLMQ_ERR_DTYPE;
     if (fp8 && a_format != LLMQ_E4M3 && a_format != LLMQ_E5M2) return LLMQ_ERR_DTYPE;
     if (!aligned16(A) || !aligned16(B)) return LLMQ_ERR_ALIGN;
-    Plan p = plan_for(static_scratch ? kStaticInt8 : op, M, N, K);
+    auto fits = [&](const Plan& pl) { return pl.splits == 1 || (ws && ws_bytes >= partials_bytes(pl, M, N)); };
+    const int planned_op = static_scratch ? kStaticInt8 : op;
+    Plan p = plan_for(planned_op, M, N, K);
+    if (!fits(p) && g_force_cfg < 0) p = rules_plan(planned_op, M, N, K);  // the caller kept the size that was enough for these
+    if (!fits(p)) return LLMQ_ERR_WORKSPACE;
     if (p.cfg >= kSkinnyCfg) {
         const SkinnyEpilogue sep{a_scale, w_scale, alpha_dev, bias, alpha, beta, bias_dtype, out_dtype, out_scale};
         const int v = p.cfg - kSkinnyCfg;
@@ -379,7 +395,6 @@ int gemm_entry(int op, int a_format, const uint8_t* A, int64_t lda, const uint8_
         p.cfg = 6;
         if (p.splits == 1) p.k_per_split = cdiv(K, 128) * 128;
     }
-    if (p.splits > 1 && (!ws || ws_bytes < partials_bytes(p, M, N))) return LLMQ_ERR_WORKSPACE;
     auto run = [&](const Plan& pl, const uint8_t* Bp, const float* wsc, const void* bs, void* o, int64_t n) {
         Epilogue ep{a_scale, wsc, alpha_dev, bs, alpha, beta, bias_dtype, out_dtype, out_scale};
         const bool dma = g_force_dma != 0;

@@ -107,3 +107,48 @@ def test_ragged_tail_behind_direct_loads(cuda, cfg, M, N, K):
             assert torch.equal(f8[0].view(torch.int16), f8[1].view(torch.int16))
     finally:
         L.llmq_gemm_force_plan(-1, 1)
+
+
+# sizes that the rules of 16 .. 128 rows serve without partial sums, or with fewer than the plan that a full workspace gets
+@pytest.mark.parametrize("kind,M,N,K,kept", [("int8", 5, 136, 13056, 0), ("int8", 66, 3896, 5120, 2057088), ("fp8", 98, 2280, 3584, 0),
+                                             ("fp8", 5, 2392, 15488, 621920), ("f16", 66, 128, 1152, 0), ("f16", 102, 1320, 10752, 2692800)])
+def test_workspace_of_the_rules_is_still_enough(cuda, kind, M, N, K, kept):
+    """A caller that kept the workspace size of the rules' plan, or has none where that needs none: the call runs and gives what the GEMM
+    with a full workspace gives (int8 bit for bit; fp32 sums in another order: half a bf16 step of the value plus what test_fp8_.. allows)."""
+    from llmqrt_amd import _abi
+    L = _abi.lib()
+    g = torch.Generator().manual_seed(N)
+    stream = torch.cuda.current_stream().cuda_stream
+    if kind == "int8":
+        a, b = _ints((M, K), 1), _ints((N, K), 2)
+        ref = R.int8_gemm_exact(a, b).float() * 2.0 ** -10
+        query = L.llmq_gemm_workspace_bytes(M, N, K)
+    elif kind == "fp8":
+        a, b = [(torch.randn(n, K, generator=g) * 30).clamp(-448, 448).to(torch.float8_e4m3fn) for n in (M, N)]
+        ref = a.double() @ b.double().t() * 2.0 ** -10
+        query = L.llmq_gemm_fp8_quantized_output_workspace_bytes(M, N, K)  # the fp8 plan's own
+    else:
+        a, b = torch.randn(M, K, generator=g).half(), torch.randn(N, K, generator=g).half()
+        ref = a.double() @ b.double().t() * 2.0 ** -10
+        query = L.llmq_gemm_f16_workspace_bytes(M, N, K)
+    a, b = a.to(cuda), b.to(cuda)
+
+    def run(nbytes):
+        out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=cuda)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=cuda) if nbytes else None
+        tail = (out.data_ptr(), _abi.BF16, N, M, N, K, None, _abi.ptr(ws), nbytes, stream)
+        if kind == "int8":
+            rc = L.llmq_gemm_w8a8(a.data_ptr(), K, b.data_ptr(), K, None, None, 2.0 ** -10, None, None, 0, 0.0, *tail)
+        elif kind == "fp8":
+            rc = L.llmq_gemm_fp8(a.data_ptr(), _abi.E4M3, K, b.data_ptr(), K, None, None, 2.0 ** -10, None, None, 0, 0.0, *tail)
+        else:
+            rc = L.llmq_gemm_f16(a.data_ptr(), K, b.data_ptr(), K, 2.0 ** -10, None, 0, 0.0, *tail)
+        _abi.check(rc, kind)
+        return out.cpu()
+    full, small = run(query), run(kept)
+    if kind == "int8":
+        assert torch.equal(small.view(torch.int16), full.view(torch.int16))
+        assert torch.equal(small.view(torch.int16), ref.to(torch.bfloat16).view(torch.int16))
+    else:
+        for y in (full, small):
+            assert ((y.double() - ref).abs() <= 2e-4 * ref.abs().max() + ref.abs() / 256).all()
