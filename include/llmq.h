@@ -150,8 +150,8 @@ int llmq_rmsnorm_quant_fp8_per_token(const void* x, int x_dtype, int64_t M, int6
  * a_scale: fp32 [M]; w_scale: fp32 [N]; alpha_dev: fp32 device scalar (removes the
  * reference's .item() host syncs, linear_sq.py:127); bias: [N] of bias_dtype (bf16/f16/f32).
  * out: [M,N] bf16/f16 (ldo >= N).  acc_dump: optional int32 [M,N] contiguous that receives
- * the raw accumulators (parity checks).  workspace: >= llmq_gemm_workspace_bytes(M,N,K)
- * bytes (may be NULL when that is 0); contents irrelevant on entry.
+ * the raw accumulators (parity checks).  workspace: >= llmq_gemm_w8a8_workspace_bytes(M,N,K)
+ * (or llmq_gemm_workspace_bytes, which covers fp8 too) bytes (may be NULL when that is 0); contents irrelevant on entry.
  * ------------------------------------------------------------------------------------ */
 int llmq_gemm_w8a8(const int8_t* A, int64_t lda, const int8_t* B, int64_t ldb,
                    const float* a_scale, const float* w_scale,
@@ -179,6 +179,9 @@ int llmq_gemm_fp8(const uint8_t* A, int a_format, int64_t lda, const uint8_t* B,
                   float* acc_dump, void* workspace, size_t workspace_bytes,
                   llmq_stream_t stream);
 
+/* Bytes that llmq_gemm_w8a8 / llmq_gemm_fp8 need for a size, and an upper bound for both. */
+size_t llmq_gemm_w8a8_workspace_bytes(int64_t M, int64_t N, int64_t K);
+size_t llmq_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t K);
 size_t llmq_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /* llmq_gemm_fp8 with the output quantization of FP8StaticLinear.forward folded into the epilogue

@@ -42,6 +42,8 @@ SIGNATURES = {
                               _i64, _i64, _i64, _vp, _vp, _sz, _vp]),
     "llmq_gemm_fp8": (_int, [_vp, _int, _i64, _vp, _i64, _vp, _vp, _f32, _vp, _vp, _int, _f32, _vp, _int, _i64,
                              _i64, _i64, _i64, _vp, _vp, _sz, _vp]),
+    "llmq_gemm_w8a8_workspace_bytes": (_sz, [_i64, _i64, _i64]),
+    "llmq_gemm_fp8_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "llmq_gemm_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "llmq_gemm_w8a8_static": (_int, [_vp, _i64, _vp, _i64, _vp, _vp, _f32, _vp, _vp, _int, _f32, _vp, _int, _i64,
                                      _i64, _i64, _i64, _vp]),

@@ -168,8 +168,7 @@ bool slab_problem(int op, int64_t M, int64_t N, int64_t K) {
     return op != 2 && (M > 16 || M * (K + 16) > 65280) && M <= 256 && K % 128 == 0 && K <= kTableMaxK && N <= (M <= 64 ? 8192 : M <= 128 ? 2048 : 1024);
 }
 
-// The plan among the configurations without the tiles of whole lines 8-10: what the table has to beat, and the bound of the workspace
-// query.  Fitted the same way to 311 000 plans of 12 600 random problems.
+// The plan among the configurations without the tiles of whole lines 8-10: what the table has to beat.  Fitted the same way to 311 000 plans of 12 600 random problems.
 //   step      time per 64 bytes of K of a round of up to 256 blocks (a partly filled round takes as long as a full one)
 //   fixed     prologue and epilogue of a round
 //   ragged    factor on step where K % 128 != 0
@@ -309,8 +308,9 @@ Plan tile_plan(int op, int64_t M, int64_t N, int64_t K) {
     double best_t;
     const size_t most = op == kStaticInt8 || (K % 128 != 0 && op != 2 && fits) ? kStaticScratchBytes : SIZE_MAX;
     const Plan best = table_plan(op, M, N, K, most, best_t);
-    // The plan without the tiles of whole lines stays unless the table's is modelled as 6 % faster: of 2100 random problems of 300-8192
-    // rows 4.4 % end more than 5 % behind it, without the margin 7.1 %, at the same mean.
+    // The plan without the tiles of whole lines stays where it is of a configuration that the table prices (4-7; 2 and 3 give way to 8-10)
+    // and the table's is not modelled as 6 % faster: of 2100 random problems of 300-8192 rows 4.4 % end more than 5 % behind it, without the
+    // margin 7.1 %, at the same mean.
     Plan old = M > 128 ? staged_plan(op, M, N, K, most) : rounds;
     if (old.cfg == 1) old.cfg = 6, old.k_per_split = cdiv(old.k_per_split, 128) * 128;  // what config 1 is launched as
     for (const TileCost& c : costs_of(op).tiles)
@@ -352,11 +352,13 @@ Plan make_plan(int op, int64_t M, int64_t N, int64_t K) {
 
 // Searching a plan takes microseconds of host time and a call needs it for its workspace and for its launch, so each host
 // thread remembers the last plans it made (a pure function of sizes and format; a forced plan is not remembered).
+constexpr int kCachedSizes = 64;
+inline int size_slot(int64_t M, int64_t N, int64_t K, int op) { return ((uint64_t)(M * 31 + N * 17 + K * 7 + op) * 0x9E3779B97F4A7C15ull) >> 58; }
 Plan plan_for(int op, int64_t M, int64_t N, int64_t K) {
     if (g_force_cfg >= 0) return make_plan(op, M, N, K);
     struct Entry { int64_t M, N, K; int op; Plan plan; };
-    static thread_local Entry cache[64] = {};
-    Entry& e = cache[((uint64_t)(M * 31 + N * 17 + K * 7 + op) * 0x9E3779B97F4A7C15ull) >> 58];
+    static thread_local Entry cache[kCachedSizes] = {};
+    Entry& e = cache[size_slot(M, N, K, op)];
     if (e.M != M || e.N != N || e.K != K || e.op != op) e = Entry{M, N, K, op, make_plan(op, M, N, K)};
     return e.plan;
 }
@@ -477,15 +479,28 @@ extern "C" int llmq_gemm_force_plan(int cfg, int splits) {
 
 extern "C" int llmq_gemm_num_configs(void) { return kNumShapes; }
 
+namespace {
+// what the plan that a call of this size runs splits into: a lookup once the size is planned
+size_t planned_bytes(int op, int64_t M, int64_t N, int64_t K) {
+    return M <= 0 || N <= 0 || K <= 0 ? 0 : partials_bytes(plan_for(op, M, N, K), M, N);
+}
+}  // namespace
+
+extern "C" size_t llmq_gemm_w8a8_workspace_bytes(int64_t M, int64_t N, int64_t K) { return planned_bytes(0, M, N, K); }
+extern "C" size_t llmq_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t K) { return planned_bytes(1, M, N, K); }
+// For both formats, and no less than what the plans of the rules split: a figure that was enough for every plan this library had for a size.
 extern "C" size_t llmq_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    if (M <= 0 || N <= 0 || K <= 0) return 0;
-    const Plan p = plan_for(0, M, N, K), p8 = plan_for(1, M, N, K);  // the int8 and the fp8 plan may differ
-    size_t most = std::max(partials_bytes(p, M, N), partials_bytes(p8, M, N));
-    // An upper bound that also covers what the configurations with a register-staged loop would split: the figure for a size stays what
-    // it was before the tiles of whole lines, for callers that keep it.
-    if (g_force_cfg < 0 && K % 128 == 0 && table_problem(0, M, N, K))
-        for (int op = 0; op < 2; op++) most = std::max(most, partials_bytes(staged_plan(op, M, N, K, SIZE_MAX), M, N));
-    return most;
+    if (g_force_cfg >= 0 || M <= 0 || N <= 0 || K <= 0) return std::max(planned_bytes(0, M, N, K), planned_bytes(1, M, N, K));
+    struct Entry { int64_t M, N, K; size_t bytes; };
+    static thread_local Entry cache[kCachedSizes] = {};
+    Entry& e = cache[size_slot(M, N, K, 0)];
+    if (e.M != M || e.N != N || e.K != K) {
+        size_t most = 0;
+        for (int op = 0; op < 2; op++)
+            most = std::max({most, planned_bytes(op, M, N, K), partials_bytes(rules_plan(op, M, N, K), M, N)});
+        e = Entry{M, N, K, most};
+    }
+    return e.bytes;
 }
 
 extern "C" int llmq_gemm_w8a8(const int8_t* A, int64_t lda, const int8_t* B, int64_t ldb, const float* a_scale,
@@ -518,17 +533,9 @@ extern "C" int llmq_gemm_fp8_quantized_output(const uint8_t* A, int a_format, in
                       inter_dtype, ldo, M, N, K, nullptr, workspace, workspace_bytes, (hipStream_t)stream, out_scale);
 }
 
-extern "C" size_t llmq_gemm_fp8_quantized_output_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    if (M <= 0 || N <= 0 || K <= 0) return 0;
-    const Plan p = plan_for(1, M, N, K);
-    return partials_bytes(p, M, N);
-}
+extern "C" size_t llmq_gemm_fp8_quantized_output_workspace_bytes(int64_t M, int64_t N, int64_t K) { return planned_bytes(1, M, N, K); }
 
-extern "C" size_t llmq_gemm_f16_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    if (M <= 0 || N <= 0 || K <= 0) return 0;
-    const Plan p = plan_for(2, M, N, 2 * K);
-    return partials_bytes(p, M, N);
-}
+extern "C" size_t llmq_gemm_f16_workspace_bytes(int64_t M, int64_t N, int64_t K) { return planned_bytes(2, M, N, 2 * K); }
 
 extern "C" int llmq_gemm_f16(const void* A, int64_t lda, const void* B, int64_t ldb, float alpha, const void* bias,
                              int bias_dtype, float beta, void* out, int out_dtype, int64_t ldo, int64_t M, int64_t N,

@@ -105,7 +105,7 @@ struct Gemm {
 };
 void gemm(const Gemm& g, Tensor& out, at::ScalarType out_dtype, const Launch& l) {
     const int64_t N = g.w.size(0);
-    const int64_t ws_bytes = (int64_t)llmq_gemm_workspace_bytes(g.M, N, g.K);
+    const int64_t ws_bytes = (int64_t)(g.fp8 ? llmq_gemm_fp8_workspace_bytes : llmq_gemm_w8a8_workspace_bytes)(g.M, N, g.K);
     Tensor ws;
     if (ws_bytes) ws = make({ws_bytes}, at::kByte, out.device());
     void* wp = ws_bytes ? ws.data_ptr() : nullptr;

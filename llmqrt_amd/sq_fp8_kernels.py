@@ -62,7 +62,7 @@ def _run(fp8: bool, x, w, a_scale, w_scale, alpha, alpha_dev, bias, beta, out_dt
     if M == 0 or N == 0:
         return out
     L = _abi.lib()
-    ws_bytes = L.llmq_gemm_workspace_bytes(M, N, K)
+    ws_bytes = (L.llmq_gemm_fp8_workspace_bytes if fp8 else L.llmq_gemm_w8a8_workspace_bytes)(M, N, K)
     ws = _abi.workspaces.get(x.device, ws_bytes)
     common = (_abi.ptr(a_scale), _abi.ptr(w_scale), float(alpha), _abi.ptr(alpha_dev), _abi.ptr(bias),
               _abi.dtype_code(bias.dtype) if bias is not None else _abi.BF16, float(beta), out.data_ptr(),

@@ -185,6 +185,35 @@ def test_plans_fit_the_static_scratch(M, N, K):
     assert L.llmq_gemm_workspace_bytes(M, N, K) <= L.llmq_gemm_static_scratch_bytes()
 
 
+def test_workspace_figures_by_format():
+    """A format's figure is what its own plan splits; the common one covers both.  200 x 512 x 3584 runs in one launch in either format."""
+    from llmqrt_amd import _abi
+    L = _abi.lib()
+    for M, N, K in [(200, 512, 3584), (109, 29600, 6144), (512, 3584, 18944), (1000, 4608, 3600), (71, 3880, 12800), (16, 896, 4864), (0, 8, 16)]:
+        i8, f8 = L.llmq_gemm_w8a8_workspace_bytes(M, N, K), L.llmq_gemm_fp8_workspace_bytes(M, N, K)
+        assert L.llmq_gemm_workspace_bytes(M, N, K) >= max(i8, f8)
+        assert f8 == L.llmq_gemm_fp8_quantized_output_workspace_bytes(M, N, K)
+        assert all(b == 0 or (b % (4 * M * N) == 0 and b > 4 * M * N) for b in (i8, f8)), "two or more partial tensors, or none"
+    assert L.llmq_gemm_w8a8_workspace_bytes(200, 512, 3584) == 0 == L.llmq_gemm_fp8_workspace_bytes(200, 512, 3584)
+
+
+def test_repeated_workspace_query_searches_no_plan():
+    """A size that is already planned costs what an unsplit one costs (a search takes several times the call itself)."""
+    import time
+    from llmqrt_amd import _abi
+    L = _abi.lib()
+
+    def cost(M, N, K):
+        best = float("inf")
+        for _ in range(30):
+            t = time.perf_counter()
+            for _ in range(300):
+                L.llmq_gemm_workspace_bytes(M, N, K)
+            best = min(best, time.perf_counter() - t)
+        return best
+    assert cost(512, 3584, 18944) < 2 * cost(8192, 37888, 3584)
+
+
 def _moved_tensors(mod, how):
     """The module's tensors where nn.Module's dictionaries do not hold them under their names."""
     if how == "replica":  # as torch.nn.parallel.replicate leaves a module: parameters are plain attributes
