@@ -110,21 +110,24 @@ const FormatCost kCosts[3] = {
      {{4, 0.160, 0.599, 4.674, 0.970}, {5, 0.125, 0.721, 3.831, 0.729}, {6, 0.742, 0.674, 4.967, 1.522}, {7, 0.420, 0.522, 4.735, 2.094},
       {8, 0.255, 0.311, 4.284, 2.477}, {9, 0.327, 0.431, 4.315, 2.575}, {10, 0.411, 0.546, 4.554, 2.606}}}};
 
-// Modelled time of configuration row `c` with K in sp splits of kps bytes.
-double table_time(const FormatCost& f, const TileCost& c, int64_t M, int64_t N, int64_t K, int sp, int kps) {
+// Modelled time of configuration row `c` with K in sp splits of kps bytes; `limit` or more where it is certain to exceed that (the roots are
+// most of a search).
+double table_time(const FormatCost& f, const TileCost& c, int64_t M, int64_t N, int64_t K, int sp, int kps, double limit = 1e300) {
     const TileShape s = kShapes[c.cfg];
     const double run = kps / 64.0 * c.step, x = (double)((int64_t)cdiv(M, s.bm) * cdiv(N, s.bn) * sp) / kNumCu;
     const double full = std::floor(x), part = x - full, weights = (double)N * K * f.weights / 1e6 + f.base;
     double t;
     if (c.cfg <= 5) t = run * (x > 1 ? std::max(x, 1 + (std::ceil(x) - 1) * c.first) : c.lo + (1 - c.lo) * x) + c.fixed;
     else t = full * (run + c.fixed) + (part > 0 ? run * (c.lo + (1 - c.lo) * part) + c.fixed : 0) + c.first;
-    const double t3 = t * t * t, w3 = weights * weights * weights;
-    t = std::cbrt(std::sqrt(t3 * t3 + w3 * w3)) + (double)M * N * 2 * f.out / 1e6;
+    double rest = (double)M * N * 2 * f.out / 1e6;
     if (sp > 1) {
         const double partials = (double)M * N * sp * 4;
-        t += f.finish + f.partial * partials * 2 / 8e6 + f.past * std::max(0.0, partials - 3.2e7) / 8e6;
+        rest += f.finish + f.partial * partials * 2 / 8e6 + f.past * std::max(0.0, partials - 3.2e7) / 8e6;
     }
-    return t;
+    const double least = (std::max(t, weights) + rest) * 0.999999;
+    if (least >= limit) return least;
+    const double t3 = t * t * t, w3 = weights * weights * weights;
+    return std::cbrt(std::sqrt(t3 * t3 + w3 * w3)) + rest;
 }
 const FormatCost& costs_of(int op) { return kCosts[op == 1 ? 1 : op == 2 ? 2 : 0]; }
 
@@ -138,14 +141,14 @@ Plan table_plan(int op, int64_t M, int64_t N, int64_t K, size_t max_partials, do
             if (sp > 1 && (K / sp < 512 || partials > (size_t)256 << 20 || partials > max_partials)) break;
             const int kps = cdiv(cdiv(K, sp), 128) * 128;
             if (cdiv(K, kps) != sp) continue;
-            const double t = table_time(f, c, M, N, K, sp, kps);
+            const double t = table_time(f, c, M, N, K, sp, kps, best_t);
             if (t < best_t) best_t = t, best = Plan{c.cfg, sp, kps};
         }
     }
     return best;
 }
 
-// Few-token kernel in slabs of 16 * mt tokens: us of a launch.  A wavefront's steps are a chain of load latencies that grows with the
+// Few-token kernel in slabs of 16 * mt tokens: modelled us of a launch.  A wavefront's steps are a chain of load latencies that grows with the
 // operands a step loads (`step` us per 16-row tile); blocks that share a CU slow each other down by `share`; a CU's loads move
 // 1000 / `bytes` bytes per us; weights as in the table.  Fitted to 16 variants each of 8500 random problems of up to 512 tokens together with
 // the tile plans of the same problems.  One launch instead of a K split and its finishing launch (us, rules alone / with slabs): int8 60 x
@@ -286,63 +289,72 @@ Plan rounds_plan(int64_t M, int64_t N, int64_t K, bool fp8) {
 // which refuses what the rounds model splits past its size and runs the rest with a plan that fits.  With a ragged 8-bit K, whose
 // price is the least certain, the other entry points stay within that size too where the rounds model does.
 constexpr int kStaticInt8 = 3;
+inline bool within_scratch(int op, int64_t K) { return op == kStaticInt8 || (op != 2 && K % 128 != 0); }
 
 // The plan without slabs and without the table of the tiles of whole lines.  Its partial sums are what a size was first served with: a
 // workspace of that size is still taken (gemm_entry) where the faster plan asks for more.
 Plan rules_plan(int op, int64_t M, int64_t N, int64_t K) {
     int t, nw;
     if (op != 2 && skinny_plan(M, N, K, t, nw)) return skinny(skinny_mt(M), t, nw, K);
-    const Plan rounds = rounds_plan(M, N, K, op == 1);
-    if (M <= 128 || (int64_t)cdiv(M, 256) * cdiv(N, 256) >= 2 * kNumCu || K > kTableMaxK * (op == 2 ? 2 : 1)) return rounds;
-    const bool fits = partials_bytes(rounds, M, N) <= kStaticScratchBytes;
-    if (op == kStaticInt8 && !fits) return rounds;
-    return staged_plan(op, M, N, K, op == kStaticInt8 || (op != 2 && K % 128 != 0 && fits) ? kStaticScratchBytes : SIZE_MAX);
+    if (M <= 128 || (int64_t)cdiv(M, 256) * cdiv(N, 256) >= 2 * kNumCu || K > kTableMaxK * (op == 2 ? 2 : 1)) return rounds_plan(M, N, K, op == 1);
+    size_t most = SIZE_MAX;
+    if (within_scratch(op, K)) {
+        const Plan rounds = rounds_plan(M, N, K, op == 1);
+        const bool fits = partials_bytes(rounds, M, N) <= kStaticScratchBytes;
+        if (op == kStaticInt8 && !fits) return rounds;
+        if (fits) most = kStaticScratchBytes;
+    }
+    return staged_plan(op, M, N, K, most);
 }
 
-Plan tile_plan(int op, int64_t M, int64_t N, int64_t K) {
-    const Plan rounds = rounds_plan(M, N, K, op == 1);
+// table_t: modelled time of the table's plan `table`, where one was searched
+Plan tile_plan(int op, int64_t M, int64_t N, int64_t K, Plan& table, double& table_t) {
     const bool forced = g_force_cfg >= 0 && g_force_cfg < 100;
-    if (forced || !table_problem(op, M, N, K)) return rounds;
-    const bool fits = partials_bytes(rounds, M, N) <= kStaticScratchBytes;
-    if (op == kStaticInt8 && !fits) return rounds;
-    double best_t;
-    const size_t most = op == kStaticInt8 || (K % 128 != 0 && op != 2 && fits) ? kStaticScratchBytes : SIZE_MAX;
-    const Plan best = table_plan(op, M, N, K, most, best_t);
+    if (forced || !table_problem(op, M, N, K)) return rounds_plan(M, N, K, op == 1);
+    size_t most = SIZE_MAX;
+    Plan old{};
+    if (M <= 128 || within_scratch(op, K)) {
+        old = rounds_plan(M, N, K, op == 1);
+        const bool fits = partials_bytes(old, M, N) <= kStaticScratchBytes;
+        if (op == kStaticInt8 && !fits) return old;
+        if (fits && within_scratch(op, K)) most = kStaticScratchBytes;
+    }
+    table = table_plan(op, M, N, K, most, table_t);
     // The plan without the tiles of whole lines stays where it is of a configuration that the table prices (4-7; 2 and 3 give way to 8-10)
     // and the table's is not modelled as 6 % faster: of 2100 random problems of 300-8192 rows 4.4 % end more than 5 % behind it, without the
     // margin 7.1 %, at the same mean.
-    Plan old = M > 128 ? staged_plan(op, M, N, K, most) : rounds;
+    if (M > 128) old = staged_plan(op, M, N, K, most);
     if (old.cfg == 1) old.cfg = 6, old.k_per_split = cdiv(old.k_per_split, 128) * 128;  // what config 1 is launched as
     for (const TileCost& c : costs_of(op).tiles)
-        if (c.cfg == old.cfg && cdiv(K, old.k_per_split) == old.splits && best_t > 0.94 * table_time(costs_of(op), c, M, N, K, old.splits, old.k_per_split)) return old;
-    return best;
+        if (c.cfg == old.cfg && cdiv(K, old.k_per_split) == old.splits && table_t > 0.94 * table_time(costs_of(op), c, M, N, K, old.splits, old.k_per_split)) return old;
+    return table;
 }
 
 Plan make_plan(int op, int64_t M, int64_t N, int64_t K) {
     int t, nw;
     if (g_force_cfg >= kSkinnyCfg && op != 2 && M <= 64) return Plan{g_force_cfg, 1, (int)K, skinny_mt(M)};
     const bool few = g_force_cfg < 0 && op != 2 && skinny_plan(M, N, K, t, nw);
-    const Plan plan = few ? skinny(skinny_mt(M), t, nw, K) : tile_plan(op, M, N, K);
+    Plan best{};
+    double best_t = -1;
+    const Plan plan = few ? skinny(skinny_mt(M), t, nw, K) : tile_plan(op, M, N, K, best, best_t);
     if (g_force_cfg >= 0 || !slab_problem(op, M, N, K)) return plan;
     if (op == kStaticInt8 && partials_bytes(plan, M, N) > kStaticScratchBytes) return plan;  // refused, as before
     // Sixteen wavefronts along a K of a few thousand in one block row: measured best there (slabs 8 % slower in the mean at 33-64 tokens of
     // more than 3000 channels, level at 2049-3000; 18-43 % faster with fewer channels, 40 % with a longer K).
     if (few && M > 32 && N > 2048 && K > 2048 && K <= 4096) return plan;
     // The plan of the rules stays unless another is modelled as clearly faster.
-    double now = 1e300, best_t;
+    double now = 1e300;
     if (few) now = skinny_time(op, M, N, K, skinny_mt(M), t, nw);
     else
         for (const TileCost& c : costs_of(op).tiles)
             if (c.cfg == plan.cfg) now = table_time(costs_of(op), c, M, N, K, plan.splits, plan.k_per_split);
-    Plan best = table_plan(op, M, N, K, op == kStaticInt8 ? kStaticScratchBytes : SIZE_MAX, best_t);
-    for (int mt = 1; mt <= 4; mt *= 2) {
-        if (mt > 1 && 16 * mt >= 2 * M) break;
-        for (t = 1; t <= 2; t++)
-            for (nw = 4; nw <= (mt * t == 8 ? 8 : 16); nw *= 2) {
-                const double s = skinny_time(op, M, N, K, mt, t, nw);
-                if (s < best_t) best_t = s, best = skinny(mt, t, nw, K);
-            }
-    }
+    if (best_t < 0) best = table_plan(op, M, N, K, op == kStaticInt8 ? kStaticScratchBytes : SIZE_MAX, best_t);
+    // Slabs of 16 or 32 tokens with four wavefronts along K: of 3 million random problems one picks another number of wavefronts, none 64 tokens.
+    for (int mt = 1; mt <= (M > 16 ? 2 : 1); mt++)
+        for (t = 1; t <= 2; t++) {
+            const double s = skinny_time(op, M, N, K, mt, t, 4);
+            if (s < best_t) best_t = s, best = skinny(mt, t, 4, K);
+        }
     // By a tenth (2.1 % of 8600 random problems here end more than 5 % behind the rules, against 4.0 % without a margin, for 1.113 of the
     // 1.118 in the mean), by more where the rules pick the few-token kernel themselves: most of those were such problems with a short K.
     // A K split gives way to one launch of slabs at the same modelled time: the gap before its finishing launch is not in the model.

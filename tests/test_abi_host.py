@@ -214,6 +214,27 @@ def test_repeated_workspace_query_searches_no_plan():
     assert cost(512, 3584, 18944) < 2 * cost(8192, 37888, 3584)
 
 
+def test_first_plan_of_a_size_is_one_search():
+    """Every prompt length is a new size for a model's projections.  Where slabs, the table and the rules compete a size is planned in about
+    the time of the rounds model's own search (1.2 times through ctypes; with two searches of the table, and the rounds model's beside them, 2.4
+    times)."""
+    import time
+    from llmqrt_amd import _abi
+    L = _abi.lib()
+
+    def cost(M, K, first):
+        best = float("inf")
+        for rep in range(20):
+            t = time.perf_counter()
+            for i in range(40):
+                L.llmq_gemm_fp8_quantized_output_workspace_bytes(M, first + 8 * (40 * rep + i), K)
+            best = min(best, time.perf_counter() - t)
+        return best
+    slabs = min(cost(129 + i, 3584, 256 + 8 * i) for i in range(3))
+    rounds = min(cost(129 + i, 20736, 256 + 8 * i) for i in range(3))
+    assert slabs < 1.8 * rounds
+
+
 def _moved_tensors(mod, how):
     """The module's tensors where nn.Module's dictionaries do not hold them under their names."""
     if how == "replica":  # as torch.nn.parallel.replicate leaves a module: parameters are plain attributes
