@@ -75,3 +75,19 @@ def test_static_scratch_takes_a_plan_that_fits(cuda):
     want = _run(L, _abi, False, p, M, N, K, cuda)
     got = _run(L, _abi, True, p, M, N, K, cuda)
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+def test_static_scratch_refusal_is_its_own(cuda):
+    """A size that needs no workspace elsewhere and is refused here, before any launch: the output stays untouched."""
+    from llmqrt_amd import _abi
+    L = _abi.lib()
+    M, N, K = 300, 29120, 17536
+    assert L.llmq_gemm_workspace_bytes(M, N, K) <= L.llmq_gemm_static_scratch_bytes()
+    a, b = (torch.zeros(n, K, dtype=torch.int8, device=cuda) for n in (M, N))
+    out = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=cuda)
+    stream = torch.cuda.current_stream().cuda_stream
+    rc = L.llmq_gemm_w8a8_static(a.data_ptr(), K, b.data_ptr(), K, None, None, 1.0, None, None, 0, 0.0, out.data_ptr(), _abi.BF16, N,
+                                 M, N, K, stream)
+    assert rc == -7
+    torch.cuda.synchronize()
+    assert bool((out == 7.0).all())
