@@ -332,7 +332,11 @@ Plan tile_plan(int op, int64_t M, int64_t N, int64_t K, Plan& table, double& tab
 
 Plan make_plan(int op, int64_t M, int64_t N, int64_t K) {
     int t, nw;
-    if (g_force_cfg >= kSkinnyCfg && op != 2 && M <= 64) return Plan{g_force_cfg, 1, (int)K, skinny_mt(M)};
+    if (g_force_cfg >= kSkinnyCfg && op != 2) {  // forced few-token variant: 16, 32 or 64 as its split are the tokens of a slab
+        const int slab = g_force_splits;
+        if (slab == 16 || slab == 32 || slab == 64) return Plan{g_force_cfg, 1, (int)K, slab / 16};
+        if (M <= 64) return Plan{g_force_cfg, 1, (int)K, skinny_mt(M)};
+    }
     const bool few = g_force_cfg < 0 && op != 2 && skinny_plan(M, N, K, t, nw);
     Plan best{};
     double best_t = -1;

@@ -7,8 +7,8 @@ from oracle import ref_math as R
 
 pytestmark = pytest.mark.gpu
 
-# 16-, 32- and 64-token slabs with a full, a one-row and a ragged last slab; ragged channels; short and long K; both sides of
-# the token and channel limits
+# what the planner picks on both sides of its token and channel limits, ragged channels, short and long K (slabs of 16 tokens, 32 for int8 at
+# 128 tokens and more, one block row, tiles); every slab variant is forced further down
 SHAPES = [(60, 640, 1664), (40, 1152, 6528), (45, 1160, 1280), (17, 520, 2048), (33, 1000, 1536), (65, 768, 1664), (82, 776, 1664),
           (128, 2048, 896), (129, 1024, 896), (200, 512, 3584), (256, 1024, 1024), (257, 1024, 1024), (5, 1024, 18944), (64, 8192, 896)]
 
@@ -54,6 +54,42 @@ def test_fp8_with_and_without_output_quantization(cuda, M, N, K):
     want = q.to(torch.bfloat16).float() * scale
     got = f8f8_tensorwise_quantized_output(a.to(cuda), b.to(cuda).t(), bias.to(cuda), alpha.to(cuda), 1.0, "bfloat16", scale)
     assert got.dtype == torch.float32 and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("slab", [16, 32, 64])
+@pytest.mark.parametrize("variant", range(6))
+@pytest.mark.parametrize("last", ["one row", "ragged", "full"])
+def test_every_slab_variant(cuda, slab, variant, last):
+    """1 + (variant & 1) channel tiles per wavefront, 4 << (variant >> 1) wavefronts along a K that ends inside a step, ragged channels: int8
+    bit for bit against the exact accumulators, fp8 against float64, its quantized output bit for bit against the steps on the GEMM result."""
+    from llmqrt_amd import _abi
+    from llmqrt_amd.quantize import static_per_tensor_quantize
+    from llmqrt_amd.sq_fp8_kernels import cutlass_f8f8bf16_tensorwise_sm89, f8f8_tensorwise_quantized_output, w8a8_int8_linear_bbf16_obf16_per_channel
+    M, N, K = {"one row": slab + 1, "ragged": 2 * slab + slab // 2 - 3, "full": 2 * slab}[last], 328, 1168
+    g = torch.Generator().manual_seed(M)
+    qx, qw = _ints((M, K), M), _ints((N, K), N)
+    sx, sw = torch.rand(M, generator=g) * 0.01 + 1e-3, torch.rand(N, generator=g) * 0.01 + 1e-3
+    bias = torch.randn(N, generator=g).bfloat16()
+    acc = R.int8_gemm_exact(qx, qw)
+    a, b = [(torch.randn(n, K, generator=g) * 30).clamp(-448, 448).to(torch.float8_e4m3fn) for n in (M, N)]
+    ref = a.double() @ b.double().t() * 0.01 + bias.double()
+    scale = torch.tensor([float(ref.abs().max()) / 300], device=cuda)
+    alpha = torch.tensor(0.01, device=cuda)
+    dump = torch.full((M, N), -1, dtype=torch.int32, device=cuda)
+    L = _abi.lib()
+    _abi.check(L.llmq_gemm_force_plan(100 + variant, slab), "force_plan")
+    try:
+        y = w8a8_int8_linear_bbf16_obf16_per_channel(qx.to(cuda), qw.to(cuda).t(), bias.to(cuda), sx.to(cuda).view(-1, 1),
+                                                     sw.to(cuda).view(1, -1), _acc_dump=dump)
+        y8 = cutlass_f8f8bf16_tensorwise_sm89(a.to(cuda), b.to(cuda).t(), bias.to(cuda), alpha, 1.0, "bfloat16")
+        got = f8f8_tensorwise_quantized_output(a.to(cuda), b.to(cuda).t(), bias.to(cuda), alpha, 1.0, "bfloat16", scale)
+    finally:
+        L.llmq_gemm_force_plan(-1, 1)
+    assert torch.equal(dump.cpu(), acc)
+    want = R.w8a8_epilogue_per_token_per_channel(acc, sx, sw, bias, torch.bfloat16)
+    assert torch.equal(y.cpu().view(torch.int16), want.view(torch.int16))
+    assert ((y8.cpu().double() - ref).abs() <= 2e-4 * ref.abs().max() + ref.abs() / 256).all()
+    assert torch.equal(got, static_per_tensor_quantize(y8, scale).to(torch.bfloat16).float() * scale)
 
 
 @pytest.mark.parametrize("cfg", [4, 5, 8, 9, 10])
