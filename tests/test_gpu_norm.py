@@ -11,10 +11,12 @@ from oracle import ref_math as R
 pytestmark = pytest.mark.gpu
 
 INV_RTOL = 5e-7  # ~4 ulp of fp32: summation order + one sqrt + one division
-# (258, 896) .. (257, 520) take the wavefront-per-row kernels (256 rows or more of at most 1024 elements), the last three
-# the half-size blocks with four chunks per thread (256 rows or more of 2056 .. 4096 elements)
+# (258, 896) .. (257, 520) take the wavefront-per-row kernels (256 rows or more of at most 1024 elements); then both sides of the row counts
+# and row lengths at which the block of a row changes: 257-512 chunks (512 threads below 256 rows, 256 below 768, 128), 513-1024, 1025-2560
+# (512 threads up to 256 rows, 256)
 SHAPES = [(1, 896), (16, 896), (7, 3584), (128, 3584), (33, 18944), (3, 8), (5, 24576), (2, 40960),
-          (258, 896), (1027, 1024), (300, 8), (257, 520), (300, 3584), (257, 2056), (256, 4096)]
+          (258, 896), (1027, 1024), (300, 8), (257, 520), (300, 3584), (257, 2056), (256, 4096),
+          (255, 4096), (767, 2056), (768, 4096), (9, 4104), (300, 8192), (256, 8200), (257, 8200), (3, 20480)]
 
 
 def _inputs(M, K, dtype, seed):
@@ -79,6 +81,23 @@ def test_rmsnorm_fp8_fused(cuda, M, K, dtype):
     assert torch.equal(y.cpu().view(torch.int16), y_ref.view(torch.int16))
     assert torch.equal(s.cpu(), s_ref)
     assert torch.equal(q.cpu().view(torch.uint8), q_ref.view(torch.uint8))
+
+
+@pytest.mark.parametrize("M,K", [(7, 3584), (300, 3584), (768, 2056), (300, 1024), (9, 4104), (9, 8200), (257, 8200), (3, 24576)])
+def test_a_nan_stays_in_its_row(cuda, M, K):
+    """One NaN makes its row's mean NaN: normalised row and scale are NaN, int8 codes 0, fp8 codes NaN; the other rows keep their bits."""
+    from llmqrt_amd.norm import rmsnorm_per_token_quantize, rmsnorm_quantize_activation_per_token_absmax
+    x, w = _inputs(M, K, torch.bfloat16, M * K)
+    bad = x.clone()
+    bad[1, K - 1] = float("nan")
+    rest = [m for m in range(M) if m != 1]
+    for fused in (rmsnorm_quantize_activation_per_token_absmax, rmsnorm_per_token_quantize):
+        q0, s0, y0 = [t.cpu() for t in fused(x.to(cuda), w.to(cuda), 1e-6, return_normed=True)]
+        q, s, y = [t.cpu() for t in fused(bad.to(cuda), w.to(cuda), 1e-6, return_normed=True)]
+        assert y[1].isnan().all() and s[1].isnan().all()
+        assert bool((q[1] == 0).all()) if q.dtype == torch.int8 else q[1].float().isnan().all()
+        for a, b in ((q, q0), (s, s0), (y, y0)):
+            assert torch.equal(a[rest].contiguous().view(torch.uint8), b[rest].contiguous().view(torch.uint8))
 
 
 def _mean_square_in_order(x, M):

@@ -13,10 +13,13 @@ def _acts(M, K, seed, dtype):
 
 
 # (258, 896) .. (257, 520) take the wavefront-per-row kernels (256 rows or more of at most 1024 elements): ragged row
-# counts, one and two chunks per lane, rows shorter than a wavefront; the last three the half-size blocks with four
-# chunks per thread (256 rows or more of 2056 .. 4096 elements): the shortest and longest such rows and K = 3584
+# counts, one and two chunks per lane, rows shorter than a wavefront; then both sides of the row counts and row lengths at which the block of a
+# row changes: 257-512 chunks (512 threads below 400 rows, 256 below 6144, 128), 513-1024, 1025-2560 (1024 threads up to 256 rows, 512 up to
+# 1024, 256)
 SHAPES = [(1, 896), (16, 896), (7, 3584), (128, 3584), (33, 18944), (3, 8), (5, 24576), (2, 40960),
-          (258, 896), (1027, 1024), (300, 8), (257, 520), (300, 3584), (257, 2056), (256, 4096)]
+          (258, 896), (1027, 1024), (300, 8), (257, 520), (300, 3584), (257, 2056), (256, 4096),
+          (399, 4096), (400, 2056), (6143, 2056), (6144, 2056), (9, 4104), (9, 8192), (256, 8200), (257, 8200), (1024, 8200), (1025, 8200),
+          (3, 20480)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -220,8 +223,9 @@ def test_sq_per_channel_module_quantizes_its_weight_on_the_gpu(cuda):
 # ---- NaN inputs: torch's max / amax propagate a NaN into the scale, so the whole row (per token) or the whole tensor
 # (per tensor) comes out as NaN scale with zero int8 codes / NaN fp8 codes.  (7, 3584): a block per row with the row
 # in registers; (300, 512): a wavefront per row; (3, 24576): a block per row, second pass re-reading the row;
-# (260, 3584): half-size blocks with four chunks per thread.
-NAN_SHAPES = [(7, 3584), (300, 512), (3, 24576), (260, 3584)]
+# (260, 3584) .. (1025, 8200): the blocks of 512, 256 and 128 threads for rows of 257-512 chunks, of 256 for 513-1024, of 1024, 512 and 256 for
+# 1025-2560.
+NAN_SHAPES = [(7, 3584), (300, 512), (3, 24576), (260, 3584), (400, 3584), (6144, 2056), (9, 4104), (9, 8200), (257, 8200), (1025, 8200)]
 
 
 def _with_nans(M, K, seed, dtype):
