@@ -5,8 +5,8 @@
 //   scale = round_dt( max(absmax, round_dt(floor)) / qmax )
 //   q     = narrow( clamp( round_dt( x / scale ) ) )
 // The kernels reproduce exactly that sequence of roundings.  They are HBM-bound:
-// 2 bytes read + 1 byte written per element, one row per 256-thread block, the row held in
-// registers between the absmax pass and the quantize pass so x is read from HBM once.
+// 2 bytes read + 1 byte written per element, one block (of 128 to 1024 threads, row_shape below) or wavefront per row, the row
+// held in registers between the absmax pass and the quantize pass so x is read from HBM once.
 #include <type_traits>
 
 #include "llmq_common.h"
@@ -38,8 +38,8 @@ __device__ __forceinline__ void store_alpha(const TensorAlpha& ta, float s) {
 
 // One block of NT threads per row.  NC > 0: the row's 16-byte chunks (8 elements) are kept in NC
 // registers per thread between the two passes; NC == 0: rows of any length, second pass
-// re-reads x (served by L2).  A tensor-wide or static scale needs no second look at the row and runs with NC == 0: fewer
-// registers and more rows in flight beat requesting the row ahead of the scale (static, 8192 x 3584: 18.0 against 21.9 us).
+// re-reads x (served by L2).  A tensor-wide or static scale needs no second look at the row: with up to 512 rows it is held in registers
+// all the same, requested ahead of the scale; with more NC == 0, whose fewer registers keep more rows in flight (launch_rows).
 template <int DT, int MODE, int SCALE, int NC, int NT = kThreads>
 __global__ __launch_bounds__(NT) void quant_rows_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, int64_t K, uint8_t* __restrict__ q,
@@ -550,11 +550,11 @@ int launch_rows(const void* x, int64_t M, int64_t K, int64_t ldx, void* q, void*
         case R512x1: LLMQ_LAUNCH_NCT(1, 512); break;
         case R256x1: LLMQ_LAUNCH_NCT(1, 256); break;
         case R256x2: LLMQ_LAUNCH_NCT(2, 256); break;
-        case R128x4: if constexpr (SCALE == SCALE_ROW) LLMQ_LAUNCH_NCT(4, 128); break;  // (M >= 6144)
+        case R128x4: LLMQ_LAUNCH_NCT((SCALE == SCALE_ROW ? 4 : 0), (SCALE == SCALE_ROW ? 128 : 256)); break;  // (M >= 6144: rows by token only)
         case R256x4: LLMQ_LAUNCH_NCT(4, 256); break;
         case R1024x3: LLMQ_LAUNCH_NCT(3, 1024); break;
         case R512x5: LLMQ_LAUNCH_NCT(5, 512); break;
-        case R256x10: if constexpr (SCALE == SCALE_ROW) LLMQ_LAUNCH_NCT(10, 256); break;  // (M > 1024)
+        case R256x10: LLMQ_LAUNCH_NCT((SCALE == SCALE_ROW ? 10 : 0), 256); break;  // (M > 1024: the same)
         default: LLMQ_LAUNCH_NCT(0, 256);
     }
     return launch_status();
