@@ -1,8 +1,8 @@
-// W8A8 int8 / FP8 GEMM for a few tokens (M <= 64): one launch, no LDS staging, no workspace.
+// W8A8 int8 / FP8 GEMM for a few tokens (up to 64 in one block row, up to 256 in slabs of 16 or 32): one launch, no LDS staging, no workspace.
 //
 //   acc[m,n] = sum_k A[m,k] * B[n,k]        A: [M,K] row-major, B: [N,K] row-major (both K-contiguous)
 //
-// With at most 64 tokens the op streams the weights once out of HBM (M*K + N*K bytes for 2*M*N*K operations) and
+// With at most 64 tokens in a block the op streams the weights once out of HBM (M*K + N*K bytes for 2*M*N*K operations) and
 // the matrix cores idle; what counts is bytes in flight and a short instruction stream.  Both operands are
 // K-contiguous, and that is the layout a lane of the 16x16 MFMAs wants (lane (r, kq) feeds 16 or 32 consecutive
 // K-bytes of row r), so the weights go from global memory straight into the operand registers:

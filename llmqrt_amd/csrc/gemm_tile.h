@@ -40,14 +40,14 @@ constexpr TileShape kShapes[] = {
     {32, 128, 128},   // 5: 4 waves x (32x32), decode
     {256, 256, 128},  // 6: 8 waves x (128x64), whole 128-byte lines per row (fp8 prefill)
     {128, 256, 128},  // 7: 8 waves x (64x64): twice the tiles of config 6 for grids that would leave CUs idle
-    {128, 128, 128},  // 8: 8 waves x (64x32)  } direct loads only: K in whole 128-byte tiles
+    {128, 128, 128},  // 8: 8 waves x (64x32)  } direct loads only (a ragged K tail goes through registers behind them)
     {192, 128, 128},  // 9: 8 waves x (96x32)  }
     {256, 128, 128},  // 10: 8 waves x (64x64) }
 };
 constexpr int kNumShapes = sizeof(kShapes) / sizeof(kShapes[0]);
 
 // One launch of the tile kernel (plus the reduction kernel of a K split) for the plan's tile configuration.
-// allow_dma = false keeps the register-staged main loop (a ragged K tail always does).
+// allow_dma = false keeps the register-staged main loop (as do 64-byte K tiles with a ragged K, and in fp8).
 #define LLMQ_GEMM_LAUNCH_ARGS                                                                                   \
     const uint8_t *A, int64_t lda, const uint8_t *B, int64_t ldb, int M, int N, int K, const Plan &p,            \
         const Epilogue &ep, void *out, int64_t ldo, void *acc_dump, void *ws, bool allow_dma, hipStream_t st

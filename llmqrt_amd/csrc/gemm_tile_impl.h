@@ -7,7 +7,7 @@
 // 16-byte chunks and nothing is ever transposed.
 //
 // Kernel shape (template GemmCfg): a block of WM x WN wavefronts owns a BM x BN output tile
-// and walks K in BK-byte steps through a double-buffered LDS ring; each wavefront owns a
+// and walks K in BK-byte steps through a ring of 2 to 4 LDS stages; each wavefront owns a
 // (BM/WM) x (BN/WN) sub-tile made of 32x32 MFMA tiles:
 //   int8: v_mfma_i32_32x32x32_i8      (16 K-bytes per lane per operand, 8 passes)
 //   fp8 : v_mfma_f32_32x32x64_f8f6f4  (32 K-bytes per lane per operand, 16 passes; the
@@ -300,7 +300,7 @@ __global__ __launch_bounds__(C::NT) void gemm_tile_kernel(
         }
     };
 
-    // ---- main loop: tile kt is computed from LDS stage kt & 1 while tile kt+1 sits in registers
+    // ---- main loop.  Register-staged: tile kt is computed from LDS stage kt & 1 while tile kt+1 sits in registers
     // and tile kt+2 is in flight from global memory.  Two tiles per iteration, no conditional
     // compute: an odd tile count is padded with a zero tile -----------------------------------
     if constexpr (C::DMA) {
@@ -908,7 +908,7 @@ int launch_gemm(const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ldb, in
     // bytes, so they have a single sub-step there and stay register-staged).
     const int bk = kShapes[p.cfg].bk;
     const bool dma = allow_dma && p.k_per_split % bk == 0 && (K % bk == 0 || bk == 128);
-    Plan staged = p;  // tiles that exist with direct loads only: a forced plan on a ragged K takes the staged tile next in size
+    Plan staged = p;  // tiles that exist with direct loads only: forced to the register-staged loop, the staged tile next in size runs
     if (p.cfg >= 8) staged.cfg = p.cfg == 8 ? 3 : 2;
     int rc = dma ? launch_shape<FP8, AFMT, true>(A, lda, B, ldb, M, N, K, p, ep, out, ldo, acc_dump, ws, st)
                  : launch_shape<FP8, AFMT, false>(A, lda, B, ldb, M, N, K, staged, ep, out, ldo, acc_dump, ws, st);
