@@ -280,10 +280,9 @@ int llmq_gemm_num_configs(void);
 /* out[m,n] = fp16( sum_k x[m,k] * fp16((q[k,n] - z[k/G,n]) * s[k/G,n]) + bias[n] ), fp32
  * accumulation in a fixed order (deterministic, unlike the reference's fp16 atomics).
  * x: fp16 [M,K] (ldx >= K, K % 32 == 0); out: fp16 [M,N] contiguous; bias: fp16 [N] or NULL.
- * Up to 64 tokens a streaming kernel runs (for group 128 the weights enter the matrix core
- * unrounded, exact (q - z) * s in fp32, instead of rounded to fp16 first); above 64 tokens
- * an fp16 tile GEMM dequantizes the weights on their way into LDS.  All are within 1e-2 of the
- * dequantize-then-matmul math.
+ * Up to 64 tokens of a group that is a multiple of 128 the weights enter the matrix core unrounded, exact (q - z) * s in
+ * fp32, instead of rounded to fp16 first; above 64 tokens either, by plan.  All are within 1e-2 of the dequantize-then-matmul
+ * math.
  * workspace: >= llmq_awq_gemm_workspace_bytes(M,N,K) bytes, 16-byte aligned.  Its first
  * llmq_awq_workspace_ticket_bytes() bytes are the arrival counters of the few-token kernel's K split:
  * they must be zero when a call starts and every call leaves them zero, so a workspace is cleared once
@@ -315,6 +314,14 @@ int llmq_awq_gemm_tickets(const void* x, int x_dtype, int64_t ldx, const int32_t
                           void* tickets, void* partials, size_t partials_bytes, llmq_stream_t stream);
 size_t llmq_awq_gemm_partials_bytes(int64_t M, int64_t N, int64_t K, int64_t group);
 
+/* llmq_awq_gemm_tickets for whole modules: bf16 x and out wherever llmq_awq_linear_bf16_supported says 1 (rows ldx elements apart),
+ * with llmq_awq_gemm_bf16's conversions (linear_awq.py:245-262): a decode batch of any group size and prompts of any length. */
+int llmq_awq_linear(const void* x, int x_dtype, int64_t ldx, const int32_t* qweight, const void* scales,
+                    const int32_t* qzeros, const void* bias, void* out,
+                    int64_t M, int64_t N, int64_t K, int64_t group,
+                    void* tickets, void* partials, size_t partials_bytes, llmq_stream_t stream);
+int llmq_awq_linear_bf16_supported(int64_t M, int64_t N, int64_t K, int64_t group, int64_t ldx);
+
 /* No counterpart in the reference (its split-K ends in fp16 atomics on the output, awq_kernels.py:253-267):
  * size of the counter area at the start of an AWQ workspace, and a launch on `stream` that zeroes it. */
 size_t llmq_awq_workspace_ticket_bytes(void);
@@ -324,7 +331,8 @@ int llmq_awq_workspace_init(void* workspace, size_t workspace_bytes, llmq_stream
  * llmq_awq_gemm for every later call of this process: v = 1 or 2 words per lane of the streaming
  * kernel in 16-token slabs, 5 or 6 = streaming kernel with 2 or 4 token tiles per wavefront,
  * 3, 7 or 4 = tile kernel with 64x128, 128x128 or 256x256 tiles (any M), 8 .. 11 = the few-token kernel
- * (M <= 64; 128- / 256-byte row segments, one / two stages ahead), 0 = heuristic; the cross-block K split
+ * (M <= 64; 128- / 256-byte row segments, one / two stages ahead), 12 .. 16 = the streaming tile kernel (K % 64 == 0; 32 tokens, 64 tokens
+ * with two / one K slice, 128 tokens with two / one), 0 = heuristic; the cross-block K split
  * (0 = heuristic); the wavefronts per block along K of the streaming kernel (4 or 8), or the K slices
  * inside a block of the few-token kernel (1, 2 or 4, v = 8 only); 0 = heuristic.
  * v + 32 keeps the tile kernel's register-staged activation loads (default: straight into LDS when K % 64 == 0).

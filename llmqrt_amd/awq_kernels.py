@@ -112,7 +112,21 @@ def awq_gemm_bf16(input: torch.Tensor, qweight: torch.Tensor, scales: torch.Tens
     return _awq_gemm(input, qweight, scales, qzeros, 1, bias)
 
 
-def _awq_gemm(input, qweight, scales, qzeros, split_k_iters, bias):
+def awq_linear_bf16_supported(M: int, N: int, K: int, group_size: int) -> bool:
+    """Whether ``awq_linear_bf16`` takes this shape: some kernel converts bf16 activations and outputs itself."""
+    return bool(_abi.lib().llmq_awq_linear_bf16_supported(M, N, K, group_size, K))
+
+
+@torch.no_grad()
+def awq_linear_bf16(input: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor, qzeros: torch.Tensor,
+                    bias: torch.Tensor | None = None) -> torch.Tensor:
+    """What the module does with bf16 activations (linear_awq.py:245-262) without launches for the conversions, for shapes that
+    awq_linear_bf16_supported takes."""
+    assert input.dtype == torch.bfloat16
+    return _awq_gemm(input, qweight, scales, qzeros, 1, bias, "llmq_awq_linear")
+
+
+def _awq_gemm(input, qweight, scales, qzeros, split_k_iters, bias, entry="llmq_awq_gemm_tickets"):
     M, K = input.shape
     N = qweight.shape[1] * 8
     group_size = qweight.shape[0] // qzeros.shape[0]
@@ -122,7 +136,7 @@ def _awq_gemm(input, qweight, scales, qzeros, split_k_iters, bias):
     _check_layout(qweight, scales, qzeros, K, N, group_size)
     assert input.device == qweight.device
     x = input
-    if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:
+    if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16 or (entry == "llmq_awq_linear" and x.stride(0) >= 1 << 22):
         x = x.contiguous()
     bias = _bias_vector(bias, N, x.device)
     if bias is not None:
@@ -133,8 +147,8 @@ def _awq_gemm(input, qweight, scales, qzeros, split_k_iters, bias):
     partials = L.llmq_awq_gemm_partials_bytes(M, N, K, group_size)
     ws = _abi.workspaces.get(x.device, partials)
     counters = host().awq_counters(x) if partials else None
-    _abi.check(L.llmq_awq_gemm_tickets(x.data_ptr(), _abi.dtype_code(input.dtype), x.stride(0), qweight.data_ptr(),
-                                       scales.data_ptr(), qzeros.data_ptr(), _abi.ptr(bias), result.data_ptr(), M, N, K,
-                                       group_size, _abi.ptr(counters), _abi.ptr(ws), ws.numel() if ws is not None else 0,
-                                       _abi.stream_of(x)), "llmq_awq_gemm")
+    _abi.check(getattr(L, entry)(x.data_ptr(), _abi.dtype_code(input.dtype), x.stride(0), qweight.data_ptr(),
+                                 scales.data_ptr(), qzeros.data_ptr(), _abi.ptr(bias), result.data_ptr(), M, N, K,
+                                 group_size, _abi.ptr(counters), _abi.ptr(ws), ws.numel() if ws is not None else 0,
+                                 _abi.stream_of(x)), "llmq_awq_gemm")
     return result

@@ -20,6 +20,8 @@
 //   * fp32 accumulation in the MFMA; the 4 wavefronts of a block split the block's K range and
 //     are summed through LDS in a fixed order; a K split across blocks goes through an fp32
 //     workspace and a finishing kernel, again in a fixed order (results are deterministic).
+#include <algorithm>
+
 #include "awq_plans.h"
 #include "llmq_common.h"
 
@@ -744,7 +746,43 @@ inline AwqDecodePlan decode16_plan(int64_t M, int64_t N, int64_t K) {
     return make_awq_decode_plan(M, N, K, cs, pd, g_force_splits, g_force_kw);
 }
 
-// More than 64 tokens go to the tile kernel (weights dequantized once per token tile on their way into LDS);
+// The streaming tile kernel (awq_stream.hip) takes what it is ahead at (us, weights out of HBM, kernel before / stream):
+//   past 64 tokens everything that it supports: 128 x 37888 x 3584 92.9 / 51.6, 128 x 3584 x 18944 51.8 / 32.7, 512 x 37888 x 3584 223 / 158,
+//     512 x 4608 x 3584 36.7 / 32.2; 300 random problems of 65-1024 tokens 1.35 times faster in the mean, seven up to 15 % slower (all of 2 MB of
+//     weights and less, 10-14 us);
+//   17-64 tokens that the few-token kernel takes as slabs of 16: with 40 million weights and more, where unpacking them once per slab costs
+//     more than a second launch for the K split (64 x 37888 x 3584 44.5 / 33.8, 64 x 3584 x 18944 29.8 / 24.2, 42 x 4608 x 21024 51.5 / 26.9; but 64
+//     x 4608 x 3584 15.0 / 15.4, 33 x 3584 x 3584 12.8 / 13.2), and with 1.5 million and fewer, which need no split (29 x 896 x 896 9.4 / 8.1);
+//   other groups and channel counts: past 16 tokens all (64 x 6400 x 4608, group 64: 31.5 / 17.8; 1.25-1.8 times in the mean), up to 16 from 24
+//     million weights on (12 x 5120 x 15488, group 32: 27.7 / 20.6; 3 x 896 x 9728, group 64: 8.8 / 11.1); groups of 128, whose register-streaming
+//     kernel is faster, past 24 tokens all (29 x 13568 x 1048 19.8 / 16.1), 17-24 from 30 million on (19 x 4992 x 1328 11.5 / 12.5), up to 16 from 150
+//     million on (5 x 17408 x 11768 45.4 / 33.7, 2 x 11264 x 3728 12.9 / 16.1).  In a bf16 model always: the kernels before have a
+//     conversion launch on either side there (12 x 4480 x 2152 20.9 / 12.6).
+inline bool stream_supported(int64_t M, int64_t N, int64_t K, int64_t group, int64_t ldx) {
+    return (g_force_v == 0 || (g_force_v >= 12 && g_force_v < 12 + kAwqStreamConfigs)) && group > 0 && awq_stream_supported(M, N, K, group, ldx);
+}
+inline bool stream_path(int64_t M, int64_t N, int64_t K, int64_t group, int64_t ldx, bool bf16_io) {
+    if (!stream_supported(M, N, K, group, ldx)) return false;
+    if (g_force_v != 0 || M > 64) return true;
+    const double weights = (double)N * K;
+    if (awq_decode_supported(M, N, K, group)) return M > 16 && (weights >= 40e6 || weights <= 1.5e6);
+    if (bf16_io) return true;
+    if (decode_path(M, group)) return M > 24 || weights >= (M > 16 ? 30e6 : 150e6);
+    return M > 16 || weights >= 24e6;
+}
+// Searching a plan takes a few microseconds of host time and a call needs it for its workspace and for its launch, so each host thread
+// remembers the last plans it made (a pure function of sizes; a forced plan is not remembered).
+AwqStreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int64_t group, size_t max_partials = SIZE_MAX) {
+    if (g_force_v >= 12) return make_awq_stream_plan(M, N, K, group, max_partials, g_force_v - 12, g_force_splits);
+    struct Entry { int64_t M, N, K, group; AwqStreamPlan plan; };
+    static thread_local Entry cache[64] = {};
+    Entry& e = cache[((uint64_t)(M * 31 + N * 17 + K * 7 + group) * 0x9E3779B97F4A7C15ull) >> 58];
+    if (e.M != M || e.N != N || e.K != K || e.group != group) e = Entry{M, N, K, group, make_awq_stream_plan(M, N, K, group, SIZE_MAX, -1, 0)};
+    if (awq_stream_workspace_bytes(e.plan, M, N) <= max_partials) return e.plan;
+    return make_awq_stream_plan(M, N, K, group, max_partials, -1, 0);
+}
+
+// More than 64 tokens that it does not take go to the tile kernel (weights dequantized once per token tile on their way into LDS);
 // llmq_awq_force_plan(3 | 4, ...) forces its 64x128 | 256x256 tile for any M, (1 | 2, ...) keeps the slabs.
 inline bool tile_path(int64_t M) { return g_force_v == 3 || g_force_v == 4 || g_force_v == 7 || (g_force_v == 0 && M > 64); }
 inline AwqTilePlan tile_plan(int64_t M, int64_t N, int64_t K) {
@@ -768,9 +806,10 @@ using namespace llmq;
 extern "C" int llmq_awq_force_plan(int v, int splits, int k_waves) {
     const int staged = v >= 0 ? (v & 32) : 0;  // + 32: the tile kernel keeps its register-staged activation loads
     if (v >= 0) v &= ~32;
-    if (v < 0 || v > 11 || splits < 0 || splits > 64) return LLMQ_ERR_SHAPE;
+    if (v < 0 || v >= 12 + kAwqStreamConfigs || splits < 0 || splits > 64) return LLMQ_ERR_SHAPE;
     // K slices of the few-token kernel: 1, 2, 4 (v = 0 or 8 .. 11); wavefronts along K of the streaming kernel: 4, 8
-    const bool few = v == 0 || v >= 8;
+    const bool few = v == 0 || (v >= 8 && v <= 11);
+    if (v >= 12 && k_waves != 0) return LLMQ_ERR_SHAPE;
     if (k_waves != 0 && !(k_waves == 4 || (few && (k_waves == 1 || k_waves == 2)) || (!few && k_waves == 8))) return LLMQ_ERR_SHAPE;
     set_awq_tile_direct_loads(staged ? 0 : 1);  // state changes only once the arguments are accepted
     g_force_v = v;
@@ -787,14 +826,13 @@ static bool awq_sizes_ok(int64_t M, int64_t N, int64_t K) {
 extern "C" size_t llmq_awq_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (!awq_sizes_ok(M, N, K)) return 0;
     size_t total = 0;
+    for (int64_t group = 32; group <= 128; group += 96)  // the group size is not known here: plans of groups that are and are not a multiple of 128
+        if (K % group == 0 && stream_supported(M, N, K, group, K)) total = std::max(total, awq_stream_workspace_bytes(stream_plan(M, N, K, group), M, N));
     if (tile_path(M)) {
         const AwqTilePlan t = tile_plan(M, N, K);
-        if (t.splits > 1) total = (size_t)t.splits * M * N * sizeof(float);
+        if (t.splits > 1) total = std::max(total, (size_t)t.splits * M * N * sizeof(float));
     }
-    if (awq_decode_supported(M, N, K, 128)) {
-        const size_t need = awq_decode_workspace_bytes(decode16_plan(M, N, K), M, N);
-        if (need > total) total = need;
-    }
+    if (awq_decode_supported(M, N, K, 128)) total = std::max(total, awq_decode_workspace_bytes(decode16_plan(M, N, K), M, N));
     for (int64_t m0 = 0; m0 < M; m0 += 64) {
         const int64_t mm = M - m0 < 64 ? M - m0 : 64;
         const AwqPlan p = make_awq_plan(mm, N, K);  // sized for either kernel (the group size is not known here)
@@ -819,9 +857,27 @@ extern "C" int llmq_awq_workspace_init(void* workspace, size_t workspace_bytes, 
 
 namespace {
 
+// Partial sums of the kernels other than the streaming tile kernel.  A workspace of that size is still taken where that one asks for more.
+size_t staged_partials_bytes(int64_t M, int64_t N, int64_t K, int64_t group) {
+    if (tile_path(M)) {
+        const AwqTilePlan t = tile_plan(M, N, K);
+        return t.splits > 1 ? (size_t)t.splits * M * N * sizeof(float) : 0;
+    }
+    if (decode16_path(M, N, K, group)) return awq_decode_workspace_bytes(decode16_plan(M, N, K), M, N);
+    size_t total = 0;
+    for (int64_t m0 = 0; m0 < M; m0 += 64) {
+        const int64_t mm = M - m0 < 64 ? M - m0 : 64;
+        const int splits = decode_path(mm, group) ? make_decode_plan(mm, N, K).splits : make_awq_plan(mm, N, K).splits;
+        const size_t need = splits > 1 ? (size_t)splits * mm * N * sizeof(float) : 0;
+        if (need > total) total = need;
+    }
+    return total;
+}
+
+// bf16_any: bf16 wherever a kernel takes it (llmq_awq_linear); otherwise only where llmq_awq_gemm_bf16_supported says so
 int awq_gemm_entry(const void* x, int64_t ldx, const int32_t* qweight, const void* scales, const int32_t* qzeros,
                    const void* bias, void* out, int64_t M, int64_t N, int64_t K, int64_t group, bool bf16_io,
-                   void* ticket_area, void* partials, size_t workspace_bytes, llmq_stream_t stream) {
+                   void* ticket_area, void* partials, size_t workspace_bytes, llmq_stream_t stream, bool bf16_any = false) {
     if (M < 0 || N < 0 || K < 0) return LLMQ_ERR_SHAPE;
     if (M == 0 || N == 0) return LLMQ_OK;
     if (!x || !qweight || !scales || !qzeros || !out) return LLMQ_ERR_NULL;
@@ -840,7 +896,17 @@ int awq_gemm_entry(const void* x, int64_t ldx, const int32_t* qweight, const voi
     const uint16_t* sc = (const uint16_t*)scales;
     const uint16_t* bs = (const uint16_t*)bias;
     const int Ni = (int)N, Ki = (int)K, Gi = (int)group;
-    if (bf16_io && (tile_path(M) || !decode16_path(M, N, K, group))) return LLMQ_ERR_DTYPE;
+    const bool stream_takes = stream_path(M, N, K, group, ldx, bf16_io);
+    if (bf16_io && !(bf16_any && stream_takes) && (tile_path(M) || !decode16_path(M, N, K, group))) return LLMQ_ERR_DTYPE;
+    if (stream_takes) {
+        const size_t given = ws ? workspace_bytes : 0;
+        AwqStreamPlan p = stream_plan(M, N, K, group);
+        if (awq_stream_workspace_bytes(p, M, N) > given) {
+            if (staged_partials_bytes(M, N, K, group) > given) return LLMQ_ERR_WORKSPACE;
+            p = stream_plan(M, N, K, group, given);
+        }
+        return launch_awq_stream(p, (const uint16_t*)x, ldx, qw, sc, qz, bs, (uint16_t*)out, ws, (int)M, Ni, Ki, Gi, bf16_io, st);
+    }
     if (tile_path(M)) {
         const AwqTilePlan t = tile_plan(M, N, K);
         if (t.splits > 1 && (!ws || workspace_bytes < (size_t)t.splits * M * N * sizeof(float))) return LLMQ_ERR_WORKSPACE;
@@ -933,19 +999,9 @@ extern "C" int llmq_awq_gemm_bf16(const void* x, int64_t ldx, const int32_t* qwe
 
 extern "C" size_t llmq_awq_gemm_partials_bytes(int64_t M, int64_t N, int64_t K, int64_t group) {
     if (!awq_sizes_ok(M, N, K)) return 0;
-    if (tile_path(M)) {
-        const AwqTilePlan t = tile_plan(M, N, K);
-        return t.splits > 1 ? (size_t)t.splits * M * N * sizeof(float) : 0;
-    }
-    if (decode16_path(M, N, K, group)) return awq_decode_workspace_bytes(decode16_plan(M, N, K), M, N);
-    size_t total = 0;
-    for (int64_t m0 = 0; m0 < M; m0 += 64) {
-        const int64_t mm = M - m0 < 64 ? M - m0 : 64;
-        const int splits = decode_path(mm, group) ? make_decode_plan(mm, N, K).splits : make_awq_plan(mm, N, K).splits;
-        const size_t need = splits > 1 ? (size_t)splits * mm * N * sizeof(float) : 0;
-        if (need > total) total = need;
-    }
-    return total;
+    // which kernel runs depends on the row stride and the dtype too: the figure covers either
+    const size_t stream = stream_path(M, N, K, group, K, true) ? awq_stream_workspace_bytes(stream_plan(M, N, K, group), M, N) : 0;
+    return std::max(stream, staged_partials_bytes(M, N, K, group));
 }
 
 extern "C" int llmq_awq_gemm_tickets(const void* x, int x_dtype, int64_t ldx, const int32_t* qweight, const void* scales,
@@ -955,6 +1011,18 @@ extern "C" int llmq_awq_gemm_tickets(const void* x, int x_dtype, int64_t ldx, co
     if (x_dtype != LLMQ_BF16 && x_dtype != LLMQ_F16) return LLMQ_ERR_DTYPE;
     return awq_gemm_entry(x, ldx, qweight, scales, qzeros, bias, out, M, N, K, group, x_dtype == LLMQ_BF16, tickets, partials,
                           tickets ? partials_bytes : 0, stream);
+}
+
+extern "C" int llmq_awq_linear_bf16_supported(int64_t M, int64_t N, int64_t K, int64_t group, int64_t ldx) {
+    return awq_sizes_ok(M, N, K) && g_force_v == 0 && (llmq_awq_gemm_bf16_supported(M, N, K, group) || stream_path(M, N, K, group, ldx, true));
+}
+
+extern "C" int llmq_awq_linear(const void* x, int x_dtype, int64_t ldx, const int32_t* qweight, const void* scales,
+                               const int32_t* qzeros, const void* bias, void* out, int64_t M, int64_t N, int64_t K, int64_t group,
+                               void* tickets, void* partials, size_t partials_bytes, llmq_stream_t stream) {
+    if (x_dtype != LLMQ_BF16 && x_dtype != LLMQ_F16) return LLMQ_ERR_DTYPE;
+    return awq_gemm_entry(x, ldx, qweight, scales, qzeros, bias, out, M, N, K, group, x_dtype == LLMQ_BF16, tickets, partials,
+                          tickets ? partials_bytes : 0, stream, true);
 }
 
 extern "C" int llmq_awq_dequant(const int32_t* qweight, const void* scales, const int32_t* qzeros, void* out,

@@ -31,4 +31,13 @@ int launch_awq_decode(const AwqDecodePlan& p, const uint16_t* x, int64_t ldx, co
                       const uint32_t* qz, const uint16_t* bias, uint16_t* out, unsigned int* tickets, float* ws, int M,
                       int N, int K, bool bf16_io, hipStream_t st);
 
+// Streaming tile kernel (awq_stream.hip): a decode batch up to a short prompt, any group; fold: the group's scale in fp32 on exact integers.
+struct AwqStreamPlan { int cfg, fold, splits, units_per_block; };
+constexpr int kAwqStreamConfigs = 5;  // 32 tokens; 64 tokens with two K slices, with one; 128 tokens with two, with one
+bool awq_stream_supported(int64_t M, int64_t N, int64_t K, int64_t group, int64_t ldx);
+AwqStreamPlan make_awq_stream_plan(int64_t M, int64_t N, int64_t K, int64_t group, size_t max_partials, int force_cfg, int force_splits);
+size_t awq_stream_workspace_bytes(const AwqStreamPlan& p, int64_t M, int64_t N);
+int launch_awq_stream(const AwqStreamPlan& p, const uint16_t* x, int64_t ldx, const uint32_t* qw, const uint16_t* scales, const uint32_t* qz,
+                      const uint16_t* bias, uint16_t* out, float* ws, int M, int N, int K, int G, bool bf16_io, hipStream_t st);
+
 }  // namespace llmq

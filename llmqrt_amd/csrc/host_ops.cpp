@@ -384,7 +384,7 @@ std::optional<Tensor> awq(const Tensor& x, const Tensor& qweight, const Tensor& 
               "llmq_gemm_f16");
         return bf16 ? out.to(at::kBFloat16) : out;
     }
-    const bool native_bf16 = bf16 && llmq_awq_gemm_bf16_supported(r.M, N, r.K, group);
+    const bool native_bf16 = bf16 && llmq_awq_linear_bf16_supported(r.M, N, r.K, group, r.K);
     const Tensor xin = bf16 && !native_bf16 ? x.to(at::kHalf) : x;
     Tensor out = make(out_size(x, N), xin.scalar_type(), dev);
     // {arrival counters, partial sums}: the partial sums of this call only
@@ -394,10 +394,10 @@ std::optional<Tensor> awq(const Tensor& x, const Tensor& qweight, const Tensor& 
         ws = make({part}, at::kByte, dev);
         tk = counters().get(dev, l.stream);
     }
-    check(llmq_awq_gemm_tickets(xin.data_ptr(), native_bf16 ? LLMQ_BF16 : LLMQ_F16, r.K, (const int32_t*)qweight.data_ptr(),
+    check(llmq_awq_linear(xin.data_ptr(), native_bf16 ? LLMQ_BF16 : LLMQ_F16, r.K, (const int32_t*)qweight.data_ptr(),
                                 scales.data_ptr(), (const int32_t*)qzeros.data_ptr(), ptr(bias), out.data_ptr(), r.M, N, r.K, group,
-                                part ? tk.data_ptr() : nullptr, part ? ws.data_ptr() : nullptr, (size_t)part, l.stream),
-          "llmq_awq_gemm");
+                          part ? tk.data_ptr() : nullptr, part ? ws.data_ptr() : nullptr, (size_t)part, l.stream),
+          "llmq_awq_linear");
     return bf16 && !native_bf16 ? out.to(at::kBFloat16) : out;
 }
 

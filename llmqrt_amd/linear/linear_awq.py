@@ -6,8 +6,8 @@ from __future__ import annotations
 import torch
 
 from .._native import host
-from ..awq_kernels import (awq_dequantize_transposed, awq_dequantize_triton, awq_gemm_bf16, awq_gemm_bf16_supported,
-                           awq_gemm_triton, gemm_f16)
+from ..awq_kernels import (awq_dequantize_transposed, awq_dequantize_triton, awq_gemm_triton, awq_linear_bf16,
+                           awq_linear_bf16_supported, gemm_f16)
 from .linear_base import LinearBase
 
 AWQ_ORDER = (0, 2, 4, 6, 1, 3, 5, 7)
@@ -33,15 +33,19 @@ def dequant_matmul_token_threshold(in_features: int, out_features: int = 0) -> i
     fused kernels on MI355X.
 
     The reference switches to dequantize + torch.matmul at 1024 tokens (linear_awq.py:22,47).  Here both sides are
-    this library's kernels; measured on the Qwen2-7B shapes (us, fused / dequantize + GEMM) the fused path (few-token
-    kernel up to 64 tokens, tile kernel with in-loop dequantization above) is ahead up to ~256 tokens for qkv / o
-    (K = 3584; o 31 / 33 at 256 tokens, 36 / 34 at 320), ~224 for down (K = 18944; 79 / 83 at 192, 92 / 90 at 256,
-    122 / 102 at 320) and ~550 for gate_up (N = 37888, where the dequantizer's 63 us take longest to amortize:
-    138 / 185 at 256 tokens, 222 / 237 at 512, 264 / 247 at 640).  Both paths are within 1e-2 (max relative) of
-    dequantize-then-matmul in fp32."""
-    if in_features > 8192:
-        return 256
-    return 576 if out_features > 8192 else 288
+    this library's kernels; measured on an MI355X (us, fused / dequantize + GEMM, weights out of HBM) the fused path (streaming
+    tile kernel past 64 tokens) is ahead up to about 2000 tokens and 0-5 % behind from 3000 on: K = 3584, N = 37888 379 / 448 at 1500,
+    524 / 560 at 2048, 755 / 771 at 3000, 1025 / 987 at 4096; K = 18944, N = 3584 156 / 183 at 1100, 273 / 282 at 2048, 452 / 437 at
+    3000; K = N = 3584 40 / 44 at 1100, 61 / 63 at 2048; K = 3584, N = 4608 59 / 66 at 1500, 88 / 83 at 2048.  Few channels: K = 3840,
+    N = 640 25 / 26 at 1541, K = 1664, N = 768 17.3 / 16.2 at 1097; few weights: K = 1152, N = 1408 14.7 / 14.3 at 430, K = N = 896 13.0 / 10.8
+    at 431.  Where the streaming kernel does not run (K no multiple of 64) the fused path is the staged tile kernel, ahead up to ~256 tokens
+    (K = N = 3584 31 / 33 at 256, 36 / 34 at 320), ~224 for a long K (92 / 90 at 256), ~550 for many channels (222 / 237 at 512,
+    264 / 247 at 640).  Both paths are within 1e-2 (max relative) of dequantize-then-matmul in fp32."""
+    if in_features % 64:
+        return 256 if in_features > 8192 else 576 if out_features > 8192 else 288
+    if out_features and in_features * out_features <= 2_000_000:
+        return 400
+    return 1000 if 0 < out_features <= 1024 else 2048
 
 
 def awq_linear_forward(x, qweight, qzeros, scales, w_bit=4, group_size=128, bias=None, out_features=0):
@@ -134,11 +138,12 @@ class WQLinear_GEMM(LinearBase):
             return torch.zeros(out_shape, dtype=x.dtype, device=x.device)
         input_dtype = x.dtype
         tokens = x.numel() // max(x.shape[-1], 1)
-        if input_dtype == torch.bfloat16 and awq_gemm_bf16_supported(tokens, self.out_features, self.in_features,
-                                                                    self.group_size):
-            # a few tokens of a bf16 model: the kernel converts in and out itself
-            return awq_gemm_bf16(x.reshape(-1, x.shape[-1]), self.qweight, self.scales, self.qzeros,
-                                 self.bias).view(out_shape)
+        many = dequant_matmul_token_threshold(self.in_features, self.out_features) if USE_DEQUANT_MATMUL else 1 << 62
+        if input_dtype == torch.bfloat16 and tokens < many and awq_linear_bf16_supported(tokens, self.out_features, self.in_features,
+                                                                                        self.group_size):
+            # up to the threshold the kernels of a bf16 model convert in and out themselves
+            return awq_linear_bf16(x.reshape(-1, x.shape[-1]), self.qweight, self.scales, self.qzeros,
+                                   self.bias).view(out_shape)
         if input_dtype != torch.float16:
             x = x.to(torch.float16)
         with torch.no_grad():
