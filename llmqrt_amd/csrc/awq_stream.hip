@@ -176,10 +176,17 @@ __global__ __launch_bounds__(C::NT, C::KS == 4 ? 4 : 2) void awq_stream_kernel(S
     };
     static_assert(NS <= 4, "wait_stage tells 0, 1, NS - 2 and NS - 1 younger stages apart");
     uint8_t* ring = smem + slice * NS * C::STAGE_BYTES;
-    auto convert = [&](int slot) __attribute__((always_inline)) {  // bf16 activations become fp16 in place: each wavefront the pieces that it loaded
+    // bf16 activations become fp16 in place, each wavefront the pieces that it loaded: read, and a sub-step later written back
+    u4 piece[C::BF ? MT : 1];
+    auto convert_read = [&](int slot) __attribute__((always_inline)) {
+        const u4* p = reinterpret_cast<const u4*>(ring + slot * C::STAGE_BYTES + C::X_AT + wv * MT * 1024) + lane;
+#pragma unroll
+        for (int i = 0; i < MT; i++) piece[C::BF ? i : 0] = p[i * kWave];
+    };
+    auto convert_write = [&](int slot) __attribute__((always_inline)) {
         u4* p = reinterpret_cast<u4*>(ring + slot * C::STAGE_BYTES + C::X_AT + wv * MT * 1024) + lane;
 #pragma unroll
-        for (int i = 0; i < MT; i++) p[i * kWave] = to_f16x8(p[i * kWave]);
+        for (int i = 0; i < MT; i++) p[i * kWave] = to_f16x8(piece[C::BF ? i : 0]);
     };
     auto lds_barrier = []() __attribute__((always_inline)) {  // orders LDS traffic only: the loads stay in flight across it
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -305,7 +312,7 @@ __global__ __launch_bounds__(C::NT, C::KS == 4 ? 4 : 2) void awq_stream_kernel(S
     for (int t = 0; t < NS; t++)
         if (t < ns) issue(t, t);
     wait_stage(min(ns, NS) - 1, std::false_type{});
-    if (C::BF && ns > 0) convert(0);
+    if (C::BF && ns > 0) convert_read(0), convert_write(0);
     lds_barrier();
 #pragma unroll
     for (int pr = 0; pr < 4; pr++) read_words(ring, 0, pr, raw[0]), read_words(ring, 1, pr, raw[1]);
@@ -322,10 +329,11 @@ __global__ __launch_bounds__(C::NT, C::KS == 4 ? 4 : 2) void awq_stream_kernel(S
         const uint8_t *cur = ring + slot * C::STAGE_BYTES, *nxt = ring + next * C::STAGE_BYTES;
         if (C::BF && kt + 1 < ns) {
             wait_stage(younger, std::integral_constant<bool, !decltype(odd_c)::value>{});
-            convert(next);
+            convert_read(next);
         }
         __builtin_amdgcn_sched_barrier(0);
         sub_step(I0{}, odd_c, cur, cur);
+        if (C::BF && kt + 1 < ns) convert_write(next);
         sub_step(I1{}, odd_c, cur, cur);
 #pragma unroll
         for (int i = 0; i < MT; i++) read_x(cur, 3, i, xa[1]);  // the last reads of the slot
@@ -533,7 +541,7 @@ double time_of(const AwqStreamPlan& p, int64_t M, int64_t N, int64_t K) {
 
 // K in whole stages; 32-bit byte offsets into a stage, the scales and the zero points; group numbers by a 32-bit reciprocal
 bool awq_stream_supported(int64_t M, int64_t N, int64_t K, int64_t group, int64_t ldx) {
-    return M >= 1 && M <= (1 << 24) && N >= 8 && N <= (1 << 24) && K >= kStageK && K % kStageK == 0 && K <= (1 << 20) && group % 32 == 0 &&
+    return M >= 1 && M <= (1 << 24) && N >= 8 && N <= (1 << 24) && K >= kStageK && K % kStageK == 0 && K <= (1 << 20) && group >= 32 && group % 32 == 0 && K % group == 0 &&
            ldx < (1 << 22) && (K / group) * N < ((int64_t)1 << 30) && (int64_t)cdiv_s(N, kTileCh) * cdiv_s(M, 32) <= (1 << 24);
 }
 
