@@ -79,7 +79,6 @@ struct Launch {
     explicit Launch(const at::Device& dev) : guard(dev), stream(c10::hip::getCurrentHIPStream(dev.index()).stream()) {}
 };
 
-bool one_launch_tensor(const Rows& r) { return r.M <= llmq_linear_per_tensor_max_tokens(r.K); }
 
 // The weight side of an 8-bit Linear: [N, K] bytes, K % 16 == 0.
 bool weight_ok(const Tensor& w, at::ScalarType dtype, const at::Device& dev, int64_t K) {
@@ -132,12 +131,12 @@ std::optional<Tensor> sq_tensor(const Tensor& x, const Tensor& w, const Tensor& 
         return std::nullopt;
     const at::ScalarType odt = bias ? bias->scalar_type() : x.scalar_type();
     const Launch l(x.device());
-    if (one_launch_tensor(r)) {
+    if (llmq_linear_one_launch_preferred(LLMQ_LINEAR_I8_TENSOR, r.M, w.size(0), r.K)) {
         Tensor out = make(out_size(x, w.size(0)), odt, x.device());
-        check(llmq_linear_per_tensor_dynamic(0, x.data_ptr(), code(x.scalar_type()), r.K, w.data_ptr(), r.K,
-                                             (const float*)w_scale.data_ptr(), ptr(bias), code(odt), out.data_ptr(), code(odt),
-                                             w.size(0), r.M, w.size(0), r.K, l.stream),
-              "llmq_linear_per_tensor_dynamic");
+        check(llmq_linear_one_launch(LLMQ_LINEAR_I8_TENSOR, x.data_ptr(), code(x.scalar_type()), r.K, w.data_ptr(), r.K,
+                                     (const float*)w_scale.data_ptr(), nullptr, ptr(bias), code(odt), nullptr, out.data_ptr(), code(odt),
+                                     w.size(0), r.M, w.size(0), r.K, l.stream),
+              "llmq_linear_one_launch");
         return out;
     }
     // codes, then {scale, alpha}, then the quantizer's partial maxima
@@ -153,11 +152,11 @@ std::optional<Tensor> sq_tensor(const Tensor& x, const Tensor& w, const Tensor& 
     return out;
 }
 
-// The line between the one-launch linear and quantizer + GEMM for per-token scales comes from the module: up to `tokens` rows
-// of fewer than `k` elements.
+// The module sets the widest range in which a per-token linear may run in one launch (up to `tokens` rows of fewer than `k` elements); inside it
+// the measured lines decide.
 struct OneLaunch {
     int64_t tokens, k;
-    bool takes(const Rows& r) const { return r.M <= tokens && r.K < k && r.M <= llmq_linear_dynamic_max_tokens(r.K); }
+    bool takes(int kind, const Rows& r, int64_t N) const { return r.M <= tokens && r.K < k && llmq_linear_one_launch_preferred(kind, r.M, N, r.K); }
 };
 
 std::optional<Tensor> sq_token(const Tensor& x, const Tensor& w, const Tensor& w_scale, const std::optional<Tensor>& bias,
@@ -171,10 +170,10 @@ std::optional<Tensor> sq_token(const Tensor& x, const Tensor& w, const Tensor& w
     const Launch l(x.device());
     const float* ws = (const float*)w_scale.data_ptr();
     Tensor out = make(out_size(x, N), odt, x.device());
-    if (line.takes(r)) {
-        check(llmq_linear_i8_dynamic(x.data_ptr(), code(x.scalar_type()), r.K, (const int8_t*)w.data_ptr(), r.K, ws, ptr(bias),
-                                     code(odt), out.data_ptr(), code(odt), N, r.M, N, r.K, nullptr, nullptr, nullptr, l.stream),
-              "llmq_linear_i8_dynamic");
+    if (line.takes(LLMQ_LINEAR_I8_TOKEN, r, N)) {
+        check(llmq_linear_one_launch(LLMQ_LINEAR_I8_TOKEN, x.data_ptr(), code(x.scalar_type()), r.K, w.data_ptr(), r.K, ws, nullptr, ptr(bias),
+                                     code(odt), nullptr, out.data_ptr(), code(odt), N, r.M, N, r.K, l.stream),
+              "llmq_linear_one_launch");
         return out;
     }
     const int64_t codes = round16(r.M * r.K);
@@ -220,11 +219,11 @@ std::optional<Tensor> fp8_token(const Tensor& x, const Tensor& w, const Tensor& 
     const Launch l(x.device());
     const float* ws = (const float*)w_scale.data_ptr();
     Tensor out = make(out_size(x, N), at::kBFloat16, x.device());
-    if (line.takes(r)) {
-        check(llmq_linear_fp8_dynamic(x.data_ptr(), code(x.scalar_type()), r.K, (const uint8_t*)w.data_ptr(), r.K, ws, ptr(bias),
-                                      bias ? code(bias->scalar_type()) : LLMQ_BF16, out.data_ptr(), LLMQ_BF16, N, r.M, N, r.K,
-                                      nullptr, nullptr, nullptr, l.stream),
-              "llmq_linear_fp8_dynamic");
+    if (line.takes(LLMQ_LINEAR_FP8_TOKEN, r, N)) {
+        check(llmq_linear_one_launch(LLMQ_LINEAR_FP8_TOKEN, x.data_ptr(), code(x.scalar_type()), r.K, w.data_ptr(), r.K, ws, nullptr, ptr(bias),
+                                     bias ? code(bias->scalar_type()) : LLMQ_BF16, nullptr, out.data_ptr(), LLMQ_BF16, N, r.M, N, r.K,
+                                     l.stream),
+              "llmq_linear_one_launch");
         return out;
     }
     const int64_t codes = round16(r.M * r.K);
@@ -249,12 +248,14 @@ std::optional<Tensor> fp8_tensor(const Tensor& x, const Tensor& w, const Tensor&
         (output_scale && !scale_ok(*output_scale, x.device(), 1)))
         return std::nullopt;
     const Launch l(x.device());
-    if (!input_scale && !output_scale && one_launch_tensor(r)) {
-        Tensor out = make(out_size(x, N), odt, x.device());
-        check(llmq_linear_per_tensor_dynamic(1, x.data_ptr(), code(x.scalar_type()), r.K, w.data_ptr(), r.K,
-                                             (const float*)w_scale.data_ptr(), ptr(bias), code(odt), out.data_ptr(), code(odt), N,
-                                             r.M, N, r.K, l.stream),
-              "llmq_linear_per_tensor_dynamic");
+    const int kind = input_scale ? LLMQ_LINEAR_FP8_STATIC : LLMQ_LINEAR_FP8_TENSOR;
+    if ((input_scale || !output_scale) && llmq_linear_one_launch_preferred(kind, r.M, N, r.K)) {
+        Tensor out = make(out_size(x, N), output_scale ? at::kFloat : odt, x.device());
+        check(llmq_linear_one_launch(kind, x.data_ptr(), code(x.scalar_type()), r.K, w.data_ptr(), r.K, (const float*)w_scale.data_ptr(),
+                                     input_scale ? (const float*)input_scale->data_ptr() : nullptr, ptr(bias), code(odt),
+                                     output_scale ? (const float*)output_scale->data_ptr() : nullptr, out.data_ptr(), code(odt), N, r.M, N,
+                                     r.K, l.stream),
+              "llmq_linear_one_launch");
         return out;
     }
     const int64_t codes = round16(r.M * r.K), part = input_scale ? 0 : (int64_t)llmq_quant_workspace_bytes();

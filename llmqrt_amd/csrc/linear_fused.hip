@@ -1,37 +1,28 @@
-// Few-token quantized linear in one launch: per-token dynamic activation quantizer + W8A8 int8 / FP8 GEMM +
-// per-token x per-channel epilogue, for up to 16 tokens (decode).
+// Few-token quantized linear in one launch: activation quantizer (dynamic per token, dynamic per tensor, or static) + W8A8 int8 /
+// FP8 GEMM + dequant epilogue, for up to 16 tokens (decode).
 //
 //   s[m]    = round_dt( max(absmax_k |x[m,k]|, round_dt(floor)) / qmax )            the row quantizers of quant.hip
 //   q[m,k]  = narrow( clamp( round_dt( x[m,k] / s[m] ) ) )
 //   out     = ((sum_k q[m,k] * B[n,k]) * s[m]) * sw[n] + bias[n]                     llmq_gemm_w8a8 / llmq_gemm_fp8
 //
-// The reference runs these as separate steps (nn_models/modules/linear/linear_sq.py:97-138: the quantizer of
-// lines 55-65, then the GEMM op; linear_fp8.py:40-63 + 199-221).  With a few tokens each step is a launch of a
+// The reference runs these as separate steps (nn_models/modules/linear/linear_sq.py:97-138: the quantizers of
+// lines 44-65, then the GEMM op; linear_fp8.py:11-63 + 199-221, 296-311).  With a few tokens each step is a launch of a
 // few microseconds that mostly waits; here the GEMM kernel quantizes its own activation operand:
-//   * a block owns 16*T output channels, its NW wavefronts own consecutive runs of K steps, and the weights stream
-//     from global memory straight into MFMA operand registers, exactly as in gemm_skinny.hip;
-//   * before its first step a block quantizes the activations itself, once, into LDS: wavefront w takes tokens w,
-//     w + NW, .., keeps the row in registers, reduces |x|, and writes the codes as the [token][K] int8 / fp8 matrix
-//     the MFMA operand reads expect (the activations are a few KB per token and sit in L2; every block repeats this,
-//     which is cheaper than a launch).  The first batch of weight loads is already in flight meanwhile;
-//   * the arithmetic is the row quantizer's (quant_math.h), so codes and scales are bit-identical to
-//     llmq_quant_*_per_token and the result is bit-identical to the two-launch form.  Block 0 can write codes and
-//     scales out for checking.
-// The quantized activations must fit in LDS: M * (K + 16) <= 64 KB (16 tokens at K = 3584, 3 at K = 18944).
-// Measured on MI355X (Qwen2-7B projections, weights out of HBM, launches back to back): level with the quantizer +
-// few-token GEMM pair at 1-3 tokens and K = 3584 (qkv 10.0 against 9.5 us, o 7.9 against 8.1, gate_up 32.5 against
-// 34.5), slower at 16 tokens (16 against 11) and for K = 18944 (30 against 20): the stream hides a second launch, while
-// the quantizer's load -> reduce -> quantize chain now precedes every block's first MFMA.  What it saves is a launch on
-// the host side.  (Quantizing in the operand registers of every wavefront instead of once per block was measured
-// 40-100 % slower: 15 of 16 MFMA rows repeat the same token's work at one token.)
+//   * a wavefront owns 16*T output channels and one of NW consecutive runs of K steps, and the weights stream
+//     from global memory straight into MFMA operand registers, exactly as in gemm_skinny.hip; a block has NG such sets of NW;
+//   * before its first step a block quantizes the activations itself, once, into LDS, with all its wavefronts and NI more that do nothing
+//     else: the codes as the [token][K] int8 / fp8 matrix the MFMA operand reads expect (the activations are a few KB per token and sit in
+//     L2; every block repeats this, which is cheaper than a launch).  The first batch of weight loads is already in flight meanwhile;
+//   * the arithmetic is the row quantizer's (quant_math.h), so codes and scales are bit-identical to llmq_quant_*, and so is
+//     the result where the few-token GEMM splits K over as many wavefronts (int32 sums always; fp32 sums are else added in another order).
 //
-// TENSOR: the same with one scale for the whole activation tensor (SqW8A8BBF16OBF16PerTensor, per-tensor
-// FP8DynamicLinear; linear_sq.py:44-54, linear_fp8.py:11-27), for M * K <= 16384.  A block spreads the tensor's 16-byte pieces
-// over all its threads and keeps them in registers from the maximum to the codes: two loads' latency and one block
-// reduction instead of a launch that every GEMM block would wait for.
-// Ahead of the pair at every size tried (us, one launch / two, int8, weights out of HBM): 1 x 3584 x 3584 7.0 / 8.0, 4 x 3584 x
-// 3584 7.7 / 9.0, 16 x 896 x 896 5.4 / 7.6, 1 x 896 x 4864 7.7 / 9.5, 16 x 9728 x 896 9.4 / 9.7, 4 x 37888 x 3584 29.9 / 31.0,
-// 1 x 4096 x 16384 14.7 / 16.3.  The line at 16384 elements is what the block holds in 32 registers a thread.
+// What bounds it is a chain: launch, activation loads, maximum, codes, barrier, the operand reads of a few steps, the sum over the
+// wavefronts.  A block of four wavefronts spent more time on its codes (14336 of them: 56 a lane, 10 instructions each) than on anything
+// else, so up to 4096 channels, where a CU has one block at most, twelve more wavefronts help (int8 / fp8, us, four wavefronts / sixteen of
+// which four multiply: 16 x 1152 x 896 6.2 / 5.5, 8 x 2304 x 2048 6.5 / 6.0, 16 x 896 x 4864 (two launches 13.7) - / 12.1).  With
+// more channels the blocks of a CU would repeat the quantizer, so a block takes as many wavefronts as its codes need and 16 or 32
+// channels (2 x 8448 x 1152 9.1 with two tiles a wavefront / 7.3, 7 x 15872 x 3840 two launches 24.1 / 16.8, 14336 codes: 16 x 9728 x 896 10.0 / 9.0).
+// Lines between one launch and two: llmq_linear_one_launch_preferred below.
 #include <algorithm>
 #include <type_traits>
 
@@ -58,29 +49,35 @@ struct FusedArgs {
     int64_t ldx, ldb, ldo;
     int M, N, K;
     int bias_dtype, out_dtype;
+    const float* in_scale;   // static: the activations' scale
+    const float* out_scale;  // device scalar or null: out is fp32 and holds the value after a round trip through e4m3fn on it
 };
+// where the activation scale comes from: every row, the whole tensor, the caller
+enum { SRC_TOKEN = 0, SRC_TENSOR = 1, SRC_STATIC = 2 };
 
-constexpr int kTensorChunks = 2048;  // TENSOR: 16-byte pieces of the activation tensor a block holds in registers
 constexpr int kRowPad = 16;        // bytes between LDS rows beyond K: consecutive tokens start 4 banks apart
-constexpr int kMaxLdsBytes = 65536 - 256;
+constexpr int kMaxLdsBytes = 65536 - 256;  // llmq_linear_*_dynamic; llmq_linear_one_launch takes more of the CU's 160 KB
 constexpr int kRowChunks = 10;     // 16-byte pieces of a row a lane keeps in registers (K <= 10 * 64 * 8 = 5120); longer rows are re-read
 
-template <bool FP8, int DT, int T, int NW, int D, bool TENSOR>
-__global__ __launch_bounds__(NW * kWave) void linear_fused_kernel(FusedArgs a) {
+// NG sets of NW wavefronts along K, NI that only quantize; SRC_TENSOR, SRC_STATIC: CH 16-byte pieces of the tensor in a thread's registers
+template <bool FP8, int DT, int T, int NW, int NG, int NI, int D, int SRC, int CH>
+__global__ __launch_bounds__((NW * NG + NI) * kWave) void linear_fused_kernel(FusedArgs a) {
+    constexpr bool TENSOR = SRC != SRC_TOKEN;  // one scale for the tensor
     constexpr int MODE = FP8 ? MODE_F8 : MODE_I8;
-    constexpr int NT = NW * kWave, KSTEP = FP8 ? 128 : 64, P = FP8 ? 2 : 1, LB = 16 * P;  // LB codes per lane and step
+    constexpr int NWT = NW * NG + NI, NT = NWT * kWave, KSTEP = FP8 ? 128 : 64, P = FP8 ? 2 : 1, LB = 16 * P;  // LB codes per lane and step
     using acc_t = typename std::conditional<FP8, v4f, v4i>::type;
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];  // [M][K + kRowPad] codes; after the main loop: red[NW][T][64]
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];  // [M][K + kRowPad] codes; after the main loop: red[NG * NW][T][64]
     __shared__ float s_scale[16];  // TENSOR: [0] = activation scale x weight scale
-    __shared__ float s_red[TENSOR ? NW : 1];
+    __shared__ float s_red[TENSOR ? NWT : 1];
 
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int r16 = lane & 15, kq = lane >> 4;
     const int M = a.M, N = a.N, K = a.K;
-    const int n0 = blockIdx.x * (16 * T);
+    const int kw = wave % NW, ng = wave / NW;  // run of K steps, set (NG and more: quantizes only)
+    const int n0 = (blockIdx.x * NG + min(ng, NG - 1)) * (16 * T);
     const int steps = (K + KSTEP - 1) / KSTEP, spw = (steps + NW - 1) / NW;
-    const int s_begin = min(steps, wave * spw), s_end = min(steps, s_begin + spw);
+    const int s_begin = ng < NG ? min(steps, kw * spw) : 0, s_end = ng < NG ? min(steps, s_begin + spw) : 0;
     const int row_bytes = K + kRowPad;
 
     const uint8_t* pb[T];
@@ -106,7 +103,6 @@ __global__ __launch_bounds__(NW * kWave) void linear_fused_kernel(FusedArgs a) {
 
     Batch ba, bb;
     // TENSOR: the activations are requested first (loads complete in order: behind the weights they would wait for HBM)
-    constexpr int CH = TENSOR ? kTensorChunks / NT : 1;
     uint4 act[CH];
     if constexpr (TENSOR) {
         const int cpr = K >> 3, total = M * cpr;
@@ -119,25 +115,40 @@ __global__ __launch_bounds__(NW * kWave) void linear_fused_kernel(FusedArgs a) {
     if (s_begin < s_end) load_batch(s_begin, ba);  // weights start streaming before the activations are quantized
     if constexpr (TENSOR) {
         const int cpr = K >> 3, total = M * cpr;
-        float amax = 0.f;
+        float s;
+        bool fin = false;  // block-uniform: the absmax behind the scale is finite, so no quotient can be NaN
+        if constexpr (SRC == SRC_STATIC) {
+            s = a.in_scale[0];
+        } else {
+            float amax = 0.f;
 #pragma unroll
-        for (int c = 0; c < CH; c++) amax = max_nonneg(amax, absmax8(act[c], DT == LLMQ_BF16));
-        amax = block_max<NW>(amax, s_red);
-        const float s = scale_from_amax<DT, MODE>(amax), inv_s = 1.0f / s;
+            for (int c = 0; c < CH; c++) amax = max_nonneg(amax, absmax8(act[c], DT == LLMQ_BF16));
+            amax = block_max<NWT>(amax, s_red);
+            s = scale_from_amax<DT, MODE>(amax);
+            fin = amax < __builtin_inff() && s > 0.f;  // (the fp8 floor rounds to 0 in fp16: an all-zero tensor has scale 0 and 0 / 0)
+        }
+        const float inv_s = 1.0f / s;
         if (tid == 0) {
             const float alpha = s * a.w_scale[0];
             s_scale[0] = FP8 ? alpha : Lo<DT>::round(alpha);  // int8: rounded to the activation dtype, as store_alpha does
         }
+        auto codes = [&](auto quot_c, auto fin_c) __attribute__((always_inline)) {
 #pragma unroll
-        for (int c = 0; c < CH; c++) {
-            const int i = tid + c * NT, m = i / cpr;
-            if (i < total) *reinterpret_cast<uint2*>(smem + m * row_bytes + 8 * (i - m * cpr)) = quant8<DT, MODE, Q_DT>(act[c], s, inv_s);
-        }
+            for (int c = 0; c < CH; c++) {
+                const int i = tid + c * NT, m = i / cpr;
+                if (i < total)
+                    *reinterpret_cast<uint2*>(smem + m * row_bytes + 8 * (i - m * cpr)) =
+                        quant8<DT, MODE, decltype(quot_c)::value, decltype(fin_c)::value>(act[c], s, inv_s);
+            }
+        };
+        if constexpr (SRC == SRC_STATIC) codes(std::integral_constant<int, Q_DIV_F32>{}, std::false_type{});
+        else if (fin) codes(std::integral_constant<int, Q_DT>{}, std::true_type{});
+        else codes(std::integral_constant<int, Q_DT>{}, std::false_type{});
     }
 
-    // ---- quantize: wavefront w takes tokens w, w + NW, ...; a lane owns the 16-byte pieces lane, lane + 64, ...
+    // ---- quantize: wavefront w takes tokens w, w + NWT, ...; a lane owns the 16-byte pieces lane, lane + 64, ...
     const int nchunk = K >> 3;
-    for (int m = TENSOR ? M : wave; m < M; m += NW) {
+    for (int m = TENSOR ? M : wave; m < M; m += NWT) {
         const uint4* row = reinterpret_cast<const uint4*>(a.x + (int64_t)m * a.ldx);
         uint4 cache[kRowChunks];
         float amax = 0.f;
@@ -223,16 +234,18 @@ __global__ __launch_bounds__(NW * kWave) void linear_fused_kernel(FusedArgs a) {
     // ---- the block's wavefronts add up in wavefront order (int32: exact; fp32: fixed order)
     __syncthreads();  // every wavefront is done reading the codes: their memory is reused
     acc_t (*red)[T][kWave] = reinterpret_cast<acc_t (*)[T][kWave]>(smem);
+    if (ng < NG) {
 #pragma unroll
-    for (int t = 0; t < T; t++) red[wave][t][lane] = acc[t];
+        for (int t = 0; t < T; t++) red[wave][t][lane] = acc[t];
+    }
     __syncthreads();
-    for (int idx = tid; idx < T * kWave; idx += NT) {
-        const int t = idx / kWave, l = idx % kWave;
-        acc_t sum = red[0][t][l];
+    for (int idx = tid; idx < NG * T * kWave; idx += NT) {
+        const int g = idx / (T * kWave), t = (idx / kWave) % T, l = idx % kWave;
+        acc_t sum = red[g * NW][t][l];
 #pragma unroll
-        for (int w = 1; w < NW; w++) sum += red[w][t][l];
-        // lane l of that accumulator: token l % 16, channels n0 + 16 t + 4 (l / 16) .. + 3
-        const int m = l & 15, n = n0 + 16 * t + 4 * (l >> 4);
+        for (int w = 1; w < NW; w++) sum += red[g * NW + w][t][l];
+        // lane l of that accumulator: token l % 16, four channels from 16 t + 4 (l / 16) of the set
+        const int m = l & 15, n = (blockIdx.x * NG + g) * (16 * T) + 16 * t + 4 * (l >> 4);
         if (m >= M || n >= N) continue;
         const float sa = TENSOR ? 1.f : s_scale[m], alpha = TENSOR ? s_scale[0] : 1.f;
         uint16_t h[4];
@@ -245,7 +258,15 @@ __global__ __launch_bounds__(NW * kWave) void linear_fused_kernel(FusedArgs a) {
             h[e] = a.out_dtype == LLMQ_BF16 ? Lo<LLMQ_BF16>::from_f32(v) : Lo<LLMQ_F16>::from_f32(v);
         }
         uint16_t* orow = reinterpret_cast<uint16_t*>(a.out) + (int64_t)m * a.ldo + n;
-        if (n + 3 < N && ((reinterpret_cast<uintptr_t>(orow) & 7u) == 0)) {
+        if (SRC == SRC_STATIC && a.out_scale) {
+            float* frow = reinterpret_cast<float*>(a.out) + (int64_t)m * a.ldo + n;
+            const float os = *a.out_scale;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float f = a.out_dtype == LLMQ_BF16 ? Lo<LLMQ_BF16>::to_f32(h[e]) : Lo<LLMQ_F16>::to_f32(h[e]);
+                if (n + e < N) frow[e] = fp8_round_trip(f, os);
+            }
+        } else if (n + 3 < N && ((reinterpret_cast<uintptr_t>(orow) & 7u) == 0)) {
             *reinterpret_cast<uint2*>(orow) = make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
         } else {
 #pragma unroll
@@ -265,25 +286,76 @@ __global__ __launch_bounds__(NW * kWave) void linear_fused_kernel(FusedArgs a) {
 
 thread_local int g_force_fused_variant = -1;  // tuning hook (per host thread): 0 = 2 channel tiles x 4 wavefronts, 1 = 1 x 8
 
-template <bool FP8, int DT, bool TENSOR>
-int launch_fused(const FusedArgs& a, hipStream_t st) {
+template <bool FP8, int DT, int T, int NW, int NG, int NI, int SRC, int CH>
+int launch_variant(const FusedArgs& a, hipStream_t st) {
     constexpr int D = FP8 ? 2 : 4;  // steps per batch: ~64 registers per batch
-    // same split as the few-token GEMM (fp32 sums in the same order): short K and many channels -> wider channel tiles,
-    // very short K -> four wavefronts, otherwise more wavefronts along K
-    const bool wide = g_force_fused_variant >= 0 ? g_force_fused_variant == 0 : a.K < 8192 && a.N >= 4096;
-    const bool four = g_force_fused_variant < 0 && a.K <= 2048 && a.N < 4096;
-    const size_t lds = std::max<size_t>((size_t)a.M * (a.K + kRowPad), (size_t)8 * 1 * kWave * 16);  // codes, then the reduction
-    if (wide) {
-        hipLaunchKernelGGL((linear_fused_kernel<FP8, DT, 2, 4, D, TENSOR>), dim3((a.N + 31) / 32), dim3(4 * kWave), lds, st, a);
-    } else if (four) {
-        hipLaunchKernelGGL((linear_fused_kernel<FP8, DT, 1, 4, D, TENSOR>), dim3((a.N + 15) / 16), dim3(4 * kWave), lds, st, a);
-    } else {
-        hipLaunchKernelGGL((linear_fused_kernel<FP8, DT, 1, 8, D, TENSOR>), dim3((a.N + 15) / 16), dim3(8 * kWave), lds, st, a);
+    auto kernel = linear_fused_kernel<FP8, DT, T, NW, NG, NI, D, SRC, CH>;
+    const size_t lds = std::max<size_t>((size_t)a.M * (a.K + kRowPad), (size_t)NW * NG * T * kWave * 16);  // codes, then the reduction
+    if (lds > 64 * 1024) {
+        // per device: the attribute belongs to the loaded code object of the current device
+        static bool raised[64] = {};
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess) return LLMQ_ERR_LAUNCH;
+        if (dev < 0 || dev >= 64 || !raised[dev]) {
+            if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024) != hipSuccess)
+                return LLMQ_ERR_LAUNCH;
+            if (dev >= 0 && dev < 64) raised[dev] = true;
+        }
     }
+    hipLaunchKernelGGL(kernel, dim3((a.N + 16 * T * NG - 1) / (16 * T * NG)), dim3((NW * NG + NI) * kWave), lds, st, a);
     return launch_status();
 }
 
-int64_t tensor_max_tokens(int64_t K) { return K <= 0 ? 0 : std::min<int64_t>(16, kTensorChunks * 8 / K); }
+constexpr int64_t kFewChannels = 4096;       // 256 blocks of 16 channels
+constexpr int64_t kMostCodes = 10 * 8192;    // codes that 1024 threads hold in 40 registers each, and their LDS
+
+template <bool FP8, int DT, int SRC>
+int launch_fused(const FusedArgs& a, hipStream_t st) {
+    const int64_t codes = (int64_t)a.M * a.K;
+    if constexpr (SRC == SRC_TOKEN) {
+        if (g_force_fused_variant == 0) return launch_variant<FP8, DT, 2, 4, 1, 0, SRC, 1>(a, st);
+        if (g_force_fused_variant == 1) return launch_variant<FP8, DT, 1, 8, 1, 0, SRC, 1>(a, st);
+        // few channels: a wavefront per row (us, 8 / 16 wavefronts: 8 x 1152 x 896 6.2 / 5.4, 11 x 3072 x 4352 12.3 / 11.0); many: four wavefronts and
+        // one channel tile each (two tiles / one: 2 x 9216 x 1792 10.6 / 9.2, 3 x 11392 x 1376 7.8 / 7.0), or two where the blocks of a CU would
+        // repeat the quantizer six times and more (3 x 23560 x 1920 11.9 / 13.3, 4 x 26112 x 6784 50.4 / 51.8)
+        if (a.N <= kFewChannels) return launch_variant<FP8, DT, 1, 4, 1, 12, SRC, 1>(a, st);
+        if (a.N > 16384) return launch_variant<FP8, DT, 2, 4, 1, 0, SRC, 1>(a, st);
+        if (a.M <= 4) return launch_variant<FP8, DT, 1, 4, 1, 0, SRC, 1>(a, st);
+        return launch_variant<FP8, DT, 1, 4, 2, 0, SRC, 1>(a, st);
+    } else {
+        if (a.N <= kFewChannels || codes > 32768) {
+            if (codes <= 16384) return launch_variant<FP8, DT, 1, 4, 1, 12, SRC, 2>(a, st);
+            if (codes <= 32768) return launch_variant<FP8, DT, 1, 4, 1, 12, SRC, 4>(a, st);
+            return launch_variant<FP8, DT, 1, 4, 1, 12, SRC, 10>(a, st);
+        }
+        if (codes <= 8192) return launch_variant<FP8, DT, 1, 4, 1, 0, SRC, 4>(a, st);
+        if (codes <= 16384) return launch_variant<FP8, DT, 1, 4, 2, 0, SRC, 4>(a, st);
+        return launch_variant<FP8, DT, 1, 4, 2, 0, SRC, 8>(a, st);
+    }
+}
+
+int64_t tensor_max_tokens(int64_t K) { return K <= 0 ? 0 : std::min<int64_t>(16, 16384 / K); }
+
+// what every entry point refuses
+int check_args(const void* x, int x_dtype, int64_t ldx, const uint8_t* B, int64_t ldb, const void* bias, int bias_dtype, const void* out,
+               int out_dtype, int64_t ldo, int64_t N, int64_t K) {
+    if (!x || !B || !out) return LLMQ_ERR_NULL;
+    if (x_dtype != LLMQ_BF16 && x_dtype != LLMQ_F16) return LLMQ_ERR_DTYPE;
+    if (out_dtype != LLMQ_BF16 && out_dtype != LLMQ_F16) return LLMQ_ERR_DTYPE;
+    if (bias && bias_dtype != LLMQ_BF16 && bias_dtype != LLMQ_F16 && bias_dtype != LLMQ_F32) return LLMQ_ERR_DTYPE;
+    if (K == 0 || (K & 15) || (ldx & 7) || (ldb & 15) || ldx < K || ldb < K || ldo < N) return LLMQ_ERR_SHAPE;
+    if (N > 0x7fffffffLL || K > 0x7fffffffLL || ldx >= (1 << 22) || ldb >= (1 << 22)) return LLMQ_ERR_SHAPE;
+    if (!aligned16(x) || !aligned16(B)) return LLMQ_ERR_ALIGN;
+    return LLMQ_OK;
+}
+
+template <int SRC>
+int dispatch(bool fp8, int x_dtype, const FusedArgs& a, hipStream_t st) {
+    if constexpr (SRC != SRC_STATIC) {
+        if (!fp8) return x_dtype == LLMQ_BF16 ? launch_fused<false, LLMQ_BF16, SRC>(a, st) : launch_fused<false, LLMQ_F16, SRC>(a, st);
+    }
+    return x_dtype == LLMQ_BF16 ? launch_fused<true, LLMQ_BF16, SRC>(a, st) : launch_fused<true, LLMQ_F16, SRC>(a, st);
+}
 
 int fused_entry(bool fp8, const void* x, int x_dtype, int64_t ldx, const uint8_t* B, int64_t ldb, const float* w_scale,
                 const void* bias, int bias_dtype, void* out, int out_dtype, int64_t ldo, int64_t M, int64_t N, int64_t K,
@@ -292,24 +364,17 @@ int fused_entry(bool fp8, const void* x, int x_dtype, int64_t ldx, const uint8_t
     if (M > 16 || M * (K + kRowPad) > kMaxLdsBytes) return LLMQ_ERR_SHAPE;  // llmq_linear_dynamic_max_tokens(K)
     if (tensor && M > tensor_max_tokens(K)) return LLMQ_ERR_SHAPE;
     if (M == 0 || N == 0) return LLMQ_OK;
-    if (!x || !B || !out || (tensor && !w_scale)) return LLMQ_ERR_NULL;
-    if (x_dtype != LLMQ_BF16 && x_dtype != LLMQ_F16) return LLMQ_ERR_DTYPE;
-    if (out_dtype != LLMQ_BF16 && out_dtype != LLMQ_F16) return LLMQ_ERR_DTYPE;
-    if (bias && bias_dtype != LLMQ_BF16 && bias_dtype != LLMQ_F16 && bias_dtype != LLMQ_F32) return LLMQ_ERR_DTYPE;
-    if (K == 0 || (K & 15) || (ldx & 7) || (ldb & 15) || ldx < K || ldb < K || ldo < N) return LLMQ_ERR_SHAPE;
-    if (N > 0x7fffffffLL || K > 0x7fffffffLL || ldx >= (1 << 22) || ldb >= (1 << 22)) return LLMQ_ERR_SHAPE;
-    if (!aligned16(x) || !aligned16(B) || (q_dump && !aligned16(q_dump))) return LLMQ_ERR_ALIGN;
+    if (tensor && !w_scale) return LLMQ_ERR_NULL;
+    const int bad = check_args(x, x_dtype, ldx, B, ldb, bias, bias_dtype, out, out_dtype, ldo, N, K);
+    if (bad != LLMQ_OK) return bad;
+    if (q_dump && !aligned16(q_dump)) return LLMQ_ERR_ALIGN;
     const FusedArgs a{(const uint16_t*)x, B, w_scale, bias, out, q_dump, scale_dump, acc_dump, ldx, ldb, ldo,
-                      (int)M, (int)N, (int)K, bias_dtype, out_dtype};
-    auto launch = [&](auto fp8_c, auto dt_c) {
-        constexpr bool F = decltype(fp8_c)::value;
-        constexpr int DT = decltype(dt_c)::value;
-        return tensor ? launch_fused<F, DT, true>(a, st) : launch_fused<F, DT, false>(a, st);
-    };
-    using BF = std::integral_constant<int, LLMQ_BF16>;
-    using HF = std::integral_constant<int, LLMQ_F16>;
-    if (fp8) return x_dtype == LLMQ_BF16 ? launch(std::true_type{}, BF{}) : launch(std::true_type{}, HF{});
-    return x_dtype == LLMQ_BF16 ? launch(std::false_type{}, BF{}) : launch(std::false_type{}, HF{});
+                      (int)M, (int)N, (int)K, bias_dtype, out_dtype, nullptr, nullptr};
+    return tensor ? dispatch<SRC_TENSOR>(fp8, x_dtype, a, st) : dispatch<SRC_TOKEN>(fp8, x_dtype, a, st);
+}
+
+bool one_launch_fits(int kind, int64_t M, int64_t N, int64_t K) {
+    return M >= 1 && M <= 16 && N >= 1 && K >= 16 && K % 16 == 0 && kind >= LLMQ_LINEAR_I8_TOKEN && kind <= LLMQ_LINEAR_FP8_STATIC && M * K <= kMostCodes;
 }
 
 }  // namespace
@@ -343,6 +408,42 @@ extern "C" int llmq_linear_fp8_dynamic(const void* x, int x_dtype, int64_t ldx, 
                                        float* acc_dump, llmq_stream_t stream) {
     return fused_entry(true, x, x_dtype, ldx, B, ldb, w_scale, bias, bias_dtype, out, out_dtype, ldo, M, N, K, q_dump,
                        scale_dump, acc_dump, (hipStream_t)stream);
+}
+
+// One launch or two.  Measured on an MI355X against quantizer + GEMM (us, two launches / one; weights out of HBM, 80 random problems and the sizes
+// of decoder layers): up to 4096 channels ahead as long as the codes are few (per tensor 6 x 3328 x 4736 12.3 / 10.0, 4 x 2096 x
+// 6272 11.2 / 9.8, 16 x 3584 x 3584 9.9 / 10.7; static, whose quotients are divisions, 2 x 1648 x 16640 18.5 / 16.8, 16 x 3584 x 3584 9.0 / 13.4; per
+// token, a wavefront per row, 11 x 3072 x 4352 12.1 / 11.0, 16 x 3584 x 3584 9.5 / 10.3, 3 x 1936 x 13824 16.4 / 21.1), and beyond
+// that where the GEMM behind the quantizer has no few-token kernel (16 x 896 x 4864 13.7 / 12.1); with more channels each CU repeats
+// the quantizer a few times (per tensor 7 x 15872 x 3840 24.1 / 16.8, 8 x 4608 x 3584 12.7 / 11.2, 8 x 5168 x 7168 16.5 / 16.9, 4 x 25728 x 7168 40.5 / 49.9; static 3 x 16128 x
+// 2048 15.1 / 10.0, 16 x 10368 x 1152 10.0 / 11.0, 2 x 8320 x 10368 25.4 / 27.0).
+extern "C" int llmq_linear_one_launch_preferred(int kind, int64_t M, int64_t N, int64_t K) {
+    if (!one_launch_fits(kind, M, N, K)) return 0;
+    const int64_t codes = M * K;
+    if (codes <= 16384 && (kind == LLMQ_LINEAR_I8_TENSOR || kind == LLMQ_LINEAR_FP8_TENSOR)) return 1;
+    if (kind == LLMQ_LINEAR_I8_TOKEN || kind == LLMQ_LINEAR_FP8_TOKEN)
+        return K < 8192 && (M <= 4 || (N <= kFewChannels && codes <= 49152));
+    if (kind == LLMQ_LINEAR_FP8_STATIC) return N <= kFewChannels ? codes <= 32768 : codes <= 14336 && K < 8192;
+    if (N > kFewChannels) return codes <= 28672 && K < 8192 && N <= 16384;
+    return codes <= 49152 || (M > 8 && N <= 1024);
+}
+
+extern "C" int llmq_linear_one_launch(int kind, const void* x, int x_dtype, int64_t ldx, const void* B, int64_t ldb, const float* w_scale,
+                                      const float* in_scale, const void* bias, int bias_dtype, const float* out_scale, void* out, int out_dtype,
+                                      int64_t ldo, int64_t M, int64_t N, int64_t K, llmq_stream_t stream) {
+    if (M < 0 || N < 0 || K < 0 || kind < LLMQ_LINEAR_I8_TOKEN || kind > LLMQ_LINEAR_FP8_STATIC) return LLMQ_ERR_SHAPE;
+    if (M == 0 || N == 0) return LLMQ_OK;
+    if (!one_launch_fits(kind, M, N, K)) return LLMQ_ERR_SHAPE;
+    const bool is_static = kind == LLMQ_LINEAR_FP8_STATIC, token = kind == LLMQ_LINEAR_I8_TOKEN || kind == LLMQ_LINEAR_FP8_TOKEN;
+    if ((!token && !w_scale) || (is_static && !in_scale)) return LLMQ_ERR_NULL;
+    if (out_scale && !is_static) return LLMQ_ERR_DTYPE;
+    const int bad = check_args(x, x_dtype, ldx, (const uint8_t*)B, ldb, bias, bias_dtype, out, out_dtype, ldo, N, K);
+    if (bad != LLMQ_OK) return bad;
+    const FusedArgs a{(const uint16_t*)x, (const uint8_t*)B, w_scale, bias, out, nullptr, nullptr, nullptr, ldx, ldb, ldo,
+                      (int)M, (int)N, (int)K, bias_dtype, out_dtype, in_scale, out_scale};
+    const bool fp8 = kind == LLMQ_LINEAR_FP8_TOKEN || kind == LLMQ_LINEAR_FP8_TENSOR || is_static;
+    hipStream_t st = (hipStream_t)stream;
+    return is_static ? dispatch<SRC_STATIC>(fp8, x_dtype, a, st) : token ? dispatch<SRC_TOKEN>(fp8, x_dtype, a, st) : dispatch<SRC_TENSOR>(fp8, x_dtype, a, st);
 }
 
 extern "C" int llmq_linear_per_tensor_max_tokens(int64_t K) { return (int)tensor_max_tokens(K); }

@@ -18,7 +18,7 @@ from ..sq_fp8_kernels import (cutlass_f8f8bf16_rowwise_sm89, cutlass_f8f8bf16_te
                               dynamic_linear_max_tokens, f8f8_tensorwise_quantized_output,
                               f8f8bf16_linear_dynamic_per_token)
 from .linear_base import LinearBase
-from .linear_sq import ONE_LAUNCH_K, ONE_LAUNCH_MAX_TOKENS, _fusable
+from .linear_sq import ONE_LAUNCH_K, ONE_LAUNCH_MAX_TOKENS, ONE_LAUNCH_TOKENS, _fusable
 
 __all__ = ["FP8DynamicLinear", "FP8StaticLinear", "per_tensor_quantize", "per_token_quantize",
            "static_per_tensor_quantize"]
@@ -121,7 +121,7 @@ class FP8DynamicLinear(_FP8LinearBase):
             y = host().fp8_tensor(x, self._qweight(), self._parameters.get("weight_scale"), self._bias_param(), self.dtype,
                                   None, None)
         else:
-            y = host().fp8_token(x, self._qweight(), self._wscale_flat(), self._bias_param(), ONE_LAUNCH_MAX_TOKENS, ONE_LAUNCH_K)
+            y = host().fp8_token(x, self._qweight(), self._wscale_flat(), self._bias_param(), ONE_LAUNCH_TOKENS, ONE_LAUNCH_K)
         return self._forward_general(x) if y is None else y
 
     @torch.no_grad()

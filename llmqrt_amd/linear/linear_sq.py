@@ -24,9 +24,10 @@ __all__ = ["SqW8A8BBF16OBF16PerTensor", "SqW8A8BBF16OBF16PerChannel",
            "quantize_activation_per_tensor_absmax", "quantize_activation_per_token_absmax"]
 
 
-# Up to this many tokens, and for shorter rows than ONE_LAUNCH_K, the one-launch linear is as fast on the GPU as quantizer +
-# GEMM and saves a launch on the host; beyond, the two launches are faster (measured on MI355X at the Qwen2-7B shapes).
-# The native forwards take both numbers from here.
+# The widest range in which a per-token linear runs in one launch: up to ONE_LAUNCH_TOKENS rows shorter than ONE_LAUNCH_K.  Inside it the native
+# forwards follow the measured lines of llmq_linear_one_launch_preferred, the general path (strided rows) stays with the number of tokens up to
+# which one launch is at least level for any number of channels.
+ONE_LAUNCH_TOKENS = 16
 ONE_LAUNCH_MAX_TOKENS = 4
 ONE_LAUNCH_K = 8192
 
@@ -129,7 +130,7 @@ class SqW8A8BBF16OBF16PerChannel(LinearBase):
     def forward(self, x):
         b = self._buffers
         y = host().sq_token(x, b.get("qweight"), b.get("weight_scale"), b["bias"] if "bias" in b else self.bias,
-                            ONE_LAUNCH_MAX_TOKENS, ONE_LAUNCH_K)
+                            ONE_LAUNCH_TOKENS, ONE_LAUNCH_K)
         return self._forward_general(x) if y is None else y
 
     @torch.no_grad()

@@ -147,3 +147,84 @@ def test_per_tensor_one_launch(cuda, M, N, K, dtype, bias):
         assert (y - ref).abs().max() <= 2.0 ** -8 * ref.abs().max()
     x[0, 3] = float("nan")
     assert torch.equal(f8(x).isnan(), f8._forward_general(x).isnan())
+
+
+# llmq_linear_one_launch in every launch shape: up to 4096 channels 2, 4 and 10 pieces a thread (the last and the first number of codes of each),
+# past that four and eight wavefronts, one row per wavefront and several; a ragged K step, ragged channels, one step, LDS past 64 KB
+@pytest.mark.parametrize("M,N,K", [(1, 24, 16), (16, 4096, 1024), (15, 1000, 1104), (16, 264, 2048), (16, 136, 2064), (16, 896, 4864), (16, 72, 5120), (1, 640, 16384),
+                                   (4, 512, 20480), (8, 4112, 1024), (9, 4104, 1040), (16, 4360, 1024), (13, 8200, 1280), (3, 9728, 912), (16, 4112, 2064)])
+@pytest.mark.parametrize("dtype,with_bias", [(torch.bfloat16, True), (torch.float16, False)])
+def test_one_launch_every_source(cuda, M, N, K, dtype, with_bias):
+    """Against quantizer + GEMM on the same operands: int8 bit for bit (exact int32 sums), fp8 within the rounding of two fp32 sums of the same
+    products in different orders, K 2^-24 of the sum of their absolute values, and one rounding to the output type (or one step of e4m3fn)."""
+    from llmqrt_amd import _abi, workloads as W
+    from llmqrt_amd.quantize import per_token_quantize, quantize_activation_per_token_absmax_f32, static_per_tensor_quantize_with_alpha
+    from llmqrt_amd.quantize import per_tensor_quantize_with_alpha
+    from llmqrt_amd.sq_fp8_kernels import w8a8_int8_linear_bbf16_obf16_per_channel, w8a8_int8_linear_bbf16_obf16_per_tensor
+    L = _abi.lib()
+    g = torch.Generator().manual_seed(M + N + K)
+    x = (torch.randn(M, K, generator=g) * 2).to(dtype).to(cuda)
+    x[-1, -1] = 40.0
+    qi, swi = (t.to(cuda) for t in W.int8_weights(N, K, N + 1))
+    qf = (torch.randn(N, K, generator=g) * 60).clamp(-448, 448).to(torch.float8_e4m3fn).to(cuda)
+    swn = (torch.rand(N, generator=g) * 0.01 + 0.001).to(cuda)
+    sw1 = torch.tensor([0.004], device=cuda)
+    sin = torch.tensor([0.0137], device=cuda)
+    sout = torch.tensor([0.9], device=cuda)
+    bias = torch.randn(N, generator=g).to(dtype).to(cuda) if with_bias else None
+    bd = bias.double() if with_bias else 0
+
+    def run(kind, w, sw, in_scale=None, out_scale=None):
+        out = torch.full((M, N), 7.0, dtype=torch.float32 if out_scale is not None else dtype, device=cuda)
+        _abi.check(L.llmq_linear_one_launch(kind, x.data_ptr(), _abi.dtype_code(dtype), K, w.data_ptr(), K, sw.data_ptr(), _abi.ptr(in_scale),
+                                            _abi.ptr(bias), _abi.dtype_code(dtype), _abi.ptr(out_scale), out.data_ptr(), _abi.dtype_code(dtype), N,
+                                            M, N, K, torch.cuda.current_stream().cuda_stream), "llmq_linear_one_launch")
+        return out
+    zeros = torch.zeros(N, dtype=dtype, device=cuda)
+    b = bias if with_bias else zeros
+    # int8
+    q, s = quantize_activation_per_token_absmax_f32(x)
+    assert torch.equal(run(0, qi, swn), w8a8_int8_linear_bbf16_obf16_per_channel(q, qi.t(), b, s, swn))
+    q, alpha = per_tensor_quantize_with_alpha(x, sw1, fp8=False)
+    assert torch.equal(run(2, qi, sw1), w8a8_int8_linear_bbf16_obf16_per_tensor(q.view(M, K), qi.t(), b, alpha, 1.0))
+    # fp8: codes and scales of the separate quantizers, fp64 sums
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+
+    def check(y, codes, scale, w_scale):
+        prod = codes.double() @ qf.double().t() * scale.double() * w_scale.double()
+        mag = codes.double().abs() @ qf.double().abs().t() * scale.double() * w_scale.double()
+        ref = prod + bd
+        # the matrix cores drop products more than 13 binary orders below the largest of a run of eight
+        tol = (K * 2.0 ** -24 + 2.0 ** -13) * mag + 2.0 * ulp * ref.abs() + 2.0 ** -20
+        assert bool(((y.double() - ref).abs() <= tol).all()), float(((y.double() - ref).abs() / tol).max())
+        return ref, tol
+    q, s = per_token_quantize(x)
+    check(run(1, qf, swn), q.float(), s.view(M, 1), swn.view(1, N))
+    q, alpha = per_tensor_quantize_with_alpha(x, sw1, fp8=True)
+    check(run(3, qf, sw1), q.view(M, K).float(), alpha.view(1, 1), torch.ones(1, device=cuda))
+    q, alpha = static_per_tensor_quantize_with_alpha(x, sin, sw1)
+    ref, tol = check(run(4, qf, sw1, sin), q.view(M, K).float(), alpha.view(1, 1), torch.ones(1, device=cuda))
+    y = run(4, qf, sw1, sin, sout)
+    codes = y / sout
+    assert torch.equal(codes.to(torch.float8_e4m3fn).float() * sout, y)  # on the grid
+    step = (ref / 0.9).abs().clamp(min=2.0 ** -6, max=448.0)
+    assert bool(((y.double() - ref.clamp(-448 * 0.9, 448 * 0.9)).abs() <= 0.9 * step * 2.0 ** -3 + tol).all())
+
+
+def test_one_launch_refuses(cuda):
+    from llmqrt_amd import _abi
+    L = _abi.lib()
+    x = torch.zeros(17, 8192, dtype=torch.bfloat16, device=cuda)
+    w = torch.zeros(64, 8192, dtype=torch.int8, device=cuda)
+    s = torch.ones(64, device=cuda)
+    out = torch.zeros(17, 64, dtype=torch.bfloat16, device=cuda)
+
+    def rc(kind, M, K, sw=s, sin=None, sout=None):
+        return L.llmq_linear_one_launch(kind, x.data_ptr(), _abi.BF16, K, w.data_ptr(), K, _abi.ptr(sw), _abi.ptr(sin), None, 0, _abi.ptr(sout), out.data_ptr(),
+                                        _abi.BF16, 64, M, 64, K, 0)
+    assert rc(2, 17, 64) == rc(2, 11, 8192) == rc(5, 1, 64) == rc(-1, 1, 64) == rc(2, 1, 40) == -3  # LLMQ_ERR_SHAPE
+    assert rc(2, 1, 64, None) == rc(4, 1, 64, s, None) == L.llmq_linear_one_launch(0, None, 0, 64, None, 64, None, None, None, 0, None, None, 0, 64, 1, 64, 64, 0)
+    assert rc(2, 1, 64, None) != 0 and rc(3, 1, 64, s, None, s) != 0
+    assert rc(2, 0, 64) == 0 and int(out.count_nonzero()) == 0
+    for kind in range(5):
+        assert L.llmq_linear_one_launch_preferred(kind, 17, 64, 64) == 0 == L.llmq_linear_one_launch_preferred(kind, 1, 64, 40)
