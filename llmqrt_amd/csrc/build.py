@@ -18,7 +18,7 @@ LIB = OUT_DIR / "libllmq_gfx950.so"
 HOST_LIB = OUT_DIR / "_llmq_host.so"  # native forward passes of the modules (host code against torch and the C ABI)
 MICROBENCH_LIB = OUT_DIR / "libllmq_microbench_gfx950.so"  # hardware microbenchmarks for `bench.py --micro`; not the product
 # the tile GEMM is instantiated per operand format in four translation units (the long poles of the build), listed first
-SOURCES = ["gemm_tile_i8.hip", "gemm_tile_fp8.hip", "gemm_tile_fp8_e5m2.hip", "gemm_tile_f16.hip", "awq_stream.hip", "gemm_mfma.hip", "abi.hip",
+SOURCES = ["gemm_tile_i8.hip", "gemm_tile_fp8.hip", "gemm_tile_fp8_e5m2.hip", "gemm_tile_f16.hip", "awq_stream.hip", "gemm_rows.hip", "gemm_mfma.hip", "abi.hip",
            "quant.hip", "gemm_skinny.hip", "linear_fused.hip", "awq.hip", "awq_decode.hip", "awq_tile.hip"]
 
 HIPCC_FLAGS = [

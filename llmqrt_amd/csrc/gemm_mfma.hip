@@ -1,28 +1,15 @@
 // W8A8 int8, FP8 (OCP e4m3fn / e5m2) and fp16 GEMMs: the planner (tile configuration, K split, few-token kernel,
 // tail split) and the C entry points.  The tile kernels live in gemm_tile_impl.h and are instantiated per operand
-// format in gemm_tile_*.hip; the few-token kernel in gemm_skinny.hip.
+// format in gemm_tile_*.hip; the few-token kernels in gemm_skinny.hip and gemm_rows.hip.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
 
+#include "gemm_rows.h"
 #include "gemm_tile.h"
 #include "llmq_common.h"
 
 namespace llmq {
-
-// Few-token kernel (gemm_skinny.hip): one launch, no workspace.
-struct SkinnyEpilogue {
-    const float* a_scale;
-    const float* w_scale;
-    const float* alpha_dev;
-    const void* bias;
-    float alpha, beta;
-    int bias_dtype, out_dtype;
-    const float* out_scale;
-};
-int launch_gemm_skinny(bool fp8, int a_format, int mt, int t, int nw, const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ldb,
-                       int M, int N, int K, const SkinnyEpilogue& ep, void* out, int64_t ldo, void* acc_dump,
-                       hipStream_t st);
 
 namespace {
 
@@ -330,9 +317,56 @@ Plan tile_plan(int op, int64_t M, int64_t N, int64_t K, Plan& table, double& tab
     return table;
 }
 
-Plan make_plan(int op, int64_t M, int64_t N, int64_t K) {
+// Long pieces of rows through LDS (gemm_rows.hip): modelled us.  `stage` is the time of a stage of a block that has its CU to itself; blocks beyond
+// the first on a CU add `share` of it each; a CU's loads take `bytes` us per KB; weights `weights` us per MB.  Fitted to the time of each
+// variant on 900 random problems of 1-64 tokens, int8 and fp8 alike, weights out of HBM (7-13 % standard deviation, 20 % for the 1024-byte pieces).
+struct RowsCost { double base, stage, bytes, weights, share; };
+const RowsCost kRowsCosts[kRowsVariants] = {
+    {2.8702, 0.2143, 0.0169, 0.1669, 1.5175},  // 1 x 1, 512 x 4
+    {3.1549, 0.0033, 0.0128, 0.2272, 0.4290},  // 1 x 1, 1024 x 4
+    {3.0883, 0.3853, 0.0000, 0.1691, 1.9517},  // 2 x 1, 512 x 4
+    {2.8773, 0.3606, 0.0001, 0.2329, 1.0927},  // 1 x 2, 512 x 3
+    {3.2079, 0.0016, 0.0121, 0.3053, 0.4101},  // 1 x 2, 1024 x 3
+    {3.2159, 0.5002, 0.0000, 0.1909, 1.7175},  // 2 x 2, 512 x 3
+    {2.8821, 0.7644, 0.0182, 0.2106, 0.6123},  // 2 x 2, 512 x 2
+    {4.0008, 0.8345, 0.0001, 0.1795, 1.7072},  // 4 x 2, 512 x 3
+    {3.4187, 0.4670, 0.0001, 0.2608, 1.6730},  // 1 x 3, 512 x 4
+    {4.0452, 0.5548, 0.0001, 0.2358, 1.8744},  // 2 x 3, 512 x 3
+    {3.3686, 0.4829, 0.0000, 0.3268, 1.7206},  // 1 x 4, 512 x 3
+    {4.0328, 0.7390, 0.0000, 0.3058, 1.3016}};  // 2 x 4, 512 x 3
+double rows_time(int v, int64_t N, int64_t K) {
+    const RowsShape& s = kRowsShapes[v];
+    const RowsCost& c = kRowsCosts[v];
+    const double x = (double)cdiv(N, 16 * s.t) / kNumCu, stages = cdiv(K, s.seg);
+    const double chain = stages * c.stage * (1 + c.share * (std::ceil(x) - 1)), supply = std::max(x, 1.0) * stages * 16 * (s.t + s.mt) * s.seg * c.bytes / 1e3;
+    const double weights = (double)N * K * c.weights / 1e6, a = chain * chain, b = supply * supply, w = weights * weights;
+    return c.base + std::sqrt(std::sqrt(a * a + b * b + w * w));
+}
+// Where it competes with the plan of tiles and gemm_skinny.hip, which takes `now` us as modelled.  Up to 64 tokens; not a short K, where a stage
+// or two are all there is: from 1040 bytes on (2048 on where K ends inside a 128-byte line), from 4096 channels or 2049 bytes up to 16 tokens, and
+// there no ragged K below 4096 (us, now / rows: fp8 2 x 1024 x 1040 3.1 / 3.6, 2 x 576 x 3184 4.2 / 4.8).  A wide N and a short K at up to
+// 16 tokens stays with the tiles, whose blocks take 128 channels (int8 3 x 16640 x 1664 9.2 / 15.6).
+// The tile times were fitted to more rows than these: below 65 they come out at 0.7 of the measured ones, those of gemm_skinny.hip at 1.15.
+// With the factors below, of the 900 problems the half that moves is 11 % faster in the mean over all, 1 % of all end more than 5 % behind.
+int rows_variant(const Plan& plan, double now, int64_t M, int64_t N, int64_t K) {
+    if (M > 64 || K <= 1024 || K > kTableMaxK || (K % 128 != 0 && K < 2048)) return -1;
+    const int mt = cdiv(M, 16);
+    if (mt == 1 && ((K <= 2048 && (N < 4096 || N > 16384)) || (K % 128 != 0 && K < 4096))) return -1;
+    double best = now * (plan.cfg >= kSkinnyCfg ? 0.95 : 1.15);
+    int variant = -1;
+    for (int v = 0; v < kRowsVariants; v++)
+        if (kRowsShapes[v].mt == mt) {
+            const double t = rows_time(v, N, K);
+            if (t < best) best = t, variant = v;
+        }
+    return variant;
+}
+inline Plan rows(int variant, int64_t K) { return Plan{kRowsCfg + variant, 1, (int)K}; }
+
+Plan tiles_or_skinny_plan(int op, int64_t M, int64_t N, int64_t K) {
     int t, nw;
-    if (g_force_cfg >= kSkinnyCfg && op != 2) {  // forced few-token variant: 16, 32 or 64 as its split are the tokens of a slab
+    if (g_force_cfg >= kRowsCfg && op != 2 && M <= 16 * kRowsShapes[g_force_cfg - kRowsCfg].mt) return rows(g_force_cfg - kRowsCfg, K);
+    if (g_force_cfg >= kSkinnyCfg && g_force_cfg < kRowsCfg && op != 2) {  // forced few-token variant: 16, 32 or 64 as its split are the tokens of a slab
         const int slab = g_force_splits;
         if (slab == 16 || slab == 32 || slab == 64) return Plan{g_force_cfg, 1, (int)K, slab / 16};
         if (M <= 64) return Plan{g_force_cfg, 1, (int)K, skinny_mt(M)};
@@ -364,6 +398,19 @@ Plan make_plan(int op, int64_t M, int64_t N, int64_t K) {
     // A K split gives way to one launch of slabs at the same modelled time: the gap before its finishing launch is not in the model.
     const bool one_launch = best.cfg >= kSkinnyCfg && plan.splits > 1;
     return best_t < (few ? (K <= 1024 ? 0.75 : 0.85) : one_launch ? 1.0 : 0.9) * now ? best : plan;
+}
+
+Plan make_plan(int op, int64_t M, int64_t N, int64_t K) {
+    const Plan plan = tiles_or_skinny_plan(op, M, N, K);
+    if (g_force_cfg >= 0 || op == 2 || M > 64) return plan;
+    if (op == kStaticInt8 && partials_bytes(plan, M, N) > kStaticScratchBytes) return plan;  // refused, as before
+    double now = 1e300;
+    if (plan.cfg >= kSkinnyCfg) now = skinny_time(op, M, N, K, plan.mt, 1 + ((plan.cfg - kSkinnyCfg) & 1), 4 << ((plan.cfg - kSkinnyCfg) >> 1));
+    else
+        for (const TileCost& c : costs_of(op).tiles)
+            if (c.cfg == plan.cfg) now = table_time(costs_of(op), c, M, N, K, plan.splits, plan.k_per_split);
+    const int variant = rows_variant(plan, now, M, N, K);
+    return variant < 0 ? plan : rows(variant, K);
 }
 
 // Searching a plan takes microseconds of host time and a call needs it for its workspace and for its launch, so each host
@@ -402,8 +449,10 @@ int gemm_entry(int op, int a_format, const uint8_t* A, int64_t lda, const uint8_
     Plan p = plan_for(planned_op, M, N, K);
     if (!fits(p) && g_force_cfg < 0) p = rules_plan(planned_op, M, N, K);  // the caller kept the size that was enough for these
     if (!fits(p)) return LLMQ_ERR_WORKSPACE;
-    if (p.cfg >= kSkinnyCfg) {
+    if (p.cfg >= kSkinnyCfg) {  // both few-token kernels
         const SkinnyEpilogue sep{a_scale, w_scale, alpha_dev, bias, alpha, beta, bias_dtype, out_dtype, out_scale};
+        if (p.cfg >= kRowsCfg)
+            return launch_gemm_rows(fp8, a_format == LLMQ_E5M2 ? 1 : 0, p.cfg - kRowsCfg, A, lda, B, ldb, (int)M, (int)N, (int)K, sep, out, ldo, acc_dump, st);
         const int v = p.cfg - kSkinnyCfg;
         return launch_gemm_skinny(fp8, a_format == LLMQ_E5M2 ? 1 : 0, p.mt, 1 + (v & 1), 4 << (v >> 1), A, lda, B, ldb, (int)M, (int)N,
                                   (int)K, sep, out, ldo, acc_dump, st);
@@ -486,7 +535,7 @@ extern "C" int llmq_gemm_w8a8_static(const int8_t* A, int64_t lda, const int8_t*
 extern "C" int llmq_gemm_force_plan(int cfg, int splits) {
     int dma = -1;
     if (cfg >= 0 && cfg < 100 && (cfg & 64)) dma = 0, cfg &= ~64;
-    if ((cfg >= kNumShapes && (cfg < 100 || cfg > 105)) || splits < 1 || splits > 64) return LLMQ_ERR_SHAPE;
+    if ((cfg >= kNumShapes && (cfg < kSkinnyCfg || (cfg > kSkinnyCfg + 5 && cfg < kRowsCfg) || cfg >= kRowsCfg + kRowsVariants)) || splits < 1 || splits > 64) return LLMQ_ERR_SHAPE;
     g_force_dma = dma;
     g_force_cfg = cfg;
     g_force_splits = splits;

@@ -18,19 +18,9 @@
 //     deterministic), and the block applies the same epilogue as the tile kernel and stores 8 bytes per lane.
 #include <type_traits>
 
-#include "llmq_common.h"
+#include "gemm_rows.h"
 
 namespace llmq {
-
-struct SkinnyEpilogue {
-    const float* a_scale;    // [M] or null
-    const float* w_scale;    // [N] or null
-    const float* alpha_dev;  // device scalar or null
-    const void* bias;        // [N] or null
-    float alpha, beta;
-    int bias_dtype, out_dtype;
-    const float* out_scale;  // device scalar or null: out is fp32 and holds the value after a round trip through e4m3fn on it
-};
 
 namespace {
 
@@ -214,8 +204,6 @@ void launch_skinny_mt(int t, int nw, const uint8_t* A, int64_t lda, const uint8_
 
 }  // namespace
 
-// mt: 16-token tiles per block (1 | 2 | 4), t: 16-channel tiles per wavefront (1 | 2), nw: wavefronts per block (4 | 8 | 16; 4 | 8 for
-// mt = 4 and t = 2); a_format: 0 e4m3, 1 e5m2 (fp8 only)
 int launch_gemm_skinny(bool fp8, int a_format, int mt, int t, int nw, const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ldb,
                        int M, int N, int K, const SkinnyEpilogue& ep, void* out, int64_t ldo, void* acc_dump,
                        hipStream_t st) {

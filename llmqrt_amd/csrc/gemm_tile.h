@@ -21,12 +21,13 @@ struct Epilogue {
 };
 
 struct Plan {
-    int cfg;     // index into the config table; kSkinnyCfg + v: the few-token kernel
+    int cfg;     // index into the config table; kSkinnyCfg + v, kRowsCfg + v: the few-token kernels
     int splits;  // K splits (1 = fused epilogue)
     int k_per_split;
-    int mt = 0;  // few-token kernel: 16-token tiles per block
+    int mt = 0;  // kSkinnyCfg + v: 16-token tiles per block
 };
 constexpr int kSkinnyCfg = 100;  // + v: 1 + (v & 1) channel tiles per wavefront, 4 << (v >> 1) wavefronts per block
+constexpr int kRowsCfg = 110;    // + v: kRowsShapes[v] (gemm_rows.h)
 
 constexpr int kNumCu = 256;
 inline int cdiv(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
