@@ -141,8 +141,10 @@ __global__ __launch_bounds__((NW * NG + NI) * kWave) void linear_fused_kernel(Fu
                         quant8<DT, MODE, decltype(quot_c)::value, decltype(fin_c)::value>(act[c], s, inv_s);
             }
         };
-        if constexpr (SRC == SRC_STATIC) codes(std::integral_constant<int, Q_DIV_F32>{}, std::false_type{});
-        else if (fin) codes(std::integral_constant<int, Q_DT>{}, std::true_type{});
+        if constexpr (SRC == SRC_STATIC) {
+            if (near_scale(s)) codes(std::integral_constant<int, Q_NEAR_F32>{}, std::false_type{});
+            else codes(std::integral_constant<int, Q_DIV_F32>{}, std::false_type{});
+        } else if (fin) codes(std::integral_constant<int, Q_DT>{}, std::true_type{});
         else codes(std::integral_constant<int, Q_DT>{}, std::false_type{});
     }
 
@@ -168,20 +170,24 @@ __global__ __launch_bounds__((NW * NG + NI) * kWave) void linear_fused_kernel(Fu
         }
         uint2* qrow = reinterpret_cast<uint2*>(smem + m * row_bytes);
         uint2* qdump = (a.q_dump && blockIdx.x == 0) ? reinterpret_cast<uint2*>(a.q_dump + (int64_t)m * K) : nullptr;
+        auto codes = [&](auto fin_c) __attribute__((always_inline)) {
 #pragma unroll
-        for (int c = 0; c < kRowChunks; c++) {
-            const int i = lane + c * kWave;
-            if (i < nchunk) {
-                const uint2 q = quant8<DT, MODE, Q_DT>(cache[c], s, inv_s);
+            for (int c = 0; c < kRowChunks; c++) {
+                const int i = lane + c * kWave;
+                if (i < nchunk) {
+                    const uint2 q = quant8<DT, MODE, Q_DT, decltype(fin_c)::value>(cache[c], s, inv_s);
+                    qrow[i] = q;
+                    if (qdump) qdump[i] = q;
+                }
+            }
+            for (int i = lane + kRowChunks * kWave; i < nchunk; i += kWave) {
+                const uint2 q = quant8<DT, MODE, Q_DT, decltype(fin_c)::value>(row[i], s, inv_s);
                 qrow[i] = q;
                 if (qdump) qdump[i] = q;
             }
-        }
-        for (int i = lane + kRowChunks * kWave; i < nchunk; i += kWave) {
-            const uint2 q = quant8<DT, MODE, Q_DT>(row[i], s, inv_s);
-            qrow[i] = q;
-            if (qdump) qdump[i] = q;
-        }
+        };
+        if (amax < __builtin_inff() && s > 0.f) codes(std::true_type{});  // wavefront-uniform: no quotient can be NaN
+        else codes(std::false_type{});
     }
     __syncthreads();
     const uint8_t* arow = smem + min(r16, M - 1) * row_bytes + kq * LB;  // rows past M repeat the last token; never stored

@@ -105,7 +105,8 @@ __global__ __launch_bounds__(NT) void quant_rows_kernel(
         }
     };
     if (SCALE == SCALE_STATIC) {
-        if (static_f32) store_row(std::integral_constant<int, Q_DIV_F32>{}, std::false_type{});
+        if (static_f32 && near_scale(s)) store_row(std::integral_constant<int, Q_NEAR_F32>{}, std::false_type{});
+        else if (static_f32) store_row(std::integral_constant<int, Q_DIV_F32>{}, std::false_type{});
         else store_row(std::integral_constant<int, Q_DIV_DT>{}, std::false_type{});
     } else if (fin) {
         store_row(std::integral_constant<int, Q_DT>{}, std::true_type{});
@@ -226,7 +227,9 @@ __global__ __launch_bounds__(kSmallThreads) void quant_tensor_small_kernel(
         else ((uint16_t*)scale_out)[0] = Lo<DT>::from_f32(s);
         store_alpha<DT>(ta, s);
     }
-    if (mine < total) q[mine] = quant8<DT, MODE, Q_DT>(own, s, 1.0f / s);
+    if (mine >= total) return;
+    if (amax < __builtin_inff() && s > 0.f) q[mine] = quant8<DT, MODE, Q_DT, true>(own, s, 1.0f / s);
+    else q[mine] = quant8<DT, MODE, Q_DT>(own, s, 1.0f / s);
 }
 
 // ---- RMSNorm fused with the per-token quantizer --------------------------------------------

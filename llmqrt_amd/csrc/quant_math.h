@@ -39,26 +39,43 @@ __device__ __forceinline__ float absmax8(uint4 r, int dt_is_bf16) {
 // Quotient rounded to the activation dtype.  bf16: x * (1/s) rounds to the same bf16 value
 // as the exact quotient for every pair of bf16 operands (the exact quotient of two 8-bit
 // significands is never closer than 2^-17 relative to a bf16 rounding boundary), so one
-// multiply replaces the division.  fp16 significands are too long for that: true division.
+// multiply replaces the division.  fp16 significands are too long for that: the product is corrected once (near_quotient) where all
+// quotients are known to be finite, else divided.
 // Q_DT: scale is itself a value of the activation dtype (dynamic quantizers).
 // Q_DIV_DT: arbitrary fp32 scale, quotient rounded to the activation dtype (tensor / Python float).
 // Q_DIV_F32: arbitrary fp32 scale, quotient kept in fp32 (tensor / fp32 tensor promotes).
-enum { Q_DT = 0, Q_DIV_DT = 1, Q_DIV_F32 = 2 };
-template <int DT, int QUOT>
-__device__ __forceinline__ float quotient(float x, float s, float inv_s) {
-    if (QUOT == Q_DIV_F32) return x / s;
-    if (QUOT == Q_DIV_DT || DT == LLMQ_F16) return Lo<DT>::round(x / s);
-    return Lo<DT>::round(x * inv_s);
-}
+// Q_NEAR_F32: the same codes for a scale in [2^-60, 2^60] (near_scale) without a division.
+enum { Q_DT = 0, Q_DIV_DT = 1, Q_DIV_F32 = 2, Q_NEAR_F32 = 3 };
+__device__ __forceinline__ bool near_scale(float s) { return s >= 0x1p-60f && s <= 0x1p60f; }  // false for NaN
+
+// x / s for a 16-bit x from inv_s = 1/s rounded to nearest: the product and one correction by its remainder, which an fma gives exactly
+// (Markstein's division, IBM J. Res. Dev. 34, 1990).  That is x / s (1 + 2^-46) rounded to fp32 once, so it is the rounded quotient unless x / s is
+// that close to the middle between two fp32 values.  With s in fp16 it never is (x - s m is a multiple of 2^-34 for a 25-bit middle m).
+// With any fp32 s it can be, but not next to a value where e4m3 rounding changes, so the codes are those of the division: there s would
+// be k / 16 + j 2^-23 with 16 <= k < 32, and x, of at most 11 bits, b s + k 2^-28 for the 5-bit b in question, so j b 32 = -k, and b 32 >= 32.
+// Three instructions where the division takes about ten: the quantizers of fp16 and static scales are bound by these.  The signs
+// of the two fmas keep that of a zero x.
+__device__ __forceinline__ float near_quotient(float x, float q, float s, float inv_s) { return fmaf(-fmaf(q, s, -x), inv_s, q); }
+
 // the quotients of a pair of elements; the two roundings to the activation dtype share one packed conversion
-template <int DT, int QUOT>
+template <int DT, int QUOT, bool FIN>
 __device__ __forceinline__ void quotient2(float x0, float x1, float s, float inv_s, float& q0, float& q1) {
     if (QUOT == Q_DIV_F32) {
         q0 = x0 / s, q1 = x1 / s;
         return;
     }
-    const bool mul = !(QUOT == Q_DIV_DT || DT == LLMQ_F16);
-    const uint32_t p = Lo<DT>::pack2(mul ? x0 * inv_s : x0 / s, mul ? x1 * inv_s : x1 / s);
+    if (QUOT == Q_NEAR_F32) {
+        // bounded, so that no remainder is inf - inf: past the bound the correction lands beyond every code's range on the same side; a NaN x
+        // comes back in through the remainder
+        const float b = 0x1p20f;
+        q0 = near_quotient(x0, __builtin_amdgcn_fmed3f(x0 * inv_s, -b, b), s, inv_s);
+        q1 = near_quotient(x1, __builtin_amdgcn_fmed3f(x1 * inv_s, -b, b), s, inv_s);
+        return;
+    }
+    uint32_t p;
+    if (QUOT == Q_DT && DT == LLMQ_BF16) p = Lo<DT>::pack2(x0 * inv_s, x1 * inv_s);
+    else if (QUOT == Q_DT && FIN) p = Lo<DT>::pack2(near_quotient(x0, x0 * inv_s, s, inv_s), near_quotient(x1, x1 * inv_s, s, inv_s));
+    else p = Lo<DT>::pack2(x0 / s, x1 / s);
     q0 = Lo<DT>::lo_f32(p), q1 = Lo<DT>::hi_f32(p);
 }
 
@@ -72,7 +89,7 @@ __device__ __forceinline__ uint2 quant8(uint4 raw, float s, float inv_s) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         float q0, q1;
-        quotient2<DT, QUOT>(Lo<DT>::lo_f32(w[i]), Lo<DT>::hi_f32(w[i]), s, inv_s, q0, q1);
+        quotient2<DT, QUOT, FIN>(Lo<DT>::lo_f32(w[i]), Lo<DT>::hi_f32(w[i]), s, inv_s, q0, q1);
         f[2 * i] = q0, f[2 * i + 1] = q1;
     }
 #pragma unroll

@@ -339,3 +339,47 @@ def test_per_tensor_with_alpha(cuda, M, K, pad, fp8, dtype):
         a_ref = (s_ref.float() * ws).to(dtype).float()
         assert torch.equal(q.cpu(), q_ref)
     assert a.dtype == torch.float32 and torch.equal(a.cpu().reshape(()), a_ref.reshape(()))
+
+
+def _same_codes(got, ref):
+    """Byte for byte, NaN codes by being NaN (their sign is the divider's)."""
+    g, r = got.cpu(), ref
+    nan = r.float().isnan()
+    return torch.equal(g.float().isnan(), nan) and torch.equal(g.view(torch.uint8)[~nan], r.view(torch.uint8)[~nan])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_static_codes_without_a_division(cuda, dtype):
+    """Every 16-bit pattern (zeros of both signs, subnormals, infinities, NaN) over fp32 scales against the fp32 quotient: the
+    neighbours of k / 16, where a quotient can be next to the middle of two fp32 values, in several binades; random ones; both sides
+    of the scales that are multiplied (2^-60 .. 2^60) instead of divided by."""
+    from llmqrt_amd.quantize import static_per_tensor_quantize
+    x = torch.arange(0, 65536, dtype=torch.int32).to(torch.int16).view(dtype).view(64, 1024)
+    near = torch.tensor([(k / 16 + j * 2.0 ** -23) * 2.0 ** e for k in range(16, 32) for j in (-2, -1, 0, 1, 2) for e in (-7, 1)])
+    g = torch.Generator().manual_seed(1)
+    rand = torch.exp2(torch.empty(200).uniform_(-24, 12, generator=g))
+    edge = torch.tensor([2.0 ** -60, 2.0 ** 60], dtype=torch.float32)
+    edge = torch.cat([edge, torch.nextafter(edge, torch.zeros(2)), torch.nextafter(edge, torch.full((2,), 3e38)), torch.tensor([1e-40, 3e38])])
+    xd = x.to(cuda)
+    for s in torch.cat([near, rand, edge]).float():
+        ref = (x.float() / s).clamp(-448.0, 448.0).to(torch.float8_e4m3fn)
+        assert _same_codes(static_per_tensor_quantize(xd, s.view(1).to(cuda)), ref), s.item()
+
+
+def test_fp16_dynamic_codes_without_a_division(cuda):
+    """The quotients of fp16 rows, 2048 values each, over 512 scales from subnormal ones to the largest, per token and per tensor."""
+    from llmqrt_amd.quantize import per_tensor_quantize, per_token_quantize, quantize_activation_per_token_absmax
+    g = torch.Generator().manual_seed(2)
+    top = torch.exp2(torch.linspace(-13, 15.99, 512)).view(-1, 1)
+    x = (torch.empty(512, 2048).uniform_(-1, 1, generator=g) * top).half()
+    x[:, 0], x[:, 1] = 0.0, -0.0
+    q, s = quantize_activation_per_token_absmax(x.to(cuda))
+    q_ref, s_ref = R.quantize_activation_per_token_absmax(x)
+    assert torch.equal(s.cpu().view(torch.int16), s_ref.view(torch.int16)) and torch.equal(q.cpu(), q_ref)
+    f, fs = per_token_quantize(x.to(cuda))
+    f_ref, fs_ref = R.fp8_per_token_quantize(x)
+    assert torch.equal(fs.cpu(), fs_ref) and _same_codes(f, f_ref)
+    for rows in (slice(0, 8), slice(256, 264), slice(300, 500)):
+        t, ts = per_tensor_quantize(x[rows].contiguous().to(cuda))
+        t_ref, ts_ref = R.fp8_per_tensor_quantize(x[rows])
+        assert ts.item() == ts_ref.item() and _same_codes(t, t_ref)
