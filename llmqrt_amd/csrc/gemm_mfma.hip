@@ -342,17 +342,28 @@ double rows_time(int v, int64_t N, int64_t K) {
     const double weights = (double)N * K * c.weights / 1e6, a = chain * chain, b = supply * supply, w = weights * weights;
     return c.base + std::sqrt(std::sqrt(a * a + b * b + w * w));
 }
-// Where it competes with the plan of tiles and gemm_skinny.hip, which takes `now` us as modelled.  Up to 64 tokens; not a short K, where a stage
-// or two are all there is: from 1040 bytes on (2048 on where K ends inside a 128-byte line), from 4096 channels or 2049 bytes up to 16 tokens, and
-// there no ragged K below 4096 (us, now / rows: fp8 2 x 1024 x 1040 3.1 / 3.6, 2 x 576 x 3184 4.2 / 4.8).  A wide N and a short K at up to
-// 16 tokens stays with the tiles, whose blocks take 128 channels (int8 3 x 16640 x 1664 9.2 / 15.6).
-// The tile times were fitted to more rows than these: below 65 they come out at 0.7 of the measured ones, those of gemm_skinny.hip at 1.15.
-// With the factors below, of the 900 problems the half that moves is 11 % faster in the mean over all, 1 % of all end more than 5 % behind.
+// Where it competes with the plan of tiles and gemm_skinny.hip, which takes `now` us as modelled: up to 64 tokens and not the shortest K, where
+// a stage or two are all there is (us, now / rows: fp8 2 x 1024 x 1040 3.1 / 3.6, 2 x 576 x 3184 4.2 / 4.8, int8 18 x 3584 x 1744 4.5 /
+// 4.8).  Up to 16 tokens a wide N and a short K stay with the tiles, whose blocks take 128 channels (int8 3 x 16640 x 1664 9.2 / 15.6).
+// `now` was fitted to more rows than these: for tiles it comes out at 0.7 of the measured time and at 0.55 where K ends inside a 128-byte line
+// and the whole K tail goes through registers (16 tokens: 2 x 9856 x 1376 10.2 / 7.1, 3 x 35200 x 7920 84 / 53; 36 x 10752 x 5792 28.8 / 24.5), for
+// gemm_skinny.hip at 1.15.  With the factors below, of the 900 problems the half that moves makes the mean over all 11 % faster; 1 % of
+// all end more than 5 % behind.
 int rows_variant(const Plan& plan, double now, int64_t M, int64_t N, int64_t K) {
-    if (M > 64 || K <= 1024 || K > kTableMaxK || (K % 128 != 0 && K < 2048)) return -1;
+    if (M > 64 || K <= 1024 || K > kTableMaxK) return -1;
     const int mt = cdiv(M, 16);
-    if (mt == 1 && ((K <= 2048 && (N < 4096 || N > 16384)) || (K % 128 != 0 && K < 4096))) return -1;
-    double best = now * (plan.cfg >= kSkinnyCfg ? 0.95 : 1.15);
+    const bool ragged = K % 128 != 0, tiles = plan.cfg < kSkinnyCfg;
+    double factor = 0.95;
+    if (mt > 1) {
+        if (ragged && K < 2048 && N < 4096) return -1;
+        if (tiles) factor = ragged ? 1.35 : 1.15;
+    } else if (tiles) {
+        if (N > 16384 && K < (ragged ? 2500 : 2049)) return -1;
+        factor = ragged ? 1.9 : 1.15;
+    } else {
+        if (N < 4096 ? K <= (ragged ? 4095 : 2048) : ragged && K < 1792) return -1;
+    }
+    double best = now * factor;
     int variant = -1;
     for (int v = 0; v < kRowsVariants; v++)
         if (kRowsShapes[v].mt == mt) {

@@ -416,20 +416,21 @@ extern "C" int llmq_linear_fp8_dynamic(const void* x, int x_dtype, int64_t ldx, 
                        scale_dump, acc_dump, (hipStream_t)stream);
 }
 
-// One launch or two.  Measured on an MI355X against quantizer + GEMM (us, two launches / one; weights out of HBM, 80 random problems and the sizes
-// of decoder layers): up to 4096 channels ahead as long as the codes are few (per tensor 6 x 3328 x 4736 12.3 / 10.0, 4 x 2096 x
-// 6272 11.2 / 9.8, 16 x 3584 x 3584 9.9 / 10.7; static, whose quotients are divisions, 2 x 1648 x 16640 18.5 / 16.8, 16 x 3584 x 3584 9.0 / 13.4; per
-// token, a wavefront per row, 11 x 3072 x 4352 12.1 / 11.0, 16 x 3584 x 3584 9.5 / 10.3, 3 x 1936 x 13824 16.4 / 21.1), and beyond
-// that where the GEMM behind the quantizer has no few-token kernel (16 x 896 x 4864 13.7 / 12.1); with more channels each CU repeats
-// the quantizer a few times (per tensor 7 x 15872 x 3840 24.1 / 16.8, 8 x 4608 x 3584 12.7 / 11.2, 8 x 5168 x 7168 16.5 / 16.9, 4 x 25728 x 7168 40.5 / 49.9; static 3 x 16128 x
-// 2048 15.1 / 10.0, 16 x 10368 x 1152 10.0 / 11.0, 2 x 8320 x 10368 25.4 / 27.0).
+// One launch or two.  Measured on an MI355X against quantizer + GEMM (us, two launches / one; weights out of HBM, 630 random problems and the
+// sizes of decoder layers).  Two launches issued from a program's own loop take 10 us of the host against 6 for one, so the line is
+// where one launch stops being ahead of max(two launches, 10).  Up to 4096 channels it is as long as the codes are few (per tensor 9 x 3584 x
+// 3584 8.8 / 9.0 on the GPU, 15 x 3584 x 3584 8.9 / 11.0; static 4 x 3584 x 3584 7.4 / 7.1, 11 x 3584 x 3584 7.5 / 10.5; per token, a wavefront per
+// row, 2 x 3584 x 3584 8.1 / 7.7, 15 x 3584 x 3584 8.1 / 10.0), and beyond that where there are few channels.  With more channels each CU repeats the quantizer a
+// few times (per tensor 7 x 9728 x 896 8.9 / 7.4, 2 x 37888 x 3584 35.2 / 31.7, 8 x 5168 x 7168 16.5 / 16.9; static 4 x 11744 x 1072 11.4 / 6.5,
+// 13 x 13016 x 2432 13.3 / 15.4, 2 x 8320 x 10368 25.4 / 27.0), past 16384 channels more often than the launch costs per token and with a
+// static scale (per token 4 x 37504 x 1408 17.0 / 22.8, 2 x 37888 x 3584 34.3 / 39.5; static 4 x 19184 x 2432 12.2 / 16.1, 9 x 34432 x 896 12.7 / 17.6).
 extern "C" int llmq_linear_one_launch_preferred(int kind, int64_t M, int64_t N, int64_t K) {
     if (!one_launch_fits(kind, M, N, K)) return 0;
     const int64_t codes = M * K;
     if (codes <= 16384 && (kind == LLMQ_LINEAR_I8_TENSOR || kind == LLMQ_LINEAR_FP8_TENSOR)) return 1;
     if (kind == LLMQ_LINEAR_I8_TOKEN || kind == LLMQ_LINEAR_FP8_TOKEN)
-        return K < 8192 && (M <= 4 || (N <= kFewChannels && codes <= 49152));
-    if (kind == LLMQ_LINEAR_FP8_STATIC) return N <= kFewChannels ? codes <= 32768 : codes <= 14336 && K < 8192;
+        return K < 8192 && ((M <= 4 && N <= 16384) || (N <= kFewChannels && codes <= 49152));
+    if (kind == LLMQ_LINEAR_FP8_STATIC) return N <= kFewChannels ? codes <= 32768 : codes <= 14336 && K < 8192 && N <= 16384;
     if (N > kFewChannels) return codes <= 28672 && K < 8192 && N <= 16384;
     return codes <= 49152 || (M > 8 && N <= 1024);
 }
