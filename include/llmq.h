@@ -275,8 +275,8 @@ int llmq_linear_dynamic_force_variant(int v);
  * process; cfg < 0 restores the built-in heuristic.  cfg | 64 keeps the register-staged main loop (8, 9 and 10 have none: they
  * run the staged configuration next in size, 3, 2 and 2).  100 .. 105 pick a variant of the few-token kernel (no K split) for int8 and
  * fp8: with `splits` 16, 32 or 64 in slabs of that many tokens, for any M, else in one block row, for up to 64 tokens (more keep the
- * built-in choice).  110 .. 121 pick a variant of the kernel that streams long pieces of weight rows through LDS, for as many tokens as the
- * variant holds (16: 110-112, 32: 113-117, 48: 118 and 119, 64: 120 and 121; more keep the built-in choice).
+ * built-in choice).  110 .. 123 pick a variant of the kernel that streams long pieces of weight rows through LDS, for as many tokens as the
+ * variant holds (16: 110-112, 122 and 123, 32: 113-117, 48: 118 and 119, 64: 120 and 121; more keep the built-in choice).
  * Per host thread (thread-local state): it affects only calls made later by the thread that set it. */
 int llmq_gemm_force_plan(int cfg, int splits);
 int llmq_gemm_num_configs(void);

@@ -321,7 +321,7 @@ Plan tile_plan(int op, int64_t M, int64_t N, int64_t K, Plan& table, double& tab
 // the first on a CU add `share` of it each; a CU's loads take `bytes` us per KB; weights `weights` us per MB.  Fitted to the time of each
 // variant on 900 random problems of 1-64 tokens, int8 and fp8 alike, weights out of HBM (7-13 % standard deviation, 20 % for the 1024-byte pieces).
 struct RowsCost { double base, stage, bytes, weights, share; };
-const RowsCost kRowsCosts[kRowsVariants] = {
+const RowsCost kRowsCosts[kRowsMany] = {
     {2.8702, 0.2143, 0.0169, 0.1669, 1.5175},  // 1 x 1, 512 x 4
     {3.1549, 0.0033, 0.0128, 0.2272, 0.4290},  // 1 x 1, 1024 x 4
     {3.0883, 0.3853, 0.0000, 0.1691, 1.9517},  // 2 x 1, 512 x 4
@@ -344,28 +344,35 @@ double rows_time(int v, int64_t N, int64_t K) {
 }
 // Where it competes with the plan of tiles and gemm_skinny.hip, which takes `now` us as modelled: up to 64 tokens and not the shortest K, where
 // a stage or two are all there is (us, now / rows: fp8 2 x 1024 x 1040 3.1 / 3.6, 2 x 576 x 3184 4.2 / 4.8, int8 18 x 3584 x 1744 4.5 /
-// 4.8).  Up to 16 tokens a wide N and a short K stay with the tiles, whose blocks take 128 channels (int8 3 x 16640 x 1664 9.2 / 15.6).
+// 4.8).
 // `now` was fitted to more rows than these: for tiles it comes out at 0.7 of the measured time and at 0.55 where K ends inside a 128-byte line
-// and the whole K tail goes through registers (16 tokens: 2 x 9856 x 1376 10.2 / 7.1, 3 x 35200 x 7920 84 / 53; 36 x 10752 x 5792 28.8 / 24.5), for
+// and the whole K tail goes through registers (36 x 10752 x 5792 28.8 / 24.5), for
 // gemm_skinny.hip at 1.15.  With the factors below, of the 900 problems the half that moves makes the mean over all 11 % faster; 1 % of
 // all end more than 5 % behind.
 int rows_variant(const Plan& plan, double now, int64_t M, int64_t N, int64_t K) {
-    if (M > 64 || K <= 1024 || K > kTableMaxK) return -1;
+    if (M > 64 || K <= (M <= 16 && N > 8192 ? 768 : 1024) || K > kTableMaxK) return -1;
     const int mt = cdiv(M, 16);
+    // Many channels: blocks that go from one group of channels to the next, from where 64 channels a block are enough blocks.  342 random problems
+    // of up to 16 tokens, plan of tiles / this (mean, least): 8193-16384 channels 1.13 (0.92), from 24577 on 1.13 (0.98); up to
+    // 8192 0.78.  16385-24576 channels make one to one and a half groups of 64 a CU, so groups of 32 there, three a block: 1.10 (0.87) against 1.08 (0.82).
+    // Up to 20480 of these the tiles of 128 channels fill the chip in one round and keep the shorter K (14 x 17920 x 4096 13.6 / 14.8, 4 x 19184 x 2432
+    // 9.7 / 10.4; 2 x 18432 x 11904 48 / 42).
     const bool ragged = K % 128 != 0, tiles = plan.cfg < kSkinnyCfg;
+    if (mt == 1 && N > 8192 && (N <= 16384 || N > 20480 || ragged || K >= 8192)) return N > 16384 && N <= 24576 ? kRowsMany + 1 : kRowsMany;
     double factor = 0.95;
     if (mt > 1) {
         if (ragged && K < 2048 && N < 4096) return -1;
         if (tiles) factor = ragged ? 1.35 : 1.15;
     } else if (tiles) {
-        if (N > 16384 && K < (ragged ? 2500 : 2049)) return -1;
+        if (N > 8192) return -1;
         factor = ragged ? 1.9 : 1.15;
     } else {
         if (N < 4096 ? K <= (ragged ? 4095 : 2048) : ragged && K < 1792) return -1;
+        if (ragged && N * K > 40000000) return -1;  // (int8 3 x 2944 x 18608 12.9 / 15.6)
     }
     double best = now * factor;
     int variant = -1;
-    for (int v = 0; v < kRowsVariants; v++)
+    for (int v = 0; v < kRowsMany; v++)
         if (kRowsShapes[v].mt == mt) {
             const double t = rows_time(v, N, K);
             if (t < best) best = t, variant = v;

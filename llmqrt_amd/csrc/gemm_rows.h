@@ -20,14 +20,17 @@ struct SkinnyEpilogue {
 int launch_gemm_skinny(bool fp8, int a_format, int mt, int t, int nw, const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ldb,
                        int M, int N, int K, const SkinnyEpilogue& ep, void* out, int64_t ldo, void* acc_dump, hipStream_t st);
 
-// Variants of gemm_rows.hip: t, mt 16-channel / 16-token tiles of a block, seg bytes of every row per stage, ns stages in LDS.
-#define LLMQ_ROWS_VARIANTS(V)                                                                                                 \
-    V(0, 1, 1, 512, 4) V(1, 1, 1, 1024, 4) V(2, 2, 1, 512, 4) V(3, 1, 2, 512, 3) V(4, 1, 2, 1024, 3) V(5, 2, 2, 512, 3)       \
-    V(6, 2, 2, 512, 2) V(7, 4, 2, 512, 3) V(8, 1, 3, 512, 4) V(9, 2, 3, 512, 3) V(10, 1, 4, 512, 3) V(11, 2, 4, 512, 3)
-constexpr int kRowsVariants = 12;
+// Variants of gemm_rows.hip: t, mt 16-channel / 16-token tiles of a block, seg bytes of every row per stage, ns stages in LDS; many: a block
+// takes several groups of channels.
+#define LLMQ_ROWS_VARIANTS(V)                                                                                                          \
+    V(0, 1, 1, 512, 4, false) V(1, 1, 1, 1024, 4, false) V(2, 2, 1, 512, 4, false) V(3, 1, 2, 512, 3, false) V(4, 1, 2, 1024, 3, false) \
+    V(5, 2, 2, 512, 3, false) V(6, 2, 2, 512, 2, false) V(7, 4, 2, 512, 3, false) V(8, 1, 3, 512, 4, false) V(9, 2, 3, 512, 3, false)   \
+    V(10, 1, 4, 512, 3, false) V(11, 2, 4, 512, 3, false) V(12, 4, 1, 512, 3, true) \
+    V(13, 2, 1, 512, 3, true)
+constexpr int kRowsVariants = 14, kRowsMany = 12;
 struct RowsShape { int t, mt, seg, ns; };
 constexpr RowsShape kRowsShapes[kRowsVariants] = {
-#define LLMQ_ROWS_SHAPE(I, T, MT, SEG, NS) {T, MT, SEG, NS},
+#define LLMQ_ROWS_SHAPE(I, T, MT, SEG, NS, MANY) {T, MT, SEG, NS},
     LLMQ_ROWS_VARIANTS(LLMQ_ROWS_SHAPE)
 #undef LLMQ_ROWS_SHAPE
 };

@@ -11,12 +11,18 @@
 //     flight while one is multiplied, and the wait is for the oldest only;
 //   * each wavefront multiplies its quarter of the bytes of each stage and the block adds the four sums in wavefront order at the end.
 // The activations are re-read by every block out of the L2: T = 2 and 4 halve and quarter that for many channels, T = 1 makes more blocks.
+// MANY: for many channels a block that ends with its channels leaves the CU without loads while the next one starts, which costs a quarter of the
+// stream (37888 channels: 592 blocks of 64).  There as many blocks as are resident take one group of channels after the other: the ring
+// runs on into the next group while the last one's sums are added beside it, and the scales of all groups are in LDS from the start, so that the
+// epilogue waits for no load.  (For 17-32 tokens, with twice the activations per stage, level with the tiles: 32 x 37888 x 3584 31.7 / 32.8 us,
+// 32 x 30000 x 2048 16.3 / 13.5; not kept.)
 // 1024-byte pieces are for few blocks over a long K (K = 18944 at N = 3584: 512 bytes 3.0 TB/s, 1024 bytes 4.2 TB/s).
 //
 // Measured (int8, weights out of HBM, us; before: the fastest plan of skinny and tile kernels the planner had):
 //   tokens        16 x 4608 x 3584   16 x 3584 x 3584   16 x 896 x 4864   16 x 3584 x 18944   32 x 4608 x 3584   64 x 3584 x 3584
 //   before              9.9                7.1                9.4               19.4               11.4               12.3
 //   this kernel         6.8                5.7                5.5               16.0                8.0                8.2
+// MANY, before / now:  1 x 37888 x 3584 30.9 / 25.0 (5.4 TB/s with launch and tail), 16 x 37888 x 3584 32.4 / 27.2, 8 x 11904 x 8192 24.9 / 19.7.
 #include <algorithm>
 #include <type_traits>
 
@@ -30,7 +36,9 @@ typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
-template <bool FP8_, int AFMT_, int T_, int MT_, int SEG_, int NS_>
+constexpr int kRowsGroups = 16;  // groups of channels a block takes at most
+
+template <bool FP8_, int AFMT_, int T_, int MT_, int SEG_, int NS_, bool MANY_ = false>
 struct RowsCfg {
     static constexpr bool FP8 = FP8_;
     static constexpr int AFMT = AFMT_;
@@ -42,9 +50,12 @@ struct RowsCfg {
     static constexpr int STEPS = SEG / NW / KSTEP;      // MFMA steps of a wavefront per stage
     static constexpr int ROWS = 16 * (T + MT), STAGE_BYTES = ROWS * SEG;
     static constexpr int LPT = STAGE_BYTES / (NT * 16);  // direct loads per thread and stage
-    static constexpr int LDS_BYTES = NS * STAGE_BYTES;
+    static constexpr bool MANY = MANY_;                 // a block takes several groups of channels, one after the other
+    static constexpr int RING_BYTES = NS * STAGE_BYTES, SUM_BYTES = NW * T * MT * kWave * 16;
+    // MANY: the ring stays in flight while the wavefronts add up, beside it, and the scales of all groups lie behind that
+    static constexpr int LDS_BYTES = RING_BYTES + (MANY ? SUM_BYTES + (kRowsGroups * 16 * T * 2 + 16 * MT) * 4 : 0);
     static_assert(STEPS >= 1 && SEG % (NW * KSTEP) == 0 && STAGE_BYTES % (NT * 16) == 0, "a stage splits evenly");
-    static_assert(LDS_BYTES <= 160 * 1024 && (NS - 1) * LPT < 64 && LDS_BYTES >= NW * T * MT * kWave * 16, "LDS, vmcnt, the final sum");
+    static_assert(LDS_BYTES <= 160 * 1024 && (NS - 1) * LPT < 64 && RING_BYTES >= SUM_BYTES, "LDS, vmcnt, the final sum");
 };
 
 template <class C>
@@ -57,8 +68,9 @@ __global__ __launch_bounds__(C::NT) void gemm_rows_kernel(const uint8_t* __restr
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int r16 = lane & 15, kq = lane >> 4;
-    const int n0 = blockIdx.x * (16 * T);
-    const int nst = (K + SEG - 1) / SEG;
+    int n0 = blockIdx.x * (16 * T);
+    const int nst = (K + SEG - 1) / SEG, step_n = C::MANY ? gridDim.x * (16 * T) : 0;
+    const int mine = C::MANY ? (N - n0 + step_n - 1) / step_n : 1, total = mine * nst;  // groups and stages of the block
 
     // ---- direct loads: piece p of a stage is row p / CPR (weights, then activations), LDS chunk p % CPR, which holds chunk
     // (p % CPR) ^ (row & 15) of the row, so that the operand reads of 16 rows hit 16 places
@@ -70,6 +82,17 @@ __global__ __launch_bounds__(C::NT) void gemm_rows_kernel(const uint8_t* __restr
         chunk[i] = 16u * (uint32_t)((p % C::CPR) ^ (row & 15));
         off[i] = row < 16 * T ? (uint32_t)min(row, N - 1 - n0) * (uint32_t)ldb : (uint32_t)min(row - 16 * T, M - 1) * (uint32_t)lda;
     }
+    int issue_n0 = n0;
+    auto next_group = [&]() __attribute__((always_inline)) {  // of the loads
+        issue_n0 += step_n;
+        wb = B + (int64_t)issue_n0 * ldb;
+        if (issue_n0 + 16 * T <= N) return;
+#pragma unroll
+        for (int i = 0; i < C::LPT; i++) {
+            const int row = ((wave * C::LPT + i) * kWave + lane) / C::CPR;
+            if (row < 16 * T) off[i] = (uint32_t)min(row, N - 1 - issue_n0) * (uint32_t)ldb;
+        }
+    };
     const uint32_t lds_base = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)smem);
     auto issue = [&](int s, int slot) __attribute__((always_inline)) {
         const bool tail = (s + 1) * SEG > K;  // uniform: chunks past the end re-read the last one of the row, masked when used
@@ -140,72 +163,103 @@ __global__ __launch_bounds__(C::NT) void gemm_rows_kernel(const uint8_t* __restr
     };
     static_assert(NS <= 8, "wait_stage");
 
+    // scales and bias of channel n0 + c of group g: MANY keeps those of all its groups in LDS, so that no load of the epilogue waits behind the ring
+    float* s_w = reinterpret_cast<float*>(smem + C::RING_BYTES + C::SUM_BYTES);
+    float* s_b = s_w + kRowsGroups * 16 * T;
+    float* s_a = s_b + kRowsGroups * 16 * T;
+    const float alpha = ep.alpha * (ep.alpha_dev ? *ep.alpha_dev : 1.0f);
+    const float out_scale = ep.out_scale ? *ep.out_scale : 1.f;
+    auto weight_scale = [&](int n) __attribute__((always_inline)) { return ep.w_scale ? ep.w_scale[min(n, N - 1)] : 1.f; };
+    auto bias_of = [&](int n) __attribute__((always_inline)) { return ep.bias ? ep.beta * load_as_f32(ep.bias, ep.bias_dtype, min(n, N - 1)) : 0.f; };
+    if constexpr (C::MANY) {
+        for (int i = tid; i < mine * 16 * T; i += C::NT) {
+            const int n = n0 + i / (16 * T) * step_n + i % (16 * T);
+            s_w[i] = weight_scale(n), s_b[i] = bias_of(n);
+        }
+        if (tid < 16 * MT) s_a[tid] = ep.a_scale ? ep.a_scale[min(tid, M - 1)] : 1.f;
+    }
+
+    // ---- the wavefronts add up in wavefront order, then scales, bias, store
+    acc_t (*red)[MT * T][kWave] = reinterpret_cast<acc_t (*)[MT * T][kWave]>(smem + (C::MANY ? C::RING_BYTES : 0));
+    auto finish = [&](int group) __attribute__((always_inline)) {
 #pragma unroll
-    for (int t = 0; t < NS - 1; t++)
-        if (t < nst) issue(t, t);
-    int slot = 0;
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int t = 0; t < T; t++) red[wave][mt * T + t][lane] = acc[mt][t];
+        lds_barrier();
+        for (int idx = tid; idx < MT * T * kWave; idx += C::NT) {
+            const int q = idx / kWave, l = idx % kWave, mt = q / T, t = q % T;
+            acc_t sum = red[0][q][l];
+#pragma unroll
+            for (int w = 1; w < C::NW; w++) sum += red[w][q][l];
+            // lane l of that accumulator: token 16 mt + l % 16, channels n0 + 16 t + 4 (l / 16) .. + 3
+            const int m = 16 * mt + (l & 15), c = 16 * t + 4 * (l >> 4), n = n0 + c;
+            if (m >= M || n >= N) continue;
+            const float sa = C::MANY ? s_a[m] : ep.a_scale ? ep.a_scale[m] : 1.f;
+            uint16_t h[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float sw = C::MANY ? s_w[group * 16 * T + c + e] : weight_scale(n + e);
+                const float bb = C::MANY ? s_b[group * 16 * T + c + e] : bias_of(n + e);
+                const float v = epi_value((float)sum[e], sa, sw, alpha, bb);
+                h[e] = ep.out_dtype == LLMQ_BF16 ? Lo<LLMQ_BF16>::from_f32(v) : Lo<LLMQ_F16>::from_f32(v);
+            }
+            uint16_t* orow = reinterpret_cast<uint16_t*>(out) + (int64_t)m * ldo + n;
+            if (ep.out_scale) {
+                float* frow = reinterpret_cast<float*>(out) + (int64_t)m * ldo + n;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float f = ep.out_dtype == LLMQ_BF16 ? Lo<LLMQ_BF16>::to_f32(h[e]) : Lo<LLMQ_F16>::to_f32(h[e]);
+                    if (n + e < N) frow[e] = fp8_round_trip(f, out_scale);
+                }
+            } else if (n + 3 < N && ((reinterpret_cast<uintptr_t>(orow) & 7u) == 0)) {
+                *reinterpret_cast<uint2*>(orow) = make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (n + e < N) orow[e] = h[e];
+            }
+            if (acc_dump) {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (n + e < N) {
+                        const auto sv = sum[e];  // scalar copy first: a bit cast applied to the vector element itself reads element 0
+                        reinterpret_cast<uint32_t*>(acc_dump)[(int64_t)m * N + n + e] = __builtin_bit_cast(uint32_t, sv);
+                    }
+            }
+        }
+    };
+
+    int issued = 0, issue_s = 0;  // stages in flight or done; the next one within its group
+    auto issue_next = [&](int slot) __attribute__((always_inline)) {
+        if (issued == total) return;
+        if (C::MANY && issue_s == nst) issue_s = 0, next_group();
+        issue(issue_s++, slot);
+        issued++;
+    };
+#pragma unroll
+    for (int t = 0; t < NS - 1; t++) issue_next(t);
+    int slot = 0, s = 0, group = 0;
 #pragma unroll 1
-    for (int s = 0; s < nst; s++) {
-        wait_stage(min(nst - 1, s + NS - 2) - s);
-        lds_barrier();  // publishes stage s; every wavefront has read the whole of stage s - 1
-        const int prev = slot == 0 ? NS - 1 : slot - 1;
-        if (s + NS - 1 < nst) issue(s + NS - 1, prev);
+    for (int f = 0; f < total; f++) {
+        wait_stage(min(total - 1, f + NS - 2) - f);
+        lds_barrier();  // publishes this stage; every wavefront has read the whole of the one before
+        issue_next(slot == 0 ? NS - 1 : slot - 1);
         if ((s + 1) * SEG > K) compute(slot, true, K - s * SEG);
         else compute(slot, false, 0);
         slot = slot == NS - 1 ? 0 : slot + 1;
+        if (C::MANY && ++s == nst) {
+            finish(group);  // its reads of the sums are done in every wavefront before the barrier of the next stage
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int t = 0; t < T; t++) acc[mt][t] = acc_t{0, 0, 0, 0};
+            n0 += step_n, group++, s = 0;
+        } else if (!C::MANY) s++;
     }
-
-    // ---- the wavefronts add up in wavefront order
-    __syncthreads();  // every wavefront is done reading the stages
-    acc_t (*red)[MT * T][kWave] = reinterpret_cast<acc_t (*)[MT * T][kWave]>(smem);
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-        for (int t = 0; t < T; t++) red[wave][mt * T + t][lane] = acc[mt][t];
-    __syncthreads();
-    const float alpha = ep.alpha * (ep.alpha_dev ? *ep.alpha_dev : 1.0f);
-    for (int idx = tid; idx < MT * T * kWave; idx += C::NT) {
-        const int q = idx / kWave, l = idx % kWave, mt = q / T, t = q % T;
-        acc_t sum = red[0][q][l];
-#pragma unroll
-        for (int w = 1; w < C::NW; w++) sum += red[w][q][l];
-        // lane l of that accumulator: token 16 mt + l % 16, channels n0 + 16 t + 4 (l / 16) .. + 3
-        const int m = 16 * mt + (l & 15), n = n0 + 16 * t + 4 * (l >> 4);
-        if (m >= M || n >= N) continue;
-        const float sa = ep.a_scale ? ep.a_scale[m] : 1.f;
-        uint16_t h[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int ne = min(n + e, N - 1);
-            const float sw = ep.w_scale ? ep.w_scale[ne] : 1.f;
-            const float bb = ep.bias ? ep.beta * load_as_f32(ep.bias, ep.bias_dtype, ne) : 0.f;
-            const float v = epi_value((float)sum[e], sa, sw, alpha, bb);
-            h[e] = ep.out_dtype == LLMQ_BF16 ? Lo<LLMQ_BF16>::from_f32(v) : Lo<LLMQ_F16>::from_f32(v);
-        }
-        uint16_t* orow = reinterpret_cast<uint16_t*>(out) + (int64_t)m * ldo + n;
-        if (ep.out_scale) {
-            float* frow = reinterpret_cast<float*>(out) + (int64_t)m * ldo + n;
-            const float os = *ep.out_scale;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float f = ep.out_dtype == LLMQ_BF16 ? Lo<LLMQ_BF16>::to_f32(h[e]) : Lo<LLMQ_F16>::to_f32(h[e]);
-                if (n + e < N) frow[e] = fp8_round_trip(f, os);
-            }
-        } else if (n + 3 < N && ((reinterpret_cast<uintptr_t>(orow) & 7u) == 0)) {
-            *reinterpret_cast<uint2*>(orow) = make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                if (n + e < N) orow[e] = h[e];
-        }
-        if (acc_dump) {
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                if (n + e < N) {
-                    const auto sv = sum[e];  // scalar copy first: a bit cast applied to the vector element itself reads element 0
-                    reinterpret_cast<uint32_t*>(acc_dump)[(int64_t)m * N + n + e] = __builtin_bit_cast(uint32_t, sv);
-                }
-        }
+    if constexpr (!C::MANY) {
+        lds_barrier();  // every wavefront is done reading the stages
+        finish(0);
     }
 }
 
@@ -224,7 +278,12 @@ int launch_rows(const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ldb, in
             if (dev >= 0 && dev < 64) raised[dev] = true;
         }
     }
-    hipLaunchKernelGGL(kernel, dim3((unsigned)((N + 16 * C::T - 1) / (16 * C::T))), dim3(C::NT), C::LDS_BYTES, st, A, lda, B, ldb, M, N, K, ep, out, ldo,
+    int blocks = (N + 16 * C::T - 1) / (16 * C::T);
+    if (C::MANY) {  // as many as are resident at once, or fewer so that all take as many groups (288 groups of 18432 x 11904: 144 blocks 43.6 us, 256 52.7)
+        const int slots = 256 * (160 * 1024 / C::LDS_BYTES), each = std::min(kRowsGroups, (blocks + slots - 1) / slots);
+        blocks = (blocks + each - 1) / each;
+    }
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(C::NT), C::LDS_BYTES, st, A, lda, B, ldb, M, N, K, ep, out, ldo,
                        acc_dump);
     return launch_status();
 }
@@ -233,8 +292,8 @@ template <bool FP8, int AFMT>
 int launch_variant(int variant, const uint8_t* A, int64_t lda, const uint8_t* B, int64_t ldb, int M, int N, int K, const SkinnyEpilogue& ep, void* out,
                    int64_t ldo, void* acc_dump, hipStream_t st) {
     switch (variant) {
-#define LLMQ_ROWS_CASE(I, T, MT, SEG, NS) \
-    case I: return launch_rows<RowsCfg<FP8, AFMT, T, MT, SEG, NS>>(A, lda, B, ldb, M, N, K, ep, out, ldo, acc_dump, st);
+#define LLMQ_ROWS_CASE(I, T, MT, SEG, NS, MANY) \
+    case I: return launch_rows<RowsCfg<FP8, AFMT, T, MT, SEG, NS, MANY>>(A, lda, B, ldb, M, N, K, ep, out, ldo, acc_dump, st);
         LLMQ_ROWS_VARIANTS(LLMQ_ROWS_CASE)
 #undef LLMQ_ROWS_CASE
     }

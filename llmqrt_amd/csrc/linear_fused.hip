@@ -421,17 +421,16 @@ extern "C" int llmq_linear_fp8_dynamic(const void* x, int x_dtype, int64_t ldx, 
 // where one launch stops being ahead of max(two launches, 10).  Up to 4096 channels it is as long as the codes are few (per tensor 9 x 3584 x
 // 3584 8.8 / 9.0 on the GPU, 15 x 3584 x 3584 8.9 / 11.0; static 4 x 3584 x 3584 7.4 / 7.1, 11 x 3584 x 3584 7.5 / 10.5; per token, a wavefront per
 // row, 2 x 3584 x 3584 8.1 / 7.7, 15 x 3584 x 3584 8.1 / 10.0), and beyond that where there are few channels.  With more channels each CU repeats the quantizer a
-// few times (per tensor 7 x 9728 x 896 8.9 / 7.4, 2 x 37888 x 3584 35.2 / 31.7, 8 x 5168 x 7168 16.5 / 16.9; static 4 x 11744 x 1072 11.4 / 6.5,
-// 13 x 13016 x 2432 13.3 / 15.4, 2 x 8320 x 10368 25.4 / 27.0), past 16384 channels more often than the launch costs per token and with a
-// static scale (per token 4 x 37504 x 1408 17.0 / 22.8, 2 x 37888 x 3584 34.3 / 39.5; static 4 x 19184 x 2432 12.2 / 16.1, 9 x 34432 x 896 12.7 / 17.6).
+// few times and the GEMM alone streams at 5-6 TB/s (per tensor 7 x 9728 x 896 8.9 / 7.4, 8 x 5168 x 7168 16.5 / 16.9, 3 x 27264 x 5120 31.4 /
+// 37.2; static 4 x 11744 x 1072 11.4 / 6.5, 13 x 13016 x 2432 13.3 / 15.4, 2 x 8320 x 10368 25.4 / 27.0), past 16384 channels too
+// often per token and with a static scale (per token 4 x 10752 x 7168 20.9 / 23.8, 4 x 37504 x 1408 17.0 / 22.8; static 4 x 19184 x 2432 12.2 / 16.1).
 extern "C" int llmq_linear_one_launch_preferred(int kind, int64_t M, int64_t N, int64_t K) {
     if (!one_launch_fits(kind, M, N, K)) return 0;
     const int64_t codes = M * K;
-    if (codes <= 16384 && (kind == LLMQ_LINEAR_I8_TENSOR || kind == LLMQ_LINEAR_FP8_TENSOR)) return 1;
     if (kind == LLMQ_LINEAR_I8_TOKEN || kind == LLMQ_LINEAR_FP8_TOKEN)
-        return K < 8192 && ((M <= 4 && N <= 16384) || (N <= kFewChannels && codes <= 49152));
+        return K < 8192 && (N <= kFewChannels ? M <= 4 || codes <= 49152 : M <= 4 && N <= 16384 && codes <= (N <= 8192 ? 14336 : 8192));
     if (kind == LLMQ_LINEAR_FP8_STATIC) return N <= kFewChannels ? codes <= 32768 : codes <= 14336 && K < 8192 && N <= 16384;
-    if (N > kFewChannels) return codes <= 28672 && K < 8192 && N <= 16384;
+    if (N > kFewChannels) return codes <= 16384 ? N <= 8192 || codes <= 8192 : codes <= 28672 && K < 8192 && N <= 8192;
     return codes <= 49152 || (M > 8 && N <= 1024);
 }
 

@@ -6,7 +6,7 @@ from oracle import ref_math as R
 
 pytestmark = pytest.mark.gpu
 
-TOKENS = [16, 16, 16, 32, 32, 32, 32, 32, 48, 48, 64, 64]  # what a block of each variant holds
+TOKENS = [16, 16, 16, 32, 32, 32, 32, 32, 48, 48, 64, 64, 16, 16]  # what a block of each variant holds
 
 
 def _ints(shape, seed):
@@ -15,7 +15,7 @@ def _ints(shape, seed):
 
 # fewer tokens than a block holds, one, all; channels that end inside a 16-channel tile, inside a store of four, inside a block; K of one MFMA
 # step's part, a stage, a stage and 16 bytes, more and fewer stages than LDS slots, a ragged end in the last of several
-@pytest.mark.parametrize("variant", range(12))
+@pytest.mark.parametrize("variant", range(14))
 @pytest.mark.parametrize("missing,N,K", [(0, 136, 16), (15, 37, 1024), (3, 72, 528), (0, 200, 2560), (1, 264, 3600), (5, 64, 7168), (0, 48, 9232)])
 def test_every_variant(cuda, variant, missing, N, K):
     """Rows further apart than K, an output inside a larger one.  int8: accumulators and results bit for bit.  fp8 (e4m3 and e5m2
@@ -64,9 +64,35 @@ def test_every_variant(cuda, variant, missing, N, K):
     assert torch.equal(quant[:, :N], static_per_tensor_quantize(padded, scale.view(1)).to(torch.bfloat16).float()[:, :N] * scale)
 
 
+# blocks that go from one group of 64 or 32 channels to the next: a block has one or two, three, more than sixteen at one block a CU (then there are more blocks), with
+# one stage, several, a ragged end, and channels that end inside the last group
+@pytest.mark.parametrize("M,N,K", [(16, 16400, 528), (3, 36904, 3600), (1, 270016, 256), (9, 33000, 2048)])
+@pytest.mark.parametrize("variant", [12, 13])
+def test_many_groups_of_channels(cuda, variant, M, N, K):
+    from llmqrt_amd import _abi
+    L = _abi.lib()
+    g = torch.Generator().manual_seed(N)
+    qx, qw = _ints((M, K), M), _ints((N, K), N)
+    sx, sw = torch.rand(M, generator=g) * 0.01 + 1e-3, torch.rand(N, generator=g) * 0.01 + 1e-3
+    bias = torch.randn(N, generator=g).bfloat16()
+    dev = [t.to(cuda) for t in (sx, sw, bias, qx, qw)]
+    p = [t.data_ptr() for t in dev]
+    out = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device=cuda)
+    _abi.check(L.llmq_gemm_force_plan(110 + variant, 1), "force_plan")
+    try:
+        _abi.check(L.llmq_gemm_w8a8(p[3], K, p[4], K, p[0], p[1], 1.0, None, p[2], 0, 1.0, out.data_ptr(), 0, N, M, N, K, None, None, 0,
+                                    torch.cuda.current_stream().cuda_stream), "int8")
+    finally:
+        L.llmq_gemm_force_plan(-1, 1)
+    acc = (qx.double() @ qw.double().t()).int()  # exact: fewer than 2^53
+    want = R.w8a8_epilogue_per_token_per_channel(acc, sx, sw, bias, torch.bfloat16)
+    assert torch.equal(out[:M].cpu().view(torch.int16), want.view(torch.int16)) and (out[M] == 7.0).all()
+
+
 # what the planner itself picks on both sides of its limits: tokens, K and channels
 @pytest.mark.parametrize("M,N,K", [(1, 3584, 3584), (16, 4104, 2048), (16, 4088, 2048), (17, 3584, 3584), (32, 4608, 3584), (33, 4608, 3584), (48, 4608, 3584),
-                                   (64, 3584, 3584), (65, 3584, 3584), (8, 896, 4864), (32, 896, 1024), (32, 896, 1152), (20, 16128, 2048), (16, 1024, 18944)])
+                                   (64, 3584, 3584), (65, 3584, 3584), (8, 896, 4864), (32, 896, 1024), (32, 896, 1152), (20, 16128, 2048), (16, 1024, 18944),
+                                   (16, 8192, 1152), (16, 8200, 1152), (16, 8200, 768), (5, 16392, 1024), (4, 24584, 1024)])
 def test_planned(cuda, M, N, K):
     from llmqrt_amd.sq_fp8_kernels import w8a8_int8_linear_bbf16_obf16_per_channel
     g = torch.Generator().manual_seed(M + N)
