@@ -418,7 +418,8 @@ extern "C" int llmq_linear_fp8_dynamic(const void* x, int x_dtype, int64_t ldx, 
 
 // One launch or two.  Measured on an MI355X against quantizer + GEMM (us, two launches / one; weights out of HBM, 630 random problems and the
 // sizes of decoder layers).  Two launches issued from a program's own loop take 10 us of the host against 6 for one, so the line is
-// where one launch stops being ahead of max(two launches, 10).  Up to 4096 channels it is as long as the codes are few (per tensor 9 x 3584 x
+// where one launch stops being ahead of max(two launches, 10).  Per tensor a little further, as a decoder layer at these sizes is bound by the
+// host (10 x 896 x 4864 9.0 on the GPU in two / 10.9 in one, but the layer with its gate_up alike, 12 tokens, 41.7 / 35.4).  Up to 4096 channels it is as long as the codes are few (per tensor 9 x 3584 x
 // 3584 8.8 / 9.0 on the GPU, 15 x 3584 x 3584 8.9 / 11.0; static 4 x 3584 x 3584 7.4 / 7.1, 11 x 3584 x 3584 7.5 / 10.5; per token, a wavefront per
 // row, 2 x 3584 x 3584 8.1 / 7.7, 15 x 3584 x 3584 8.1 / 10.0), and beyond that where there are few channels.  With more channels each CU repeats the quantizer a
 // few times and the GEMM alone streams at 5-6 TB/s (per tensor 7 x 9728 x 896 8.9 / 7.4, 8 x 5168 x 7168 16.5 / 16.9, 3 x 27264 x 5120 31.4 /
@@ -430,7 +431,7 @@ extern "C" int llmq_linear_one_launch_preferred(int kind, int64_t M, int64_t N, 
     if (kind == LLMQ_LINEAR_I8_TOKEN || kind == LLMQ_LINEAR_FP8_TOKEN)
         return K < 8192 && (N <= kFewChannels ? M <= 4 || codes <= 49152 : M <= 4 && N <= 16384 && codes <= (N <= 8192 ? 14336 : 8192));
     if (kind == LLMQ_LINEAR_FP8_STATIC) return N <= kFewChannels ? codes <= 32768 : codes <= 14336 && K < 8192 && N <= 16384;
-    if (N > kFewChannels) return codes <= 16384 ? N <= 8192 || codes <= 8192 : codes <= 28672 && K < 8192 && N <= 8192;
+    if (N > kFewChannels) return codes <= 16384 ? N <= 16384 || codes <= 8192 : codes <= 28672 && K < 8192 && N <= 8192;
     return codes <= 49152 || (M > 8 && N <= 1024);
 }
 
