@@ -280,6 +280,9 @@ int llmq_linear_dynamic_force_variant(int v);
  * Per host thread (thread-local state): it affects only calls made later by the thread that set it. */
 int llmq_gemm_force_plan(int cfg, int splits);
 int llmq_gemm_num_configs(void);
+/* The configuration (as llmq_gemm_force_plan numbers them) that a call of llmq_gemm_w8a8 or llmq_gemm_fp8 of this size runs with a
+ * workspace of the query's size; LLMQ_ERR_SHAPE for sizes that are refused. */
+int llmq_gemm_planned_config(int fp8, int64_t M, int64_t N, int64_t K);
 
 /* ------------------------------------------------------------------------------------
  * AWQ W4A16.  Replaces awq_gemm_triton / awq_dequantize_triton

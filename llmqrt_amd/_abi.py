@@ -63,6 +63,7 @@ SIGNATURES = {
     "llmq_gemm_fp8_quantized_output_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "llmq_gemm_force_plan": (_int, [_int, _int]),
     "llmq_gemm_num_configs": (_int, []),
+    "llmq_gemm_planned_config": (_int, [_int, _i64, _i64, _i64]),
     "llmq_awq_gemm": (_int, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _sz, _vp]),
     "llmq_awq_gemm_bf16": (_int, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _sz, _vp]),
     "llmq_awq_gemm_bf16_supported": (_int, [_i64, _i64, _i64, _i64]),

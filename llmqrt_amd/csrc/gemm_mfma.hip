@@ -349,16 +349,60 @@ double rows_time(int v, int64_t N, int64_t K) {
 // and the whole K tail goes through registers (36 x 10752 x 5792 28.8 / 24.5), for
 // gemm_skinny.hip at 1.15.  With the factors below, of the 900 problems the half that moves makes the mean over all 11 % faster; 1 % of
 // all end more than 5 % behind.
-int rows_variant(const Plan& plan, double now, int64_t M, int64_t N, int64_t K) {
+// Row lengths for which the same piece of the rows of a block falls on few memory channels: a few rows span a whole number of 32 KB, exactly or
+// to 256 bytes.  Long pieces of many rows, all blocks at the same place of K, suffer more from it than the tiles' 128 bytes.
+inline bool crowded_rows(int64_t K) {
+    const auto near = [](int64_t v) { return (v + 256) % 32768 <= 512; };
+    return K % 4096 == 0 || near(2 * K) || near(3 * K);
+}
+// Sizes at which the plan of tiles and gemm_skinny.hip (before) was measured ahead of this kernel (rows), in 10 000 random problems of 1-64 tokens that
+// the lines of rows_variant give to it; us, before / rows.  With these the problems that end more than 3 % behind go from 819 to
+// 181, more than 10 % from 262 to 7.
+bool rows_behind(bool fp8, const Plan& plan, bool many, int64_t M, int64_t N, int64_t K) {
+    const bool ragged = K % 128 != 0, tiles = plan.cfg < kSkinnyCfg;
+    if (M > 16) {
+        // three and four token tiles of few channels are few blocks over a long K (int8 61 x 960 x 8704 11.6 / 14.2, 50 x 512 x 9104 11.3 / 15.2; but fp8
+        // 59 x 3472 x 7552 14.5 / 13.7), and over a short one wait for four wavefronts' sums (fp8 57 x 952 x 1920 4.4 / 5.1); many short ragged rows
+        // (int8 49 x 9400 x 1984 12.6 / 14.4); the 4 KB stride (fp8 57 x 968 x 4096 7.1 / 8.3)
+        if (M > 32) {
+            if (tiles && K > 5632 && (M > 48 ? 3 : 4) * N < K && !(ragged && K <= 8192)) return true;
+            if (plan.cfg == kSkinnyCfg && N <= 1280 && K <= 2048) return true;
+            if (N > 8192 && K < 2560) return true;
+            if (!ragged && N <= 1536 && K % 4096 == 0) return true;
+        }
+        // more than 256 tiles of 64 channels (int8 20 x 16808 x 1280 9.2 / 11.5, 29 x 24528 x 2000 16.4 / 18.8); 22 x 1080 x 15296 13.0 / 15.1
+        return N > 16384 || (K > 10240 && 5 * N <= K);
+    }
+    if (many) {
+        if (ragged) return false;
+        // two stages or three of which the last is mostly empty, in more rounds than one (fp8 1 x 29256 x 1152 9.5 / 10.4, 2 x 25824 x 896 8.1 / 8.5;
+        // but 2 x 25544 x 1024 8.7 / 8.3)
+        if (N > 20480 && K < 1280 && K % 512) return true;
+        // crowded rows, up to two groups a block: int8 2 x 14408 x 11008 33.1 / 38.9, 7 x 25576 x 8192 39.3 / 42.4, 4 x 22384 x 16384 66.5 / 80.0, 2 x 30896 x
+        // 4096 24.9 / 28.1; fp8 8 x 8512 x 20480 37.9 / 42.7, 2 x 20544 x 16384 65.7 / 74.6; with three groups ahead again (int8 16 x 34104 x 8192 66.3 / 57.7)
+        if (!crowded_rows(K) || N > 32768) return false;
+        if (N <= 16384) return K > 10240 && !(fp8 && K >= 12288 && K <= 16512);
+        if (fp8) return K == 16384 && N <= 24576;
+        return K >= 16000 || 3 * K % 32768 <= 256 || (K == 8192 && N > 20480) || (K % 4096 == 0 && N > 24576);
+    }
+    if (ragged || tiles) return false;
+    // eight or sixteen wavefronts along K that own no more than seven steps each (fp8 1 x 2760 x 3456 5.0 / 5.5, 4 x 3384 x 3456 5.4 / 5.7)
+    if (K > 3136 && K <= 4096 && N < 4096 && ((M <= 2 && K < 4096) || (M <= 6 && N * K > 8800000))) return true;
+    // crowded rows again (int8 1 x 3624 x 11008 11.1 / 13.1, 2 x 7984 x 16384 25.9 / 33.3, 3 x 8000 x 8192 14.7 / 16.7; fp8 2 x 7112 x 16384 26.0 / 30.2)
+    if (K % 4096 != 0 && 3 * K % 32768 > 256) return false;
+    return (M <= 3 && K >= 8192 && N > 2400 && N < 4096) || (M <= 8 && N > 6716 && (!fp8 || K >= 16384));
+}
+int rows_variant(int op, const Plan& plan, double now, int64_t M, int64_t N, int64_t K) {
     if (M > 64 || K <= (M <= 16 && N > 8192 ? 768 : 1024) || K > kTableMaxK) return -1;
     const int mt = cdiv(M, 16);
-    // Many channels: blocks that go from one group of channels to the next, from where 64 channels a block are enough blocks.  342 random problems
-    // of up to 16 tokens, plan of tiles / this (mean, least): 8193-16384 channels 1.13 (0.92), from 24577 on 1.13 (0.98); up to
-    // 8192 0.78.  16385-24576 channels make one to one and a half groups of 64 a CU, so groups of 32 there, three a block: 1.10 (0.87) against 1.08 (0.82).
+    // Many channels: blocks that go from one group of channels to the next, from where 64 channels a block are enough blocks.  3400 random problems
+    // of up to 16 tokens, plan of tiles / this in the mean: 8193-16384 channels 1.20, 16385-24576 1.11, more 1.09; up to 8192 0.78.  16385-24576 channels
+    // make one to one and a half groups of 64 a CU, so groups of 32 there, three a block: 1.10 against 1.08.
     // Up to 20480 of these the tiles of 128 channels fill the chip in one round and keep the shorter K (14 x 17920 x 4096 13.6 / 14.8, 4 x 19184 x 2432
     // 9.7 / 10.4; 2 x 18432 x 11904 48 / 42).
     const bool ragged = K % 128 != 0, tiles = plan.cfg < kSkinnyCfg;
-    if (mt == 1 && N > 8192 && (N <= 16384 || N > 20480 || ragged || K >= 8192)) return N > 16384 && N <= 24576 ? kRowsMany + 1 : kRowsMany;
+    if (mt == 1 && N > 8192 && (N <= 16384 || N > 20480 || ragged || K >= 8192))
+        return rows_behind(op == 1, plan, true, M, N, K) ? -1 : N > 16384 && N <= 24576 ? kRowsMany + 1 : kRowsMany;
     double factor = 0.95;
     if (mt > 1) {
         if (ragged && K < 2048 && N < 4096) return -1;
@@ -370,6 +414,7 @@ int rows_variant(const Plan& plan, double now, int64_t M, int64_t N, int64_t K) 
         if (N < 4096 ? K <= (ragged ? 4095 : 2048) : ragged && K < 1792) return -1;
         if (ragged && N * K > 40000000) return -1;  // (int8 3 x 2944 x 18608 12.9 / 15.6)
     }
+    if (rows_behind(op == 1, plan, false, M, N, K)) return -1;
     double best = now * factor;
     int variant = -1;
     for (int v = 0; v < kRowsMany; v++)
@@ -427,7 +472,7 @@ Plan make_plan(int op, int64_t M, int64_t N, int64_t K) {
     else
         for (const TileCost& c : costs_of(op).tiles)
             if (c.cfg == plan.cfg) now = table_time(costs_of(op), c, M, N, K, plan.splits, plan.k_per_split);
-    const int variant = rows_variant(plan, now, M, N, K);
+    const int variant = rows_variant(op, plan, now, M, N, K);
     return variant < 0 ? plan : rows(variant, K);
 }
 
@@ -561,6 +606,10 @@ extern "C" int llmq_gemm_force_plan(int cfg, int splits) {
 }
 
 extern "C" int llmq_gemm_num_configs(void) { return kNumShapes; }
+
+extern "C" int llmq_gemm_planned_config(int fp8, int64_t M, int64_t N, int64_t K) {
+    return M <= 0 || N <= 0 || K <= 0 || K % 16 ? LLMQ_ERR_SHAPE : plan_for(fp8 ? 1 : 0, M, N, K).cfg;
+}
 
 namespace {
 // what the plan that a call of this size runs splits into: a lookup once the size is planned

@@ -58,6 +58,28 @@ def test_argument_validation_needs_no_gpu():
     assert L.llmq_awq_gemm_workspace_bytes(1, 4608, 3584) > 0
 
 
+# (fp8, M, N, K, whether the row-streaming kernel runs): both sides of the lines beyond which the kernels before it were measured ahead: many tokens of few
+# channels over a long and a short K, more channels than 17-64 tokens stream, short rows that leave the last stage empty, rows that fall on few
+# memory channels
+@pytest.mark.parametrize("fp8,M,N,K,rows", [
+    (0, 61, 960, 8704, False), (0, 61, 2560, 4096, True), (0, 50, 512, 9104, False), (0, 50, 512, 7216, True), (1, 57, 952, 1920, False), (1, 57, 2304, 1920, True),
+    (0, 49, 9400, 1984, False), (0, 30, 9400, 1984, True), (1, 57, 968, 4096, False), (0, 20, 16808, 1280, False), (0, 20, 16128, 1280, True),
+    (0, 22, 1080, 15296, False), (1, 1, 29256, 1152, False), (1, 1, 29256, 1024, True), (1, 1, 29256, 1280, True), (0, 2, 14408, 11008, False), (0, 2, 14408, 10752, True),
+    (0, 7, 25576, 8192, False), (1, 7, 25576, 8192, True), (0, 4, 22384, 16384, False), (0, 2, 30896, 4096, False), (0, 16, 34104, 8192, True),
+    (1, 8, 8512, 20480, False), (1, 2, 20544, 16384, False), (1, 2, 14408, 16384, True), (1, 1, 2760, 3456, False), (1, 8, 2760, 3456, True), (0, 1, 3624, 11008, False),
+    (0, 2, 7984, 16384, False), (0, 2, 7984, 14336, True), (0, 1, 37888, 3584, True), (0, 16, 3584, 3584, True), (0, 65, 3584, 3584, False)])
+def test_few_token_gemm_lines(fp8, M, N, K, rows):
+    from llmqrt_amd import _abi
+    cfg = _abi.lib().llmq_gemm_planned_config(fp8, M, N, K)
+    assert (110 <= cfg <= 123) == rows, cfg
+
+
+def test_planned_config_refuses():
+    from llmqrt_amd import _abi
+    plan = _abi.lib().llmq_gemm_planned_config
+    assert plan(0, 0, 64, 64) == plan(0, 4, 64, 40) == plan(1, 4, -1, 64) == -3
+
+
 def test_wrappers_fail_loudly_off_gpu():
     from llmqrt_amd import sq_fp8_kernels as ops
     from llmqrt_amd.quantize import quantize_activation_per_token_absmax
