@@ -4,6 +4,8 @@ and split-K arguments are accepted (and validated as the reference validates the
 gfx950 kernels choose their own tiling."""
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _abi
@@ -109,7 +111,7 @@ def awq_gemm_bf16(input: torch.Tensor, qweight: torch.Tensor, scales: torch.Tens
                   bias: torch.Tensor | None = None) -> torch.Tensor:
     """``awq_gemm_triton(input.half(), ...).bfloat16()`` in one launch, for shapes that awq_gemm_bf16_supported takes."""
     assert input.dtype == torch.bfloat16
-    return _awq_gemm(input, qweight, scales, qzeros, 1, bias)
+    return _awq_gemm(input, qweight, scales, qzeros, 1, bias, "llmq_awq_gemm_tickets")
 
 
 def awq_linear_bf16_supported(M: int, N: int, K: int, group_size: int) -> bool:
@@ -123,10 +125,10 @@ def awq_linear_bf16(input: torch.Tensor, qweight: torch.Tensor, scales: torch.Te
     """What the module does with bf16 activations (linear_awq.py:245-262) without launches for the conversions, for shapes that
     awq_linear_bf16_supported takes."""
     assert input.dtype == torch.bfloat16
-    return _awq_gemm(input, qweight, scales, qzeros, 1, bias, "llmq_awq_linear")
+    return _awq_gemm(input, qweight, scales, qzeros, 1, bias)
 
 
-def _awq_gemm(input, qweight, scales, qzeros, split_k_iters, bias, entry="llmq_awq_gemm_tickets"):
+def _awq_gemm(input, qweight, scales, qzeros, split_k_iters, bias, entry="llmq_awq_linear"):
     M, K = input.shape
     N = qweight.shape[1] * 8
     group_size = qweight.shape[0] // qzeros.shape[0]
@@ -136,7 +138,8 @@ def _awq_gemm(input, qweight, scales, qzeros, split_k_iters, bias, entry="llmq_a
     _check_layout(qweight, scales, qzeros, K, N, group_size)
     assert input.device == qweight.device
     x = input
-    if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16 or (entry == "llmq_awq_linear" and x.stride(0) >= 1 << 22):
+    if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16 or (entry == "llmq_awq_linear" and x.dtype == torch.bfloat16
+                                                                             and x.stride(0) >= 1 << 22):
         x = x.contiguous()
     bias = _bias_vector(bias, N, x.device)
     if bias is not None:
@@ -144,10 +147,16 @@ def _awq_gemm(input, qweight, scales, qzeros, split_k_iters, bias, entry="llmq_a
     result = torch.empty((M, N), dtype=input.dtype, device=input.device)
     L = _abi.lib()
     # the arrival counters are the native forwards' own, one set per stream and one per capture; the partial sums are this call's
-    partials = L.llmq_awq_gemm_partials_bytes(M, N, K, group_size)
+    dt = _abi.dtype_code(input.dtype)
+    if entry == "llmq_awq_linear":
+        needs = ctypes.c_int(0)
+        partials = L.llmq_awq_linear_partials_bytes(dt, M, N, K, group_size, x.stride(0), ctypes.byref(needs))
+        counters = host().awq_counters(x) if needs.value else None
+    else:
+        partials = L.llmq_awq_gemm_partials_bytes(M, N, K, group_size)
+        counters = host().awq_counters(x) if partials else None
     ws = _abi.workspaces.get(x.device, partials)
-    counters = host().awq_counters(x) if partials else None
-    _abi.check(getattr(L, entry)(x.data_ptr(), _abi.dtype_code(input.dtype), x.stride(0), qweight.data_ptr(),
+    _abi.check(getattr(L, entry)(x.data_ptr(), dt, x.stride(0), qweight.data_ptr(),
                                  scales.data_ptr(), qzeros.data_ptr(), _abi.ptr(bias), result.data_ptr(), M, N, K,
                                  group_size, _abi.ptr(counters), _abi.ptr(ws), ws.numel() if ws is not None else 0,
                                  _abi.stream_of(x)), "llmq_awq_gemm")

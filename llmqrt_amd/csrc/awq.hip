@@ -874,10 +874,11 @@ size_t staged_partials_bytes(int64_t M, int64_t N, int64_t K, int64_t group) {
     return total;
 }
 
-// bf16_any: bf16 wherever a kernel takes it (llmq_awq_linear); otherwise only where llmq_awq_gemm_bf16_supported says so
+// linear (llmq_awq_linear): bf16 wherever a kernel takes it, partial sums without counters where none are used; otherwise bf16 only where
+// llmq_awq_gemm_bf16_supported says so, and no workspace without counters
 int awq_gemm_entry(const void* x, int64_t ldx, const int32_t* qweight, const void* scales, const int32_t* qzeros,
                    const void* bias, void* out, int64_t M, int64_t N, int64_t K, int64_t group, bool bf16_io,
-                   void* ticket_area, void* partials, size_t workspace_bytes, llmq_stream_t stream, bool bf16_any = false) {
+                   void* ticket_area, void* partials, size_t workspace_bytes, llmq_stream_t stream, bool linear = false) {
     if (M < 0 || N < 0 || K < 0) return LLMQ_ERR_SHAPE;
     if (M == 0 || N == 0) return LLMQ_OK;
     if (!x || !qweight || !scales || !qzeros || !out) return LLMQ_ERR_NULL;
@@ -890,14 +891,14 @@ int awq_gemm_entry(const void* x, int64_t ldx, const int32_t* qweight, const voi
         return LLMQ_ERR_ALIGN;
     hipStream_t st = (hipStream_t)stream;
     unsigned int* tickets = (unsigned int*)ticket_area;
-    float* ws = tickets ? (float*)partials : nullptr;
+    float* ws = tickets || linear ? (float*)partials : nullptr;
     const uint32_t* qw = (const uint32_t*)qweight;
     const uint32_t* qz = (const uint32_t*)qzeros;
     const uint16_t* sc = (const uint16_t*)scales;
     const uint16_t* bs = (const uint16_t*)bias;
     const int Ni = (int)N, Ki = (int)K, Gi = (int)group;
     const bool stream_takes = stream_path(M, N, K, group, ldx, bf16_io);
-    if (bf16_io && !(bf16_any && stream_takes) && (tile_path(M) || !decode16_path(M, N, K, group))) return LLMQ_ERR_DTYPE;
+    if (bf16_io && !(linear && stream_takes) && (tile_path(M) || !decode16_path(M, N, K, group))) return LLMQ_ERR_DTYPE;
     if (stream_takes) {
         const size_t given = ws ? workspace_bytes : 0;
         AwqStreamPlan p = stream_plan(M, N, K, group);
@@ -923,7 +924,7 @@ int awq_gemm_entry(const void* x, int64_t ldx, const int32_t* qweight, const voi
     }
     if (decode16_path(M, N, K, group)) {
         const AwqDecodePlan d = decode16_plan(M, N, K);
-        if (d.splits > 1 && (!ws || workspace_bytes < awq_decode_workspace_bytes(d, M, N))) return LLMQ_ERR_WORKSPACE;
+        if (d.splits > 1 && (!ws || !tickets || workspace_bytes < awq_decode_workspace_bytes(d, M, N))) return LLMQ_ERR_WORKSPACE;
         return launch_awq_decode(d, (const uint16_t*)x, ldx, qw, sc, qz, bs, (uint16_t*)out, tickets, ws, (int)M, Ni, Ki, bf16_io, st);
     }
     // tokens are processed in slabs of at most 64 rows (4 MFMA token tiles per weight pass)
@@ -1022,7 +1023,16 @@ extern "C" int llmq_awq_linear(const void* x, int x_dtype, int64_t ldx, const in
                                void* tickets, void* partials, size_t partials_bytes, llmq_stream_t stream) {
     if (x_dtype != LLMQ_BF16 && x_dtype != LLMQ_F16) return LLMQ_ERR_DTYPE;
     return awq_gemm_entry(x, ldx, qweight, scales, qzeros, bias, out, M, N, K, group, x_dtype == LLMQ_BF16, tickets, partials,
-                          tickets ? partials_bytes : 0, stream, true);
+                          partials ? partials_bytes : 0, stream, true);
+}
+
+extern "C" size_t llmq_awq_linear_partials_bytes(int x_dtype, int64_t M, int64_t N, int64_t K, int64_t group, int64_t ldx, int* counters) {
+    *counters = 0;
+    if (!awq_sizes_ok(M, N, K) || group <= 0) return 0;
+    if (stream_path(M, N, K, group, ldx, x_dtype == LLMQ_BF16)) return awq_stream_workspace_bytes(stream_plan(M, N, K, group), M, N);
+    const size_t staged = staged_partials_bytes(M, N, K, group);
+    *counters = staged > 0 && !tile_path(M) && decode16_path(M, N, K, group);
+    return staged;
 }
 
 extern "C" int llmq_awq_dequant(const int32_t* qweight, const void* scales, const int32_t* qzeros, void* out,

@@ -388,16 +388,16 @@ std::optional<Tensor> awq(const Tensor& x, const Tensor& qweight, const Tensor& 
     const bool native_bf16 = bf16 && llmq_awq_linear_bf16_supported(r.M, N, r.K, group, r.K);
     const Tensor xin = bf16 && !native_bf16 ? x.to(at::kHalf) : x;
     Tensor out = make(out_size(x, N), xin.scalar_type(), dev);
-    // {arrival counters, partial sums}: the partial sums of this call only
-    const int64_t part = (int64_t)llmq_awq_gemm_partials_bytes(r.M, N, r.K, group);
+    // the partial sums of this call, and the arrival counters where the kernel that runs uses them
+    const int xdt = native_bf16 ? LLMQ_BF16 : LLMQ_F16;
+    int count = 0;
+    const int64_t part = (int64_t)llmq_awq_linear_partials_bytes(xdt, r.M, N, r.K, group, r.K, &count);
     Tensor ws, tk;
-    if (part) {
-        ws = make({part}, at::kByte, dev);
-        tk = counters().get(dev, l.stream);
-    }
-    check(llmq_awq_linear(xin.data_ptr(), native_bf16 ? LLMQ_BF16 : LLMQ_F16, r.K, (const int32_t*)qweight.data_ptr(),
-                                scales.data_ptr(), (const int32_t*)qzeros.data_ptr(), ptr(bias), out.data_ptr(), r.M, N, r.K, group,
-                          part ? tk.data_ptr() : nullptr, part ? ws.data_ptr() : nullptr, (size_t)part, l.stream),
+    if (part) ws = make({part}, at::kByte, dev);
+    if (count) tk = counters().get(dev, l.stream);
+    check(llmq_awq_linear(xin.data_ptr(), xdt, r.K, (const int32_t*)qweight.data_ptr(), scales.data_ptr(), (const int32_t*)qzeros.data_ptr(),
+                          ptr(bias), out.data_ptr(), r.M, N, r.K, group, count ? tk.data_ptr() : nullptr, part ? ws.data_ptr() : nullptr,
+                          (size_t)part, l.stream),
           "llmq_awq_linear");
     return bf16 && !native_bf16 ? out.to(at::kBFloat16) : out;
 }

@@ -158,3 +158,56 @@ def test_workspace_rule(cuda):
     assert rc == 0 and ((out4.float() - out.float()).abs().max() <= 2e-3 * out.float().abs().max())
     rc, none = call(few // 4)
     assert rc == -4 and int(none.count_nonzero()) == 0
+
+
+@pytest.mark.parametrize("M,K,N,G,dtype,most", [(777, 1024, 2048, 128, torch.float16, 1), (64, 18944, 3584, 128, torch.float16, 2), (12, 896, 1152, 32, torch.float16, 1),
+                                                (12, 896, 1152, 32, torch.bfloat16, 2)])
+def test_module_allocates_what_runs(cuda, M, K, N, G, dtype, most):
+    """The output, and partial sums only where the kernel that runs splits K; arrival counters only for the kernel that counts (the 7B-class sizes
+    above): a streaming call makes none."""
+    from llmqrt_amd._native import host
+    from llmqrt_amd.linear import WQLinear_GEMM
+    qw, qz, s, x, _ = _problem(M, K, N, G, M + N)
+    mod = WQLinear_GEMM(4, G, K, N, False, cuda)
+    mod.qweight.copy_(qw); mod.qzeros.copy_(qz); mod.scales.copy_(s)
+    xd = x.to(dtype).to(cuda).view(1, M, K)
+    ref = mod(xd)
+    torch.cuda.synchronize()
+    host().release_tickets()
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    y = mod(xd)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] - before == most
+    assert torch.equal(y, ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_exact_workspace_without_counters(cuda, dtype):
+    """llmq_awq_linear with the bytes that its query names and no counters gives what it gives with more of both; with no workspace at all it runs
+    without a split or refuses, as the kernels before need one; the few-token kernel refuses a split without counters."""
+    import ctypes
+    from llmqrt_amd import _abi
+    L = _abi.lib()
+    stream = torch.cuda.current_stream().cuda_stream
+    tickets = torch.zeros(L.llmq_awq_workspace_ticket_bytes(), dtype=torch.uint8, device=cuda)
+
+    def call(M, K, N, G, tick, ws, nbytes):
+        qw, qz, s, x, _ = (t.to(cuda) for t in _problem(M, K, N, G, M))
+        out = torch.zeros((M, N), dtype=dtype, device=cuda)
+        rc = L.llmq_awq_linear(x.to(dtype).data_ptr(), _abi.dtype_code(dtype), K, qw.data_ptr(), s.data_ptr(), qz.data_ptr(), None, out.data_ptr(), M, N, K, G,
+                               _abi.ptr(tick), _abi.ptr(ws), nbytes, stream)
+        return rc, out
+    flag = ctypes.c_int(0)
+    for M, K, N, G in ((64, 18944, 3584, 128), (200, 3584, 1152, 64), (130, 1024, 520, 128)):
+        need = L.llmq_awq_linear_partials_bytes(_abi.dtype_code(dtype), M, N, K, G, K, ctypes.byref(flag))
+        assert flag.value == 0
+        guard = torch.full((need + 256,), 0x5A, dtype=torch.uint8, device=cuda)
+        rc, exact = call(M, K, N, G, None, guard, need)
+        big = torch.empty(max(need, L.llmq_awq_gemm_partials_bytes(M, N, K, G), 16), dtype=torch.uint8, device=cuda)
+        rc2, ref = call(M, K, N, G, tickets, big, big.numel())
+        assert rc == rc2 == 0 and torch.equal(exact, ref) and bool((guard[need:] == 0x5A).all())
+        rc, _ = call(M, K, N, G, None, None, 0)
+        assert rc == (-4 if L.llmq_awq_gemm_partials_bytes(M, N, K, G) else 0)
+    need = L.llmq_awq_linear_partials_bytes(_abi.dtype_code(dtype), 4, 3584, 3584, 128, 3584, ctypes.byref(flag))
+    assert need and flag.value == 1
+    rc, none = call(4, 3584, 3584, 128, None, torch.empty(need, dtype=torch.uint8, device=cuda), need)
+    assert rc == -4 and int(none.count_nonzero()) == 0
