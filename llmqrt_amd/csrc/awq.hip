@@ -748,8 +748,8 @@ inline AwqDecodePlan decode16_plan(int64_t M, int64_t N, int64_t K) {
 
 // The streaming tile kernel (awq_stream.hip) takes what it is ahead at (us, weights out of HBM, kernel before / stream):
 //   past 64 tokens everything that it supports: 128 x 37888 x 3584 92.9 / 51.6, 128 x 3584 x 18944 51.8 / 32.7, 512 x 37888 x 3584 223 / 158,
-//     512 x 4608 x 3584 36.7 / 32.2; 300 random problems of 65-1024 tokens 1.35 times faster in the mean, seven up to 15 % slower (all of 2 MB of
-//     weights and less, 10-14 us);
+//     512 x 4608 x 3584 36.7 / 32.2; 300 random problems of 65-1024 tokens 1.35 times faster in the mean; 1200 of up to 600 tokens and 4 million
+//     weights (8-14 us) 1.08 times, 187 of them more than 3 % slower, 18 more than 8 %, and no line through tokens, K and channels tells which;
 //   17-64 tokens that the few-token kernel takes as slabs of 16: with 40 million weights and more, where unpacking them once per slab costs
 //     more than a second launch for the K split (64 x 37888 x 3584 44.5 / 33.8, 64 x 3584 x 18944 29.8 / 24.2, 42 x 4608 x 21024 51.5 / 26.9; but 64
 //     x 4608 x 3584 15.0 / 15.4, 33 x 3584 x 3584 12.8 / 13.2), and with 1.5 million and fewer, which need no split (29 x 896 x 896 9.4 / 8.1);

@@ -563,7 +563,12 @@ AwqStreamPlan make_awq_stream_plan(int64_t M, int64_t N, int64_t K, int64_t grou
                 return plan_of(cfg, fold, K, 1);
             }
             if (force_splits > 0) return p;
-            const double t = time_of(p, M, N, K);
+            double t = time_of(p, M, N, K);
+            // Past 64 tokens with few weights and a short K a K split of two 64-token blocks a CU comes out cheaper than the table has it, most where the
+            // alternative is one launch over eight to twelve stages (us, one launch / split: 148 x 632 x 512 10.0 / 8.5, 79 x 1560 x 512 10.0 / 8.7).
+            // 1200 random problems of 65-600 tokens and up to 4 million weights, against the tile kernel: more than 8 % behind 62 -> 18, more than 3 %
+            // 266 -> 187, in the mean 1.07 -> 1.08 times ahead.  With a longer K such a split loses 2-6 % (391 x 512 x 2432 13.3 / 14.3).
+            if (cfg == 2 && p.splits > 1 && M > 64 && K <= 1024 && N * K <= 4000000) t -= 0.9;
             if (t < best_t) best_t = t, best = p;
         }
     }
