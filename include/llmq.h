@@ -336,6 +336,9 @@ int llmq_awq_linear(const void* x, int x_dtype, int64_t ldx, const int32_t* qwei
                     int64_t M, int64_t N, int64_t K, int64_t group,
                     void* tickets, void* partials, size_t partials_bytes, llmq_stream_t stream);
 int llmq_awq_linear_bf16_supported(int64_t M, int64_t N, int64_t K, int64_t group, int64_t ldx);
+/* The kernel that a call of llmq_awq_linear of this size runs with a workspace of the query's size, numbered as llmq_awq_force_plan numbers them
+ * (8 for every form of the few-token kernel, 1 for every form of the register-streaming one); LLMQ_ERR_SHAPE or _DTYPE where it is refused. */
+int llmq_awq_planned_config(int x_dtype, int64_t M, int64_t N, int64_t K, int64_t group, int64_t ldx);
 /* What one call of llmq_awq_linear uses: bytes of partial sums, and in *counters 1 where it needs the arrival counters too (else
  * `tickets` may be null).  Like the other queries it knows nothing of pointers: no size is refused here that a call would refuse. */
 size_t llmq_awq_linear_partials_bytes(int x_dtype, int64_t M, int64_t N, int64_t K, int64_t group, int64_t ldx, int* counters);

@@ -70,6 +70,7 @@ SIGNATURES = {
     "llmq_awq_gemm_tickets": (_int, [_vp, _int, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _sz, _vp]),
     "llmq_awq_linear": (_int, [_vp, _int, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _sz, _vp]),
     "llmq_awq_linear_bf16_supported": (_int, [_i64, _i64, _i64, _i64, _i64]),
+    "llmq_awq_planned_config": (_int, [_int, _i64, _i64, _i64, _i64, _i64]),
     "llmq_awq_linear_partials_bytes": (_sz, [_int, _i64, _i64, _i64, _i64, _i64, ctypes.POINTER(_int)]),
     "llmq_awq_gemm_partials_bytes": (_sz, [_i64, _i64, _i64, _i64]),
     "llmq_awq_gemm_workspace_bytes": (_sz, [_i64, _i64, _i64]),

@@ -751,13 +751,18 @@ inline AwqDecodePlan decode16_plan(int64_t M, int64_t N, int64_t K) {
 //     512 x 4608 x 3584 36.7 / 32.2; 300 random problems of 65-1024 tokens 1.35 times faster in the mean; 1200 of up to 600 tokens and 4 million
 //     weights (8-14 us) 1.08 times, 187 of them more than 3 % slower, 18 more than 8 %, and no line through tokens, K and channels tells which;
 //   17-64 tokens that the few-token kernel takes as slabs of 16: with 40 million weights and more, where unpacking them once per slab costs
-//     more than a second launch for the K split (64 x 37888 x 3584 44.5 / 33.8, 64 x 3584 x 18944 29.8 / 24.2, 42 x 4608 x 21024 51.5 / 26.9; but 64
-//     x 4608 x 3584 15.0 / 15.4, 33 x 3584 x 3584 12.8 / 13.2), and with 1.5 million and fewer, which need no split (29 x 896 x 896 9.4 / 8.1);
-//   other groups and channel counts: past 16 tokens all (64 x 6400 x 4608, group 64: 31.5 / 17.8; 1.25-1.8 times in the mean), up to 16 from 24
-//     million weights on (12 x 5120 x 15488, group 32: 27.7 / 20.6; 3 x 896 x 9728, group 64: 8.8 / 11.1); groups of 128, whose register-streaming
-//     kernel is faster, past 24 tokens all (29 x 13568 x 1048 19.8 / 16.1), 17-24 from 30 million on (19 x 4992 x 1328 11.5 / 12.5), up to 16 from 150
-//     million on (5 x 17408 x 11768 45.4 / 33.7, 2 x 11264 x 3728 12.9 / 16.1).  In a bf16 model always: the kernels before have a
-//     conversion launch on either side there (12 x 4480 x 2152 20.9 / 12.6).
+//     more than a second launch for the K split (64 x 37888 x 3584 44.5 / 33.8, 64 x 3584 x 18944 29.8 / 24.2, 42 x 21024 x 4608 51.5 / 26.9; but 64
+//     x 4608 x 3584 15.0 / 15.4, 33 x 3584 x 3584 12.8 / 13.2), and with 1.5 million and fewer, which need no split (29 x 896 x 896 9.4 / 8.1), but
+//     not few channels over a long K;
+//   other groups: past 16 tokens all (64 x 4608 x 6400, group 64: 31.5 / 17.8; 1.25-1.8 times in the mean), up to 16 from 24 million weights on (12 x
+//     15488 x 5120, group 32: 27.7 / 20.6; 3 x 9728 x 896, group 64: 8.8 / 11.1);
+//   groups of 128 with channels that are no multiple of 32, whose register-streaming kernel is faster (tokens x channels x K, 3000 random problems): past
+//     24 tokens with a long K and from 6.5 to 11 million weights on, the more the fewer 16-token slabs that kernel has, and more for a short K (29 x 1048 x
+//     13568 19.8 / 16.1, 56 x 9224 x 1664 18 / 14; 35 x 3792 x 768 7.0 / 9.6, 62 x 3624 x 1024 8.9 / 11.3, 39 x 9744 x 896 8.5 / 11.4); 17-24 from 30
+//     million on (0.77 of the time in the mean); up to 16 from 150 million on (5 x 11768 x 17408 45.4 / 33.7), up to 6 from 210 where that kernel's blocks
+//     fill the chip once (1 x 9904 x 17792, 234 blocks, 29.9 / 36.3), but not where that kernel has a block a CU and more without a split and whole pieces of 128 bytes (1 x 32776 x 7424 38.4 / 54.3, 10 x 31800 x 7296 37.5 /
+//     45.3, 7 x 33296 x 7040 45.1 / 53.1; 6 x 35976 x 16640 124.8 / 93.2).  In a bf16 model always but for the last: the kernels before have a
+//     conversion launch on either side there (1500 random problems 0.67 of the time in the mean, 12 x 2152 x 4480 20.9 / 12.6; 2 x 36208 x 7552 53.4 / 64.2).
 inline bool stream_supported(int64_t M, int64_t N, int64_t K, int64_t group, int64_t ldx) {
     return (g_force_v == 0 || (g_force_v >= 12 && g_force_v < 12 + kAwqStreamConfigs)) && group > 0 && awq_stream_supported(M, N, K, group, ldx);
 }
@@ -765,10 +770,16 @@ inline bool stream_path(int64_t M, int64_t N, int64_t K, int64_t group, int64_t 
     if (!stream_supported(M, N, K, group, ldx)) return false;
     if (g_force_v != 0 || M > 64) return true;
     const double weights = (double)N * K;
-    if (awq_decode_supported(M, N, K, group)) return M > 16 && (weights >= 40e6 || weights <= 1.5e6);
-    if (bf16_io) return true;
-    if (decode_path(M, group)) return M > 24 || weights >= (M > 16 ? 30e6 : 150e6);
-    return M > 16 || weights >= 24e6;
+    if (awq_decode_supported(M, N, K, group)) return M > 16 && (weights >= 40e6 || (weights <= 1.5e6 && (K <= 1088 || 5 * N > 2 * K)));
+    const bool wide = weights >= 150e6 && N > 22000 && (N <= 33000 || N % 16 == 0);
+    if (bf16_io) return !(group == 128 && M <= 2 && wide);
+    if (!decode_path(M, group)) return M > 16 || weights >= 24e6;
+    if (M > 24) return K >= 8192 || weights > (M > 48 ? 6.5e6 : M > 32 ? 8e6 : 11e6) * (K < 1000 ? 1.4 : 1.0);
+    if (M > 16) return weights >= 30e6;
+    if (weights < 150e6 || wide) return false;
+    const DecodePlan d = make_decode_plan(M, N, K);
+    const int blocks = cdiv(N / 8, 16 * d.v) * d.splits;
+    return M > 6 || weights >= 210e6 || blocks <= 200 || blocks > 256;
 }
 // Searching a plan takes a few microseconds of host time and a call needs it for its workspace and for its launch, so each host thread
 // remembers the last plans it made (a pure function of sizes; a forced plan is not remembered).
@@ -1024,6 +1035,14 @@ extern "C" int llmq_awq_linear(const void* x, int x_dtype, int64_t ldx, const in
     if (x_dtype != LLMQ_BF16 && x_dtype != LLMQ_F16) return LLMQ_ERR_DTYPE;
     return awq_gemm_entry(x, ldx, qweight, scales, qzeros, bias, out, M, N, K, group, x_dtype == LLMQ_BF16, tickets, partials,
                           partials ? partials_bytes : 0, stream, true);
+}
+
+extern "C" int llmq_awq_planned_config(int x_dtype, int64_t M, int64_t N, int64_t K, int64_t group, int64_t ldx) {
+    if (!awq_sizes_ok(M, N, K) || K % kChunkK || N % 8 || group <= 0 || K % group || group % kChunkK) return LLMQ_ERR_SHAPE;
+    if (stream_path(M, N, K, group, ldx, x_dtype == LLMQ_BF16)) return 12 + stream_plan(M, N, K, group).cfg;
+    if (x_dtype == LLMQ_BF16 && !llmq_awq_gemm_bf16_supported(M, N, K, group)) return LLMQ_ERR_DTYPE;
+    if (tile_path(M)) return tile_plan(M, N, K).cfg == 0 ? 3 : tile_plan(M, N, K).cfg == 1 ? 4 : 7;
+    return decode16_path(M, N, K, group) ? 8 : 1;
 }
 
 extern "C" size_t llmq_awq_linear_partials_bytes(int x_dtype, int64_t M, int64_t N, int64_t K, int64_t group, int64_t ldx, int* counters) {

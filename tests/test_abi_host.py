@@ -88,8 +88,27 @@ def test_awq_linear_workspace(bf16, M, N, K, group, some, counters):
     assert need <= L.llmq_awq_gemm_partials_bytes(M, N, K, group)
 
 
+# (bf16, tokens, channels, K, group, kernel: s streaming tiles, f few-token, r register-streaming, t tiles): both sides of the lines between the kernels; group 128
+# with channels off the few-token kernel's grid of 32 among them
+@pytest.mark.parametrize("bf16,M,N,K,group,kernel", [
+    (0, 35, 3792, 768, 128, "r"), (0, 62, 3624, 1024, 128, "r"), (0, 29, 13576, 1024, 128, "s"), (1, 35, 3792, 768, 128, "s"), (0, 35, 3792, 768, 64, "s"),
+    (0, 1, 32776, 7424, 128, "r"), (0, 10, 31800, 7296, 128, "r"), (0, 10, 33800, 7296, 128, "s"), (0, 7, 33296, 7040, 128, "r"), (0, 5, 14088, 17408, 128, "s"), (0, 5, 11768, 17408, 128, "s"), (0, 1, 9904, 17792, 128, "r"),
+    (0, 8, 11768, 17408, 128, "s"), (0, 42, 616, 10624, 128, "s"), (0, 39, 9744, 896, 128, "r"), (1, 2, 36208, 7552, 128, None), (1, 3, 36208, 7552, 128, "s"), (0, 1, 32768, 7424, 128, "f"), (0, 18, 4992, 1024, 128, "f"), (0, 37, 896, 896, 128, "s"), (0, 60, 256, 3584, 128, "f"),
+    (0, 64, 37888, 3584, 128, "s"), (0, 65, 896, 896, 32, "s"), (0, 65, 896, 992, 32, "t"), (0, 8, 4096, 4096, 64, "r"), (0, 8, 8192, 4096, 64, "s")])
+def test_awq_lines(bf16, M, N, K, group, kernel):
+    from llmqrt_amd import _abi
+    L, dt = _abi.lib(), _abi.BF16 if bf16 else _abi.F16
+    cfg = L.llmq_awq_planned_config(dt, M, N, K, group, K)
+    if kernel is None:  # the module converts around the fp16 kernel
+        assert cfg == -2 and not L.llmq_awq_linear_bf16_supported(M, N, K, group, K)
+        return
+    assert kernel == ("s" if cfg >= 12 else "f" if cfg == 8 else "t" if cfg in (3, 4, 7) else "r" if cfg == 1 else "?"), cfg
+
+
 def test_planned_config_refuses():
     from llmqrt_amd import _abi
+    awq = _abi.lib().llmq_awq_planned_config
+    assert awq(_abi.F16, 4, 64, 100, 100, 100) == awq(_abi.F16, 4, 60, 128, 128, 128) == awq(_abi.F16, 0, 64, 128, 128, 128) == -3
     plan = _abi.lib().llmq_gemm_planned_config
     assert plan(0, 0, 64, 64) == plan(0, 4, 64, 40) == plan(1, 4, -1, 64) == -3
 
