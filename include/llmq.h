@@ -260,12 +260,15 @@ int llmq_linear_per_tensor_max_tokens(int64_t K);
  * in_scale: device scalar; out_scale: device scalar or null, then out is fp32 [M, N] and holds the out_dtype result after a round trip through
  * e4m3fn on it, as llmq_gemm_fp8_quantized_output gives it).  w_scale: [N] per token, one device scalar otherwise.  Codes and
  * scales are those of llmq_quant_*; fp32 sums may be added in another order than the separate GEMM's.  Up to 16 tokens and M * K <=
- * 81920, K % 16 == 0; more return LLMQ_ERR_SHAPE.  llmq_linear_one_launch_preferred: 1 where it was measured ahead of quantizer + GEMM. */
+ * 81920, K % 16 == 0; more return LLMQ_ERR_SHAPE.  llmq_linear_one_launch_ahead: 1 where it was measured ahead of quantizer + GEMM on the GPU, for
+ * calls that are captured; llmq_linear_one_launch_preferred: 1 also where it is not, but by less than the host takes to issue a second
+ * launch, for calls that a program issues one by one. */
 enum { LLMQ_LINEAR_I8_TOKEN = 0, LLMQ_LINEAR_FP8_TOKEN = 1, LLMQ_LINEAR_I8_TENSOR = 2, LLMQ_LINEAR_FP8_TENSOR = 3, LLMQ_LINEAR_FP8_STATIC = 4 };
 int llmq_linear_one_launch(int kind, const void* x, int x_dtype, int64_t ldx, const void* B, int64_t ldb, const float* w_scale,
                            const float* in_scale, const void* bias, int bias_dtype, const float* out_scale, void* out,
                            int out_dtype, int64_t ldo, int64_t M, int64_t N, int64_t K, llmq_stream_t stream);
 int llmq_linear_one_launch_preferred(int kind, int64_t M, int64_t N, int64_t K);
+int llmq_linear_one_launch_ahead(int kind, int64_t M, int64_t N, int64_t K);
 /* Tuning / test hook: 0 = two 16-channel tiles per wavefront x 4 wavefronts per block, 1 = one tile x 8 wavefronts,
  * -1 = built-in choice.  Per host thread (thread-local state): it affects only calls made later by the thread that set it. */
 int llmq_linear_dynamic_force_variant(int v);

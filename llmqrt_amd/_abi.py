@@ -56,6 +56,7 @@ SIGNATURES = {
     "llmq_linear_per_tensor_dynamic": (_int, [_int, _vp, _int, _i64, _vp, _i64, _vp, _vp, _int, _vp, _int, _i64, _i64, _i64, _i64, _vp]),
     "llmq_linear_one_launch": (_int, [_int, _vp, _int, _i64, _vp, _i64, _vp, _vp, _vp, _int, _vp, _vp, _int, _i64, _i64, _i64, _i64, _vp]),
     "llmq_linear_one_launch_preferred": (_int, [_int, _i64, _i64, _i64]),
+    "llmq_linear_one_launch_ahead": (_int, [_int, _i64, _i64, _i64]),
     "llmq_linear_per_tensor_max_tokens": (_int, [_i64]),
     "llmq_linear_dynamic_force_variant": (_int, [_int]),
     "llmq_gemm_fp8_quantized_output": (_int, [_vp, _int, _i64, _vp, _i64, _vp, _vp, _f32, _vp, _vp, _int, _f32, _vp, _vp, _int,

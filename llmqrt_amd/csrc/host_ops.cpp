@@ -78,7 +78,12 @@ struct Launch {
     llmq_stream_t stream;
     explicit Launch(const at::Device& dev) : guard(dev), stream(c10::hip::getCurrentHIPStream(dev.index()).stream()) {}
 };
-
+// Whether a linear runs in one launch: where that is ahead on the GPU, and where the saved launch is worth more to the host than it costs the
+// GPU, which no replayed graph gets back.  The current device is the stream's (Launch).
+bool one_launch(int kind, int64_t M, int64_t N, int64_t K) {
+    return llmq_linear_one_launch_preferred(kind, M, N, K) &&
+           (llmq_linear_one_launch_ahead(kind, M, N, K) || c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None);
+}
 
 // The weight side of an 8-bit Linear: [N, K] bytes, K % 16 == 0.
 bool weight_ok(const Tensor& w, at::ScalarType dtype, const at::Device& dev, int64_t K) {
@@ -131,7 +136,7 @@ std::optional<Tensor> sq_tensor(const Tensor& x, const Tensor& w, const Tensor& 
         return std::nullopt;
     const at::ScalarType odt = bias ? bias->scalar_type() : x.scalar_type();
     const Launch l(x.device());
-    if (llmq_linear_one_launch_preferred(LLMQ_LINEAR_I8_TENSOR, r.M, w.size(0), r.K)) {
+    if (one_launch(LLMQ_LINEAR_I8_TENSOR, r.M, w.size(0), r.K)) {
         Tensor out = make(out_size(x, w.size(0)), odt, x.device());
         check(llmq_linear_one_launch(LLMQ_LINEAR_I8_TENSOR, x.data_ptr(), code(x.scalar_type()), r.K, w.data_ptr(), r.K,
                                      (const float*)w_scale.data_ptr(), nullptr, ptr(bias), code(odt), nullptr, out.data_ptr(), code(odt),
@@ -156,7 +161,7 @@ std::optional<Tensor> sq_tensor(const Tensor& x, const Tensor& w, const Tensor& 
 // the measured lines decide.
 struct OneLaunch {
     int64_t tokens, k;
-    bool takes(int kind, const Rows& r, int64_t N) const { return r.M <= tokens && r.K < k && llmq_linear_one_launch_preferred(kind, r.M, N, r.K); }
+    bool takes(int kind, const Rows& r, int64_t N) const { return r.M <= tokens && r.K < k && one_launch(kind, r.M, N, r.K); }
 };
 
 std::optional<Tensor> sq_token(const Tensor& x, const Tensor& w, const Tensor& w_scale, const std::optional<Tensor>& bias,
@@ -249,7 +254,7 @@ std::optional<Tensor> fp8_tensor(const Tensor& x, const Tensor& w, const Tensor&
         return std::nullopt;
     const Launch l(x.device());
     const int kind = input_scale ? LLMQ_LINEAR_FP8_STATIC : LLMQ_LINEAR_FP8_TENSOR;
-    if ((input_scale || !output_scale) && llmq_linear_one_launch_preferred(kind, r.M, N, r.K)) {
+    if ((input_scale || !output_scale) && one_launch(kind, r.M, N, r.K)) {
         Tensor out = make(out_size(x, N), output_scale ? at::kFloat : odt, x.device());
         check(llmq_linear_one_launch(kind, x.data_ptr(), code(x.scalar_type()), r.K, w.data_ptr(), r.K, (const float*)w_scale.data_ptr(),
                                      input_scale ? (const float*)input_scale->data_ptr() : nullptr, ptr(bias), code(odt),

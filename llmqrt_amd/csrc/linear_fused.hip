@@ -22,7 +22,7 @@
 // which four multiply: 16 x 1152 x 896 6.2 / 5.5, 8 x 2304 x 2048 6.5 / 6.0, 16 x 896 x 4864 (two launches 13.7) - / 12.1).  With
 // more channels the blocks of a CU would repeat the quantizer, so a block takes as many wavefronts as its codes need and 16 or 32
 // channels (2 x 8448 x 1152 9.1 with two tiles a wavefront / 7.3, 7 x 15872 x 3840 two launches 24.1 / 16.8, 14336 codes: 16 x 9728 x 896 10.0 / 9.0).
-// Lines between one launch and two: llmq_linear_one_launch_preferred below.
+// Lines between one launch and two: llmq_linear_one_launch_preferred and _ahead below.
 #include <algorithm>
 #include <type_traits>
 
@@ -416,23 +416,40 @@ extern "C" int llmq_linear_fp8_dynamic(const void* x, int x_dtype, int64_t ldx, 
                        scale_dump, acc_dump, (hipStream_t)stream);
 }
 
-// One launch or two.  Measured on an MI355X against quantizer + GEMM (us, two launches / one; weights out of HBM, 630 random problems and the
-// sizes of decoder layers).  Two launches issued from a program's own loop take 10 us of the host against 6 for one, so the line is
-// where one launch stops being ahead of max(two launches, 10).  Per tensor a little further, as a decoder layer at these sizes is bound by the
-// host (10 x 896 x 4864 9.0 on the GPU in two / 10.9 in one, but the layer with its gate_up alike, 12 tokens, 41.7 / 35.4).  Up to 4096 channels it is as long as the codes are few (per tensor 9 x 3584 x
-// 3584 8.8 / 9.0 on the GPU, 15 x 3584 x 3584 8.9 / 11.0; static 4 x 3584 x 3584 7.4 / 7.1, 11 x 3584 x 3584 7.5 / 10.5; per token, a wavefront per
-// row, 2 x 3584 x 3584 8.1 / 7.7, 15 x 3584 x 3584 8.1 / 10.0), and beyond that where there are few channels.  With more channels each CU repeats the quantizer a
-// few times and the GEMM alone streams at 5-6 TB/s (per tensor 7 x 9728 x 896 8.9 / 7.4, 8 x 5168 x 7168 16.5 / 16.9, 3 x 27264 x 5120 31.4 /
-// 37.2; static 4 x 11744 x 1072 11.4 / 6.5, 13 x 13016 x 2432 13.3 / 15.4, 2 x 8320 x 10368 25.4 / 27.0), past 16384 channels too
-// often per token and with a static scale (per token 4 x 10752 x 7168 20.9 / 23.8, 4 x 37504 x 1408 17.0 / 22.8; static 4 x 19184 x 2432 12.2 / 16.1).
+// One launch or two.  Measured on an MI355X against quantizer + GEMM, in graphs, weights out of HBM, 4000 random problems of up to 16 tokens.
+//
+// On the GPU alone (llmq_linear_one_launch_ahead; us, two launches / one): one is ahead as long as the codes that every block makes are few for the
+// launch they save.  Per token, a wavefront per row: a short K (0.81 of the time up to 1888 elements), longer rows only with up to 24576 codes (8.1 /
+// 7.7 at 2 x 3584 x 3584, 8.1 / 10.0 at 15 x 3584 x 3584, 10.2 / 12.4 at 5 x 688 x 7936).  Per tensor up to 32768 codes (0.79 up to 18416, 0.95 up to 33000, 1.09-1.2 past
+// that: 8.3 / 11.6 at 14 x 416 x 4096, 9.0 / 12.3 at 16 x 896 x 4864), with a static scale up to 20480.  With more than 4096 channels each CU repeats
+// the quantizer and the GEMM alone streams at 5-6 TB/s, so few codes and short rows (8.9 / 7.4 at 7 x 9728 x 896; 19.4 / 23.4 at 2 x 8704 x 6464, 38.7 / 46.1
+// at 1 x 14200 x 13088), and past 16384 channels only where the GEMM has a ragged K (9.1 / 8.0 at 2 x 22368 x 400, 13.3 / 11.6 at 3 x 18064 x 1600; 12.2 / 18.2 at
+// 1 x 26176 x 1280).
+//
+// From a program's own loop (llmq_linear_one_launch_preferred) a second launch takes the host 4 us more, 10 instead of 6, and a decoder layer of small
+// projections waits for the host: one launch also where it costs the GPU less than that, up to 49152 codes and with up to 1024 channels all (a layer
+// of hidden size 896, 10 tokens: 34.5, with two launches for gate_up and down 42.3), but not for rows so long that the GPU takes more than 10 us either
+// way (14.1 / 16.0 at 2 x 312 x 17408, 15.0 / 17.5 at 2 x 1040 x 19456).  The larger of GPU and host time of the same problems is 1.0 % over that of the better choice.
 extern "C" int llmq_linear_one_launch_preferred(int kind, int64_t M, int64_t N, int64_t K) {
     if (!one_launch_fits(kind, M, N, K)) return 0;
     const int64_t codes = M * K;
-    if (kind == LLMQ_LINEAR_I8_TOKEN || kind == LLMQ_LINEAR_FP8_TOKEN)
-        return K < 8192 && (N <= kFewChannels ? M <= 4 || codes <= 49152 : M <= 4 && N <= 16384 && codes <= (N <= 8192 ? 14336 : 8192));
+    if (kind == LLMQ_LINEAR_I8_TOKEN || kind == LLMQ_LINEAR_FP8_TOKEN) {
+        if (K >= 8192) return 0;
+        if (N <= kFewChannels) return M <= 4 || (codes <= 49152 && K <= 6144);
+        if (N > 16384) return M >= 2 && M <= 4 && N <= 24576 && K % 128 != 0 && codes <= 4800;
+        return M <= 4 && codes <= (N <= 8192 ? 14336 : 8192);
+    }
     if (kind == LLMQ_LINEAR_FP8_STATIC) return N <= kFewChannels ? codes <= 32768 : codes <= 14336 && K < 8192 && N <= 16384;
-    if (N > kFewChannels) return codes <= 16384 ? N <= 16384 || codes <= 8192 : codes <= 28672 && K < 8192 && N <= 8192;
-    return codes <= 49152 || (M > 8 && N <= 1024);
+    if (N > kFewChannels) return codes <= 8192 || (K < 6144 && codes <= (N <= 8192 ? 28672 : 16384) && N <= 16384);
+    return K <= 5120 ? codes <= 49152 || N <= 1024 : codes <= 32768;
+}
+
+extern "C" int llmq_linear_one_launch_ahead(int kind, int64_t M, int64_t N, int64_t K) {
+    if (!llmq_linear_one_launch_preferred(kind, M, N, K)) return 0;
+    const int64_t codes = M * K;
+    if (kind == LLMQ_LINEAR_I8_TOKEN || kind == LLMQ_LINEAR_FP8_TOKEN) return K <= 1888 || (N <= kFewChannels && K <= 5824 && codes <= 24576);
+    if (kind == LLMQ_LINEAR_FP8_STATIC) return codes <= (N <= kFewChannels ? 20480 : 9216);
+    return codes <= 32768 && N <= 16384;
 }
 
 extern "C" int llmq_linear_one_launch(int kind, const void* x, int x_dtype, int64_t ldx, const void* B, int64_t ldb, const float* w_scale,

@@ -105,6 +105,31 @@ def test_awq_lines(bf16, M, N, K, group, kernel):
     assert kernel == ("s" if cfg >= 12 else "f" if cfg == 8 else "t" if cfg in (3, 4, 7) else "r" if cfg == 1 else "?"), cfg
 
 
+# kind (0 int8 per token, 1 fp8 per token, 2 int8 per tensor, 3 fp8 per tensor, 4 static), tokens, channels, K, one launch from a program's loop, in a graph
+@pytest.mark.parametrize("kind,M,N,K,loop,graph", [
+    (2, 16, 896, 4864, 1, 0), (3, 14, 416, 4096, 1, 0), (3, 10, 896, 3072, 1, 1), (2, 9, 232, 6160, 0, 0), (2, 2, 312, 17408, 0, 0), (2, 1, 3584, 18944, 1, 1),
+    (3, 8, 896, 8192, 0, 0), (3, 9, 896, 8192, 0, 0), (2, 1, 3584, 3584, 1, 1), (2, 1, 37888, 3584, 1, 0), (3, 2, 8704, 6464, 0, 0), (3, 1, 14200, 13088, 0, 0),
+    (3, 16, 9728, 896, 1, 1), (0, 5, 688, 7936, 0, 0), (0, 5, 688, 1600, 1, 1), (1, 10, 3584, 3584, 1, 0), (1, 2, 3584, 3584, 1, 1), (0, 4, 3584, 7936, 1, 0),
+    (0, 2, 22368, 400, 1, 1), (0, 3, 18064, 1600, 1, 1), (0, 2, 22368, 384, 0, 0), (1, 4, 37504, 1408, 0, 0), (4, 8, 3584, 3584, 1, 0), (4, 4, 3584, 3584, 1, 1),
+    (4, 17, 64, 64, 0, 0), (5, 1, 64, 64, 0, 0)])
+def test_one_launch_lines(kind, M, N, K, loop, graph):
+    from llmqrt_amd import _abi
+    L = _abi.lib()
+    assert (L.llmq_linear_one_launch_preferred(kind, M, N, K), L.llmq_linear_one_launch_ahead(kind, M, N, K)) == (loop, graph)
+
+
+@pytest.mark.parametrize("kind", range(5))
+def test_one_launch_lines_have_no_holes(kind):
+    """More tokens of the same sizes make more codes for every block: a size that takes two launches takes two with more tokens as well."""
+    from llmqrt_amd import _abi
+    L = _abi.lib()
+    for line in (L.llmq_linear_one_launch_preferred, L.llmq_linear_one_launch_ahead):
+        for N in (64, 896, 1024, 1032, 3584, 4096, 4104, 8192, 9728, 16384, 37888):
+            for K in (64, 896, 1888, 1904, 3584, 4864, 5120, 5136, 6144, 8192, 18944):
+                taken = [line(kind, M, N, K) for M in range(1, 18)]
+                assert taken == sorted(taken, reverse=True), (N, K, taken)
+
+
 def test_planned_config_refuses():
     from llmqrt_amd import _abi
     awq = _abi.lib().llmq_awq_planned_config

@@ -298,3 +298,48 @@ def test_native_forward_from_threads(cuda):
     done.set()
     releaser.join(10)
     assert not wrong and not any(t.is_alive() for t in threads + [releaser])
+
+
+# 16 x 896 x 4864 and 14 x 416 x 4096 run in one launch from a program's loop and in two inside a graph, where no host waits for the second
+@pytest.mark.parametrize("M,n,k", [(16, 896, 4864), (14, 416, 4096), (16, 3584, 2304)])
+@pytest.mark.parametrize("name", ["sq", "fp8", "sq_channel", "fp8_token", "static", "static_out"])
+def test_captured_forward_follows_the_gpu(cuda, M, n, k, name):
+    """int8 results are the eager ones bit for bit; fp8 sums may be added in another order (twice K 2^-24 of the sum of absolute products, a step of the output type).
+    Every replay equals the first, with eager calls between them."""
+    from llmqrt_amd.linear import FP8DynamicLinear, FP8StaticLinear, SqW8A8BBF16OBF16PerChannel, SqW8A8BBF16OBF16PerTensor
+    g = torch.Generator(device="cuda").manual_seed(n)
+    lin = torch.nn.Linear(k, n, bias=False, device="cuda")
+    lin.weight.data = 0.02 * torch.randn(n, k, device="cuda", generator=g)
+    if name.startswith("sq"):
+        mod = (SqW8A8BBF16OBF16PerTensor if name == "sq" else SqW8A8BBF16OBF16PerChannel).from_linear(lin, 8, 0, False, dtype=torch.bfloat16)
+    elif name.startswith("static"):
+        mod = FP8StaticLinear.from_linear(lin, init_only=False, dtype=torch.bfloat16, quantize_output=name == "static_out")
+        mod.input_scale.data.fill_(0.02)
+        mod.output_scale.data.fill_(0.02)
+    else:
+        mod = FP8DynamicLinear.from_linear(lin, init_only=False, dtype=torch.bfloat16, per_tensor=name == "fp8")
+    x = torch.randn(M, 1, k, device=cuda, generator=g).bfloat16()
+    eager = mod(x)
+    st = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        before = _allocations()
+        y = mod(x)
+        made = _allocations() - before
+    if name in ("sq", "fp8") and n < 1024:
+        assert made == 2  # the output, and the codes of a separate quantizer
+    graph.replay()
+    torch.cuda.synchronize()
+    first = y.clone()
+    if name.startswith("sq"):
+        assert torch.equal(first, eager)
+    else:
+        mag = x.double().abs() @ (mod._qweight().double() * mod.weight_scale.double().reshape(-1, 1)).abs().t()
+        tol = (2 * k * 2.0 ** -24 + 2.0 ** -12) * mag + 2.0 ** -8 * eager.double().abs() + (eager.double().abs() / 8 + 0.02 * 2.0 ** -9 if name == "static_out" else 0)
+        assert bool(((first.double() - eager.double()).abs() <= tol).all())
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        again = mod(x)
+        torch.cuda.synchronize()
+        assert torch.equal(y, first) and torch.equal(again, eager)
