@@ -235,9 +235,9 @@ size_t llmq_gemm_f16_workspace_bytes(int64_t M, int64_t N, int64_t K);
  * fit in 64 KB of LDS: 3 at K = 18944).  Replaces the two steps of
  * SqW8A8BBF16OBF16PerChannel.forward / the per-token branch of FP8DynamicLinear.forward
  * (nn_models/modules/linear/linear_sq.py:97-138 with the quantizer of lines 55-65;
- * nn_models/modules/linear/linear_fp8.py:40-63 and 199-221) and gives, bit for bit, what
- * llmq_quant_i8_per_token (llmq_quant_fp8_per_token) followed by llmq_gemm_w8a8 (llmq_gemm_fp8) with a_scale = the
- * quantizer's scales, alpha = beta = 1 gives:
+ * nn_models/modules/linear/linear_fp8.py:40-63 and 199-221): llmq_quant_i8_per_token (llmq_quant_fp8_per_token) followed by
+ * llmq_gemm_w8a8 (llmq_gemm_fp8) with a_scale = the quantizer's scales, alpha = beta = 1.  Codes and scales are those of the two calls bit for
+ * bit, and so are int8 results; the fp32 sums of fp8 may be added in another order than the GEMM's, whose order depends on its plan:
  *   out[m, n] = out_dtype( ((sum_k q[m, k] B[n, k]) * s[m]) * w_scale[n] + bias[n] ).
  * x: bf16 / f16 [M, K], row stride ldx (K % 16 == 0, ldx % 8 == 0); B: int8 / e4m3 [N, K], row stride ldb; w_scale: [N]
  * or null; bias: [N] or null; out: bf16 / f16 [M, N].  Optional outputs for checking: q_dump [M, K] (the codes),

@@ -126,6 +126,14 @@ def stream_of(t: torch.Tensor) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
+def capturing(device: torch.device) -> bool:
+    """Whether the current stream of `device` is being captured into a graph."""
+    if device.index == torch.cuda.current_device():
+        return torch.cuda.is_current_stream_capturing()
+    with torch.cuda.device(device):
+        return torch.cuda.is_current_stream_capturing()
+
+
 class _Workspaces:
     """One grow-only scratch tensor per (device, stream): the C library never allocates.  Under capture every call gets
     memory of the graph instead: an eager call's buffer may be replaced by a larger one while the graph still replays on
@@ -139,17 +147,10 @@ class _Workspaces:
     def release(self):
         self._buf.clear()
 
-    @staticmethod
-    def _capturing(device: torch.device) -> bool:
-        if device.index == torch.cuda.current_device():
-            return torch.cuda.is_current_stream_capturing()
-        with torch.cuda.device(device):
-            return torch.cuda.is_current_stream_capturing()
-
     def get(self, device: torch.device, nbytes: int) -> torch.Tensor | None:
         if nbytes == 0:
             return None
-        if self._capturing(device):
+        if capturing(device):
             return torch.empty(nbytes, dtype=torch.uint8, device=device)
         key = (device.index, torch.cuda.current_stream(device).cuda_stream)
         buf = self._buf.get(key)

@@ -157,15 +157,7 @@ std::optional<Tensor> sq_tensor(const Tensor& x, const Tensor& w, const Tensor& 
     return out;
 }
 
-// The module sets the widest range in which a per-token linear may run in one launch (up to `tokens` rows of fewer than `k` elements); inside it
-// the measured lines decide.
-struct OneLaunch {
-    int64_t tokens, k;
-    bool takes(int kind, const Rows& r, int64_t N) const { return r.M <= tokens && r.K < k && one_launch(kind, r.M, N, r.K); }
-};
-
-std::optional<Tensor> sq_token(const Tensor& x, const Tensor& w, const Tensor& w_scale, const std::optional<Tensor>& bias,
-                               const OneLaunch& line) {
+std::optional<Tensor> sq_token(const Tensor& x, const Tensor& w, const Tensor& w_scale, const std::optional<Tensor>& bias) {
     const Rows r = rows_of(x);
     if (!r.ok || !is16(x.scalar_type()) || !weight_ok(w, at::kChar, x.device(), r.K)) return std::nullopt;
     const int64_t N = w.size(0);
@@ -175,7 +167,7 @@ std::optional<Tensor> sq_token(const Tensor& x, const Tensor& w, const Tensor& w
     const Launch l(x.device());
     const float* ws = (const float*)w_scale.data_ptr();
     Tensor out = make(out_size(x, N), odt, x.device());
-    if (line.takes(LLMQ_LINEAR_I8_TOKEN, r, N)) {
+    if (one_launch(LLMQ_LINEAR_I8_TOKEN, r.M, N, r.K)) {
         check(llmq_linear_one_launch(LLMQ_LINEAR_I8_TOKEN, x.data_ptr(), code(x.scalar_type()), r.K, w.data_ptr(), r.K, ws, nullptr, ptr(bias),
                                      code(odt), nullptr, out.data_ptr(), code(odt), N, r.M, N, r.K, l.stream),
               "llmq_linear_one_launch");
@@ -213,8 +205,7 @@ std::optional<Tensor> prequantized(bool fp8, const Tensor& q, const Tensor& a_sc
 }
 
 // ---- FP8 (e4m3fn) ----------------------------------------------------------------------------------------------
-std::optional<Tensor> fp8_token(const Tensor& x, const Tensor& w, const Tensor& w_scale, const std::optional<Tensor>& bias,
-                                const OneLaunch& line) {
+std::optional<Tensor> fp8_token(const Tensor& x, const Tensor& w, const Tensor& w_scale, const std::optional<Tensor>& bias) {
     const Rows r = rows_of(x);
     if (!r.ok || !is16(x.scalar_type()) || !weight_ok(w, at::kFloat8_e4m3fn, x.device(), r.K)) return std::nullopt;
     const int64_t N = w.size(0);
@@ -224,7 +215,7 @@ std::optional<Tensor> fp8_token(const Tensor& x, const Tensor& w, const Tensor& 
     const Launch l(x.device());
     const float* ws = (const float*)w_scale.data_ptr();
     Tensor out = make(out_size(x, N), at::kBFloat16, x.device());
-    if (line.takes(LLMQ_LINEAR_FP8_TOKEN, r, N)) {
+    if (one_launch(LLMQ_LINEAR_FP8_TOKEN, r.M, N, r.K)) {
         check(llmq_linear_one_launch(LLMQ_LINEAR_FP8_TOKEN, x.data_ptr(), code(x.scalar_type()), r.K, w.data_ptr(), r.K, ws, nullptr, ptr(bias),
                                      bias ? code(bias->scalar_type()) : LLMQ_BF16, nullptr, out.data_ptr(), LLMQ_BF16, N, r.M, N, r.K,
                                      l.stream),
@@ -496,14 +487,12 @@ LLMQ_PY(py_sq_tensor, 5)
     return wrap(std::move(y));
 LLMQ_PY_END
 
-LLMQ_PY(py_sq_token, 6)
+LLMQ_PY(py_sq_token, 4)
     const Tensor &x = in.tensor(0), &w = in.tensor(1), &s = in.tensor(2);
     const auto bias = in.optional(3);
     LLMQ_PY_TENSORS;
-    const OneLaunch line{PyLong_AsLongLong(argv[4]), PyLong_AsLongLong(argv[5])};
-    if (PyErr_Occurred()) return nullptr;
     std::optional<Tensor> y;
-    { NoGil g; y = sq_token(x, w, s, bias, line); }
+    { NoGil g; y = sq_token(x, w, s, bias); }
     return wrap(std::move(y));
 LLMQ_PY_END
 
@@ -526,14 +515,12 @@ LLMQ_PY(py_fp8_prequantized, 5)
     return wrap(std::move(y));
 LLMQ_PY_END
 
-LLMQ_PY(py_fp8_token, 6)
+LLMQ_PY(py_fp8_token, 4)
     const Tensor &x = in.tensor(0), &w = in.tensor(1), &s = in.tensor(2);
     const auto bias = in.optional(3);
     LLMQ_PY_TENSORS;
-    const OneLaunch line{PyLong_AsLongLong(argv[4]), PyLong_AsLongLong(argv[5])};
-    if (PyErr_Occurred()) return nullptr;
     std::optional<Tensor> y;
-    { NoGil g; y = fp8_token(x, w, s, bias, line); }
+    { NoGil g; y = fp8_token(x, w, s, bias); }
     return wrap(std::move(y));
 LLMQ_PY_END
 

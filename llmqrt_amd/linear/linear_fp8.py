@@ -14,11 +14,9 @@ import torch
 from .._native import host
 from ..quantize import (per_tensor_quantize, per_tensor_quantize_with_alpha, per_token_quantize, static_per_tensor_quantize,
                         static_per_tensor_quantize_with_alpha)
-from ..sq_fp8_kernels import (cutlass_f8f8bf16_rowwise_sm89, cutlass_f8f8bf16_tensorwise_sm89,
-                              dynamic_linear_max_tokens, f8f8_tensorwise_quantized_output,
-                              f8f8bf16_linear_dynamic_per_token)
+from ..sq_fp8_kernels import (FP8_STATIC, FP8_TENSOR, FP8_TOKEN, cutlass_f8f8bf16_rowwise_sm89, cutlass_f8f8bf16_tensorwise_sm89,
+                              f8f8_tensorwise_quantized_output, one_launch_linear)
 from .linear_base import LinearBase
-from .linear_sq import ONE_LAUNCH_K, ONE_LAUNCH_MAX_TOKENS, ONE_LAUNCH_TOKENS, _fusable
 
 __all__ = ["FP8DynamicLinear", "FP8StaticLinear", "per_tensor_quantize", "per_token_quantize",
            "static_per_tensor_quantize"]
@@ -121,7 +119,7 @@ class FP8DynamicLinear(_FP8LinearBase):
             y = host().fp8_tensor(x, self._qweight(), self._parameters.get("weight_scale"), self._bias_param(), self.dtype,
                                   None, None)
         else:
-            y = host().fp8_token(x, self._qweight(), self._wscale_flat(), self._bias_param(), ONE_LAUNCH_TOKENS, ONE_LAUNCH_K)
+            y = host().fp8_token(x, self._qweight(), self._wscale_flat(), self._bias_param())
         return self._forward_general(x) if y is None else y
 
     @torch.no_grad()
@@ -133,17 +131,19 @@ class FP8DynamicLinear(_FP8LinearBase):
         if x.shape[0] == 0:
             return torch.zeros(out_shape, dtype=x.dtype, device=x.device)
         qweight = self._qweight_t()
+        x2 = x.reshape(-1, x_shape[-1])
+        # per tensor, strided rows: what contiguous rows of these values run natively, bit for bit
+        if not self.per_tensor or not x.is_contiguous():
+            output = one_launch_linear(FP8_TENSOR if self.per_tensor else FP8_TOKEN, x2, self._qweight(),
+                                       self.weight_scale if self.per_tensor else self._wscale_flat(), self.bias,
+                                       self.dtype if self.per_tensor else torch.bfloat16)
+            if output is not None:
+                return output.view(*x_shape[:-1], -1)
         if self.per_tensor:
             qinput, alpha = per_tensor_quantize_with_alpha(x, self.weight_scale, fp8=True)
             output = cutlass_f8f8bf16_tensorwise_sm89(qinput.view(-1, x_shape[-1]), qweight, self.bias, alpha, 1.0,
                                                       dtype_to_str.get(self.dtype))
         else:
-            x2 = x.reshape(-1, x_shape[-1])
-            if (self.qdtype == torch.float8_e4m3fn and _fusable(x2)
-                    and x2.shape[0] <= min(ONE_LAUNCH_MAX_TOKENS, dynamic_linear_max_tokens(x2.shape[-1]))):
-                # a few tokens: quantizer and GEMM in one launch (same bits as the two calls below)
-                output = f8f8bf16_linear_dynamic_per_token(x2, qweight, self.bias, self._wscale_flat())
-                return output.view(*x_shape[:-1], -1)
             qinput, x_scale = per_token_quantize(x)
             output = cutlass_f8f8bf16_rowwise_sm89(qinput.view(-1, x_shape[-1]), qweight, self.bias,
                                                    x_scale.view(-1, 1), self.weight_scale.to(torch.float32).t(), True)
@@ -208,6 +208,11 @@ class FP8StaticLinear(_FP8LinearBase):
         if x.shape[0] == 0:
             return torch.zeros(out_shape, dtype=x.dtype, device=x.device)
         assert self.per_tensor, "[error!!] static activation quant only support per tensor!"
+        if not x.is_contiguous():  # what contiguous rows of these values run natively, bit for bit
+            output = one_launch_linear(FP8_STATIC, x.reshape(-1, x_shape[-1]), self._qweight(), self.weight_scale, self.bias, self.dtype,
+                                       self.input_scale, self.output_scale if self.quantize_output else None)
+            if output is not None:
+                return output.view(*x_shape[:-1], -1)
         qinput, alpha = static_per_tensor_quantize_with_alpha(x, self.input_scale, self.weight_scale)
         if self.quantize_output:
             # output / output_scale -> e4m3fn -> * output_scale (linear_fp8.py:309-311) inside the GEMM epilogue:

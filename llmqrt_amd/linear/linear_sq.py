@@ -16,27 +16,12 @@ from .._native import host
 from ..quantize import (per_tensor_quantize_with_alpha, quantize_activation_per_tensor_absmax,
                         quantize_activation_per_token_absmax, quantize_activation_per_token_absmax_f32,
                         quantize_weight_per_channel_absmax)
-from ..sq_fp8_kernels import (dynamic_linear_max_tokens, w8a8_int8_linear_bbf16_obf16_per_channel,
-                              w8a8_int8_linear_bbf16_obf16_per_tensor, w8a8_int8_linear_dynamic_per_token)
+from ..sq_fp8_kernels import (I8_TENSOR, I8_TOKEN, one_launch_linear, w8a8_int8_linear_bbf16_obf16_per_channel,
+                              w8a8_int8_linear_bbf16_obf16_per_tensor)
 from .linear_base import LinearBase
 
 __all__ = ["SqW8A8BBF16OBF16PerTensor", "SqW8A8BBF16OBF16PerChannel",
            "quantize_activation_per_tensor_absmax", "quantize_activation_per_token_absmax"]
-
-
-# The widest range in which a per-token linear runs in one launch: up to ONE_LAUNCH_TOKENS rows shorter than ONE_LAUNCH_K.  Inside it the native
-# forwards follow the measured lines of llmq_linear_one_launch_preferred, the general path (strided rows) stays with the number of tokens up to
-# which one launch is at least level for any number of channels.
-ONE_LAUNCH_TOKENS = 16
-ONE_LAUNCH_MAX_TOKENS = 4
-ONE_LAUNCH_K = 8192
-
-
-def _fusable(x2: torch.Tensor) -> bool:
-    """Layout the one-launch linear takes: 16-bit activations, contiguous rows, K % 16 == 0, 16-byte aligned."""
-    return (x2.is_cuda and x2.dtype in (torch.bfloat16, torch.float16) and x2.stride(-1) == 1 and x2.shape[-1] % 16 == 0
-            and x2.shape[-1] < ONE_LAUNCH_K
-            and x2.stride(0) % 8 == 0 and x2.data_ptr() % 16 == 0)
 
 
 class SqW8A8BBF16OBF16PerTensor(LinearBase):
@@ -81,6 +66,10 @@ class SqW8A8BBF16OBF16PerTensor(LinearBase):
         assert self.input_scale.device == self.qweight.device, "when sq linear fwd, scale and qweight must be same device!"
         x_shape = x.shape
         x2 = x.reshape(-1, x_shape[-1])
+        if not x.is_contiguous():  # what contiguous rows of these values run natively, bit for bit
+            y = one_launch_linear(I8_TENSOR, x2, self.qweight, self.weight_scale, self.bias, x.dtype if self.bias is None else self.bias.dtype)
+            if y is not None:
+                return y.view(*x_shape[:-1], -1)
         # alpha stays on the device: the quantizer forms the product, rounded to the activation dtype as the
         # reference's `input_scale * weight_scale.item()` is, and the GEMM reads it
         qx, alpha = per_tensor_quantize_with_alpha(x2, self.weight_scale, fp8=False)
@@ -129,8 +118,7 @@ class SqW8A8BBF16OBF16PerChannel(LinearBase):
 
     def forward(self, x):
         b = self._buffers
-        y = host().sq_token(x, b.get("qweight"), b.get("weight_scale"), b["bias"] if "bias" in b else self.bias,
-                            ONE_LAUNCH_TOKENS, ONE_LAUNCH_K)
+        y = host().sq_token(x, b.get("qweight"), b.get("weight_scale"), b["bias"] if "bias" in b else self.bias)
         return self._forward_general(x) if y is None else y
 
     @torch.no_grad()
@@ -139,10 +127,8 @@ class SqW8A8BBF16OBF16PerChannel(LinearBase):
         assert self.weight_scale.device == self.qweight.device, "when sq linear fwd, scale and qweight must be same device!"
         x_shape = x.shape
         x2 = x.reshape(-1, x_shape[-1])
-        if 0 < x2.shape[0] <= min(ONE_LAUNCH_MAX_TOKENS, dynamic_linear_max_tokens(x2.shape[-1])) and _fusable(x2):
-            # a few tokens: quantizer and GEMM in one launch (same bits as the two calls below)
-            y = w8a8_int8_linear_dynamic_per_token(x2, self.qweight.t(), self._bias_or_zeros(x.dtype, x.device),
-                                                   self.weight_scale)
+        y = one_launch_linear(I8_TOKEN, x2, self.qweight, self.weight_scale, self.bias, x.dtype if self.bias is None else self.bias.dtype)
+        if y is not None:
             return y.view(*x_shape[:-1], -1)
         qx, input_scale = quantize_activation_per_token_absmax_f32(x2)
         y = w8a8_int8_linear_bbf16_obf16_per_channel(qx, self.qweight.t(), self._bias_or_zeros(x.dtype, x.device),

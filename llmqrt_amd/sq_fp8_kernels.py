@@ -223,7 +223,7 @@ def _run_dynamic(fp8: bool, x, w, bias, w_scale, out_dtype, q_dump, scale_dump, 
 def w8a8_int8_linear_dynamic_per_token(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, w_scale: torch.Tensor,
                                        *, _q_dump=None, _scale_dump=None, _acc_dump=None) -> torch.Tensor:
     """quantize_activation_per_token_absmax (linear_sq.py:55-65) + w8a8_int8_linear_bbf16_obf16_per_channel in one
-    launch, for up to dynamic_linear_max_tokens(K) tokens; bit-identical to the two calls.  ``x``: bf16 / fp16 [M, K];
+    launch, for up to dynamic_linear_max_tokens(K) tokens; the same bits as the two calls.  ``x``: bf16 / fp16 [M, K];
     ``weight``: int8 [K, N] view of an [N, K] row-major tensor; ``bias``: [N], its dtype is the output dtype."""
     what = "w8a8_int8_linear_dynamic_per_token"
     _check(weight.dtype == torch.int8, f"{what}: weight must be int8")
@@ -237,8 +237,45 @@ def f8f8bf16_linear_dynamic_per_token(x: torch.Tensor, WQ: torch.Tensor, bias: O
                                       w_scale: torch.Tensor, *, _q_dump=None, _scale_dump=None,
                                       _acc_dump=None) -> torch.Tensor:
     """per_token_quantize (linear_fp8.py:40-63) + cutlass_f8f8bf16_rowwise_sm89 in one launch, for up to
-    dynamic_linear_max_tokens(K) tokens; bit-identical to the two calls.  Output bf16."""
+    dynamic_linear_max_tokens(K) tokens.  Codes and scales are those of the two calls; the fp32 sums over K may be added in another
+    order than the GEMM's, which depends on its plan.  Output bf16."""
     what = "f8f8bf16_linear_dynamic_per_token"
     _check(WQ.dtype == torch.float8_e4m3fn, f"{what}: WQ must be float8_e4m3fn")
     _check_bias(bias, WQ, WQ.size(1), (torch.bfloat16, torch.float32), what)
     return _run_dynamic(True, x, WQ, bias, w_scale, torch.bfloat16, _q_dump, _scale_dump, _acc_dump, what)
+
+
+# kinds of llmq_linear_one_launch
+I8_TOKEN, FP8_TOKEN, I8_TENSOR, FP8_TENSOR, FP8_STATIC = range(5)
+
+
+@torch.no_grad()
+def one_launch_linear(kind: int, x: torch.Tensor, w: torch.Tensor, w_scale, bias, out_dtype: torch.dtype, in_scale=None,
+                      out_scale=None) -> Optional[torch.Tensor]:
+    """A quantized linear of a few tokens (``x`` [M, K], rows any multiple of 16 bytes apart; ``w`` [N, K]) in the one launch that the native forwards
+    use for these sizes, by the same rule; None where the rule says two launches or the tensors are not the kernel's."""
+    M, K = x.shape
+    N = w.shape[0]
+    L, dev = _abi.lib(), x.device
+
+    def values(t, n):
+        return t.dtype == torch.float32 and t.numel() == n and t.device == dev and t.is_contiguous()
+    halves = (torch.bfloat16, torch.float16)
+    if not (x.is_cuda and x.dtype in halves and out_dtype in halves and x.data_ptr() % 16 == 0
+            and (M == 1 or (x.stride(0) % 8 == 0 and K <= x.stride(0) < 1 << 22)) and x.stride(1) == 1
+            and L.llmq_linear_one_launch_preferred(kind, M, N, K)
+            and (L.llmq_linear_one_launch_ahead(kind, M, N, K) or not _abi.capturing(dev))):
+        return None
+    fp8 = kind not in (I8_TOKEN, I8_TENSOR)
+    if not (w.dtype == (torch.float8_e4m3fn if fp8 else torch.int8) and w.shape[1] == K and w.device == dev and w.is_contiguous()
+            and w.data_ptr() % 16 == 0 and values(w_scale, N if kind in (I8_TOKEN, FP8_TOKEN) else 1)
+            and (bias is None or (bias.dim() == 1 and bias.numel() == N and bias.device == dev and bias.is_contiguous()
+                                  and bias.dtype in ((torch.bfloat16, torch.float32) if kind == FP8_TOKEN else (out_dtype,))))
+            and (in_scale is None or (values(in_scale, 1) and in_scale.dim() > 0)) and (out_scale is None or values(out_scale, 1))):
+        return None
+    out = torch.empty((M, N), dtype=out_dtype if out_scale is None else torch.float32, device=dev)
+    dt = _abi.dtype_code(out_dtype)
+    _abi.check(L.llmq_linear_one_launch(kind, x.data_ptr(), _abi.dtype_code(x.dtype), K if M == 1 else x.stride(0), w.data_ptr(), K, w_scale.data_ptr(),
+                                        _abi.ptr(in_scale), _abi.ptr(bias), dt if bias is None else _abi.dtype_code(bias.dtype), _abi.ptr(out_scale),
+                                        out.data_ptr(), dt, N, M, N, K, _abi.stream_of(x)), "llmq_linear_one_launch")
+    return out

@@ -109,7 +109,7 @@ def test_dynamic_linear_rejects_more_tokens_and_bad_layout(cuda):
 
 @pytest.mark.parametrize("tokens", [1, 4, 5])
 def test_modules_take_the_one_launch_path_with_identical_results(cuda, tokens):
-    """SqW8A8BBF16OBF16PerChannel and FP8DynamicLinear (per token) switch to the one-launch kernel up to 4 tokens:
+    """SqW8A8BBF16OBF16PerChannel and FP8DynamicLinear (per token) run these tokens in one launch and 17 in two:
     the result must not depend on which side of the switch a batch falls (rows of a 17-token batch = the same rows
     computed alone)."""
     from llmqrt_amd.linear import FP8DynamicLinear, SqW8A8BBF16OBF16PerChannel
@@ -118,14 +118,14 @@ def test_modules_take_the_one_launch_path_with_identical_results(cuda, tokens):
     x = torch.randn(17, 512, device=cuda).to(torch.bfloat16)
     sq = SqW8A8BBF16OBF16PerChannel.from_linear(dense, 8, 0, init_only=False, dtype=torch.bfloat16)
     f8 = FP8DynamicLinear.from_linear(dense, init_only=False, dtype=torch.bfloat16, per_tensor=False)
-    full, part = sq(x), sq(x[:tokens])    # 17 tokens: quantizer + GEMM; up to 4: one launch
+    full, part = sq(x), sq(x[:tokens])    # 17 tokens: quantizer + GEMM; up to 5: one launch
     assert torch.equal(part, full[:tokens])   # int32 accumulation is exact, the epilogue arithmetic is shared
     full, part = f8(x), f8(x[:tokens])    # fp32 accumulation: the two kernels add in different orders
     assert ((part.float() - full[:tokens].float()).abs().max() / full.float().abs().max()).item() <= 1e-2
 
 
-# One launch with a tensor-wide scale (M * K <= 16384): one token, the most tokens of a K, rows past the MFMA's 16-byte steps,
-# one channel tile / two / ragged N; one token more runs as quantizer + GEMM.  int8: the same bits as quantizer + GEMM; fp8: fp32
+# One launch with a tensor-wide scale, native, against quantizer + GEMM, the general path of contiguous rows: one token, several, rows past the MFMA's 16-byte
+# steps, one channel tile / two / ragged N; 2 x 4104 x 8192 takes two launches either way.  int8: the same bits as quantizer + GEMM; fp8: fp32
 # sums of the same products, in another order where the GEMM is the tile kernel, then one rounding: a bf16 step is 2^-8.
 @pytest.mark.parametrize("M,N,K", [(1, 3584, 3584), (4, 3584, 3584), (5, 3584, 3584), (16, 896, 896), (16, 1000, 1024), (2, 4104, 8192),
                                    (1, 520, 16384), (3, 9728, 912), (1, 5000, 2064), (16, 24, 16)])
@@ -228,3 +228,97 @@ def test_one_launch_refuses(cuda):
     assert rc(2, 0, 64) == 0 and int(out.count_nonzero()) == 0
     for kind in range(5):
         assert L.llmq_linear_one_launch_preferred(kind, 17, 64, 64) == 0 == L.llmq_linear_one_launch_preferred(kind, 1, 64, 40)
+
+
+def _modules(N, K, dtype, bias, cuda):
+    from llmqrt_amd.linear import FP8DynamicLinear, FP8StaticLinear, SqW8A8BBF16OBF16PerChannel, SqW8A8BBF16OBF16PerTensor
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    lin = torch.nn.Linear(K, N, bias=bias, device="cuda")
+    lin.weight.data = 0.02 * torch.randn(N, K, device="cuda", generator=g)
+    if bias:
+        lin.bias.data = torch.randn(N, device="cuda", generator=g)
+    mods = {"sq": SqW8A8BBF16OBF16PerTensor.from_linear(lin, 8, 0, False, dtype=dtype),
+            "sq_channel": SqW8A8BBF16OBF16PerChannel.from_linear(lin, 8, 0, False, dtype=dtype),
+            "fp8": FP8DynamicLinear.from_linear(lin, init_only=False, dtype=dtype)}
+    if dtype == torch.bfloat16:
+        mods["fp8_token"] = FP8DynamicLinear.from_linear(lin, init_only=False, dtype=dtype, per_tensor=False)
+    for name, quantized in (("static", False), ("static_out", True)):
+        m = mods[name] = FP8StaticLinear.from_linear(lin, init_only=False, dtype=dtype, quantize_output=quantized)
+        m.input_scale.data.fill_(0.03)
+        m.output_scale.data.fill_(0.05)
+    return mods
+
+
+# one launch and two by every rule: few and many codes, up to 4096 channels and past them, more than 4 tokens, a ragged K, a K past 8192
+@pytest.mark.parametrize("M,N,K", [(3, 896, 3584), (10, 3072, 3008), (16, 896, 4864), (8, 3584, 3584), (16, 9728, 896), (4, 20488, 1040), (2, 520, 12288), (13, 512, 2064)])
+@pytest.mark.parametrize("dtype,bias", [(torch.bfloat16, True), (torch.float16, False)])
+def test_strided_rows_give_the_bits_of_contiguous_ones(cuda, M, N, K, dtype, bias):
+    """The same values in rows that are further apart (and start 16 bytes into the buffer) run the same kernels as contiguous ones, eager and captured."""
+    wide = torch.zeros(M, 1, K + 24, dtype=dtype, device=cuda)
+    wide[..., 8:8 + K] = (torch.randn(M, 1, K, device=cuda, generator=torch.Generator(device="cuda").manual_seed(M)) * 2).to(dtype)
+    strided = wide[..., 8:8 + K]
+    x = strided.contiguous()
+    for name, mod in _modules(N, K, dtype, bias, cuda).items():
+        want = mod(x)
+        got = mod(strided)
+        assert got.dtype == want.dtype and got.shape == want.shape and torch.equal(got, want), name
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            a, b = mod(x), mod(strided)
+        for _ in range(2):
+            graph.replay()
+            mod(strided)
+            torch.cuda.synchronize()
+            assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 896, 3584), (10, 3072, 3008), (16, 896, 4864), (16, 9728, 896), (4, 37504, 1408)])
+def test_strided_rows_take_the_launch_of_contiguous_ones(cuda, M, N, K):
+    """Where the rule says one launch a strided call makes its output and nothing else; where it says two (the per-token kinds of the last size), codes and
+    scales as well."""
+    from llmqrt_amd import _abi
+    kinds = {"sq_channel": 0, "fp8_token": 1, "sq": 2, "fp8": 3, "static": 4, "static_out": 4}
+    strided = torch.randn(M, K + 24, device=cuda, generator=torch.Generator(device="cuda").manual_seed(M)).bfloat16()[:, 8:8 + K]
+    for name, mod in _modules(N, K, torch.bfloat16, True, cuda).items():
+        mod(strided)
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        mod(strided)
+        made = torch.cuda.memory_stats()["allocation.all.allocated"] - before
+        one = _abi.lib().llmq_linear_one_launch_preferred(kinds[name], M, N, K)
+        assert (made == 1) == bool(one), (name, made)
+
+
+def test_strided_rows_off_the_kernel_still_run(cuda):
+    """Rows, columns and addresses that no one-launch kernel takes: the general path copies or quantizes separately, as for any size."""
+    M, N, K = 5, 640, 1024
+    g = torch.Generator(device="cuda").manual_seed(1)
+    wide = torch.randn(M, 2 * K + 13, device=cuda, generator=g).bfloat16()
+    views = {"odd address": wide[:, 1:1 + K], "odd stride": wide[:, :K], "every other column": wide[:, :2 * K:2],
+             "transposed": torch.randn(K, M, device=cuda, generator=g).bfloat16().t()}
+    for name, mod in _modules(N, K, torch.bfloat16, True, cuda).items():
+        for what, x in views.items():
+            y, ref = mod(x).double(), mod(x.contiguous().clone()).double()
+            assert y.shape == (M, N) and (y - ref).abs().max() <= 2.0 ** -7 * ref.abs().max() + (0.05 * 2.0 ** -3 if name == "static_out" else 0), (name, what)
+
+
+@pytest.mark.parametrize("fp8", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(1, 24, 16), (16, 896, 1024), (4, 4104, 4096), (5, 9728, 912)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_per_tensor_entry_point(cuda, fp8, M, N, K, dtype):
+    """llmq_linear_per_tensor_dynamic is llmq_linear_one_launch for up to llmq_linear_per_tensor_max_tokens tokens, and refuses more."""
+    from llmqrt_amd import _abi
+    L = _abi.lib()
+    g = torch.Generator().manual_seed(N)
+    x = torch.randn(M, K + 8, generator=g).to(dtype).to(cuda)
+    w = (torch.randn(N, K, generator=g) * 40).clamp(-127, 127)
+    w = (w.to(torch.float8_e4m3fn) if fp8 else w.to(torch.int8)).to(cuda)
+    s = torch.tensor([0.01], device=cuda)
+    bias = torch.randn(N, generator=g).to(dtype).to(cuda)
+    a, b = (torch.zeros(M, N, dtype=dtype, device=cuda) for _ in range(2))
+    dt, st = _abi.dtype_code(dtype), torch.cuda.current_stream().cuda_stream
+
+    def entry(tokens):
+        return L.llmq_linear_per_tensor_dynamic(fp8, x.data_ptr(), dt, K + 8, w.data_ptr(), K, s.data_ptr(), bias.data_ptr(), dt, a.data_ptr(), dt, N, tokens, N, K, st)
+    assert entry(M) == 0 and entry(L.llmq_linear_per_tensor_max_tokens(K) + 1) == -3
+    assert L.llmq_linear_one_launch(2 + fp8, x.data_ptr(), dt, K + 8, w.data_ptr(), K, s.data_ptr(), None, bias.data_ptr(), dt, None, b.data_ptr(), dt, N, M, N, K, st) == 0
+    assert torch.equal(a, b) and int(a.count_nonzero()) > 0
