@@ -341,7 +341,7 @@ __global__ __launch_bounds__(KW * kWave) void awq_gemv_kernel(
         for (int r = 0; r < 8; r++) voff[r] = (uint32_t)(((8 * kb + r) * Nw + cwc) * 4);
         uint32_t xoff[MS];
 #pragma unroll
-        for (int a = 0; a < MS; a++) xoff[a] = (uint32_t)((min(16 * a + li, M - 1) * (int)ldx + 8 * kb) * 2);
+        for (int a = 0; a < MS; a++) xoff[a] = 2u * ((uint32_t)min(16 * a + li, M - 1) * (uint32_t)ldx + 8u * (uint32_t)kb);
         // loads past the last group of this wavefront re-read that group (results unused): no branches
         auto load_chunk = [&](int g, int u, wvec* wdst, uint4* xdst) {
             const int c = (g < ngroups ? g : g - gstride) * RING + u;
@@ -922,14 +922,19 @@ int awq_gemm_entry(const void* x, int64_t ldx, const int32_t* qweight, const voi
     if (tile_path(M)) {
         const AwqTilePlan t = tile_plan(M, N, K);
         if (t.splits > 1 && (!ws || workspace_bytes < (size_t)t.splits * M * N * sizeof(float))) return LLMQ_ERR_WORKSPACE;
-        const int rc = launch_awq_tile(t, (const uint16_t*)x, ldx, qw, sc, qz, bs, (uint16_t*)out, ws, (int)M, Ni, Ki, Gi, st);
-        if (rc != LLMQ_OK) return rc;
-        if (t.splits > 1) {
-            const int64_t total = M * N;
-            const int blocks = (int)((total + 255) / 256 < 2048 ? (total + 255) / 256 : 2048);
-            hipLaunchKernelGGL(awq_finish_kernel, dim3(blocks), dim3(256), 0, st, ws, t.splits, total, Ni, bs,
-                               (uint16_t*)out);
-            if (launch_status() != LLMQ_OK) return LLMQ_ERR_LAUNCH;
+        // offsets of a tile's rows are 32-bit element counts: rows further apart than 2^23 elements go through in launches of as many as fit
+        const int64_t reach = 0x7fffffffLL / ldx, step = reach >= 256 ? M : reach;  // at least 15 (ldx * 16 fits)
+        for (int64_t m0 = 0; m0 < M; m0 += step) {
+            const int64_t mm = M - m0 < step ? M - m0 : step;
+            uint16_t* os = (uint16_t*)out + m0 * N;
+            const int rc = launch_awq_tile(t, (const uint16_t*)x + m0 * ldx, ldx, qw, sc, qz, bs, os, ws, (int)mm, Ni, Ki, Gi, st);
+            if (rc != LLMQ_OK) return rc;
+            if (t.splits > 1) {
+                const int64_t total = mm * N;
+                const int blocks = (int)((total + 255) / 256 < 2048 ? (total + 255) / 256 : 2048);
+                hipLaunchKernelGGL(awq_finish_kernel, dim3(blocks), dim3(256), 0, st, ws, t.splits, total, Ni, bs, os);
+                if (launch_status() != LLMQ_OK) return LLMQ_ERR_LAUNCH;
+            }
         }
         return LLMQ_OK;
     }
@@ -948,7 +953,7 @@ int awq_gemm_entry(const void* x, int64_t ldx, const int32_t* qweight, const voi
             const DecodePlan d = make_decode_plan(mm, N, K);
             splits = d.splits;
             if (splits > 1 && (!ws || workspace_bytes < (size_t)splits * mm * N * sizeof(float))) return LLMQ_ERR_WORKSPACE;
-            const int ms = d.ms;
+            const int ms = ldx > (1 << 25) ? 1 : d.ms;  // 32-bit byte offsets of 16 ms rows
             const int slabs = cdiv(mm, 16 * ms);
             const dim3 grid(cdiv(Ni / 8, 16 * d.v) * slabs, splits);
 #define LLMQ_AWQ_DECODE(VV, KWW, MSS) \

@@ -559,3 +559,23 @@ def test_bias_is_checked_and_converted(cuda):
                      lambda: awq_gemm_bf16(x.bfloat16(), qw, s, qz, b)):
             with pytest.raises(RuntimeError, match="bias"):
                 call()
+
+
+# (tokens, K, channels, group, row stride in elements, forced kernel): rows so far apart that 32-bit offsets of a block's rows overflow: the tile kernel (64- and
+# 256-token tiles, with and without a K split), two and four token tiles a wavefront of the register-streaming kernel, the few-token kernel
+@pytest.mark.parametrize("M,K,N,G,ldx,force", [(70, 96, 64, 32, 1 << 26, None), (300, 1056, 264, 32, 8808032, 4), (300, 1056, 264, 32, 8808032, 3), (40, 8192, 264, 128, (1 << 26) + 8, 6),
+                                               (20, 8192, 264, 128, (1 << 27) - 8, None), (33, 256, 64, 128, 1 << 26, None)])
+def test_rows_far_apart(cuda, force_awq_plan, M, K, N, G, ldx, force):
+    from llmqrt_amd import workloads as W
+    from llmqrt_amd.awq_kernels import awq_gemm_triton
+    qw, qz, s = W.awq_weights(N, K, 21 * M + N, group=G)
+    x = W.activations(M, K, 22 * M + K, dtype=torch.float16, outliers=False)
+    store = torch.empty((M - 1) * ldx + K, dtype=torch.float16, device=cuda)
+    far = store.as_strided((M, K), (ldx, 1))
+    far.copy_(x)
+    args = (qw.to(cuda), s.to(cuda), qz.to(cuda))
+    if force is not None:
+        force_awq_plan(force, 0)
+    out = awq_gemm_triton(far, *args, split_k_iters=8)
+    assert rel_err(out, R.awq_gemm(x, qw, qz, s, G)) <= REL_TOL
+    assert rel_err(out, awq_gemm_triton(x.to(cuda), *args, split_k_iters=8).cpu()) <= 2e-3
