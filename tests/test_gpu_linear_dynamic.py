@@ -150,8 +150,8 @@ def test_per_tensor_one_launch(cuda, M, N, K, dtype, bias):
 
 
 # llmq_linear_one_launch in every launch shape: up to 4096 channels 2, 4 and 10 pieces a thread (the last and the first number of codes of each),
-# past that four and eight wavefronts, one row per wavefront and several; a ragged K step, ragged channels, one step, LDS past 64 KB
-@pytest.mark.parametrize("M,N,K", [(1, 24, 16), (16, 4096, 1024), (15, 1000, 1104), (16, 264, 2048), (16, 136, 2064), (16, 896, 4864), (16, 72, 5120), (1, 640, 16384),
+# past that four and eight wavefronts, one row per wavefront and several; a ragged K step, ragged channels, one step, LDS past 64 KB and codes of 64 KB exactly
+@pytest.mark.parametrize("M,N,K", [(1, 24, 16), (16, 4096, 1024), (15, 1000, 1104), (16, 264, 2048), (16, 136, 2064), (16, 896, 4864), (16, 72, 5120), (16, 40, 4080), (8, 40, 8176), (1, 640, 16384),
                                    (4, 512, 20480), (8, 4112, 1024), (9, 4104, 1040), (16, 4360, 1024), (13, 8200, 1280), (3, 9728, 912), (16, 4112, 2064)])
 @pytest.mark.parametrize("dtype,with_bias", [(torch.bfloat16, True), (torch.float16, False)])
 def test_one_launch_every_source(cuda, M, N, K, dtype, with_bias):
