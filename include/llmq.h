@@ -359,7 +359,7 @@ int llmq_awq_workspace_init(void* workspace, size_t workspace_bytes, llmq_stream
  * with two / one K slice, 128 tokens with two / one), 0 = heuristic; the cross-block K split
  * (0 = heuristic); the wavefronts per block along K of the streaming kernel (4 or 8), or the K slices
  * inside a block of the few-token kernel (1, 2 or 4, v = 8 only); 0 = heuristic.
- * v + 32 keeps the tile kernel's register-staged activation loads (default: straight into LDS when K % 64 == 0).
+ * v + 32 is v (it named a form of the tile kernel's loads that is the only one now).
  * Per host thread (thread-local state): it affects only calls made later by the thread that set it. */
 int llmq_awq_force_plan(int v, int splits, int k_waves);
 

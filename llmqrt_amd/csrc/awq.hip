@@ -710,7 +710,8 @@ DecodePlan make_decode_plan(int64_t M, int64_t N, int64_t K) {
     // Token tiles of 16 per wavefront.  Above 16 tokens, for a long K that is split across blocks anyway
     // (down), one wavefront feeds every unpacked weight operand to 2 or 4 token tiles instead of running
     // one block per 16-token slab: measured at 64 tokens with the weights coming from HBM, down 30.5 -> 27 us.
-    // For K = 3584 the slabs are as fast or faster (qkv 19 vs 21.6 us, gate_up 57 vs 65 us).
+    // For K = 3584 the slabs are as fast or faster (qkv 19 vs 21.6 us, gate_up 57 vs 65 us).  Two tiles serve 17-24 tokens; past 24 such a K streams
+    // (awq_stream.hip), and four are for rows too far apart for that.
     p.ms = (cdiv(Nw, 16) < 128 && K >= 8192) ? (M > 32 ? 4 : (M > 16 ? 2 : 1)) : 1;
     if (g_force_v == 5) p.ms = 2;
     if (g_force_v == 6) p.ms = 4;
@@ -815,15 +816,13 @@ void launch_awq(const AwqPlan& p, const uint16_t* x, int64_t ldx, const uint32_t
 using namespace llmq;
 
 extern "C" int llmq_awq_force_plan(int v, int splits, int k_waves) {
-    const int staged = v >= 0 ? (v & 32) : 0;  // + 32: the tile kernel keeps its register-staged activation loads
-    if (v >= 0) v &= ~32;
+    if (v >= 0) v &= ~32;  // + 32 named the tile kernel's register-staged activation loads, the only ones it has
     if (v < 0 || v >= 12 + kAwqStreamConfigs || splits < 0 || splits > 64) return LLMQ_ERR_SHAPE;
     // K slices of the few-token kernel: 1, 2, 4 (v = 0 or 8 .. 11); wavefronts along K of the streaming kernel: 4, 8
     const bool few = v == 0 || (v >= 8 && v <= 11);
     if (v >= 12 && k_waves != 0) return LLMQ_ERR_SHAPE;
     if (k_waves != 0 && !(k_waves == 4 || (few && (k_waves == 1 || k_waves == 2)) || (!few && k_waves == 8))) return LLMQ_ERR_SHAPE;
-    set_awq_tile_direct_loads(staged ? 0 : 1);  // state changes only once the arguments are accepted
-    g_force_v = v;
+    g_force_v = v;  // state changes only once the arguments are accepted
     g_force_splits = splits;
     g_force_kw = k_waves;
     return LLMQ_OK;

@@ -87,7 +87,7 @@ __device__ __forceinline__ uint16_t finish_value(float v, bool has_bias, float b
 __device__ __forceinline__ int channel_of(int byte, int p) { return 4 * (byte & 1) + (byte >> 1) + 2 * p; }  // nibble 2 byte + p of a word
 
 template <class C>
-__global__ __launch_bounds__(C::NT, C::KS == 4 ? 4 : 2) void awq_stream_kernel(StreamArgs a) {
+__global__ __launch_bounds__(C::NT, 2) void awq_stream_kernel(StreamArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     constexpr int MT = C::MT, KS = C::KS, NS = C::NS;
     const int lane = threadIdx.x & (kWave - 1);

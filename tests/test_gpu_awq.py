@@ -235,9 +235,8 @@ def test_tile_kernel_every_shape_and_split(cuda, force_awq_plan, tile, splits, M
 @pytest.mark.parametrize("M,K,N,G,xstride", [(65, 64, 8, 64, 64), (257, 512, 264, 512, 1024), (130, 3584, 4608, 128, 3584),
                                             (300, 1088, 520, 32, 1096), (600, 1024, 1000, 128, 1024)])
 def test_tile_kernel_direct_loads_equal_register_staging(cuda, force_awq_plan, tile, M, K, N, G, xstride):
-    """With K a multiple of 64 the tile kernel fetches its activation tiles straight into LDS; variant + 32 keeps the
-    register-staged loop.  Same products, same order: equal on every element, for every tile shape, ragged token /
-    channel edges, several token tiles, and a row stride larger than K."""
+    """The tile kernel with K a multiple of 64, where only the hook and rows far apart lead to it: variant + 32 names the same register-staged loop.  Equal on
+    every element and close to the oracle for every tile shape, ragged token / channel edges, several token tiles, and a row stride larger than K."""
     from llmqrt_amd import workloads as W
     from llmqrt_amd.awq_kernels import awq_gemm_triton
     qw, qz, s = W.awq_weights(N, K, 9 * M + N, group=G)
