@@ -89,6 +89,74 @@ def test_many_groups_of_channels(cuda, variant, M, N, K):
     assert torch.equal(out[:M].cpu().view(torch.int16), want.view(torch.int16)) and (out[M] == 7.0).all()
 
 
+# the same with fp8 operands and the other forms of the epilogue: e4m3 and e5m2 activations, one scale for the tensor read from the device and none per row or
+# channel, fp16 results, the quantized fp32 output, raw sums, rows and outputs further apart than they are long
+@pytest.mark.parametrize("M,N,K", [(16, 16400, 528), (3, 36904, 1040), (5, 33000, 2048)])
+@pytest.mark.parametrize("variant", [12, 13])
+def test_many_groups_fp8_and_every_epilogue(cuda, variant, M, N, K):
+    from llmqrt_amd import _abi
+    from llmqrt_amd.quantize import static_per_tensor_quantize
+    L = _abi.lib()
+    ld, ldo = K + 32, N + 8
+    g = torch.Generator().manual_seed(N + K)
+    a, b = [(torch.randn(n, ld, generator=g) * 30).clamp(-448, 448).to(torch.float8_e4m3fn).to(cuda) for n in (M, N)]
+    a5 = a.float().to(torch.float8_e5m2)
+    qx, qw = _ints((M, ld), M).to(cuda), _ints((N, ld), N).to(cuda)
+    sx, sw = (torch.rand(M, generator=g) * 0.01 + 1e-3).to(cuda), (torch.rand(N, generator=g) * 0.01 + 1e-3).to(cuda)
+    alpha, bias = torch.tensor([3e-4], device=cuda), torch.randn(N, generator=g).bfloat16().to(cuda)
+    stream = torch.cuda.current_stream().cuda_stream
+    names = {torch.bfloat16: 0, torch.float16: 1}
+
+    def fp8(x, fmt, rows, channels, scalar, out_dtype, dump=None):
+        out = torch.full((M, ldo), 7.0, dtype=out_dtype, device=cuda)
+        _abi.check(L.llmq_gemm_fp8(x.data_ptr(), fmt, ld, b.data_ptr(), ld, _abi.ptr(rows), _abi.ptr(channels), 1.0, _abi.ptr(scalar), bias.data_ptr(), 0, 1.0,
+                                   out.data_ptr(), names[out_dtype], ldo, M, N, K, _abi.ptr(dump), None, 0, stream), "fp8")
+        assert bool((out[:, N:] == 7.0).all())
+        return out[:, :N]
+    _abi.check(L.llmq_gemm_force_plan(110 + variant, 1), "force_plan")
+    try:
+        dump, dump8 = torch.full((M, N), -1, dtype=torch.int32, device=cuda), torch.full((M, N), -1.0, device=cuda)
+        token = fp8(a, 0, sx, sw, None, torch.bfloat16, dump8)
+        wide = fp8(a5, 1, sx, sw, None, torch.bfloat16)
+        tensor = fp8(a, 0, None, None, alpha, torch.float16)
+        i8 = torch.full((M, ldo), 7.0, dtype=torch.float16, device=cuda)
+        _abi.check(L.llmq_gemm_w8a8(qx.data_ptr(), ld, qw.data_ptr(), ld, None, None, 1.0, alpha.data_ptr(), bias.data_ptr(), 0, 1.0, i8.data_ptr(), 1, ldo, M, N, K,
+                                    dump.data_ptr(), None, 0, stream), "int8")
+        scale = tensor.float().abs().max().view(1) / 300
+        quant = torch.full((M, ldo), 7.0, device=cuda)
+        _abi.check(L.llmq_gemm_fp8_quantized_output(a.data_ptr(), 0, ld, b.data_ptr(), ld, None, None, 1.0, alpha.data_ptr(), bias.data_ptr(), 0, 1.0, scale.data_ptr(),
+                                                    quant.data_ptr(), 1, ldo, M, N, K, None, 0, stream), "quantized output")
+    finally:
+        L.llmq_gemm_force_plan(-1, 1)
+    prod, prod5 = (x[:, :K].double() @ b[:, :K].double().t() for x in (a, a5))
+    per = sx.double().view(-1, 1) * sw.double()
+    for got, p, scales, half_ulp in ((token, prod, per, 2.0 ** -9), (wide, prod5, per, 2.0 ** -9), (tensor, prod, alpha.double(), 2.0 ** -12)):
+        p = p * scales
+        ref = p + bias.double()
+        # exact products; what the matrix cores' accumulation window loses, fp32 sums, one rounding to the output type
+        assert bool(((got.double() - ref).abs() <= 2e-4 * p.abs().max() + 2 * half_ulp * ref.abs()).all())
+    assert bool(((dump8.double() - prod).abs() <= 2e-4 * prod.abs().max()).all())
+    acc = qx[:, :K].double() @ qw[:, :K].double().t()
+    assert torch.equal(dump, acc.int())
+    want = (acc.float().double() * alpha.double() + bias.double()).float().half()  # one fma, then the output type
+    assert torch.equal(i8[:, :N], want)
+    padded = torch.nn.functional.pad(tensor, (0, -N % 8))
+    assert torch.equal(quant[:, :N], static_per_tensor_quantize(padded, scale).to(torch.float16).float()[:, :N] * scale) and bool((quant[:, N:] == 7.0).all())
+
+
+# fp8 on both sides of the planner's lines of channels
+@pytest.mark.parametrize("M,N,K", [(7, 8192, 2048), (7, 8200, 2048), (7, 16384, 1024), (7, 16392, 1040), (7, 20480, 8192), (7, 20488, 1536), (7, 24576, 2048), (7, 24584, 2048),
+                                   (7, 32776, 1152), (7, 29256, 1152)])
+def test_planned_fp8(cuda, M, N, K):
+    from llmqrt_amd.sq_fp8_kernels import cutlass_f8f8bf16_rowwise_sm89
+    g = torch.Generator().manual_seed(M + N)
+    a, b = [(torch.randn(n, K, generator=g) * 30).clamp(-448, 448).to(torch.float8_e4m3fn).to(cuda) for n in (M, N)]
+    sx, sw = (torch.rand(M, generator=g) * 0.01 + 1e-3).to(cuda), (torch.rand(N, generator=g) * 0.01 + 1e-3).to(cuda)
+    y = cutlass_f8f8bf16_rowwise_sm89(a, b.t(), None, sx.view(-1, 1), sw.view(1, -1), True)
+    ref = a.double() @ b.double().t() * sx.double().view(-1, 1) * sw.double()
+    assert bool(((y.double() - ref).abs() <= 2e-4 * ref.abs().max() + 2.0 ** -8 * ref.abs()).all())
+
+
 # what the planner itself picks on both sides of its limits: tokens, K and channels
 @pytest.mark.parametrize("M,N,K", [(1, 3584, 3584), (16, 4104, 2048), (16, 4088, 2048), (17, 3584, 3584), (32, 4608, 3584), (33, 4608, 3584), (48, 4608, 3584),
                                    (64, 3584, 3584), (65, 3584, 3584), (8, 896, 4864), (32, 896, 1024), (32, 896, 1152), (20, 16128, 2048), (16, 1024, 18944),

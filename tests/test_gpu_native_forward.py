@@ -32,13 +32,15 @@ def _modules(dtype, bias):
     return mods
 
 
-# 1 / 4 tokens: one-launch linears; 5: quantizer + few-token kernel; 70: tile kernels; 300: AWQ dequantize + GEMM
-@pytest.mark.parametrize("M", [1, 4, 5, 70, 300])
+# 1 - 5 tokens: one-launch linears; 70 and 300: tile kernels, AWQ streaming; 450: AWQ dequantize + GEMM
+@pytest.mark.parametrize("M", [1, 4, 5, 70, 300, 450])
 @pytest.mark.parametrize("dtype,bias", [(torch.bfloat16, True), (torch.float16, False)])
 def test_native_forward_equals_general_path(cuda, M, dtype, bias):
     x = torch.randn(M, 1, K, device=cuda, generator=torch.Generator(device="cuda").manual_seed(M)).to(dtype)
     strided = torch.zeros(M, 1, K + 8, dtype=dtype, device=cuda)
     strided[..., :K] = x
+    from llmqrt_amd.linear.linear_awq import dequant_matmul_token_threshold
+    assert 300 < dequant_matmul_token_threshold(K, N) <= 450
     for name, mod in _modules(dtype, bias).items():
         y, ref = mod(x), mod._forward_general(x)
         assert y.shape == (M, 1, N) and y.dtype == ref.dtype, name
@@ -343,3 +345,81 @@ def test_captured_forward_follows_the_gpu(cuda, M, n, k, name):
         again = mod(x)
         torch.cuda.synchronize()
         assert torch.equal(y, first) and torch.equal(again, eager)
+
+
+def _route_modules(dtype):
+    """(name, module, activations) of calls that run the kernels of few tokens and short prompts: the row-streaming GEMM with one group of channels a block, with
+    several and in three token tiles, the streaming AWQ kernel with a K split and without, for groups of 128 and 32."""
+    import ctypes
+    from llmqrt_amd import _abi
+    from llmqrt_amd.linear import FP8DynamicLinear, SqW8A8BBF16OBF16PerChannel, WQLinear_GEMM
+    L = _abi.lib()
+    g = torch.Generator(device="cuda").manual_seed(12)
+    calls = []
+    for fp8, M, n, k in ((False, 24, 1536, 2048), (True, 24, 1536, 2048), (False, 9, 16640, 1168), (True, 9, 16640, 8192), (True, 40, 2304, 2048)):
+        assert 110 <= L.llmq_gemm_planned_config(int(fp8), M, n, k) <= 123
+        lin = torch.nn.Linear(k, n, bias=False, device="cuda")
+        lin.weight.data = 0.02 * torch.randn(n, k, device="cuda", generator=g)
+        mod = FP8DynamicLinear.from_linear(lin, init_only=False, dtype=torch.bfloat16, per_tensor=False) if fp8 else \
+            SqW8A8BBF16OBF16PerChannel.from_linear(lin, 8, 0, False, dtype=torch.bfloat16)
+        calls.append((f"rows {M} x {n} x {k} {fp8}", mod, [torch.randn(M, k, device="cuda", generator=g).bfloat16() for _ in range(2)]))
+    for M, n, k, group in ((64, 1024, 4096, 32), (48, 384, 2048, 64), (777, 2048, 1024, 128), (40, 896, 896, 128)):
+        need = ctypes.c_int(0)
+        assert L.llmq_awq_planned_config(_abi.dtype_code(dtype), M, n, k, group, k) >= 12
+        split = L.llmq_awq_linear_partials_bytes(_abi.dtype_code(dtype), M, n, k, group, k, ctypes.byref(need)) > 0
+        mod = WQLinear_GEMM(4, group, k, n, False, "cuda")
+        mod.qweight.random_(generator=g)
+        mod.qzeros.random_(generator=g)
+        mod.scales.uniform_(0.001, 0.01, generator=g)
+        calls.append((f"stream {M} x {n} x {k} {group} split {split}", mod, [torch.randn(M, k, device="cuda", generator=g).to(dtype) for _ in range(2)]))
+    assert {name.endswith("split True") for name, _, _ in calls if name.startswith("stream")} == {True, False}
+    return calls
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_streaming_kernels_captured_and_on_two_streams(cuda, dtype):
+    """Captured calls replayed beside eager ones on two streams: every result is the one of a lone call, bit for bit."""
+    calls = _route_modules(dtype)
+    refs = [[mod(x) for x in xs] for _, mod, xs in calls]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=streams[0]):
+        captured = [mod(xs[1]) for _, mod, xs in calls]
+    for _ in range(4):
+        for y in captured:
+            y.zero_()
+        torch.cuda.synchronize()
+        outs = [[], []]
+        for i, (_, mod, xs) in enumerate(calls):
+            for j, st in enumerate(streams):
+                with torch.cuda.stream(st):
+                    outs[j].append(mod(xs[j]))
+        with torch.cuda.stream(streams[1]):
+            graph.replay()
+        torch.cuda.synchronize()
+        for i, (name, _, _) in enumerate(calls):
+            assert torch.equal(outs[0][i], refs[i][0]) and torch.equal(outs[1][i], refs[i][1]), name
+            assert torch.equal(captured[i], refs[i][1]), name
+
+
+def test_streaming_kernels_from_threads(cuda):
+    """Four threads on a stream each, each its own plans and scratch."""
+    import threading
+    calls = _route_modules(torch.bfloat16)
+    refs = [[mod(x) for x in xs] for _, mod, xs in calls]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(5):
+                ys = [mod(xs[i % 2]) for _, mod, xs in calls]
+                torch.cuda.current_stream().synchronize()
+                wrong.extend((i, name) for (name, _, _), y, ref in zip(calls, ys, refs) if not torch.equal(y, ref[i % 2]))
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not wrong and not any(t.is_alive() for t in threads)
