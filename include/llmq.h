@@ -6,8 +6,8 @@
  *  - The caller owns every buffer (inputs, outputs, workspaces); the library allocates
  *    nothing, never synchronises with the host and launches on the stream it is given
  *    (0 = the null stream).  Calls are asynchronous.  State kept between calls, all of
- *    it per host thread: the *_force_plan tuning hooks, and the last GEMM plans (a function of sizes
- *    and format alone).  llmq_gemm_w8a8_static has a scratch array per GPU.
+ *    it per host thread: the *_force_plan tuning hooks, and the last GEMM and AWQ plans (a function of
+ *    sizes and format alone).  llmq_gemm_w8a8_static has a scratch array per GPU.
  *  - Matrices are row-major; `ld*` is the row stride in ELEMENTS.
  *  - Return value: LLMQ_OK (0) or a negative llmq_status; llmq_status_string() names it.
  *  - Paths below are relative to the reference's runtime/ directory.
@@ -274,8 +274,8 @@ int llmq_linear_one_launch_ahead(int kind, int64_t M, int64_t N, int64_t K);
 int llmq_linear_dynamic_force_variant(int v);
 
 /* Tuning / test hook with no counterpart in the reference: force tile configuration `cfg`
- * (0 .. llmq_gemm_num_configs()-1) and K split `splits` for every later GEMM call of this
- * process; cfg < 0 restores the built-in heuristic.  cfg | 64 keeps the register-staged main loop (8, 9 and 10 have none: they
+ * (0 .. llmq_gemm_num_configs()-1) and K split `splits` for every later GEMM call;
+ * cfg < 0 restores the built-in heuristic.  cfg | 64 keeps the register-staged main loop (8, 9 and 10 have none: they
  * run the staged configuration next in size, 3, 2 and 2).  100 .. 105 pick a variant of the few-token kernel (no K split) for int8 and
  * fp8: with `splits` 16, 32 or 64 in slabs of that many tokens, for any M, else in one block row, for up to 64 tokens (more keep the
  * built-in choice).  110 .. 123 pick a variant of the kernel that streams long pieces of weight rows through LDS, for as many tokens as the
@@ -298,8 +298,8 @@ int llmq_gemm_planned_config(int fp8, int64_t M, int64_t N, int64_t K);
 /* out[m,n] = fp16( sum_k x[m,k] * fp16((q[k,n] - z[k/G,n]) * s[k/G,n]) + bias[n] ), fp32
  * accumulation in a fixed order (deterministic, unlike the reference's fp16 atomics).
  * x: fp16 [M,K] (ldx >= K, K % 32 == 0); out: fp16 [M,N] contiguous; bias: fp16 [N] or NULL.
- * Up to 64 tokens of a group that is a multiple of 128 the weights enter the matrix core unrounded, exact (q - z) * s in
- * fp32, instead of rounded to fp16 first; above 64 tokens either, by plan.  All are within 1e-2 of the dequantize-then-matmul
+ * In most plans of up to 64 tokens and in some of more, always of a group that is a multiple of 128, the weights enter the matrix
+ * core unrounded, exact (q - z) * s in fp32, instead of rounded to fp16 first.  All are within 1e-2 of the dequantize-then-matmul
  * math.
  * workspace: >= llmq_awq_gemm_workspace_bytes(M,N,K) bytes, 16-byte aligned.  Its first
  * llmq_awq_workspace_ticket_bytes() bytes are the arrival counters of the few-token kernel's K split:
@@ -352,7 +352,7 @@ size_t llmq_awq_workspace_ticket_bytes(void);
 int llmq_awq_workspace_init(void* workspace, size_t workspace_bytes, llmq_stream_t stream);
 
 /* Tuning / test hook with no counterpart in the reference: force the kernel variant of
- * llmq_awq_gemm for every later call of this process: v = 1 or 2 words per lane of the streaming
+ * llmq_awq_gemm: v = 1 or 2 words per lane of the streaming
  * kernel in 16-token slabs, 5 or 6 = streaming kernel with 2 or 4 token tiles per wavefront,
  * 3, 7 or 4 = tile kernel with 64x128, 128x128 or 256x256 tiles (any M), 8 .. 11 = the few-token kernel
  * (M <= 64; 128- / 256-byte row segments, one / two stages ahead), 12 .. 16 = the streaming tile kernel (K % 64 == 0; 32 tokens, 64 tokens
