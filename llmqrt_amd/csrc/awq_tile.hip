@@ -314,9 +314,9 @@ AwqTilePlan make_awq_tile_plan(int64_t M, int64_t N, int64_t K, int force_cfg, i
     p.cfg = cost256 <= cost128 && cost256 <= cost64 ? 1 : (cost128 <= cost64 ? 2 : 0);
     if (force_cfg >= 0) p.cfg = force_cfg;
     const int bm = p.cfg == 1 ? 256 : (p.cfg == 2 ? 128 : 64), bn = p.cfg == 1 ? 256 : 128;
-    const int blocks = cdiv(M, bm) * cdiv(N, bn);
+    const int64_t blocks = (int64_t)cdiv(M, bm) * cdiv(N, bn);
     const int want = p.cfg == 1 ? 256 : 512;  // blocks that fill the 256 CUs
-    int splits = force_splits > 0 ? force_splits : (blocks >= want * 3 / 4 ? 1 : cdiv(want, blocks));
+    int splits = force_splits > 0 ? force_splits : (blocks >= want * 3 / 4 ? 1 : cdiv(want, (int)blocks));
     const int max_splits = (int)(K / 256) > 0 ? (int)(K / 256) : 1;  // at least 4 K tiles per block
     if (splits > max_splits) splits = max_splits;
     if (splits > 32) splits = 32;

@@ -607,14 +607,17 @@ extern "C" int llmq_gemm_force_plan(int cfg, int splits) {
 
 extern "C" int llmq_gemm_num_configs(void) { return kNumShapes; }
 
+// Sizes (K in bytes) of which a call can be taken; the planners count in 32 bits.
+static bool plannable(int64_t M, int64_t N, int64_t K) { return M > 0 && N > 0 && K > 0 && M <= 0x7fffffffLL && N <= 0x7fffffffLL && K < (1 << 22); }
+
 extern "C" int llmq_gemm_planned_config(int fp8, int64_t M, int64_t N, int64_t K) {
-    return M <= 0 || N <= 0 || K <= 0 || K % 16 ? LLMQ_ERR_SHAPE : plan_for(fp8 ? 1 : 0, M, N, K).cfg;
+    return !plannable(M, N, K) || K % 16 ? LLMQ_ERR_SHAPE : plan_for(fp8 ? 1 : 0, M, N, K).cfg;
 }
 
 namespace {
 // what the plan that a call of this size runs splits into: a lookup once the size is planned
 size_t planned_bytes(int op, int64_t M, int64_t N, int64_t K) {
-    return M <= 0 || N <= 0 || K <= 0 ? 0 : partials_bytes(plan_for(op, M, N, K), M, N);
+    return !plannable(M, N, K) ? 0 : partials_bytes(plan_for(op, M, N, K), M, N);
 }
 }  // namespace
 
@@ -622,7 +625,7 @@ extern "C" size_t llmq_gemm_w8a8_workspace_bytes(int64_t M, int64_t N, int64_t K
 extern "C" size_t llmq_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t K) { return planned_bytes(1, M, N, K); }
 // For both formats, and no less than what the plans of the rules split: a figure that was enough for every plan this library had for a size.
 extern "C" size_t llmq_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    if (g_force_cfg >= 0 || M <= 0 || N <= 0 || K <= 0) return std::max(planned_bytes(0, M, N, K), planned_bytes(1, M, N, K));
+    if (g_force_cfg >= 0 || !plannable(M, N, K)) return std::max(planned_bytes(0, M, N, K), planned_bytes(1, M, N, K));
     struct Entry { int64_t M, N, K; size_t bytes; };
     static thread_local Entry cache[kCachedSizes] = {};
     Entry& e = cache[size_slot(M, N, K, 0)];

@@ -395,6 +395,26 @@ def test_awq_size_queries_answer_for_any_sizes():
     assert r.returncode == 0, r.stderr[-2000:]
 
 
+def test_queries_answer_for_the_largest_sizes():
+    """Tile counts past 32 bits: sizes that no call takes need nothing, and a plan's division by a wrapped count would end the process."""
+    import subprocess
+    import sys
+    code = ("import ctypes, itertools; from llmqrt_amd import _abi; L = _abi.lib(); c = ctypes.c_int()\n"
+            "v = (1, 64, 70000, 2**24, 2**31 - 8, 2**31 - 1, 2**31, 2**40)\n"
+            "for m, n, k in itertools.product(v, v, (64, 128, 2**22 - 16, 2**22, 2**31 - 32, 2**40)):\n"
+            "    refused = max(m, n) >= 2**31 or k >= 2**22\n"
+            "    for f in (0, 1): assert (L.llmq_gemm_planned_config(f, m, n, k) < 0) == refused\n"
+            "    for q in ('gemm_w8a8', 'gemm_fp8', 'gemm', 'gemm_f16', 'gemm_fp8_quantized_output'):\n"
+            "        assert getattr(L, f'llmq_{q}_workspace_bytes')(m, n, k) == 0 or not refused\n"
+            "    if m > 2**24: continue  # the AWQ queries go over M in steps\n"
+            "    L.llmq_awq_gemm_workspace_bytes(m, n, k)\n"
+            "    for g in (32, 128):\n"
+            "        L.llmq_awq_gemm_partials_bytes(m, n, k, g); L.llmq_awq_linear_partials_bytes(1, m, n, k, g, k, ctypes.byref(c))\n"
+            "        L.llmq_awq_planned_config(1, m, n, k, g, k)\n")
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+
+
 def test_captured_calls_keep_no_shared_workspace(monkeypatch):
     """A capture neither uses a cached buffer, which a larger eager call would replace under the graph, nor leaves one."""
     from llmqrt_amd import _abi
